@@ -18,6 +18,7 @@
 //     buffered over K-steps of 128 so that the global loads of step s+1 overlap step s.
 #include <cstdlib>
 #include <type_traits>
+#include "gemm_convert.h"
 #include "qproj_device.h"
 #include "qproj_internal.h"
 #include "gemm_tiles.h"
@@ -26,11 +27,6 @@
 namespace qproj {
 
 namespace {
-
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 constexpr int BM = 128, BN = 128, BK = 128;
 constexpr int LDT = BK + 16;  // LDS row stride in bytes, padded against bank conflicts
@@ -346,11 +342,6 @@ __global__ __launch_bounds__(kGemmThreads, 4) void gemm_per32_kernel(const Weigh
 //     I_lo = sum_k (sc_lo*q) * a,   I_hi = sum_k (sc_hi*q) * a,   sum_k sc*q*a = 8*I_hi + I_lo,
 // so the vector ALU only works once per 256 weights (shift-add, int->float, one fma with dx*d).
 // Twice the matrix instructions of the per-32 kernel, a third of its vector instructions.
-typedef unsigned short v2us __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t pk_mul_u16(uint32_t x, uint32_t s2) {
-    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2us, x) * __builtin_bit_cast(v2us, s2));
-}
-
 // The weights never become an LDS tile: they are converted in registers.  Inside a super-block
 // the order of the 256 products is free (both chains run over all of it), so a lane may feed the matrix
 // instruction with whichever 16 weights it likes as long as the activation operand carries the
@@ -383,11 +374,6 @@ struct DirectB {     // one super-block of the lane's weight row
     v4i hdr;         // d, dmin, 12 bytes of 6-bit scales and mins
     v4i q[4];        // 64 nibble bytes: q[2*gg + half] = bytes 16*half.. of the 32-byte group 2*(l/32) + gg
 };
-
-__device__ __forceinline__ uint32_t byte_to_u16x2(uint32_t word, int i) {
-    // byte i of word -> both 16-bit halves (v_perm_b32: selector 0x0c yields a zero byte)
-    return __builtin_amdgcn_perm(0u, word, 0x0c000c00u | (uint32_t)(i << 16) | (uint32_t)i);
-}
 
 // Up to three matrices that multiply the same activation rows (q/k/v, gate/up) ride in one launch: a matrix of
 // 1024 rows against 512 tokens is 64 tiles, an eighth of the workgroups the chip holds, and took as long alone

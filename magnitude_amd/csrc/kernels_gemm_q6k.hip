@@ -21,6 +21,7 @@
 // super-block of activations, double-buffered: one workgroup barrier per 256 weights.
 #include <type_traits>
 
+#include "gemm_convert.h"
 #include "qproj_device.h"
 #include "qproj_internal.h"
 #include "gemm_tiles.h"
@@ -29,11 +30,6 @@
 namespace qproj {
 
 namespace {
-
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v2i __attribute__((ext_vector_type(2)));
-typedef int v16i __attribute__((ext_vector_type(16)));
-typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int LA = 256 + 16;   // activation row stride in LDS (bytes)
 constexpr int SQL = 128 + 16;  // strip row strides
@@ -47,42 +43,6 @@ struct Q6Smem {
     uint8_t qh[NW][32 * SQH];
     int8_t sc[NW][32 * 16];
 };
-
-// two 16-bit lanes: x * s + c, each lane modulo 2^16
-__device__ __forceinline__ uint32_t pk_mad_u16(uint32_t x, uint32_t s, uint32_t c) {
-    uint32_t r;
-    asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(r) : "v"(x), "v"(s), "v"(c));
-    return r;
-}
-
-// The 16 + 16 weights that one 16-byte piece of ql (group gl of the half, bytes 16e .. 16e+15) holds in its low and
-// high nibbles, with the matching piece of qh, into both int8 operands.  Step t of a lane is sub-block 8f + t of its
-// half f = group g = t/2 (ql byte 32*(g%2) + l, nibble g/2, qh bits 2g and 2g+1), bytes l = 16*(t%2) .. +15; `scq`
-// holds the eight scales of the half.
-__device__ __forceinline__ void convert_pieces(const v4i &lq, const v4i &hq, const v2i &scq, int gl, int e, v4i (&cl)[8], v4i (&ch)[8]) {
-#pragma unroll
-    for (int nib = 0; nib < 2; ++nib) {
-        const int g = gl + 2 * nib, t = 2 * g + e;
-        const int s = (int)(int8_t)((uint32_t)scq[t >> 2] >> (8 * (t & 3)));
-        const uint32_t s16 = __builtin_amdgcn_perm((uint32_t)s, (uint32_t)s, 0x01000100u);
-        const int cc = 128 - 32 * s;
-        const uint32_t c16 = __builtin_amdgcn_perm((uint32_t)cc, (uint32_t)cc, 0x01000100u);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const uint32_t lw = (uint32_t)lq[c], hw = (uint32_t)hq[c];
-            const uint32_t x = nib ? (lw >> 4) & 0x0f0f0f0fu : lw & 0x0f0f0f0fu;
-            const uint32_t hs = g == 0 ? hw << 4 : g == 1 ? hw << 2 : g == 2 ? hw : hw >> 2;
-            const uint32_t q = (hs & 0x30303030u) | x;                          // four codes 0..63
-            // codes 0, 2 and 1, 3 in 16-bit lanes: byte permutes over zeros (a mask for the first pair made the compiler
-            // build the four codes twice, once for each pair)
-            const uint32_t e0 = __builtin_amdgcn_perm(0u, q, 0x0c020c00u), e1 = __builtin_amdgcn_perm(0u, q, 0x0c030c01u);
-            const uint32_t w0 = pk_mad_u16(e0, s16, c16), w1 = pk_mad_u16(e1, s16, c16);   // sc * (q - 32) + 128
-            // low bytes (bit 7 flipped: minus 128 modulo 256) and high bytes, back in the order of the codes
-            cl[t][c] = (int)(__builtin_amdgcn_perm(w1, w0, 0x06020400u) ^ 0x80808080u);
-            ch[t][c] = (int)__builtin_amdgcn_perm(w1, w0, 0x07030501u);
-        }
-    }
-}
 
 template <int NW, int JT>
 __global__ __launch_bounds__(64 * NW, 2) void gemm_q6k_q8k_kernel(const WeightView w, const ActView a, int64_t M,
@@ -183,7 +143,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_q6k_q8k_kernel(const WeightVi
 #pragma unroll
             for (int gl = 0; gl < 2; ++gl) {
                 const v4i lq = *reinterpret_cast<const v4i *>(pql + l32 * SQL + 64 * lh + 32 * gl + 16 * e);
-                convert_pieces(lq, hq, scq, gl, e, cl, ch);
+                convert_q6k(lq, hq, scq, gl, e, cl, ch);
             }
         }
         const float dn = h2f(dbits);
@@ -354,7 +314,7 @@ __global__ __launch_bounds__(512, 1) void gemm_q6k_q8k_wide_kernel(const WeightV
 #pragma unroll
             for (int gl = 0; gl < 2; ++gl) {
                 const v4i lq = *reinterpret_cast<const v4i *>(pql + qlrow + 16 * ((4 * lh + 2 * gl + e) ^ qlx));
-                convert_pieces(lq, hq, scq, gl, e, cl, ch);
+                convert_q6k(lq, hq, scq, gl, e, cl, ch);
             }
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the strip has been read: it may be overwritten

@@ -418,14 +418,22 @@ bool takes_tiled(const qproj_weight *t, int64_t M) {
     return t->type != kTypeQ8_0 || t->K % 128 == 0;
 }
 
+// The streaming kernel's share of those batches: the matrices it takes go in one launch, the others follow on the tiled
+// kernels.  Decided matrix by matrix, so that a matrix gets the same kernel whatever rides along with it.
+bool takes_stream(const qproj_weight *t, int64_t M) { return takes_tiled(t, M) && stream_takes(t->type, t->K, M, t->N); }
+
 size_t dense_scratch_bytes(int n, const qproj_weight *const *w, int64_t M) {
     if (takes_tiled(w[0], M)) {
-        if (w[0]->type == kTypeQ8_0) return per32_scratch_max(n, w, M);
-        size_t need = 0;
-        for (int i = 0; i < n; ++i)
-            need = std::max(need, w[0]->type == kTypeQ6_K ? q6k_tile_scratch_bytes(w[i]->K, M, w[i]->N)
-                                                          : q4k_tile_scratch_bytes(w[i]->K, M, w[i]->N));
-        return need;
+        size_t need = 0, streamed = 0;   // the launches follow one another: the same bytes serve all of them
+        for (int i = 0; i < n; ++i) {
+            const int t = w[i]->type;
+            if (takes_stream(w[i], M)) streamed += stream_scratch_bytes(t, w[i]->K, M, w[i]->N);
+            else
+                need = std::max(need, t == kTypeQ8_0   ? per32_scratch_bytes(w[i]->K, M, w[i]->N)
+                                      : t == kTypeQ6_K ? q6k_tile_scratch_bytes(w[i]->K, M, w[i]->N)
+                                                       : q4k_tile_scratch_bytes(w[i]->K, M, w[i]->N));
+        }
+        return std::max(need, streamed);
     }
     if (!use_mfma_kernel(w[0]->type, M, w[0]->K)) return 0;
     int64_t sum_n = 0, rgs = 0;
@@ -482,19 +490,24 @@ bool dense_clears_rows(int n, const qproj_weight *const *w, int64_t M, float *co
 // Returns the mask of those matrices and fills `z` with their rows.
 uint32_t tiled_clears_rows(int n, const qproj_weight *const *w, int64_t M, float *const *y, const float *x, bool have_scratch, ZeroJob &z) {
     WeightView views[kMaxTargets];
-    for (int i = 0; i < n; ++i) views[i] = w[i]->view;
-    uint32_t mask = q4k_multi_adds(n, views, M, have_scratch);
-    z.count = 0;
+    int index[kMaxTargets], count = 0;
     for (int i = 0; i < n; ++i) {
-        if (!((mask >> i) & 1u)) continue;
+        if (takes_stream(w[i], M)) continue;
+        index[count] = i;
+        views[count++] = w[i]->view;
+    }
+    const uint32_t adds = count ? q4k_multi_adds(count, views, M, have_scratch) : 0;
+    uint32_t mask = 0;
+    z.count = 0;
+    for (int c = 0; c < count; ++c) {
+        if (!((adds >> c) & 1u)) continue;
+        const int i = index[c];
         const int64_t cnt = M * w[i]->N;
-        if (cnt % 4 != 0 || (reinterpret_cast<uintptr_t>(y[i]) & 15) != 0 || overlaps(y[i], cnt, x, M * w[0]->K)) {
-            mask &= ~(1u << i);
-            continue;
-        }
+        if (cnt % 4 != 0 || (reinterpret_cast<uintptr_t>(y[i]) & 15) != 0 || overlaps(y[i], cnt, x, M * w[0]->K)) continue;
         z.p[z.count] = y[i];
         z.n[z.count] = cnt;
         ++z.count;
+        mask |= 1u << i;
     }
     return mask;
 }
@@ -506,20 +519,32 @@ int run_dense_q8act(qproj_ctx *ctx, int n, const qproj_weight *const *w, const A
     // Beyond the rows one pass of the small-batch kernel takes: the tiled product, weights reused across a tile of
     // tokens, K cut into stretches where the grid would leave the chip idle.  (Measured, 8B shapes, 33 rows: Q6_K
     // 14336 -> 4096 50.9 us in two passes of the small-batch kernel against 41 us tiled, Q4_K 4096 -> 14336 42 against 29.)
-    const auto tiled = [&](const qproj_weight *t) { return takes_tiled(t, M); };
-    if (tiled(w[0])) {
-        if (w[0]->type == kTypeQ4_K && n >= 2 && n <= 3) {   // q/k/v, gate/up: one launch where the tiles allow it
-            WeightView views[3];
-            for (int i = 0; i < n; ++i) views[i] = w[i]->view;
-            QP_HIP(ctx, launch_gemm_q8k_multi(n, views, a, M, y, sc, ctx->stream));
+    if (takes_tiled(w[0], M)) {
+        const int type = w[0]->type;
+        WeightView streamed[kMaxTargets], rest[kMaxTargets];
+        float *ys[kMaxTargets], *yr[kMaxTargets];
+        int n_streamed = 0, n_rest = 0;
+        Scratch scr = sc;
+        scr.zeroed = 0;   // its bits follow the matrices that are left
+        for (int i = 0; i < n; ++i) {
+            if (takes_stream(w[i], M)) {
+                streamed[n_streamed] = w[i]->view;
+                ys[n_streamed++] = y[i];
+            } else {
+                scr.zeroed |= ((sc.zeroed >> i) & 1u) << n_rest;
+                rest[n_rest] = w[i]->view;
+                yr[n_rest++] = y[i];
+            }
+        }
+        if (n_streamed) QP_HIP(ctx, launch_gemm_stream(n_streamed, streamed, a, M, ys, sc, ctx->stream));
+        if (type == kTypeQ4_K && n_rest >= 2 && n_rest <= 3) {   // q/k/v, gate/up: one launch where the tiles allow it
+            QP_HIP(ctx, launch_gemm_q8k_multi(n_rest, rest, a, M, yr, scr, ctx->stream));
             return QPROJ_OK;
         }
-        for (int i = 0; i < n; ++i) {
-            const int t = w[0]->type;
-            QP_HIP(ctx, t == kTypeQ4_K   ? launch_gemm_q8k(w[i]->view, a, M, y[i], sc.for_target(i), ctx->stream)
-                        : t == kTypeQ6_K ? launch_gemm_q6k_q8k(w[i]->view, a, M, y[i], sc, ctx->stream)
-                                         : launch_gemm_q8_0(w[i]->view, a, M, y[i], sc, ctx->stream));
-        }
+        for (int i = 0; i < n_rest; ++i)
+            QP_HIP(ctx, type == kTypeQ4_K   ? launch_gemm_q8k(rest[i], a, M, yr[i], scr.for_target(i), ctx->stream)
+                        : type == kTypeQ6_K ? launch_gemm_q6k_q8k(rest[i], a, M, yr[i], scr, ctx->stream)
+                                            : launch_gemm_q8_0(rest[i], a, M, yr[i], scr, ctx->stream));
         return QPROJ_OK;
     }
     if (use_mfma_kernel(w[0]->type, M, w[0]->K)) {

@@ -230,6 +230,11 @@ hipError_t launch_gemm_q8k(const WeightView &w, const ActView &a, int64_t M, flo
 hipError_t launch_gemm_q8k_multi(int n, const WeightView *w, const ActView &a, int64_t M, float *const *y,
                                  const Scratch &scratch, hipStream_t s);
 hipError_t launch_gemm_q8_0(const WeightView &w, const ActView &a, int64_t M, float *y, const Scratch &scratch, hipStream_t s);
+// 33..256 rows of Q4_K / Q6_K weights: all matrices of a call in one launch, K cut per matrix
+bool stream_takes(int type, int64_t K, int64_t M, int64_t N);
+size_t stream_scratch_bytes(int type, int64_t K, int64_t M, int64_t N);   // per matrix; the launcher wants the sum
+hipError_t launch_gemm_stream(int n, const WeightView *w, const ActView &a, int64_t M, float *const *y, const Scratch &scratch,
+                              hipStream_t s);
 size_t q6k_tile_scratch_bytes(int64_t K, int64_t M, int64_t N);   // what launch_gemm_q6k_q8k asks of its scratch
 hipError_t launch_gemm_q6k_q8k(const WeightView &w, const ActView &a, int64_t M, float *y, const Scratch &scratch, hipStream_t s);
 

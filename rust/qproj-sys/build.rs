@@ -5,10 +5,10 @@ use std::{env, path::PathBuf, process::Command};
 const SOURCES: &[&str] = &[
     "qproj_api.hip", "kernels_dequant.hip", "kernels_actquant.hip", "kernels_gemv.hip", "kernels_decode.hip",
     "kernels_gemv_mfma.hip", "kernels_gemv_f32.hip", "kernels_moe.hip", "kernels_moe_decode.hip", "kernels_gemm.hip", "kernels_gemm_q6k.hip",
-    "kernels_rmsnorm.hip",
+    "kernels_gemm_stream.hip", "kernels_rmsnorm.hip",
 ];
 const HEADERS: &[&str] = &[
-    "qproj_internal.h", "qproj_device.h", "gemv_frags.h", "actquant_device.h", "gemm_tiles.h", "lds_direct.h",
+    "qproj_internal.h", "qproj_device.h", "gemv_frags.h", "actquant_device.h", "gemm_tiles.h", "gemm_convert.h", "lds_direct.h",
 ];
 const HIPFLAGS: &[&str] = &[
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",

@@ -358,6 +358,40 @@ def test_mul_mat_ggml_mode_prefill_sized_batches(ctx, orc, qtype, m, k, n):
     w.free()
 
 
+@pytest.mark.parametrize("qtype,m,k,ns,tile", [
+    (Q4_K, 33, 256, (9,), "2 token tiles, 2 K parts"),              # one super-block: the second K part has none of its own
+    (Q4_K, 64, 768, (203, 128), "2 token tiles, 2 K parts"),        # an odd number of them, ragged rows, two matrices
+    (Q4_K, 65, 5120, (77,), "2 token tiles, 2 K parts"),            # K whole (odd output): the chunk of scales is refilled
+    (Q4_K, 256, 4096, (1024, 260), "2 token tiles, 2 K parts"),     # K in stretches of two steps
+    (Q4_K, 96, 512, (33000,), "3 token tiles, 1 K parts"),          # more tiles than a round
+    (Q4_K, 40, 2304, (33001,), "2 token tiles, 1 K parts"),
+    (Q6_K, 33, 256, (5,), "2 token tiles, 2 K parts"),
+    (Q6_K, 70, 5376, (131,), "2 token tiles, 2 K parts"),
+    (Q6_K, 100, 256, (33000,), "4 token tiles, 1 K parts"),
+    (Q6_K, 161, 8192, (300, 33), "3 token tiles, 1 K parts"),
+    (Q6_K, 250, 8448, (100,), "4 token tiles, 1 K parts"),
+])
+def test_streamed_batches_of_33_to_256_rows(ctx, orc, qtype, m, k, ns, tile):
+    """The streaming kernel at the edges of its tiles, K parts, stretches and chunks of scales, against the oracle: exact
+    integer dots, fp32 sums in another order (the min term adds 22-bit products: 2e-5 like the other tiled kernels); rows
+    behind a matrix stay untouched; several matrices in a launch are bitwise the matrices one by one."""
+    from magnitude_amd import ACT_GGML, qproj
+    assert f"gemm_stream_kernel<{'Q4_K' if qtype == Q4_K else 'Q6_K'}, {tile}>" in qproj.plan_mul_mat(qtype, k, list(ns), m, ACT_GGML)
+    blocks = [make_weight(orc, qtype, n, k, seed=2600 + k + n) for n in ns]
+    ws = [ctx.upload(qtype, k, n, b) for n, b in zip(ns, blocks)]
+    x = np.random.default_rng(m + k).standard_normal((m, k)).astype(np.float32)
+    x[:, :: 61] *= 20.0
+    bufs = [torch.full((m * n + 64,), 7.0, dtype=torch.float32, device="cuda") for n in ns]
+    outs = [b[: m * n].view(m, n) for b, n in zip(bufs, ns)]
+    ctx.mul_mat_multi(ws, dev(x), ACT_GGML, outs=outs)
+    some = np.unique(np.concatenate([np.arange(min(m, 3)), [31, 32, m - 1], np.arange(m - 1, 0, -17)]))
+    for w, b, o, n, blk in zip(ws, bufs, outs, ns, blocks):
+        close(o.cpu().numpy()[some], orc.mul_mat(qtype, blk, k, x[some], orc.ACT_GGML), 2e-5)
+        assert bool((b[m * n:] == 7.0).all())
+        assert torch.equal(o, ctx.mul_mat(w, dev(x), ACT_GGML))
+        w.free()
+
+
 @pytest.mark.parametrize("m,k,n", [(1000, 256, 6200), (900, 768, 6200)])
 def test_mul_mat_ggml_mode_q4k_wide_tiles(ctx, orc, m, k, n):
     """Q4_K with enough 128-token x 256-row tiles (>= 192) to take the wide prefill kernel: one and three
