@@ -6,16 +6,19 @@
 // A workgroup owns a 128 (tokens) x 128 (weight rows) tile; each of its 8 waves a 32x64
 // sub-tile = two v_mfma_i32_32x32x32_i8 products per 32-wide sub-block.  Both operands change
 // scale every 32 K-elements, so an int32 accumulator is meaningful for ONE product only: each
-// product is folded into the fp32 accumulators right away (cvt, scale product, fma per output).
-// That fp32 work, not the matrix cores, bounds this kernel, so everything else is kept off the
-// vector ALU:
+// product is folded into the fp32 accumulators right away.  That fp32 work, not the matrix cores,
+// bounds this kernel (the vector ALU issues in 91 % of its cycles; at this load the clock sinks to
+// 1.8 - 2.05 GHz), so everything else is kept off the vector ALU:
+//   - two instructions an output and block instead of three (see `product`);
+//   - activations go from global memory straight into LDS, addresses are one register an operand
+//     and immediate offsets, the four sub-blocks of a K-step are unrolled;
 //   - the min term is a separate small GEMM over K/32 (activation block sums x mins) done on the
 //     fp16 matrix cores before the main loop, with both operands split into fp16 high and low
 //     parts (the mins are 17-bit products, split exactly; the sums keep 22 bits);
-//   - the weight-side scales d*sc of a lane's own output column are unpacked from the block
-//     header by that lane and held in registers for the 8 sub-blocks of a super-block;
-//   - LDS holds only the two int8 operand tiles and the transposed activation scales, double
-//     buffered over K-steps of 128 so that the global loads of step s+1 overlap step s.
+//   - LDS holds only the two int8 operand tiles and the transposed scales, double buffered over
+//     K-steps of 128 so that the global loads of step s+1 overlap step s.
+// Measured, three instructions and operands through registers -> this, same card in turn:
+// 4096 x 4096 against 14336 rows 783 -> 684 us (614 -> 703 TOPS), vector instructions 105 -> 85 a pair of products.
 #include <cstdlib>
 #include <type_traits>
 #include "gemm_convert.h"
@@ -29,24 +32,24 @@ namespace qproj {
 namespace {
 
 constexpr int BM = 128, BN = 128, BK = 128;
-constexpr int LDT = BK + 16;  // LDS row stride in bytes, padded against bank conflicts
 
+// Rows of 128 bytes; the 16-byte segment `seg` of row r sits in slot seg ^ ((r / 2) % 8) (a load straight into LDS
+// cannot pad rows; 16 consecutive rows reading the same segment hit 16 different quadwords of the 64 banks).
 struct GemmStage {
-    int8_t a[BM * LDT];  // activations  [m][k]
-    int8_t b[BN * LDT];  // weights      [n][k], nibbles expanded
-    float a_d[4][BM];    // da           [sub-block][m]
+    int8_t a[BM * BK];   // activations  [m][k]
+    int8_t b[BN * BK];   // weights      [n][k], nibbles expanded
+    float sc[8][BM];     // 0..3: da [sub-block][m]; 4..7: d*sc (Q8_0: d) [sub-block][n]
 };
+static_assert(BM == BN, "one array of scales");
 
 struct GemmSmem {
     GemmStage st[2];
-    float w_s[8][BN];  // d*sc of the 8 sub-blocks of the current super-block [n]
 };
 
 // registers one thread carries from global memory to LDS for one K-step
 struct StageRegs {
-    uint4 act[2];
-    uint4 wq, wq2;   // wq2: Q8_0 only (its rows are 128 bytes per K-step, Q4_K's 64)
-    float4 ad;  // threads 0..127: activation scales; threads 128..255: block header of a weight row
+    v4i wq;   // Q4_K: 16 nibble bytes of a weight row
+    v4i ad;   // threads 0..127: activation scales; threads 128..255: block header (Q8_0: four scales) of a weight row
 };
 
 __device__ __forceinline__ void split_h(float v, _Float16 &hi, _Float16 &lo) {
@@ -55,6 +58,7 @@ __device__ __forceinline__ void split_h(float v, _Float16 &hi, _Float16 &lo) {
 }
 
 constexpr int kGemmThreads = 512;
+constexpr float kMagic = 12582912.f;   // 1.5 * 2^23: one integer step is one step of the float
 
 // QT = Q4_K: per-32 int8 activations with fp32 scales and block sums (the prefill format).
 // QT = Q8_0: ggml's Q8_0 activation blocks against Q8_0 weights: the same product without nibbles,
@@ -181,137 +185,150 @@ __global__ __launch_bounds__(kGemmThreads, 4) void gemm_per32_kernel(const Weigh
     // end of a tile read the last valid row: their results are never stored.
     const int mrow_cap = (int)(M - 1 - m0 < BM - 1 ? M - 1 - m0 : BM - 1);
     const int nrow_cap = (int)(N - 1 - n0 < BN - 1 ? N - 1 - n0 : BN - 1);
-    const global_ptr<int8_t> abase_s = scalar_global(a.qs + m0 * K);
+    const int8_t *abase_s = scalar_pointer(a.qs + m0 * K);
     const global_ptr<float> adbase_s = scalar_global(a.d + m0 * kb32);
-    uint32_t aoffg[2];
+    // requests straight into LDS: chunk wave + 8*i of a tile = its rows 8*(wave + 8*i) .. +7
+    const int swave = __builtin_amdgcn_readfirstlane(wave);
+    const int seg = (lane & 7) ^ ((lane >> 4) | ((swave & 1) << 2));   // slot lane%8 of row r holds segment slot ^ (r/2)%8
+    uint32_t aoffg[2], w8offg[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const int idx = tid + kGemmThreads * i, row = idx >> 3, seg = idx & 7;
+        const int row = 8 * (wave + 8 * i) + (lane >> 3);
         aoffg[i] = (uint32_t)(row < mrow_cap ? row : mrow_cap) * (uint32_t)K + 16u * seg;
+        w8offg[i] = (uint32_t)(row < nrow_cap ? row : nrow_cap) * (uint32_t)K + 16u * seg;   // Q8_0 only
     }
-    const uint32_t wrow = (uint32_t)((tid >> 2) < nrow_cap ? (tid >> 2) : nrow_cap);
-    const uint32_t hrow = (uint32_t)(tid - BM < 0 ? 0 : (tid - BM < nrow_cap ? tid - BM : nrow_cap));
-    const uint32_t adoffg = (uint32_t)(tid < mrow_cap ? tid : mrow_cap) * (uint32_t)kb32;
+    // threads 0..127: byte offset of a token's activation scales; 128..255: of a weight row's header (Q8_0: scales)
     global_ptr<uint8_t> wbase_s = nullptr;
-    global_ptr<int8_t> w8base_s = nullptr;
+    const int8_t *w8base_s = nullptr;
     global_ptr<uint16_t> w8d_s = nullptr;
-    uint32_t woffg, hoffg;
+    uint32_t woffg = 0, doffg = (uint32_t)min(tid, mrow_cap) * (uint32_t)kb32 * 4u;
     if constexpr (kQ4) {
         wbase_s = scalar_global(w.q4k + n0 * w.nb * 144);
-        woffg = wrow * (uint32_t)w.nb * 144u + 16u + 16u * (tid & 3);
-        hoffg = hrow * (uint32_t)w.nb * 144u;
+        woffg = (uint32_t)min(tid >> 2, nrow_cap) * (uint32_t)w.nb * 144u + 16u + 16u * (tid & 3);
+        if (tid >= BM) doffg = (uint32_t)min(tid - BM, nrow_cap) * (uint32_t)w.nb * 144u;
     } else {
-        w8base_s = scalar_global(w.q8_qs + n0 * K);
+        w8base_s = scalar_pointer(w.q8_qs + n0 * K);
         w8d_s = scalar_global(w.q8_d + n0 * w.nb);
-        woffg = wrow * (uint32_t)K + 32u * (tid & 3);
-        hoffg = hrow * (uint32_t)w.nb;
+        if (tid >= BM) doffg = (uint32_t)min(tid - BM, nrow_cap) * (uint32_t)w.nb * 2u;
     }
-    auto load_stage = [&](StageRegs &r, int64_t k0) {
+    // the half of a super-block a K-step is (its parity) is known at compile time
+    auto load_stage = [&](StageRegs &r, uint32_t ks, auto parity) {
+        constexpr int P = decltype(parity)::value;
+        GemmStage &st = sm.st[P];
 #pragma unroll
         for (int i = 0; i < 2; ++i)   // activations: 128 rows x 128 B
-            r.act[i] = load_global<uint4>(abase_s + k0, aoffg[i]);
+            global_to_lds16(abase_s + (aoffg[i] + ks * BK), st.a + (swave + 8 * i) * 1024);
         if constexpr (kQ4) {  // weights: 128 rows x 64 packed bytes (two 64-weight chunks of the super-block)
-            const int c2 = (int)((k0 & 255) >> 5);  // 32-byte chunk pair index * 2
-            r.wq = load_global<uint4>(wbase_s + ((k0 >> 8) * 144 + 16 * c2), woffg);
+            r.wq = load_global<v4i>(wbase_s, woffg + ((ks >> 1) * 144u + 64u * P));
         } else {              // weights: 128 rows x 128 int8
-            r.wq = load_global<uint4>(w8base_s + k0, woffg);
-            r.wq2 = load_global<uint4>(w8base_s + k0 + 16, woffg);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) global_to_lds16(w8base_s + (w8offg[i] + ks * BK), st.b + (swave + 8 * i) * 1024);
         }
-        r.ad = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (tid < BM) {
-            r.ad = load_global<float4>(adbase_s + (k0 >> 5), 4u * adoffg);
-        } else if (tid < BM + BN && (!kQ4 || (k0 & 255) == 0)) {
-            if constexpr (kQ4) {   // a new super-block starts: its header
-                r.ad = load_global<float4>(wbase_s + (k0 >> 8) * 144, hoffg);
-            } else {               // the four fp16 scales of this K-step
-                const uint2 d4 = load_global<uint2>(w8d_s + (k0 >> 5), 2u * hoffg);
-                r.ad.x = __uint_as_float(d4.x);
-                r.ad.y = __uint_as_float(d4.y);
+        if (swave < 4) {   // scalar branches: one base, one lane offset
+            if (kQ4 || swave < 2) {
+                r.ad = load_global<v4i>(swave < 2 ? (global_ptr<uint8_t>)adbase_s : wbase_s, doffg + (swave < 2 ? ks * 16u : (ks >> 1) * 144u));
+            } else {           // the four fp16 scales of this K-step
+                const v2i d4 = load_global<v2i>(w8d_s, doffg + ks * 8u);
+                r.ad[0] = d4[0];
+                r.ad[1] = d4[1];
             }
         }
     };
-    auto store_stage = [&](const StageRegs &r, GemmStage &st, int64_t k0) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int idx = tid + kGemmThreads * i;
-            const int row = idx >> 3, seg = idx & 7;
-            *reinterpret_cast<uint4 *>(st.a + row * LDT + 16 * seg) = r.act[i];
-        }
-        if constexpr (!kQ4) {
-            const int row = tid >> 2, part = tid & 3;
-            *reinterpret_cast<uint4 *>(st.b + row * LDT + 32 * part) = r.wq;
-            *reinterpret_cast<uint4 *>(st.b + row * LDT + 32 * part + 16) = r.wq2;
-        } else {
+    auto store_stage = [&](const StageRegs &r, auto parity) {
+        constexpr int P = decltype(parity)::value;
+        GemmStage &st = sm.st[P];
+        if constexpr (kQ4) {
             // 16 packed bytes = bytes 16*(part&1).. of chunk (part>>1): low nibbles -> sub-block 2c, high -> 2c+1
-            const int row = tid >> 2, part = tid & 3, ch = part >> 1, half = part & 1;
-            int8_t *base = st.b + row * LDT + 64 * ch + 16 * half;
-            *reinterpret_cast<uint4 *>(base) = make_uint4(r.wq.x & 0x0f0f0f0fu, r.wq.y & 0x0f0f0f0fu, r.wq.z & 0x0f0f0f0fu, r.wq.w & 0x0f0f0f0fu);
-            *reinterpret_cast<uint4 *>(base + 32) = make_uint4((r.wq.x >> 4) & 0x0f0f0f0fu, (r.wq.y >> 4) & 0x0f0f0f0fu,
-                                                               (r.wq.z >> 4) & 0x0f0f0f0fu, (r.wq.w >> 4) & 0x0f0f0f0fu);
-        }
-        if (tid < BM) {
-            st.a_d[0][tid] = r.ad.x;
-            st.a_d[1][tid] = r.ad.y;
-            st.a_d[2][tid] = r.ad.z;
-            st.a_d[3][tid] = r.ad.w;
-        } else if (tid < BM + BN && (!kQ4 || (k0 & 255) == 0)) {
-            if constexpr (kQ4) {
-                const uint32_t h0 = __float_as_uint(r.ad.x);
-                const ScalesK4 sc = unpack_scales_k4(__float_as_uint(r.ad.y), __float_as_uint(r.ad.z), __float_as_uint(r.ad.w));
-                const float d = h2f(h0);
-                float *dst = &sm.w_s[0][tid - BM];
+            const int row = tid >> 2, part = tid & 3, slot = ((part >> 1) * 4 + (part & 1)) ^ ((row >> 1) & 7);
+            int8_t *base = st.b + row * BK;
+            v4i lo, hi;
 #pragma unroll
-                for (int t = 0; t < 8; ++t) dst[t * BN] = d * (float)scale_k4(sc, t);
-            } else {   // scale slots 0..3 and 4..7 alternate with the K-steps, like the operand stages
-                const uint32_t lo = __float_as_uint(r.ad.x), hi = __float_as_uint(r.ad.y);
-                float *dst = &sm.w_s[(int)((k0 / BK) & 1) * 4][tid - BM];
-                dst[0] = h2f(lo & 0xffffu);
-                dst[BN] = h2f(lo >> 16);
-                dst[2 * BN] = h2f(hi & 0xffffu);
-                dst[3 * BN] = h2f(hi >> 16);
+            for (int c = 0; c < 4; ++c) {
+                lo[c] = r.wq[c] & 0x0f0f0f0f;
+                hi[c] = (int)((uint32_t)r.wq[c] >> 4) & 0x0f0f0f0f;
+            }
+            *reinterpret_cast<v4i *>(base + 16 * slot) = lo;
+            *reinterpret_cast<v4i *>(base + 16 * (slot ^ 2)) = hi;
+        }
+        float *const dst = &st.sc[0][0] + tid;   // (thread BM + i: entry i of rows 1.. , so rows 4..7 are three further on)
+        if (swave < 2) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) dst[t * BM] = __int_as_float(r.ad[t]);
+        } else if (swave < 4) {
+            if constexpr (kQ4) {
+                const ScalesK4 sc = unpack_scales_k4((uint32_t)r.ad[1], (uint32_t)r.ad[2], (uint32_t)r.ad[3]);
+                const float d = h2f((uint32_t)r.ad[0]);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) dst[(3 + t) * BM] = d * (float)scale_k4(sc, 4 * P + t);
+            } else {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) dst[(3 + t) * BM] = h2f(((uint32_t)r.ad[t >> 1] >> (16 * (t & 1))) & 0xffffu);
             }
         }
     };
 
-    const int64_t ks_begin = u_begin * 2, n_ksteps = min(u_end * 2, K / BK);
+    // Q4_K: the integer sums leave the matrix instruction as the bits of the float kMagic + I (its addend is kMagic's
+    // bits), and (kMagic + I) * w - kMagic * w in one fma is I * w rounded once: kMagic * w is exact, w = fp16 scale x
+    // 6-bit sub-block scale has 17 significant bits, |I| < 2^16.  Two vector instructions an output and block where
+    // int -> float, scale product and fma are three, and as many roundings.  For Q8_0 they are one rounding more, since
+    // the product of its two fp16 scales is exact: it keeps the three.
+    v16i addend;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) addend[v] = kQ4 ? __float_as_int(kMagic) : 0;
+    if constexpr (kQ4) asm volatile("" : "+v"(addend));   // in registers: rebuilt for every product it costs eight moves
+    auto product = [&](const v4i &af, const v4i &bf, float ws, const v4i (&ad)[4], float (&sum)[16]) {
+        const v16i I = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bf, addend, 0, 0, 0);
+        const float nws = -kMagic * ws;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const float da = __int_as_float(ad[v >> 2][v & 3]);
+            sum[v] = kQ4 ? fmaf(fmaf(__int_as_float(I[v]), ws, nws), da, sum[v]) : fmaf((float)I[v], da * ws, sum[v]);
+        }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) asm volatile("" : "+v"(sum[v]));
+    };
+    const uint32_t ks_begin = (uint32_t)u_begin * 2, ks_end = (uint32_t)min(u_end * 2, K / BK);
+    float sum[2][16];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sum[j][v] = acc[j][v];
+    // segment 2*kb + lh of row l%32 (of the wave's tokens, of its first 32 weight rows): offset ^ 32*kb
+    int fa = (wm * 32 + l32) * BK + 16 * (lh ^ ((l32 >> 1) & 7)), fb = (wn * 64 + l32) * BK + 16 * (lh ^ ((l32 >> 1) & 7));
     StageRegs regs;
-    if (ks_begin < n_ksteps) {
-        load_stage(regs, ks_begin * BK);
-        store_stage(regs, sm.st[ks_begin & 1], ks_begin * BK);
+    auto step = [&](uint32_t ks, auto parity) {
+        constexpr int P = decltype(parity)::value;
+        const std::integral_constant<int, 1 - P> other{};
+        const GemmStage &st = sm.st[P];
+        const bool more = ks + 1 < ks_end;
+        if (more) load_stage(regs, ks + 1, other);   // in flight during the arithmetic below
+        asm volatile("" : "+v"(fa), "+v"(fb));   // the eight addresses are worked out on the spot, not kept in registers
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+            const v4i af = *reinterpret_cast<const v4i *>(st.a + (fa ^ (32 * kb)));
+            const v4i bf0 = *reinterpret_cast<const v4i *>(st.b + (fb ^ (32 * kb)));
+            const v4i bf1 = *reinterpret_cast<const v4i *>(st.b + (fb ^ (32 * kb)) + 32 * BK);
+            const float w0 = st.sc[4 + kb][wn * 64 + l32], w1 = st.sc[4 + kb][wn * 64 + 32 + l32];
+            v4i ad[4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) ad[g] = *reinterpret_cast<const v4i *>(&st.sc[kb][wm * 32 + 8 * g + 4 * lh]);
+            // (the empty asm statements keep the sums of a block together: left alone the compiler postpones the last
+            // fma of every output and spills hundreds of registers)
+            product(af, bf0, w0, ad, sum[0]);
+            product(af, bf1, w1, ad, sum[1]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (more) store_stage(regs, other);
+        __syncthreads();   // (waits for the requests into LDS as well)
+    };
+    if (ks_begin < ks_end) {
+        load_stage(regs, ks_begin, std::integral_constant<int, 0>{});
+        store_stage(regs, std::integral_constant<int, 0>{});
     }
     __syncthreads();
-
-    for (int64_t ks = ks_begin; ks < n_ksteps; ++ks) {
-        const int64_t k0 = ks * BK;
-        const GemmStage &st = sm.st[ks & 1];
-        if (ks + 1 < n_ksteps) load_stage(regs, k0 + BK);  // in flight during the arithmetic below
-        const float *wsp = &sm.w_s[kQ4 ? (int)((k0 & 255) >> 5) : (int)(ks & 1) * 4][wn * 64 + l32];
-#pragma unroll 1
-        for (int kb = 0; kb < 4; ++kb) {
-            const v4i af = *reinterpret_cast<const v4i *>(st.a + (wm * 32 + l32) * LDT + kb * 32 + 16 * lh);
-            v4i bf[2];
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-                bf[j] = *reinterpret_cast<const v4i *>(st.b + (wn * 64 + j * 32 + l32) * LDT + kb * 32 + 16 * lh);
-            const float w0 = wsp[kb * BN], w1 = wsp[kb * BN + 32];
-            float ad[16];
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const float4 d4 = *reinterpret_cast<const float4 *>(&st.a_d[kb][wm * 32 + 8 * g + 4 * lh]);
-                ad[4 * g + 0] = d4.x; ad[4 * g + 1] = d4.y; ad[4 * g + 2] = d4.z; ad[4 * g + 3] = d4.w;
-            }
-            const v16i z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-            const v16i I0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bf[0], z, 0, 0, 0);
-            const v16i I1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bf[1], z, 0, 0, 0);
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[0][v] = fmaf((float)I0[v], ad[v] * w0, acc[0][v]);
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[1][v] = fmaf((float)I1[v], ad[v] * w1, acc[1][v]);
-        }
-        // the next step starts a new super-block: its scales replace the ones other waves may still read
-        if (kQ4 && ((k0 + BK) & 255) == 0) __syncthreads();
-        if (ks + 1 < n_ksteps) store_stage(regs, sm.st[(ks + 1) & 1], k0 + BK);
-        __syncthreads();
+    for (uint32_t ks = ks_begin; ks < ks_end; ks += 2) {
+        step(ks, std::integral_constant<int, 0>{});
+        if (ks + 1 < ks_end) step(ks + 1, std::integral_constant<int, 1>{});
     }
 
     // ---- store: accumulator register v of lane l is row 8*(v/4) + 4*(l/32) + v%4, column l%32
@@ -326,7 +343,7 @@ __global__ __launch_bounds__(kGemmThreads, 4) void gemm_per32_kernel(const Weigh
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             const int64_t m = m0 + wm_s * 32 + 8 * (v >> 2) + 4 * lh_s + (v & 3);
-            if (m < M && n < N) y[m * N + n] = acc[j][v];
+            if (m < M && n < N) y[m * N + n] = sum[j][v];
         }
     }
 }

@@ -599,6 +599,34 @@ def test_prefill_gemm_q8x32_matches_oracle(ctx, orc, m, k, n):
     gate(got, want)
 
 
+@pytest.mark.parametrize("qtype,m,k,n", [(Q8_0, 40, 128, 130), (Q8_0, 300, 640, 129), (Q8_0, 129, 1152, 260), (Q4_K, 33, 256, 1),
+                                         (Q4_K, 129, 512, 257), (Q4_K, 500, 4352, 128)])
+def test_per32_tiles_hold_the_largest_block_sums(ctx, orc, qtype, m, k, n):
+    """The per-32 tiles at one K-step, an odd number of them and ragged edges, with codes at the ends of their ranges
+    (Q8_0: -128 and 127, which no encoder writes together; Q4_K: nibbles 0 and 15 under any scale) against activations
+    whose codes are all +-127: the block sums are the largest there are.  They are exact integers on both sides; the fp32
+    sums over K / 32 blocks differ by order (5e-5 of the larger of 1 and the result, as in the test above)."""
+    from magnitude_amd import ACT_GGML, ACT_Q8X32, qproj
+    act, oact = (ACT_GGML, orc.ACT_GGML) if qtype == Q8_0 else (ACT_Q8X32, orc.ACT_Q8X32)
+    assert "gemm_per32_kernel" in qproj.plan_mul_mat(qtype, k, [n], m, act)
+    rng = np.random.default_rng(m + k + n)
+    blocks = make_weight(orc, qtype, n, k, seed=6200 + n).copy().reshape(n, -1, 34 if qtype == Q8_0 else 144)
+    if qtype == Q8_0:
+        blocks[:, :, 2:] = rng.choice([128, 127], (n, k // 32, 1)).astype(np.uint8)   # a block's codes: all -128 or all 127
+    else:
+        blocks[:, :, 16:] = rng.choice([0, 15, 240, 255], (n, k // 256, 128)).astype(np.uint8)
+    blocks = blocks.reshape(n, -1)
+    x = (rng.choice([-1.0, 1.0], (m, 1)) * rng.choice([-1.0, 1.0], (m, k // 32)) * rng.uniform(0.25, 4.0, (m, k // 32))).astype(np.float32)
+    x = np.repeat(x, 32, axis=1)
+    w = ctx.upload(qtype, k, n, blocks)
+    buf = torch.full((m * n + 64,), 7.0, dtype=torch.float32, device="cuda")
+    ctx.mul_mat(w, dev(x), act, out=buf[: m * n].view(m, n))
+    some = np.unique([0, 1, 31, 32, m // 2, m - 2, m - 1])
+    close(buf[: m * n].view(m, n).cpu().numpy()[some], orc.mul_mat(qtype, blocks, k, x[some], oact), 5e-5)
+    assert bool((buf[m * n:] == 7.0).all())
+    w.free()
+
+
 # ---------------------------------------------------------------- MUL_MAT_ID and the MoE FFN
 
 @pytest.fixture(scope="module")
