@@ -63,26 +63,55 @@ constexpr float kMagic = 12582912.f;   // 1.5 * 2^23: one integer step is one st
 // QT = Q4_K: per-32 int8 activations with fp32 scales and block sums (the prefill format).
 // QT = Q8_0: ggml's Q8_0 activation blocks against Q8_0 weights: the same product without nibbles,
 // without a min term, and with a weight scale per 32 instead of d*sc per sub-block.
-// blockIdx.y selects one of gridDim.y equal stretches of K (whole super-blocks for Q4_K); with more than one
-// the tile goes to part[blockIdx.y][M][N] and sum_parts_kernel adds the stretches up in order.
+// K of a matrix goes in n_split equal stretches (whole super-blocks for Q4_K); with more than one the tiles go to
+// out[stretch][M][N] and an adding pass puts the stretches together in order.  The matrices of a call (q/k/v, gate/up)
+// share a launch: at 33 .. 256 tokens one of them alone leaves most of the chip's 512 places (two workgroups a compute
+// unit) empty, and every launch pays the latency of its K loop again.  Four layers of 3072 / 1024 / 8192 Q8_0 weights
+// at 187 tokens, a launch and an adding pass a matrix -> this: 774 -> 558 us.
+struct Per32Target {
+    WeightView w;
+    float *out;   // the output, or [n_split][M][N] partial tiles
+    int tiles_pad, n_split, first_wg;   // tiles_pad: workgroups of one stretch, a multiple of the 8 XCDs
+};
+struct Per32Args {
+    int n;
+    Per32Target t[kMaxTargets];
+    ActView a;
+    int64_t M;
+};
 template <int QT>
-__global__ __launch_bounds__(kGemmThreads, 4) void gemm_per32_kernel(const WeightView w, const ActView a, int64_t M,
-                                                                   float *__restrict__ y, float *__restrict__ part) {
+__global__ __launch_bounds__(kGemmThreads, 4) void gemm_per32_kernel(const Per32Args g) {
     constexpr bool kQ4 = QT == kTypeQ4_K;
     extern __shared__ __align__(16) uint8_t smem_raw[];
     GemmSmem &sm = *reinterpret_cast<GemmSmem *>(smem_raw);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;  // 4 x 2 waves
-    const int64_t N = w.N, K = w.K;
+    int ti = 0;
+    if constexpr (!kQ4) {   // (Q4_K launches carry one matrix)
+#pragma unroll
+        for (int i = 1; i < kMaxTargets; ++i)
+            if (i < g.n && (int)blockIdx.x >= g.t[i].first_wg) ti = i;
+    }
+    const Per32Target &t = g.t[ti];
+    const WeightView w = t.w;
+    const ActView a = g.a;
+    const int64_t N = w.N, K = w.K, M = g.M;
+    const int tiles_n = (int)((N + BN - 1) / BN), tiles_m = (int)((M + BM - 1) / BM);
+    int split = 0, pid = (int)blockIdx.x - t.first_wg;
+    if (t.n_split > 1) {
+        split = pid / t.tiles_pad;
+        pid -= split * t.tiles_pad;
+    }
+    if (pid >= tiles_n * tiles_m) return;   // padding: the whole workgroup leaves
     int tile_n, tile_m;
-    tile_of_workgroup((int)((N + BN - 1) / BN), (int)((M + BM - 1) / BM), tile_n, tile_m);
+    tile_of_workgroup(tiles_n, tiles_m, pid, tile_n, tile_m);
     const int64_t n0 = (int64_t)tile_n * BN, m0 = (int64_t)tile_m * BM;
     const int64_t kb32 = K / 32;
     const int l32 = lane & 31, lh = lane >> 5;
     // this workgroup's stretch of K, in units of 256 (Q4_K super-blocks; two K-steps)
-    const int64_t n_units = (K + 255) / 256, per = (n_units + gridDim.y - 1) / gridDim.y;
-    const int64_t u_begin = min((int64_t)blockIdx.y * per, n_units), u_end = min(u_begin + per, n_units);
-    if (gridDim.y > 1) y = part + (size_t)blockIdx.y * M * N;
+    const int64_t n_units = (K + 255) / 256, per = (n_units + t.n_split - 1) / t.n_split;
+    const int64_t u_begin = min((int64_t)split * per, n_units), u_end = min(u_begin + per, n_units);
+    float *const y = t.out + (size_t)split * M * N;
 
     v16f acc[2];
 #pragma unroll
@@ -878,41 +907,67 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_q4k_q8k_wide_kernel(const Wei
 }  // namespace
 
 namespace {
-// y[i] = part[0][i] + part[1][i] + ... in that order
-__global__ __launch_bounds__(256) void sum_parts_kernel(const float *__restrict__ part, int n_split, size_t n4,
-                                                        float *__restrict__ y) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n4) return;
-    float4 s = reinterpret_cast<const float4 *>(part)[i];
-    for (int c = 1; c < n_split; ++c) {
-        const float4 v = reinterpret_cast<const float4 *>(part)[(size_t)c * n4 + i];
-        s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
-    }
-    reinterpret_cast<float4 *>(y)[i] = s;
-}
-
+// n matrices of one type and K over the same rows.  A launch takes as many of them as have room for their partial
+// tiles in the scratch; the next launch uses the same bytes again, behind the adding passes.
 template <int QT>
-hipError_t launch_per32(const WeightView &w, const ActView &a, int64_t M, float *y, const Scratch &sc, hipStream_t s) {
-    if (w.K > (1 << 24)) return hipErrorInvalidValue;   // 32-bit lane offsets: 128 rows of K bytes
-    const int n_split = sc.p ? per32_splits(w.K, M, w.N) : 1;
-    if (n_split > 1 && (size_t)n_split * M * w.N * 4 > sc.bytes) return hipErrorInvalidValue;   // partial tiles would not fit
-    if (dry_run()) {
-        if (n_split > 1) plan_note_cut();
-        plan_note("gemm_per32_kernel<%s>: tile 128 tokens x 128 rows, %lld tiles x %d K stretches%s", plan_type_name(QT),
-                  (long long)(((w.N + BN - 1) / BN) * ((M + BM - 1) / BM)), n_split, n_split > 1 ? " + sum_parts_kernel" : "");
-        return hipSuccess;
-    }
+hipError_t launch_per32(int n, const WeightView *w, const ActView &a, int64_t M, float *const *y, const Scratch &sc, hipStream_t s) {
+    if (n < 1 || n > kMaxTargets || w[0].K > (1 << 24)) return hipErrorInvalidValue;   // 32-bit lane offsets: 128 rows of K bytes
     const auto kern = &gemm_per32_kernel<QT>;
-    static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GemmSmem));
-    if (attr != hipSuccess) return attr;
-    const dim3 grid((unsigned)(((w.N + BN - 1) / BN) * ((M + BM - 1) / BM)), (unsigned)n_split);
-    hipLaunchKernelGGL(kern, grid, dim3(kGemmThreads), sizeof(GemmSmem), s, w, a, M, y, sc.p);
-    if (n_split > 1) {
-        const size_t n4 = (size_t)M * w.N / 4;
-        hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, sc.p, n_split, n4, y);
+    if (!dry_run()) {
+        static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GemmSmem));
+        if (attr != hipSuccess) return attr;
     }
-    return hipGetLastError();
+    int64_t all_tiles = 0;
+    for (int i = 0; i < n; ++i) all_tiles += per32_tiles(M, w[i].N);
+    for (int first = 0; first < n;) {
+        Per32Args g{};
+        g.a = a;
+        g.M = M;
+        SumTargets sums{};
+        size_t used = 0;
+        int64_t wg = 0;
+        int i = first;
+        for (; i < n; ++i) {
+            if (w[i].K != w[0].K) return hipErrorInvalidValue;
+            const int n_split = sc.p ? per32_splits(QT, w[i].K, M, w[i].N, all_tiles) : 1;
+            const size_t bytes = n_split > 1 ? (size_t)n_split * M * w[i].N * 4 : 0;
+            if (used + bytes > sc.bytes && bytes) {
+                if (i == first) return hipErrorInvalidValue;   // partial tiles would not fit
+                break;
+            }
+            const int64_t tiles = per32_tiles(M, w[i].N), pad = (tiles + 7) / 8 * 8;
+            if (wg + pad * n_split >= 0x7fffffff) {
+                if (i == first) return hipErrorInvalidValue;
+                break;
+            }
+            Per32Target &t = g.t[g.n++];
+            t.w = w[i];
+            t.out = y[i];
+            if (bytes) {
+                if (!dry_run()) t.out = sc.p + used / 4;
+                add_sum(sums, t.out, y[i], n_split, M * w[i].N);
+                used += bytes;
+            }
+            t.tiles_pad = (int)pad;
+            t.n_split = n_split;
+            t.first_wg = (int)wg;
+            wg += pad * n_split;
+            if (dry_run())
+                plan_note("gemm_per32_kernel<%s>%s: tile 128 tokens x 128 rows, %lld tiles x %d K stretches%s", plan_type_name(QT),
+                          g.n > 1 ? " (same launch)" : "", (long long)tiles, n_split, n_split > 1 ? " + sum_parts_kernel" : "");
+        }
+        first = i;
+        if (dry_run()) {
+            if (sums.n) plan_note_cut();
+            continue;
+        }
+        hipLaunchKernelGGL(kern, dim3((unsigned)wg), dim3(kGemmThreads), sizeof(GemmSmem), s, g);
+        hipError_t e = hipGetLastError();
+        if (e == hipSuccess && sums.n) e = launch_sum_parts(sums, s);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 }  // namespace
 
@@ -921,9 +976,9 @@ hipError_t launch_sum_parts(const float *part, int n_split, size_t n, float *y, 
         plan_note("sum_parts_kernel: adds %d partial results of %zu outputs in order", n_split, n);
         return hipSuccess;
     }
-    const size_t n4 = n / 4;   // callers only split when n is a multiple of 4
-    hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, part, n_split, n4, y);
-    return hipGetLastError();
+    SumTargets g{};
+    add_sum(g, part, y, n_split, (int64_t)n);   // callers only split when n is a multiple of 4
+    return launch_sum_parts(g, s);
 }
 
 // K stretches for the kernels that take ggml-format activations (64-token x 128-row tiles, two workgroups per
@@ -961,30 +1016,36 @@ size_t q8k_tile_scratch_bytes(int64_t K, int64_t M, int64_t N) {
 
 // A grid of fewer than 192 tiles leaves the 256 compute units mostly idle and a workgroup's K loop is
 // latency-bound: K is then cut into stretches done by different workgroups, as many as fill one round (32 tiles of
-// K = 14336, Q8_0 at 64 - 128 tokens: 8 stretches instead of 3).
-int per32_splits(int64_t K, int64_t M, int64_t N) {
+// K = 14336, Q8_0 at 64 - 128 tokens: 8 stretches instead of 3).  `all_tiles`: the tiles of every matrix that shares the
+// launch - gate and up of 8192 rows at 187 tokens are 256 tiles together and stay whole (cut in two, as each is alone, a
+// layer took 152 us instead of 141), while 4096 -> 14336 alone at 64 tokens needs its two stretches (35 us; whole 55).
+int64_t per32_tiles(int64_t M, int64_t N) { return ((N + BN - 1) / BN) * ((M + BM - 1) / BM); }
+int per32_splits(int type, int64_t K, int64_t M, int64_t N, int64_t all_tiles) {
     static const int forced = tuning_int("QPROJ_PER32_SPLITS", 0);
-    const int64_t tiles = ((N + BN - 1) / BN) * ((M + BM - 1) / BM);
     // as many stretches as fill one round of workgroups (one a compute unit), eight at most
-    int n = forced > 0 ? forced : tiles >= 192 ? 1 : (int)std::min<int64_t>(8, std::max<int64_t>(1, cu_count() / tiles));
+    int n = forced > 0 ? forced : all_tiles >= 192 ? 1 : (int)std::min<int64_t>(8, std::max<int64_t>(1, cu_count() / all_tiles));
     if ((M * N) % 4 != 0) n = 1;
-    while (n > 1 && K / 256 < 4 * n) --n;   // at least four super-blocks a stretch
+    // at least two times 256 weights a stretch, Q4_K four (its min term is a loop of its own over the stretch).  Q8_0,
+    // four -> two, us: 4096 -> 1024 at 64 tokens 21.2 -> 16.8, 2560 x 2560 at 250 27.2 -> 22.5, 4096 x 4096 at 100 24.5 -> 22.4.
+    const int least = type == kTypeQ8_0 ? 2 : 4;
+    while (n > 1 && K / 256 < least * n) --n;
     return n;
 }
-size_t per32_scratch_bytes(int64_t K, int64_t M, int64_t N) {
-    const int n = per32_splits(K, M, N);
+size_t per32_scratch_bytes(int type, int64_t K, int64_t M, int64_t N, int64_t all_tiles) {
+    const int n = per32_splits(type, K, M, N, all_tiles);
     return n > 1 ? (size_t)n * M * N * 4 : 0;
 }
 
 hipError_t launch_gemm_q8x32(const WeightView &w, const ActView &a, int64_t M, float *y, const Scratch &scratch, hipStream_t s) {
     if (w.type != kTypeQ4_K || w.K % 256 != 0 || M <= 0 || !a.msum || !a.rs) return hipErrorInvalidValue;
-    return launch_per32<kTypeQ4_K>(w, a, M, y, scratch, s);
+    return launch_per32<kTypeQ4_K>(1, &w, a, M, &y, scratch, s);
 }
 
 // Q8_0 weights x ggml Q8_0 activation blocks (planes in `a`), K a multiple of 128
-hipError_t launch_gemm_q8_0(const WeightView &w, const ActView &a, int64_t M, float *y, const Scratch &scratch, hipStream_t s) {
-    if (w.type != kTypeQ8_0 || a.kind != kActKindQ8_0 || w.K % BK != 0 || M <= 0) return hipErrorInvalidValue;
-    return launch_per32<kTypeQ8_0>(w, a, M, y, scratch, s);
+hipError_t launch_gemm_q8_0(int n, const WeightView *w, const ActView &a, int64_t M, float *const *y, const Scratch &scratch, hipStream_t s) {
+    for (int i = 0; i < n; ++i)
+        if (w[i].type != kTypeQ8_0 || a.kind != kActKindQ8_0 || w[i].K % BK != 0 || M <= 0) return hipErrorInvalidValue;
+    return launch_per32<kTypeQ8_0>(n, w, a, M, y, scratch, s);
 }
 
 // Which Q4_K kernel and how many stretches of K (one rule for the launcher and for the scratch sizing).  The

@@ -499,18 +499,7 @@ __global__ __launch_bounds__(512, 1) void gemm_stream_kernel(const StreamArgs g)
 }
 
 // y_i = part_i[0] + part_i[1] + ... in that order, all matrices of a call in one launch
-struct SumTarget {
-    const float *part;
-    float *y;
-    int n_split;
-    int64_t n4;         // float4s of one partial result
-    int64_t first;      // first thread
-};
-struct SumArgs {
-    int n;
-    SumTarget t[kMaxTargets];
-};
-__global__ __launch_bounds__(256) void sum_stretches_kernel(const SumArgs g) {
+__global__ __launch_bounds__(256) void sum_parts_kernel(const SumTargets g) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     SumTarget t = g.t[0];
 #pragma unroll
@@ -598,8 +587,7 @@ hipError_t launch_gemm_stream(int n, const WeightView *w, const ActView &a, int6
     if (n < 1 || n > kMaxTargets || a.kind != kActKindQ8_K || M <= 0) return hipErrorInvalidValue;
     const bool q4 = w[0].type == kTypeQ4_K;
     if (q4 && (!a.msum || !a.rs)) return hipErrorInvalidValue;
-    SumArgs sg{};
-    int64_t sum_threads = 0;
+    SumTargets sg{};
     size_t part = 0;
     StreamPlan plans[kMaxTargets];
     float *out[kMaxTargets];
@@ -611,13 +599,7 @@ hipError_t launch_gemm_stream(int n, const WeightView *w, const ActView &a, int6
         const size_t bytes = (size_t)plans[i].n_split * M * w[i].N * 4;
         if (part + bytes > scratch.bytes || (!scratch.p && !dry_run())) return hipErrorInvalidValue;   // partial tiles would not fit
         if (!dry_run()) out[i] = scratch.p + part / 4;
-        SumTarget &st = sg.t[sg.n++];
-        st.part = out[i];
-        st.y = y[i];
-        st.n_split = plans[i].n_split;
-        st.n4 = M * w[i].N / 4;
-        st.first = sum_threads;
-        sum_threads += (st.n4 + 255) / 256 * 256;
+        add_sum(sg, out[i], y[i], plans[i].n_split, M * w[i].N);
         part += bytes;
     }
     if (sg.n && dry_run()) plan_note_cut();
@@ -652,7 +634,7 @@ hipError_t launch_gemm_stream(int n, const WeightView *w, const ActView &a, int6
             wg += (int64_t)t.tiles_pad * t.n_split;
             plan_note("gemm_stream_kernel<%s, %d token tiles, %d K parts>%s: tile %d tokens x %d rows, %d tiles x %d K stretches%s", plan_type_name(w[0].type),
                       p0.jt, p0.kw, g.n > 1 ? " (same launch)" : "", 32 * p0.jt, rows, t.tiles_n * g.tiles_m, t.n_split,
-                      t.n_split > 1 ? " + sum_stretches_kernel" : "");
+                      t.n_split > 1 ? " + sum_parts_kernel" : "");
         }
         if (wg >= 0x7fffffff) return hipErrorInvalidValue;
         if (dry_run()) continue;
@@ -668,7 +650,11 @@ hipError_t launch_gemm_stream(int n, const WeightView *w, const ActView &a, int6
         if (e != hipSuccess) return e;
     }
     if (dry_run() || sg.n == 0) return hipSuccess;
-    hipLaunchKernelGGL(sum_stretches_kernel, dim3((unsigned)(sum_threads / 256)), dim3(256), 0, s, sg);
+    return launch_sum_parts(sg, s);
+}
+
+hipError_t launch_sum_parts(const SumTargets &g, hipStream_t s) {
+    hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)(g.threads / 256)), dim3(256), 0, s, g);
     return hipGetLastError();
 }
 

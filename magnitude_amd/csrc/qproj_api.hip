@@ -383,7 +383,7 @@ bool use_mfma_kernel(int type, int64_t M, int64_t K) {
 // scratch bytes run_dense_q8act needs for M rows against these tensors
 size_t per32_scratch_max(int n, const qproj_weight *const *w, int64_t M) {   // the targets run one after the other
     size_t need = 0;
-    for (int i = 0; i < n; ++i) need = std::max(need, per32_scratch_bytes(w[i]->K, M, w[i]->N));
+    for (int i = 0; i < n; ++i) need = std::max(need, per32_scratch_bytes(w[i]->type, w[i]->K, M, w[i]->N, per32_tiles(M, w[i]->N)));
     return need;
 }
 
@@ -424,14 +424,22 @@ bool takes_stream(const qproj_weight *t, int64_t M) { return takes_tiled(t, M) &
 
 size_t dense_scratch_bytes(int n, const qproj_weight *const *w, int64_t M) {
     if (takes_tiled(w[0], M)) {
+        int64_t all_tiles = 0;   // Q8_0: the matrices share a launch
+        for (int i = 0; i < n; ++i) all_tiles += per32_tiles(M, w[i]->N);
         size_t need = 0, streamed = 0;   // the launches follow one another: the same bytes serve all of them
         for (int i = 0; i < n; ++i) {
             const int t = w[i]->type;
             if (takes_stream(w[i], M)) streamed += stream_scratch_bytes(t, w[i]->K, M, w[i]->N);
             else
-                need = std::max(need, t == kTypeQ8_0   ? per32_scratch_bytes(w[i]->K, M, w[i]->N)
+                need = std::max(need, t == kTypeQ8_0   ? per32_scratch_bytes(t, w[i]->K, M, w[i]->N, all_tiles)
                                       : t == kTypeQ6_K ? q6k_tile_scratch_bytes(w[i]->K, M, w[i]->N)
                                                        : q4k_tile_scratch_bytes(w[i]->K, M, w[i]->N));
+        }
+        if (w[0]->type == kTypeQ8_0) {   // one launch for all of them, unless that asks more than the
+            // allocation-free entry point has: then one after the other in the room of the largest
+            size_t all = 0;
+            for (int i = 0; i < n; ++i) all += per32_scratch_bytes(kTypeQ8_0, w[i]->K, M, w[i]->N, all_tiles);
+            if (act_planes(kActKindQ8_0, M, w[0]->K).total + all <= (size_t)QPROJ_NOALLOC_SCRATCH_BYTES) need = all;
         }
         return std::max(need, streamed);
     }
@@ -541,10 +549,13 @@ int run_dense_q8act(qproj_ctx *ctx, int n, const qproj_weight *const *w, const A
             QP_HIP(ctx, launch_gemm_q8k_multi(n_rest, rest, a, M, yr, scr, ctx->stream));
             return QPROJ_OK;
         }
+        if (type == kTypeQ8_0 && n_rest > 0) {
+            QP_HIP(ctx, launch_gemm_q8_0(n_rest, rest, a, M, yr, scr, ctx->stream));
+            return QPROJ_OK;
+        }
         for (int i = 0; i < n_rest; ++i)
             QP_HIP(ctx, type == kTypeQ4_K   ? launch_gemm_q8k(rest[i], a, M, yr[i], scr.for_target(i), ctx->stream)
-                        : type == kTypeQ6_K ? launch_gemm_q6k_q8k(rest[i], a, M, yr[i], scr, ctx->stream)
-                                            : launch_gemm_q8_0(rest[i], a, M, yr[i], scr, ctx->stream));
+                                            : launch_gemm_q6k_q8k(rest[i], a, M, yr[i], scr, ctx->stream));
         return QPROJ_OK;
     }
     if (use_mfma_kernel(w[0]->type, M, w[0]->K)) {

@@ -215,8 +215,9 @@ hipError_t launch_moe_decode(const GemvArgs &args, int n_expert, bool swiglu, co
 hipError_t launch_moe_combine(const float *e, const float *weights, int64_t B, int64_t n_used, int64_t N,
                               float *y, hipStream_t s);
 // `scratch`: per32_scratch_bytes(K, M, N) bytes (null: K is never split)
-int per32_splits(int64_t K, int64_t M, int64_t N);
-size_t per32_scratch_bytes(int64_t K, int64_t M, int64_t N);
+int64_t per32_tiles(int64_t M, int64_t N);
+int per32_splits(int type, int64_t K, int64_t M, int64_t N, int64_t all_tiles);   // all_tiles: of every matrix of the launch
+size_t per32_scratch_bytes(int type, int64_t K, int64_t M, int64_t N, int64_t all_tiles);
 hipError_t launch_gemm_q8x32(const WeightView &w, const ActView &a, int64_t M, float *y, const Scratch &scratch, hipStream_t s);
 // Q4_K weights x ggml Q8_K activations (`a`), large M
 // `scratch`: q8k_tile_scratch_bytes(K, M, N) bytes (null: K is never split)
@@ -229,7 +230,32 @@ uint32_t q4k_multi_adds(int n, const WeightView *w, int64_t M, bool have_scratch
 hipError_t launch_gemm_q8k(const WeightView &w, const ActView &a, int64_t M, float *y, const Scratch &scratch, hipStream_t s);
 hipError_t launch_gemm_q8k_multi(int n, const WeightView *w, const ActView &a, int64_t M, float *const *y,
                                  const Scratch &scratch, hipStream_t s);
-hipError_t launch_gemm_q8_0(const WeightView &w, const ActView &a, int64_t M, float *y, const Scratch &scratch, hipStream_t s);
+// n Q8_0 matrices of one K; `scratch`: at least the largest per32_scratch_bytes, their sum for one launch and one adding pass
+hipError_t launch_gemm_q8_0(int n, const WeightView *w, const ActView &a, int64_t M, float *const *y, const Scratch &scratch, hipStream_t s);
+// y_i = part_i[0] + part_i[1] + ... in that order (n_split partial results of `count` floats, a multiple of 4 and 16-byte
+// aligned), several matrices in one launch
+struct SumTarget {
+    const float *part;
+    float *y;
+    int n_split;
+    int64_t n4;         // float4s of one partial result
+    int64_t first;      // first thread, a multiple of 256
+};
+struct SumTargets {
+    int n;
+    int64_t threads;
+    SumTarget t[kMaxTargets];
+};
+inline void add_sum(SumTargets &g, const float *part, float *y, int n_split, int64_t count) {
+    SumTarget &t = g.t[g.n++];
+    t.part = part;
+    t.y = y;
+    t.n_split = n_split;
+    t.n4 = count / 4;
+    t.first = g.threads;
+    g.threads += (t.n4 + 255) / 256 * 256;
+}
+hipError_t launch_sum_parts(const SumTargets &g, hipStream_t s);
 // 33..256 rows of Q4_K / Q6_K weights: all matrices of a call in one launch, K cut per matrix
 bool stream_takes(int type, int64_t K, int64_t M, int64_t N);
 size_t stream_scratch_bytes(int type, int64_t K, int64_t M, int64_t N);   // per matrix; the launcher wants the sum

@@ -136,3 +136,13 @@ def test_routing_table_of_the_benchmark_configurations_is_pinned():
 def test_plan_reports_a_refused_call():
     with pytest.raises(qproj.QprojError):
         qproj.plan_mul_mat(Q6_K, 4096, (4096,), 64, Q8X32)
+
+
+def test_q8_0_matrices_share_a_launch_only_while_their_partial_results_have_room():
+    # 256 rows of K = 196608: the activation planes leave 10 MB of the allocation-free entry point's 64 MiB, one matrix's
+    # partial results are 4 MB, four matrices' 16
+    k, ns = 196608, [1024] * 4
+    plan = qproj.plan_mul_mat(Q8_0, k, ns, 256)
+    assert plan.count("gemm_per32_kernel") == 4 and "(same launch)" not in plan
+    assert 0 < qproj.workspace_bytes(Q8_0, k, ns, 256) <= 64 << 20
+    assert qproj.plan_mul_mat(Q8_0, k // 2, ns, 256).count("(same launch)") == 3

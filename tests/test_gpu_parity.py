@@ -627,6 +627,27 @@ def test_per32_tiles_hold_the_largest_block_sums(ctx, orc, qtype, m, k, n):
     w.free()
 
 
+@pytest.mark.parametrize("m,k,ns", [(33, 512, (130, 128, 1)), (187, 3072, (640, 256, 256)), (64, 1152, (129, 260, 4, 384)),
+                                    (256, 640, (1024, 1024))])
+def test_q8_0_matrices_of_a_call_share_a_launch(ctx, orc, m, k, ns):
+    """Ragged row counts, outputs that are no multiple of four floats (K whole) beside ones whose K is cut, an odd number
+    of K-steps, two to four matrices: one launch, each result against the oracle (5e-5 of the larger of 1 and the result:
+    exact block sums, K / 32 fp32 addends in another order), nothing written behind an output."""
+    from magnitude_amd import ACT_GGML, qproj
+    plan = qproj.plan_mul_mat(Q8_0, k, list(ns), m, ACT_GGML)
+    assert plan.count("gemm_per32_kernel") == len(ns) and plan.count("(same launch)") == len(ns) - 1
+    x = np.random.default_rng(m + k).standard_normal((m, k)).astype(np.float32)
+    blocks = [make_weight(orc, Q8_0, n, k, seed=6300 + i) for i, n in enumerate(ns)]
+    ws = [ctx.upload(Q8_0, k, n, b) for n, b in zip(ns, blocks)]
+    bufs = [torch.full((m * n + 64,), 7.0, dtype=torch.float32, device="cuda") for n in ns]
+    ctx.mul_mat_multi(ws, dev(x), ACT_GGML, outs=[b[: m * n].view(m, n) for b, n in zip(bufs, ns)])
+    some = np.unique([0, 1, 31, 32, m // 2, m - 2, m - 1])
+    for w, n, b, bl in zip(ws, ns, bufs, blocks):
+        close(b[: m * n].view(m, n).cpu().numpy()[some], orc.mul_mat(Q8_0, bl, k, x[some], orc.ACT_GGML), 5e-5)
+        assert bool((b[m * n:] == 7.0).all())
+        w.free()
+
+
 # ---------------------------------------------------------------- MUL_MAT_ID and the MoE FFN
 
 @pytest.fixture(scope="module")
