@@ -652,12 +652,12 @@ def main():
                           "headline_rel_mad": head["rel_mad"], "samples_per_shape": MIN_SAMPLES, "statistic": "median",
                           # What bounds this format (not the matrix cores): both operands change scale every 32 weights, so
                           # an int32 result is good for ONE matrix instruction and each of its 16 outputs a lane costs
-                          # convert + scale product + fma on the vector ALU: 48 vector instructions behind every
-                          # 32 x 32 x 32 product (52.8 measured with addresses and loads).  With a matrix instruction holding
-                          # the issue port 16 of its 32 cycles and a vector instruction 4, the floor is
-                          # 5000 TOPS x 32 / (16 + 4 x 52.8) = 704 TOPS (profiles/prefill_gemm_kernels.txt, section 2).
-                          "bound": "valu", "floor_tops": 704.0,
-                          "floor": "5000 x 32 / (16 + 4 x 52.8): 48 of 52.8 vector instr. per matrix instr. are the per-32 flush",
+                          # two fmas on the vector ALU (the sum arrives as float bits): 32 vector instructions behind every
+                          # 32 x 32 x 32 product, 42.5 with addresses, staging and scales (85 a pair of products).  With a matrix
+                          # instruction holding the issue port 16 of its 32 cycles and a vector instruction 4, the floor is
+                          # 5000 TOPS x 32 / (16 + 4 x 42.5) = 860 TOPS.
+                          "bound": "valu", "floor_tops": 860.0,
+                          "floor": "5000 x 32 / (16 + 4 x 42.5): 32 of 42.5 vector instr. per matrix instr. are the per-32 flush",
                           "peak_tops": INT8_PEAK_TOPS, "shapes": res}
         # the same shapes in the ggml activation format (Q8_K, one scale per 256): the reference's own arithmetic
         # (plus the layer's Q6_K down projection, which a Q4_K_M model runs through the same operator, and
