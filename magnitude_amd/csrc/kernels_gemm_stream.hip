@@ -572,6 +572,7 @@ hipError_t launch_stream_kernel(const StreamArgs &g, int wgs, hipStream_t s) {
 bool stream_takes(int type, int64_t K, int64_t M, int64_t N) {
     const int lo = tuning_int("QPROJ_STREAM_MIN_M", 33), hi = tuning_int("QPROJ_STREAM_MAX_M", 256);
     if ((type != kTypeQ4_K && type != kTypeQ6_K) || K % 256 != 0 || K > (1 << 22) || M < lo || M > hi) return false;
+    if (N > (1 << 24)) return false;   // row and tile numbers are ints, a tile's outputs are indexed with 32 bits: 127 * N + 31 at most
     return type == kTypeQ6_K || M <= 96 || stream_tiles(M, N, 2, 2) <= 256;
 }
 

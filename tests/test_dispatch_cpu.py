@@ -146,3 +146,13 @@ def test_q8_0_matrices_share_a_launch_only_while_their_partial_results_have_room
     assert plan.count("gemm_per32_kernel") == 4 and "(same launch)" not in plan
     assert 0 < qproj.workspace_bytes(Q8_0, k, ns, 256) <= 64 << 20
     assert qproj.plan_mul_mat(Q8_0, k // 2, ns, 256).count("(same launch)") == 3
+
+
+@pytest.mark.parametrize("qtype,m", [(Q4_K, 64), (Q6_K, 48), (Q6_K, 128), (Q6_K, 256)])
+def test_outputs_beyond_32_bit_indices_stay_on_the_kernels_with_64_bit_ones(qtype, m):
+    """The streaming kernel indexes a tile's outputs with 32 bits (127 rows * N + 31 at most): matrices beyond 2^24 rows
+    take the tiled kernels, whose output index has 64."""
+    assert "gemm_stream_kernel" in qproj.plan_mul_mat(qtype, 256, [1 << 24], m)
+    for n in ((1 << 24) + 1, 33_800_000, 40_000_000, 1 << 30):
+        plan = qproj.plan_mul_mat(qtype, 256, [n], m)
+        assert "gemm_stream_kernel" not in plan and "q8k" in plan, plan
