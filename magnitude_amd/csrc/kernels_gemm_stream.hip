@@ -547,6 +547,8 @@ StreamPlan stream_plan(int type, int64_t K, int64_t M, int64_t N) {
     int64_t n = std::max<int64_t>(1, wgs / stream_tiles(M, N, p.jt, p.kw));
     n = tuning_int("QPROJ_STREAM_SPLIT", (int)n);
     n = std::min<int64_t>(n, std::max<int64_t>(1, nb / (2 * p.kw)));   // two steps a stretch at least
+    // never more partial tiles than the allocation-free entry point has room for beside the activation planes
+    n = std::min<int64_t>(n, std::max<int64_t>(1, (int64_t)(q8k_scratch_room(M, K) / ((size_t)M * N * 4))));
     const auto steps = [&](int64_t parts) { return ((nb + parts - 1) / parts + p.kw - 1) / p.kw; };
     while (n > 1 && steps(n - 1) == steps(n)) --n;   // no more stretches than it takes
     if ((M * N) % 4 != 0) n = 1;
@@ -576,36 +578,56 @@ bool stream_takes(int type, int64_t K, int64_t M, int64_t N) {
     return type == kTypeQ6_K || M <= 96 || stream_tiles(M, N, 2, 2) <= 256;
 }
 
-size_t stream_scratch_bytes(int type, int64_t K, int64_t M, int64_t N) {
-    const StreamPlan p = stream_plan(type, K, M, N);
-    return p.n_split > 1 ? (size_t)p.n_split * M * N * 4 : 0;
+namespace {
+size_t partial_bytes(const StreamPlan &p, int64_t M, int64_t N) { return p.n_split > 1 ? (size_t)p.n_split * M * N * 4 : 0; }
+
+// How many of the matrices from `first` on have room for their partial tiles in `bytes` of scratch; the next ones follow
+// in launches of their own, behind the adding pass, through the same bytes.
+int matrices_that_fit(int n, const StreamPlan *plans, int64_t M, const int64_t *N, int first, size_t bytes, size_t *used) {
+    *used = 0;
+    int i = first;
+    for (; i < n; ++i) {
+        const size_t b = partial_bytes(plans[i], M, N[i]);
+        if (*used + b > bytes) break;
+        *used += b;
+    }
+    return i - first;
+}
+}  // namespace
+
+// Scratch for the matrices of one call: all partial tiles side by side where the allocation-free entry point has the
+// room, else the largest run of matrices that has it (8192 -> 8192 / 1024 / 1024, Q6_K, 256 rows: 33.5 + 16.8 + 16.8 MB)
+size_t stream_scratch_bytes(int type, int64_t K, int64_t M, int n, const int64_t *N) {
+    StreamPlan plans[kMaxTargets];
+    for (int i = 0; i < n; ++i) plans[i] = stream_plan(type, K, M, N[i]);
+    size_t need = 0;
+    for (int first = 0; first < n;) {
+        size_t used = 0;
+        first += std::max(1, matrices_that_fit(n, plans, M, N, first, q8k_scratch_room(M, K), &used));   // (alone each fits: stream_plan)
+        need = std::max(need, used);
+    }
+    return need;
 }
 
-// n matrices of one type over the same activation rows; `scratch` holds the partial tiles of all of them one behind
-// the other (the sum of stream_scratch_bytes)
-hipError_t launch_gemm_stream(int n, const WeightView *w, const ActView &a, int64_t M, float *const *y, const Scratch &scratch,
-                              hipStream_t s) {
-    if (n < 1 || n > kMaxTargets || a.kind != kActKindQ8_K || M <= 0) return hipErrorInvalidValue;
+namespace {
+// the matrices of one launch group, their partial tiles side by side in `part`: a launch for all of one tile shape
+// (q/k/v, gate/up: all of them), then one adding pass
+hipError_t launch_group(int n, const WeightView *w, const StreamPlan *plans, const ActView &a, int64_t M, float *const *y, float *part, hipStream_t s) {
     const bool q4 = w[0].type == kTypeQ4_K;
-    if (q4 && (!a.msum || !a.rs)) return hipErrorInvalidValue;
     SumTargets sg{};
-    size_t part = 0;
-    StreamPlan plans[kMaxTargets];
     float *out[kMaxTargets];
     for (int i = 0; i < n; ++i) {
-        if (w[i].type != w[0].type || w[i].K != w[0].K || !stream_takes(w[i].type, w[i].K, M, w[i].N)) return hipErrorInvalidValue;
-        plans[i] = stream_plan(w[i].type, w[i].K, M, w[i].N);
         out[i] = y[i];
         if (plans[i].n_split == 1) continue;
-        const size_t bytes = (size_t)plans[i].n_split * M * w[i].N * 4;
-        if (part + bytes > scratch.bytes || (!scratch.p && !dry_run())) return hipErrorInvalidValue;   // partial tiles would not fit
-        if (!dry_run()) out[i] = scratch.p + part / 4;
+        if (!dry_run()) {
+            out[i] = part;
+            part += partial_bytes(plans[i], M, w[i].N) / 4;
+        }
         add_sum(sg, out[i], y[i], plans[i].n_split, M * w[i].N);
-        part += bytes;
     }
     if (sg.n && dry_run()) plan_note_cut();
     bool done[kMaxTargets] = {};
-    for (int first = 0; first < n; ++first) {   // one launch for all matrices of one tile shape (q/k/v, gate/up: all of them)
+    for (int first = 0; first < n; ++first) {
         if (done[first]) continue;
         const StreamPlan &p0 = plans[first];
         const int rows = 32 * (8 / p0.kw);
@@ -652,6 +674,30 @@ hipError_t launch_gemm_stream(int n, const WeightView *w, const ActView &a, int6
     }
     if (dry_run() || sg.n == 0) return hipSuccess;
     return launch_sum_parts(sg, s);
+}
+}  // namespace
+
+// n matrices of one type over the same activation rows; `scratch`: stream_scratch_bytes
+hipError_t launch_gemm_stream(int n, const WeightView *w, const ActView &a, int64_t M, float *const *y, const Scratch &scratch,
+                              hipStream_t s) {
+    if (n < 1 || n > kMaxTargets || a.kind != kActKindQ8_K || M <= 0) return hipErrorInvalidValue;
+    if (w[0].type == kTypeQ4_K && (!a.msum || !a.rs)) return hipErrorInvalidValue;
+    StreamPlan plans[kMaxTargets];
+    int64_t N[kMaxTargets];
+    for (int i = 0; i < n; ++i) {
+        if (w[i].type != w[0].type || w[i].K != w[0].K || !stream_takes(w[i].type, w[i].K, M, w[i].N)) return hipErrorInvalidValue;
+        plans[i] = stream_plan(w[i].type, w[i].K, M, w[i].N);
+        N[i] = w[i].N;
+    }
+    for (int first = 0; first < n;) {
+        size_t used = 0;
+        const int count = matrices_that_fit(n, plans, M, N, first, scratch.bytes, &used);
+        if (count == 0 || (used && !scratch.p && !dry_run())) return hipErrorInvalidValue;   // partial tiles would not fit
+        const hipError_t e = launch_group(count, w + first, plans + first, a, M, y + first, scratch.p, s);
+        if (e != hipSuccess) return e;
+        first += count;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_sum_parts(const SumTargets &g, hipStream_t s) {

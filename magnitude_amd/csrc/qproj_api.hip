@@ -357,6 +357,15 @@ int upload_common(qproj_ctx *ctx, int type, int64_t K, int64_t N, int64_t n_expe
     return QPROJ_OK;
 }
 
+}  // namespace
+
+size_t qproj::q8k_scratch_room(int64_t M, int64_t K) {
+    const size_t planes = act_planes(kActKindQ8_K, M, K).total;
+    return planes < (size_t)QPROJ_NOALLOC_SCRATCH_BYTES ? (size_t)QPROJ_NOALLOC_SCRATCH_BYTES - planes : 0;
+}
+
+namespace {
+
 // dense mul_mat over quantized activations already sitting in `a` (M rows)
 bool use_decode_kernel(int type, int64_t M, int64_t K) {
     static const bool off = tuning_int("QPROJ_NO_DECODE_KERNEL", 0) != 0;
@@ -426,10 +435,12 @@ size_t dense_scratch_bytes(int n, const qproj_weight *const *w, int64_t M) {
     if (takes_tiled(w[0], M)) {
         int64_t all_tiles = 0;   // Q8_0: the matrices share a launch
         for (int i = 0; i < n; ++i) all_tiles += per32_tiles(M, w[i]->N);
-        size_t need = 0, streamed = 0;   // the launches follow one another: the same bytes serve all of them
+        size_t need = 0;   // the launches follow one another: the same bytes serve all of them
+        int64_t streamed[kMaxTargets];
+        int n_streamed = 0;
         for (int i = 0; i < n; ++i) {
             const int t = w[i]->type;
-            if (takes_stream(w[i], M)) streamed += stream_scratch_bytes(t, w[i]->K, M, w[i]->N);
+            if (takes_stream(w[i], M)) streamed[n_streamed++] = w[i]->N;
             else
                 need = std::max(need, t == kTypeQ8_0   ? per32_scratch_bytes(t, w[i]->K, M, w[i]->N, all_tiles)
                                       : t == kTypeQ6_K ? q6k_tile_scratch_bytes(w[i]->K, M, w[i]->N)
@@ -441,7 +452,7 @@ size_t dense_scratch_bytes(int n, const qproj_weight *const *w, int64_t M) {
             for (int i = 0; i < n; ++i) all += per32_scratch_bytes(kTypeQ8_0, w[i]->K, M, w[i]->N, all_tiles);
             if (act_planes(kActKindQ8_0, M, w[0]->K).total + all <= (size_t)QPROJ_NOALLOC_SCRATCH_BYTES) need = all;
         }
-        return std::max(need, streamed);
+        return n_streamed ? std::max(need, stream_scratch_bytes(w[0]->type, w[0]->K, M, n_streamed, streamed)) : need;
     }
     if (!use_mfma_kernel(w[0]->type, M, w[0]->K)) return 0;
     int64_t sum_n = 0, rgs = 0;

@@ -156,3 +156,25 @@ def test_outputs_beyond_32_bit_indices_stay_on_the_kernels_with_64_bit_ones(qtyp
     for n in ((1 << 24) + 1, 33_800_000, 40_000_000, 1 << 30):
         plan = qproj.plan_mul_mat(qtype, 256, [n], m)
         assert "gemm_stream_kernel" not in plan and "q8k" in plan, plan
+
+
+@pytest.mark.parametrize("qtype", [Q4_K, Q6_K])
+def test_streamed_batches_fit_the_fixed_scratch_while_their_activation_planes_do(qtype):
+    """The partial tiles of a streamed call share what the 64 MiB of the allocation-free entry point leave beside the
+    activation planes: one matrix's K is cut in no more stretches than fit there, and matrices whose partial tiles do
+    not fit side by side go one after the other through the same bytes."""
+    lib = qproj.load_library()
+    apart = checked = 0
+    for k, m in itertools.product([4096, 8192, 14336, 16384, 28672, 65536, 131072, 163840, 196608], [33, 64, 65, 96, 128, 187, 250, 256]):
+        planes = lib.qproj_act_bytes(GGML, qtype, m, k)
+        for ns in [(1024,), (8192,), (77,), (128,), (512,), (8192, 8192), (8192, 1024, 1024), (4096, 4096), (4096,) * 4, (512,) * 4, (28672, 28672)]:
+            plan = qproj.plan_mul_mat(qtype, k, ns, m)
+            if plan.count("gemm_stream_kernel") < len(ns):
+                continue
+            checked += 1
+            nbytes = qproj.workspace_bytes(qtype, k, ns, m)
+            assert planes <= nbytes <= max(planes, qproj.NOALLOC_SCRATCH_BYTES), (k, m, ns, nbytes)
+            apart += plan.count("(same launch)") < len(ns) - 1
+    assert checked > 300 and apart > 10
+    assert qproj.workspace_bytes(Q6_K, 8192, (8192, 1024, 1024), 256) <= qproj.NOALLOC_SCRATCH_BYTES
+    assert "(same launch)" in qproj.plan_mul_mat(Q6_K, 8192, (8192, 1024, 1024), 128)   # with room: one launch

@@ -119,3 +119,19 @@ def test_noalloc_scratch_belongs_to_one_context_at_a_time(ctx):
     again = ctx.mul_mat_multi([w], x, ACT_GGML, noalloc=True)[0]
     assert torch.equal(again.view(torch.int32), want.view(torch.int32))
     w.free()
+
+
+@pytest.mark.parametrize("qtype,k,ns,m", [(Q6_K, 8192, (2048, 1024, 1024), 256), (Q6_K, 8192, (1024, 1024, 2048, 77), 250)])
+def test_noalloc_streams_matrices_one_after_the_other_where_their_partial_tiles_do_not_fit_together(ctx, qtype, k, ns, m):
+    """The partial tiles of all matrices are 67 MB, the room beside the activation planes is 61.8 MiB: they go in two
+    launches through the same bytes.  Bar: the call is served and every matrix has the bits of a call of its own."""
+    from magnitude_amd import ACT_GGML, qproj
+    plan = qproj.plan_mul_mat(qtype, k, list(ns), m, ACT_GGML)
+    assert plan.count("gemm_stream_kernel") == len(ns) and plan.count("(same launch)") == len(ns) - 2
+    ws = [upload(ctx, qtype, n, k, seed=7 * i + n) for i, n in enumerate(ns)]
+    x = torch.randn((m, k), generator=torch.Generator(device="cuda").manual_seed(m), device="cuda")
+    outs = [torch.full((m, n), float("nan"), device="cuda") for n in ns]
+    ctx.mul_mat_multi(ws, x, ACT_GGML, outs=outs, noalloc=True)
+    for w, y in zip(ws, outs):
+        assert torch.equal(y.view(torch.int32), ctx.mul_mat(w, x, ACT_GGML).view(torch.int32))
+        w.free()
