@@ -67,7 +67,7 @@ constexpr float kMagic = 12582912.f;   // 1.5 * 2^23: one integer step is one st
 // out[stretch][M][N] and an adding pass puts the stretches together in order.  The matrices of a call (q/k/v, gate/up)
 // share a launch: at 33 .. 256 tokens one of them alone leaves most of the chip's 512 places (two workgroups a compute
 // unit) empty, and every launch pays the latency of its K loop again.  Four layers of 3072 / 1024 / 8192 Q8_0 weights
-// at 187 tokens, a launch and an adding pass a matrix -> this: 774 -> 558 us.
+// at 187 tokens, a launch and an adding pass a matrix -> this: 828 -> 565 us.
 struct Per32Target {
     WeightView w;
     float *out;   // the output, or [n_split][M][N] partial tiles
@@ -918,8 +918,6 @@ hipError_t launch_per32(int n, const WeightView *w, const ActView &a, int64_t M,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GemmSmem));
         if (attr != hipSuccess) return attr;
     }
-    int64_t all_tiles = 0;
-    for (int i = 0; i < n; ++i) all_tiles += per32_tiles(M, w[i].N);
     for (int first = 0; first < n;) {
         Per32Args g{};
         g.a = a;
@@ -930,7 +928,7 @@ hipError_t launch_per32(int n, const WeightView *w, const ActView &a, int64_t M,
         int i = first;
         for (; i < n; ++i) {
             if (w[i].K != w[0].K) return hipErrorInvalidValue;
-            const int n_split = sc.p ? per32_splits(QT, w[i].K, M, w[i].N, all_tiles) : 1;
+            const int n_split = sc.p ? per32_splits(QT, w[i].K, M, w[i].N) : 1;
             const size_t bytes = n_split > 1 ? (size_t)n_split * M * w[i].N * 4 : 0;
             if (used + bytes > sc.bytes && bytes) {
                 if (i == first) return hipErrorInvalidValue;   // partial tiles would not fit
@@ -1016,14 +1014,16 @@ size_t q8k_tile_scratch_bytes(int64_t K, int64_t M, int64_t N) {
 
 // A grid of fewer than 192 tiles leaves the 256 compute units mostly idle and a workgroup's K loop is
 // latency-bound: K is then cut into stretches done by different workgroups, as many as fill one round (32 tiles of
-// K = 14336, Q8_0 at 64 - 128 tokens: 8 stretches instead of 3).  `all_tiles`: the tiles of every matrix that shares the
-// launch - gate and up of 8192 rows at 187 tokens are 256 tiles together and stay whole (cut in two, as each is alone, a
-// layer took 152 us instead of 141), while 4096 -> 14336 alone at 64 tokens needs its two stretches (35 us; whole 55).
+// K = 14336, Q8_0 at 64 - 128 tokens: 8 stretches instead of 3).  The cut follows the matrix and the row count alone,
+// whatever shares the launch: the order of a result's fp32 sums is the same in a call of its own, and the shorter
+// chains keep the error down (8192 -> 8192 / 1024 / 1024 at 256 rows against 64 bits: 2.1e-7; with the cut by the tiles of
+// the whole launch, which was tried, 2.9e-7).
 int64_t per32_tiles(int64_t M, int64_t N) { return ((N + BN - 1) / BN) * ((M + BM - 1) / BM); }
-int per32_splits(int type, int64_t K, int64_t M, int64_t N, int64_t all_tiles) {
+int per32_splits(int type, int64_t K, int64_t M, int64_t N) {
     static const int forced = tuning_int("QPROJ_PER32_SPLITS", 0);
     // as many stretches as fill one round of workgroups (one a compute unit), eight at most
-    int n = forced > 0 ? forced : all_tiles >= 192 ? 1 : (int)std::min<int64_t>(8, std::max<int64_t>(1, cu_count() / all_tiles));
+    const int64_t tiles = per32_tiles(M, N);
+    int n = forced > 0 ? forced : tiles >= 192 ? 1 : (int)std::min<int64_t>(8, std::max<int64_t>(1, cu_count() / tiles));
     if ((M * N) % 4 != 0) n = 1;
     // at least two times 256 weights a stretch, Q4_K four (its min term is a loop of its own over the stretch).  Q8_0,
     // four -> two, us: 4096 -> 1024 at 64 tokens 21.2 -> 16.8, 2560 x 2560 at 250 27.2 -> 22.5, 4096 x 4096 at 100 24.5 -> 22.4.
@@ -1031,8 +1031,8 @@ int per32_splits(int type, int64_t K, int64_t M, int64_t N, int64_t all_tiles) {
     while (n > 1 && K / 256 < least * n) --n;
     return n;
 }
-size_t per32_scratch_bytes(int type, int64_t K, int64_t M, int64_t N, int64_t all_tiles) {
-    const int n = per32_splits(type, K, M, N, all_tiles);
+size_t per32_scratch_bytes(int type, int64_t K, int64_t M, int64_t N) {
+    const int n = per32_splits(type, K, M, N);
     return n > 1 ? (size_t)n * M * N * 4 : 0;
 }
 

@@ -392,7 +392,7 @@ bool use_mfma_kernel(int type, int64_t M, int64_t K) {
 // scratch bytes run_dense_q8act needs for M rows against these tensors
 size_t per32_scratch_max(int n, const qproj_weight *const *w, int64_t M) {   // the targets run one after the other
     size_t need = 0;
-    for (int i = 0; i < n; ++i) need = std::max(need, per32_scratch_bytes(w[i]->type, w[i]->K, M, w[i]->N, per32_tiles(M, w[i]->N)));
+    for (int i = 0; i < n; ++i) need = std::max(need, per32_scratch_bytes(w[i]->type, w[i]->K, M, w[i]->N));
     return need;
 }
 
@@ -428,13 +428,12 @@ bool takes_tiled(const qproj_weight *t, int64_t M) {
 }
 
 // The streaming kernel's share of those batches: the matrices it takes go in one launch, the others follow on the tiled
-// kernels.  Decided matrix by matrix, so that a matrix gets the same kernel whatever rides along with it.
+// kernels.  Decided matrix by matrix, as its cut of K is (stream_plan; per32_splits for Q8_0): a matrix gets the same
+// kernel and the same order of its fp32 sums whatever rides along with it.
 bool takes_stream(const qproj_weight *t, int64_t M) { return takes_tiled(t, M) && stream_takes(t->type, t->K, M, t->N); }
 
 size_t dense_scratch_bytes(int n, const qproj_weight *const *w, int64_t M) {
     if (takes_tiled(w[0], M)) {
-        int64_t all_tiles = 0;   // Q8_0: the matrices share a launch
-        for (int i = 0; i < n; ++i) all_tiles += per32_tiles(M, w[i]->N);
         size_t need = 0;   // the launches follow one another: the same bytes serve all of them
         int64_t streamed[kMaxTargets];
         int n_streamed = 0;
@@ -442,14 +441,14 @@ size_t dense_scratch_bytes(int n, const qproj_weight *const *w, int64_t M) {
             const int t = w[i]->type;
             if (takes_stream(w[i], M)) streamed[n_streamed++] = w[i]->N;
             else
-                need = std::max(need, t == kTypeQ8_0   ? per32_scratch_bytes(t, w[i]->K, M, w[i]->N, all_tiles)
+                need = std::max(need, t == kTypeQ8_0   ? per32_scratch_bytes(t, w[i]->K, M, w[i]->N)
                                       : t == kTypeQ6_K ? q6k_tile_scratch_bytes(w[i]->K, M, w[i]->N)
                                                        : q4k_tile_scratch_bytes(w[i]->K, M, w[i]->N));
         }
         if (w[0]->type == kTypeQ8_0) {   // one launch for all of them, unless that asks more than the
             // allocation-free entry point has: then one after the other in the room of the largest
             size_t all = 0;
-            for (int i = 0; i < n; ++i) all += per32_scratch_bytes(kTypeQ8_0, w[i]->K, M, w[i]->N, all_tiles);
+            for (int i = 0; i < n; ++i) all += per32_scratch_bytes(kTypeQ8_0, w[i]->K, M, w[i]->N);
             if (act_planes(kActKindQ8_0, M, w[0]->K).total + all <= (size_t)QPROJ_NOALLOC_SCRATCH_BYTES) need = all;
         }
         return n_streamed ? std::max(need, stream_scratch_bytes(w[0]->type, w[0]->K, M, n_streamed, streamed)) : need;

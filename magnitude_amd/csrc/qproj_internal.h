@@ -214,10 +214,10 @@ hipError_t launch_moe_decode(const GemvArgs &args, int n_expert, bool swiglu, co
                              hipStream_t s);
 hipError_t launch_moe_combine(const float *e, const float *weights, int64_t B, int64_t n_used, int64_t N,
                               float *y, hipStream_t s);
-// `scratch`: per32_scratch_bytes(K, M, N) bytes (null: K is never split)
+// `scratch`: per32_scratch_bytes bytes (null: K is never split)
 int64_t per32_tiles(int64_t M, int64_t N);
-int per32_splits(int type, int64_t K, int64_t M, int64_t N, int64_t all_tiles);   // all_tiles: of every matrix of the launch
-size_t per32_scratch_bytes(int type, int64_t K, int64_t M, int64_t N, int64_t all_tiles);
+int per32_splits(int type, int64_t K, int64_t M, int64_t N);
+size_t per32_scratch_bytes(int type, int64_t K, int64_t M, int64_t N);
 hipError_t launch_gemm_q8x32(const WeightView &w, const ActView &a, int64_t M, float *y, const Scratch &scratch, hipStream_t s);
 // Q4_K weights x ggml Q8_K activations (`a`), large M
 // `scratch`: q8k_tile_scratch_bytes(K, M, N) bytes (null: K is never split)

@@ -178,3 +178,22 @@ def test_streamed_batches_fit_the_fixed_scratch_while_their_activation_planes_do
     assert checked > 300 and apart > 10
     assert qproj.workspace_bytes(Q6_K, 8192, (8192, 1024, 1024), 256) <= qproj.NOALLOC_SCRATCH_BYTES
     assert "(same launch)" in qproj.plan_mul_mat(Q6_K, 8192, (8192, 1024, 1024), 128)   # with room: one launch
+
+
+@pytest.mark.parametrize("qtype", [Q8_0, Q4_K, Q6_K])
+def test_a_matrix_is_cut_the_same_way_alone_and_beside_others(qtype):
+    """Tile and stretches of K decide the order of a result's fp32 sums.  Q8_0 tiles and the streaming kernel take both
+    from the matrix and the row count alone, so a call with several matrices gives the bits of separate calls."""
+    def cuts(ns, k, m):
+        lines = [l for l in qproj.plan_mul_mat(qtype, k, ns, m).splitlines() if "gemm_" in l]
+        return [l.replace(" (same launch)", "") for l in lines]
+
+    checked = 0
+    for k, m in itertools.product([512, 3072, 4096, 8192, 14336], [33, 64, 100, 187, 256, 500, 2048]):
+        for ns in [(4096, 1024, 1024), (8192, 8192), (3072, 1024, 1024), (28672, 28672), (512, 77, 2048, 256)]:
+            together, alone = cuts(ns, k, m), [cuts((n,), k, m) for n in ns]
+            if qtype != Q8_0 and any("gemm_stream_kernel" not in a[0] for a in alone):
+                continue
+            assert together == sum(alone, []), (k, m, ns)
+            checked += 1
+    assert checked > 30

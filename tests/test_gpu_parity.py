@@ -628,11 +628,12 @@ def test_per32_tiles_hold_the_largest_block_sums(ctx, orc, qtype, m, k, n):
 
 
 @pytest.mark.parametrize("m,k,ns", [(33, 512, (130, 128, 1)), (187, 3072, (640, 256, 256)), (64, 1152, (129, 260, 4, 384)),
-                                    (256, 640, (1024, 1024))])
+                                    (256, 640, (1024, 1024)), (187, 3072, (3072, 1024, 1024)), (129, 2048, (8192, 8192))])
 def test_q8_0_matrices_of_a_call_share_a_launch(ctx, orc, m, k, ns):
     """Ragged row counts, outputs that are no multiple of four floats (K whole) beside ones whose K is cut, an odd number
     of K-steps, two to four matrices: one launch, each result against the oracle (5e-5 of the larger of 1 and the result:
-    exact block sums, K / 32 fp32 addends in another order), nothing written behind an output."""
+    exact block sums, K / 32 fp32 addends in another order), nothing written behind an output.  K is cut by the matrix and
+    the row count alone, so the results have the bits of separate calls."""
     from magnitude_amd import ACT_GGML, qproj
     plan = qproj.plan_mul_mat(Q8_0, k, list(ns), m, ACT_GGML)
     assert plan.count("gemm_per32_kernel") == len(ns) and plan.count("(same launch)") == len(ns) - 1
@@ -645,6 +646,7 @@ def test_q8_0_matrices_of_a_call_share_a_launch(ctx, orc, m, k, ns):
     for w, n, b, bl in zip(ws, ns, bufs, blocks):
         close(b[: m * n].view(m, n).cpu().numpy()[some], orc.mul_mat(Q8_0, bl, k, x[some], orc.ACT_GGML), 5e-5)
         assert bool((b[m * n:] == 7.0).all())
+        assert torch.equal(b[: m * n].view(m, n), ctx.mul_mat(w, dev(x), ACT_GGML))
         w.free()
 
 
