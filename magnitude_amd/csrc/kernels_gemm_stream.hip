@@ -8,7 +8,8 @@
 //     step and asks for the block after next into the same strip, so 8 waves keep 2 x 37 KB a compute unit in flight;
 //   - activations of a step (one super-block a K part) are double-buffered in LDS, shared by the row groups of the
 //     workgroup, one barrier a step;
-//   - a workgroup is 8 waves = RW row groups of 32 weight rows x KW K parts (summed through LDS at the end), K is cut
+//   - a workgroup is 8 waves (4 where the launch leaves room for twice the workgroups) = RW row groups of 32 weight
+//     rows x KW K parts (summed through LDS at the end), K is cut
 //     further over workgroups where the tiles would not fill the chip, and all matrices of a call (q/k/v, gate/up)
 //     share the launch and the launch that adds the partial tiles.
 // The arithmetic is that of the tiled kernels: Q4_K scales in base 8 as two int8 operands, Q6_K products as high and
@@ -134,24 +135,24 @@ struct Strip<kTypeQ6_K> {
 // LDS of a workgroup: [2][KW] activation tiles (32 * JT tokens x 256, 16-byte segments XOR-swizzled by the token),
 // [2][KW] min-term tiles (Q4_K), the scales of kScaleSb super-blocks (activations [super-block][token]; Q6_K weights
 // [wave][super-block][row]), then the strips
-template <int QT, int JT, int KW, int SW>
+template <int QT, int JT, int KW, int SW, int NW>
 struct StreamLds {
     static constexpr int kScaleSb = JT <= 2 ? 16 : 8;
     static constexpr int kAct = JT * 8192, kMs = QT == kTypeQ4_K ? JT * 1024 : 0, kDx = JT * 128;
     static constexpr int kDwWave = QT == kTypeQ6_K ? kScaleSb / KW * 64 : 0;
     static constexpr int kOffMs = 2 * KW * kAct, kOffDx = kOffMs + 2 * KW * kMs, kOffDw = kOffDx + kScaleSb * kDx,
-                         kOffStrip = kOffDw + 8 * kDwWave;
-    static constexpr int kTotal = kOffStrip + 8 * SW * Strip<QT>::kBytes;
+                         kOffStrip = kOffDw + NW * kDwWave;
+    static constexpr int kTotal = kOffStrip + NW * SW * Strip<QT>::kBytes;
     static_assert(kTotal <= 160 * 1024, "one workgroup's LDS");
-    static_assert(8 * JT * 4096 <= kOffStrip || KW == 1, "the K parts meet in the same LDS at the end");
+    static_assert(NW * JT * 4096 <= kOffStrip || KW == 1, "the K parts meet in the same LDS at the end");
 };
 
-template <int QT, int JT, int KW, int SW>
-__global__ __launch_bounds__(512, 1) void gemm_stream_kernel(const StreamArgs g) {
+template <int QT, int JT, int KW, int SW, int NW>
+__global__ __launch_bounds__(64 * NW, 1) void gemm_stream_kernel(const StreamArgs g) {
     using S = Strip<QT>;
-    using L = StreamLds<QT, JT, KW, SW>;
+    using L = StreamLds<QT, JT, KW, SW, NW>;
     constexpr bool kQ4 = QT == kTypeQ4_K;
-    constexpr int RW = 8 / KW, TM = 32 * JT;
+    constexpr int RW = NW / KW, TM = 32 * JT, NT = 64 * NW;
     extern __shared__ __align__(16) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, lh = lane >> 5, rg = wave % RW, kp = wave / RW;
@@ -175,28 +176,30 @@ __global__ __launch_bounds__(512, 1) void gemm_stream_kernel(const StreamArgs g)
         const int row0 = min(n0, t.N - 1);   // rows past the edge of the matrix repeat its last row (never stored)
         strip_src.init(t, nb, row0, min(t.N - 1 - row0, 31), lane);
     }
-    uint8_t *strip = smem + L::kOffStrip + wave * S::kBytes;   // second buffer 8 * kBytes further on
+    uint8_t *strip = smem + L::kOffStrip + wave * S::kBytes;   // second buffer NW * kBytes further on
     auto my_sb = [&](int s) { return (uint32_t)min(sb_begin + s * KW + kp, sb_end - 1); };
 
-    // activations: chunk wave + 8*p of a step = K part p / JT, tokens 4*(wave + 8*(p % JT)) .. +3 of the tile
+    // activations: request p of a wave = K part p / AP, tokens 4*(wave + NW*(p % AP)) .. +3 of the tile
+    constexpr int AP = 8 * JT / NW;
     const int mcap = min(M - 1 - m0, TM - 1);
     const int8_t *abase = scalar_pointer(g.a.qs + (int64_t)m0 * K);
-    uint32_t aoff[JT];
+    uint32_t aoff[AP];
 #pragma unroll
-    for (int j = 0; j < JT; ++j) {
-        const int row = 4 * (wave + 8 * j) + (lane >> 4), seg = (lane & 15) ^ (row & 15);
+    for (int j = 0; j < AP; ++j) {
+        const int row = 4 * (wave + NW * j) + (lane >> 4), seg = (lane & 15) ^ (row & 15);
         aoff[j] = (uint32_t)(min(row, mcap) * (int)K + 16 * seg);
     }
     auto request_acts = [&](int s) {
 #pragma unroll
-        for (int p = 0; p < KW * JT; ++p) {
-            const uint32_t sb = (uint32_t)min(sb_begin + s * KW + p / JT, sb_end - 1);
-            global_to_lds16(abase + (aoff[p % JT] + sb * 256u), smem + ((s & 1) * KW + p / JT) * L::kAct + (wave + 8 * (p % JT)) * 1024);
+        for (int p = 0; p < KW * AP; ++p) {
+            const uint32_t sb = (uint32_t)min(sb_begin + s * KW + p / AP, sb_end - 1);
+            global_to_lds16(abase + (aoff[p % AP] + sb * 256u), smem + ((s & 1) * KW + p / AP) * L::kAct + (wave + NW * (p % AP)) * 1024);
         }
     };
     const uint8_t *msbase = nullptr;
     uint32_t msoff = 0;
     if constexpr (kQ4) {
+        static_assert(KW * JT <= NW, "a wave requests one tile of the min-term plane at most");
         msbase = scalar_pointer(reinterpret_cast<const uint8_t *>(g.a.msum) + (int64_t)m0 * nb * 32);
         msoff = (uint32_t)(min((wave % JT) * 32 + (lane >> 1), mcap) * nb * 32 + 16 * (lane & 1));
     }
@@ -220,13 +223,12 @@ __global__ __launch_bounds__(512, 1) void gemm_stream_kernel(const StreamArgs g)
         inv_rs = 1.0f / rs_mine;
     }
     auto load_scales = [&](int sb0) {
-        constexpr int kPer = (L::kScaleSb * TM + 511) / 512;
-        // thread -> token tid % TM of super-blocks tid / TM, + 512 / TM, ... (threads past the last whole group idle)
-        constexpr int kGroups = 512 / TM;
+        // thread -> token tid % TM of super-blocks tid / TM, + NT / TM, ... (threads past the last whole group idle)
+        constexpr int kGroups = NT / TM;
         if (tid < kGroups * TM) {
             const int tok = tid % TM;
 #pragma unroll
-            for (int i = 0; i < kPer + (512 % TM ? 1 : 0); ++i) {
+            for (int i = 0; i < (L::kScaleSb + kGroups - 1) / kGroups; ++i) {
                 const int q = tid / TM + i * kGroups;
                 if (q < L::kScaleSb)
                     dx_lds[q * TM + tok] = load_global<float>(dxbase, 4u * (uint32_t)(min(tok, mcap) * nb + min(sb0 + q, sb_end - 1))) * inv_rs;
@@ -390,7 +392,7 @@ __global__ __launch_bounds__(512, 1) void gemm_stream_kernel(const StreamArgs g)
     request_ms(0);
     load_scales(sb_begin);
     if constexpr (SW == 2) {
-        strip_src.request(my_sb(1), strip + 8 * S::kBytes);
+        strip_src.request(my_sb(1), strip + NW * S::kBytes);
         wait_vmcnt<S::kLoads>();
     } else {
         wait_vmcnt<0>();
@@ -403,7 +405,7 @@ __global__ __launch_bounds__(512, 1) void gemm_stream_kernel(const StreamArgs g)
         // MORE1: another step follows; MORE2: so does one whose strip is requested now
         auto step = [&](int s, auto more1, auto more2) {
             constexpr bool MORE1 = decltype(more1)::value, MORE2 = decltype(more2)::value;
-            uint8_t *sbuf = strip + (SW == 2 ? (s & 1) * 8 * S::kBytes : 0);
+            uint8_t *sbuf = strip + (SW == 2 ? (s & 1) * NW * S::kBytes : 0);
             const typename S::Raw raw = S::read(sbuf, l32, lh);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the strip has been read: it may be overwritten
             if constexpr (MORE1) {
@@ -441,8 +443,12 @@ __global__ __launch_bounds__(512, 1) void gemm_stream_kernel(const StreamArgs g)
         step(s, std::false_type{}, std::false_type{});
         if constexpr (LATE) flush(s);
     };
-    if (wave < 4) run(std::false_type{});
-    else run(std::true_type{});
+    if constexpr (NW <= 4) {   // a wave a SIMD
+        run(std::false_type{});
+    } else {
+        if (wave < 4) run(std::false_type{});
+        else run(std::true_type{});
+    }
 
     // ---- the K parts meet in LDS: part q of a row group keeps token tiles j % KW == q, the others hand theirs over
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (a single step leaves its second strip request behind)
@@ -556,13 +562,13 @@ StreamPlan stream_plan(int type, int64_t K, int64_t M, int64_t N) {
     return p;
 }
 
-template <int QT, int JT, int KW, int SW>
+template <int QT, int JT, int KW, int SW, int NW>
 hipError_t launch_stream_kernel(const StreamArgs &g, int wgs, hipStream_t s) {
-    constexpr int lds = StreamLds<QT, JT, KW, SW>::kTotal;
-    const auto kern = &gemm_stream_kernel<QT, JT, KW, SW>;
+    constexpr int lds = StreamLds<QT, JT, KW, SW, NW>::kTotal;
+    const auto kern = &gemm_stream_kernel<QT, JT, KW, SW, NW>;
     static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (attr != hipSuccess) return attr;
-    hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(512), lds, s, g);
+    hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(64 * NW), lds, s, g);
     return hipGetLastError();
 }
 
@@ -630,12 +636,20 @@ hipError_t launch_group(int n, const WeightView *w, const StreamPlan *plans, con
     for (int first = 0; first < n; ++first) {
         if (done[first]) continue;
         const StreamPlan &p0 = plans[first];
-        const int rows = 32 * (8 / p0.kw);
         StreamArgs g{};
         g.a = a;
         g.M = (int)M;
         g.nb = (int)(w[0].K / 256);
         g.tiles_m = (int)((M + 32 * p0.jt - 1) / (32 * p0.jt));
+        const auto tiles_pad = [&](int i, int rows) { return ((w[i].N + rows - 1) / rows * g.tiles_m + 7) / 8 * 8; };
+        // Four waves a workgroup (half the weight rows) where that many workgroups are still one round: the same sums, on
+        // twice the compute units.  Eight waves -> four, us a call: Q4_K 4096 -> 14336 alone at 48 rows 27.8 -> 23.3, 4096 x
+        // 4096 18.4 -> 16.6; Q6_K 4096 -> 14336 33.5 -> 27.8 at 48 rows, 69.3 -> 52.0 at 160; Q4_K 4096 -> 32000 at 96 rows
+        // 69.6 -> 50.8.  (A matrix is cut as if its usual neighbours rode along; alone it left half the chip idle.)
+        int64_t halves = 0;
+        for (int i = first; i < n; ++i)
+            if (plans[i].jt == p0.jt && plans[i].kw == p0.kw) halves += tiles_pad(i, 128 / p0.kw) * plans[i].n_split;
+        const int waves = tuning_int("QPROJ_STREAM_WAVES", halves <= cu_count() ? 4 : 8), rows = 32 * waves / p0.kw;
         int64_t wg = 0;
         for (int i = first; i < n; ++i) {
             if (plans[i].jt != p0.jt || plans[i].kw != p0.kw) continue;
@@ -650,7 +664,7 @@ hipError_t launch_group(int n, const WeightView *w, const StreamPlan *plans, con
             }
             t.N = (int)w[i].N;
             t.tiles_n = (int)((w[i].N + rows - 1) / rows);
-            t.tiles_pad = (t.tiles_n * g.tiles_m + 7) / 8 * 8;
+            t.tiles_pad = (int)tiles_pad(i, rows);
             t.n_split = plans[i].n_split;
             t.first_wg = (int)wg;
             t.out = out[i];
@@ -662,13 +676,22 @@ hipError_t launch_group(int n, const WeightView *w, const StreamPlan *plans, con
         if (wg >= 0x7fffffff) return hipErrorInvalidValue;
         if (dry_run()) continue;
         hipError_t e = hipErrorInvalidValue;
-#define QP_STREAM(JT, KW, SW6)                                                                                            \
-    if (p0.jt == JT && p0.kw == KW)                                                                                       \
-        e = q4 ? launch_stream_kernel<kTypeQ4_K, JT, KW, 2>(g, (int)wg, s) : launch_stream_kernel<kTypeQ6_K, JT, KW, SW6>(g, (int)wg, s)
-        QP_STREAM(2, 1, 2);
-        QP_STREAM(2, 2, 1);
-        QP_STREAM(3, 1, 1);
-        QP_STREAM(4, 1, 1);
+#define QP_STREAM(QT, JT, KW, SW, NW)                                             \
+    if (w[0].type == QT && p0.jt == JT && p0.kw == KW && waves == NW)             \
+        e = launch_stream_kernel<QT, JT, KW, SW, NW>(g, (int)wg, s)
+        // (64-token tiles with K in one part are only taken by grids beyond a round of the halves)
+        QP_STREAM(kTypeQ4_K, 2, 1, 2, 8);
+        QP_STREAM(kTypeQ4_K, 2, 2, 2, 8);
+        QP_STREAM(kTypeQ4_K, 2, 2, 2, 4);
+        QP_STREAM(kTypeQ4_K, 3, 1, 2, 8);
+        QP_STREAM(kTypeQ4_K, 3, 1, 2, 4);
+        QP_STREAM(kTypeQ6_K, 2, 1, 2, 8);
+        QP_STREAM(kTypeQ6_K, 2, 2, 1, 8);
+        QP_STREAM(kTypeQ6_K, 2, 2, 1, 4);
+        QP_STREAM(kTypeQ6_K, 3, 1, 1, 8);
+        QP_STREAM(kTypeQ6_K, 3, 1, 1, 4);
+        QP_STREAM(kTypeQ6_K, 4, 1, 1, 8);
+        QP_STREAM(kTypeQ6_K, 4, 1, 1, 4);
 #undef QP_STREAM
         if (e != hipSuccess) return e;
     }

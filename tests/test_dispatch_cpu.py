@@ -5,6 +5,7 @@ launching: every launcher works out its demand from the variables that pick its 
 too small, so a sizing rule and a dispatch rule that disagree show up here, on the CPU, as a non-zero status --
 not as a write past a device buffer."""
 import itertools
+import re
 
 import pytest
 
@@ -184,9 +185,9 @@ def test_streamed_batches_fit_the_fixed_scratch_while_their_activation_planes_do
 def test_a_matrix_is_cut_the_same_way_alone_and_beside_others(qtype):
     """Tile and stretches of K decide the order of a result's fp32 sums.  Q8_0 tiles and the streaming kernel take both
     from the matrix and the row count alone, so a call with several matrices gives the bits of separate calls."""
-    def cuts(ns, k, m):
+    def cuts(ns, k, m):   # kernel, tokens a tile, K parts, K stretches (how many rows a workgroup takes may follow the launch)
         lines = [l for l in qproj.plan_mul_mat(qtype, k, ns, m).splitlines() if "gemm_" in l]
-        return [l.replace(" (same launch)", "") for l in lines]
+        return [re.sub(r" x \d+ rows, \d+ tiles", "", l.replace(" (same launch)", "")) for l in lines]
 
     checked = 0
     for k, m in itertools.product([512, 3072, 4096, 8192, 14336], [33, 64, 100, 187, 256, 500, 2048]):
@@ -197,3 +198,10 @@ def test_a_matrix_is_cut_the_same_way_alone_and_beside_others(qtype):
             assert together == sum(alone, []), (k, m, ns)
             checked += 1
     assert checked > 30
+
+
+def test_streamed_launches_that_would_fill_half_the_chip_take_half_the_rows_a_workgroup():
+    for qtype, k, ns, m, rows in [(Q4_K, 4096, (14336,), 48, 64), (Q4_K, 4096, (14336, 14336), 48, 128), (Q6_K, 4096, (14336,), 160, 128),
+                                  (Q6_K, 4096, (14336, 14336), 160, 256), (Q4_K, 4096, (32000,), 96, 128)]:
+        plan = qproj.plan_mul_mat(qtype, k, ns, m)
+        assert plan.count(f"x {rows} rows") == len(ns), plan

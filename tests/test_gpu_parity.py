@@ -7,6 +7,8 @@ from its scalar path in the same way); fp32-activation mode against the fp64 dot
 Both are far inside the stated gate (max relative error 1e-3, max abs 1e-2 where |y| < 1),
 which is asserted as well.
 """
+import re
+
 import numpy as np
 import pytest
 import torch
@@ -390,6 +392,27 @@ def test_streamed_batches_of_33_to_256_rows(ctx, orc, qtype, m, k, ns, tile):
         assert bool((b[m * n:] == 7.0).all())
         assert torch.equal(o, ctx.mul_mat(w, dev(x), ACT_GGML))
         w.free()
+
+
+@pytest.mark.parametrize("qtype,m,k,ns,tile,rows", [
+    (Q4_K, 64, 512, (16600,), "2 token tiles, 2 K parts", 128),     # eight waves: one row group more than a round of halves
+    (Q4_K, 50, 4608, (9001, 8999), "2 token tiles, 2 K parts", 128),  # together eight waves, each matrix alone four
+    (Q4_K, 96, 2304, (16511,), "3 token tiles, 1 K parts", 128),    # four waves, K whole, the scale chunk refilled, a ragged edge
+    (Q4_K, 70, 2304, (33001,), "3 token tiles, 1 K parts", 256),
+    (Q6_K, 64, 512, (16600,), "2 token tiles, 2 K parts", 128),
+    (Q6_K, 50, 4864, (9001, 8999), "2 token tiles, 2 K parts", 128),
+    (Q6_K, 40, 2304, (33001,), "2 token tiles, 1 K parts", 256),
+    (Q6_K, 96, 2304, (16511,), "3 token tiles, 1 K parts", 128),
+    (Q6_K, 70, 2304, (33001,), "3 token tiles, 1 K parts", 256),
+    (Q6_K, 128, 2304, (16511,), "4 token tiles, 1 K parts", 128),
+    (Q6_K, 100, 2304, (33001,), "4 token tiles, 1 K parts", 256),
+])
+def test_streamed_workgroups_of_four_and_eight_waves(ctx, orc, qtype, m, k, ns, tile, rows):
+    """Every instance of the streaming kernel in both workgroup sizes, with K beyond one chunk of scales: the bounds of the
+    test above, and a matrix's bits do not depend on the workgroup size its launch takes."""
+    from magnitude_amd import ACT_GGML, qproj
+    assert re.search(rf"{tile}>: tile \d+ tokens x {rows} rows", qproj.plan_mul_mat(qtype, k, list(ns), m, ACT_GGML))
+    test_streamed_batches_of_33_to_256_rows(ctx, orc, qtype, m, k, ns, tile)
 
 
 @pytest.mark.parametrize("m,k,n", [(1000, 256, 6200), (900, 768, 6200)])
