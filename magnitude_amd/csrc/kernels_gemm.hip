@@ -1072,6 +1072,11 @@ Q4Plan q4k_plan(int64_t K, int64_t M, int64_t N, bool have_scratch, bool add_ok 
 }  // namespace
 
 
+bool q4k_fills_wide(int64_t K, int64_t M, int64_t N) {
+    const Q4Plan p = q4k_plan(K, M, N, true);
+    return p.wide && ((N + 255) / 256) * ((M + 127) / 128) * p.n_split * 8 >= (int64_t)cu_count() * 5;
+}
+
 size_t q4k_tile_scratch_bytes(int64_t K, int64_t M, int64_t N) {
     const Q4Plan p = q4k_plan(K, M, N, true);
     return p.n_split > 1 ? (size_t)p.n_split * M * N * 4 : 0;

@@ -476,6 +476,11 @@ Q6Plan q6k_plan(int64_t K, int64_t M, int64_t N, bool have_scratch) {
 }
 }  // namespace
 
+bool q6k_fills_wide(int64_t K, int64_t M, int64_t N) {
+    const Q6Plan p = q6k_plan(K, M, N, true);
+    return p.wide && (p.n_split == 1 || K >= 12288) && ((N + 255) / 256) * ((M + 127) / 128) * p.n_split * 8 >= (int64_t)cu_count() * 5;
+}
+
 size_t q6k_tile_scratch_bytes(int64_t K, int64_t M, int64_t N) {
     const Q6Plan p = q6k_plan(K, M, N, true);
     return p.n_split > 1 ? (size_t)p.n_split * M * N * 4 : 0;

@@ -525,36 +525,48 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const SumTargets g) {
 struct StreamPlan {
     int jt, kw, n_split;
 };
-int64_t stream_tiles(int64_t M, int64_t N, int jt, int kw) { return ((N + 256 / kw - 1) / (256 / kw)) * ((M + 32 * jt - 1) / (32 * jt)); }
+// token tiles a workgroup of the larger tile shape: as few as cover M in as few workgroups
+int large_token_tiles(int64_t M) { return (int)std::max<int64_t>(2, ((M + 31) / 32 + (M + 127) / 128 - 1) / ((M + 127) / 128)); }
+// workgroups of one stretch of K: tiles, filled up to the same number on each of the 8 XCDs
+int64_t stream_tiles(int64_t M, int64_t N, int jt, int kw) {
+    return ((N + 256 / kw - 1) / (256 / kw) * ((M + 32 * jt - 1) / (32 * jt)) + 7) / 8 * 8;
+}
 
 // One matrix's cut.  It depends on the matrix and the row count alone: a matrix is cut the same way whatever rides
 // along with it, so the results of a call with several matrices are bit for bit those of separate calls.
 StreamPlan stream_plan(int type, int64_t K, int64_t M, int64_t N) {
     StreamPlan p;
-    const int64_t nb = K / 256;
+    const int64_t nb = K / 256, cus = cu_count();
     // Two K parts a workgroup (128 rows x 64 tokens) while that is one round of workgroups; beyond, 256 rows and as few
-    // token tiles as cover M, so that a converted weight serves more tokens.  (Q6_K conversions are dear: long rows of
-    // more than 128 tokens always take the larger tile - 14336 -> 4096 at 192 tokens 53.5 us in 64-token tiles, 44.1 in
-    // 96-token ones, 28672 -> 8192 186.5 against 133.7.)
-    p.jt = 2;
-    p.kw = 2;
-    if (stream_tiles(M, N, 2, 2) > 256 || (type == kTypeQ6_K && M > 128 && K >= 8192)) {
-        p.kw = 1;
-        p.jt = (int)std::max<int64_t>(2, ((M + 31) / 32 + ((M + 127) / 128) - 1) / ((M + 127) / 128));
-    }
+    // token tiles as cover M, so that a converted weight serves more tokens.
+    const int large_jt = large_token_tiles(M);
+    const int64_t small_tiles = stream_tiles(M, N, 2, 2);
+    bool large = small_tiles > cus;
+    // Q6_K conversions are dear: beyond 128 tokens long rows take the larger tile as well (14336 -> 4096 at 192 tokens 53.5 us
+    // in 64-token tiles, 44.1 in 96-token ones, 28672 -> 8192 186.5 against 133.7), unless that means twelve and more
+    // stretches: their partial tiles cost more than they bring (8192 -> 1024 at 160 / 250 tokens 25.3 / 28.6 us, in 64-token tiles
+    // 22.8 / 24.3; 8192 -> 2048 29.1 / 33.3 and 27.5 / 29.3) and lengthen the sums (14336 -> 1024 against 64 bits 1.07e-7 and 8.0e-8).
+    if (type == kTypeQ6_K && M > 128 && K >= 8192)
+        large = large || !(N > 512 && K <= 16384 && stream_tiles(M, N, large_jt, 1) * 12 <= cus);
+    p.jt = large ? large_jt : 2;
+    p.kw = large ? 1 : 2;
     p.jt = tuning_int("QPROJ_STREAM_JT", p.jt);
     p.kw = tuning_int("QPROJ_STREAM_KW", p.kw);
-    // Stretches of K over workgroups, by what usually shares the launch: a matrix with N > K has a sibling of its size
+    // Stretches of K over workgroups, by what usually shares the launch (a matrix has to be cut without knowing it, and
+    // launch_group evens out the workgroups where the guess leaves half the chip idle): a matrix with N > K has a sibling of its size
     // (gate / up) and takes half the chip, a square one (q, o) leaves room for k and v, a down projection or a matrix of
     // long rows takes all of it.  Measured, us, 160 / 256 workgroups: q/k/v of 4096 at 96 tokens 21.5 / 25.6, o 17.4 / 15.9;
     // gate + up 4096 -> 14336 at 64 tokens 27.3 / 38.3; 14336 -> 4096 39.0 / 26.3 at 96 tokens; 8192 x 8192 40.1 / 28.3.
     const bool whole_chip = K > N || K >= 8192 || (K == N && type == kTypeQ6_K);
-    const int64_t wgs = tuning_int("QPROJ_STREAM_WGS", whole_chip ? 256 : K == N ? 160 : 128);
+    const int64_t wgs = tuning_int("QPROJ_STREAM_WGS", whole_chip ? (int)cus : (int)(K == N ? cus * 5 / 8 : cus / 2));
     int64_t n = std::max<int64_t>(1, wgs / stream_tiles(M, N, p.jt, p.kw));
     n = tuning_int("QPROJ_STREAM_SPLIT", (int)n);
     n = std::min<int64_t>(n, std::max<int64_t>(1, nb / (2 * p.kw)));   // two steps a stretch at least
     // never more partial tiles than the allocation-free entry point has room for beside the activation planes
     n = std::min<int64_t>(n, std::max<int64_t>(1, (int64_t)(q8k_scratch_room(M, K) / ((size_t)M * N * 4))));
+    // (a cut in two of short rows leaves no room for k and v in the round: 2560 -> 2560 / 1024 / 1024 at 250 tokens 34.9 -> 25.5
+    // us with it whole, 3072 -> 3072 / 1024 / 1024 at 192 31.0 -> 27.9)
+    if (K == N && n == 2 && nb < 14 && stream_tiles(M, N, p.jt, p.kw) * 4 > cus) n = 1;
     const auto steps = [&](int64_t parts) { return ((nb + parts - 1) / parts + p.kw - 1) / p.kw; };
     while (n > 1 && steps(n - 1) == steps(n)) --n;   // no more stretches than it takes
     if ((M * N) % 4 != 0) n = 1;
@@ -576,12 +588,24 @@ hipError_t launch_stream_kernel(const StreamArgs &g, int wgs, hipStream_t s) {
 
 // Which products the streaming kernel takes.  From 33 tokens (below, the small-batch kernel) to 256; of the grids beyond
 // one round of workgroups Q4_K keeps the older tiles from 97 tokens on, where arithmetic and not latency is the limit
-// (4096 -> 32000 at 128 tokens 51.0 us there, 54.0 here; at 96 tokens 50.1 against 45.3).
+// (4096 -> 32000 at 128 tokens 51.0 us there, 54.0 here; at 96 tokens 50.1 against 45.3).  The 128-token kernels
+// keep the grids they fill (q4k_fills_wide, q6k_fills_wide) where they are as fast or faster, us there / here: Q4_K beyond
+// 128 tokens (28672 -> 8192 at 192 / 256 tokens 147 / 159, 151 / 166) and from 65 on for very long rows (28672 -> 16384 at 112
+// tokens 155 / 165); Q6_K where the tokens fill 128-token tiles (8192 -> 2 x 28672 at 256 tokens 334 / 346, 4096 -> 32000
+// 91.5 / 96.1) and from 65 on for long rows (12288 x 12288 at 96 tokens 79 / 88, 16384 x 16384 109 / 124).  At 129..192 tokens
+// Q6_K has tiles of 96 here: 4096 -> 32000 at 160 tokens 91.7 / 83.
 bool stream_takes(int type, int64_t K, int64_t M, int64_t N) {
     const int lo = tuning_int("QPROJ_STREAM_MIN_M", 33), hi = tuning_int("QPROJ_STREAM_MAX_M", 256);
     if ((type != kTypeQ4_K && type != kTypeQ6_K) || K % 256 != 0 || K > (1 << 22) || M < lo || M > hi) return false;
     if (N > (1 << 24)) return false;   // row and tile numbers are ints, a tile's outputs are indexed with 32 bits: 127 * N + 31 at most
-    return type == kTypeQ6_K || M <= 96 || stream_tiles(M, N, 2, 2) <= 256;
+    if (type == kTypeQ6_K) {
+        const int jt = large_token_tiles(M);
+        // half a round of 128-token tiles and, with more than four times K rows (an output head), nothing that rides along
+        const bool alone = M <= 128 && jt == 4 && N > 4 * K && stream_tiles(M, N, 4, 1) * 2 <= cu_count() && stream_tiles(M, N, 2, 2) > cu_count();
+        return !alone && !((jt == 4 || (jt == 3 && M <= 96 && K >= 12288)) && q6k_fills_wide(K, M, N));
+    }
+    if ((M > 128 || (M > 64 && K >= 16384)) && q4k_fills_wide(K, M, N)) return false;
+    return M <= 96 || stream_tiles(M, N, 2, 2) <= cu_count();
 }
 
 namespace {

@@ -258,6 +258,8 @@ inline void add_sum(SumTargets &g, const float *part, float *y, int n_split, int
 hipError_t launch_sum_parts(const SumTargets &g, hipStream_t s);
 // 33..256 rows of Q4_K / Q6_K weights: all matrices of a call in one launch, K cut per matrix
 bool stream_takes(int type, int64_t K, int64_t M, int64_t N);
+bool q4k_fills_wide(int64_t K, int64_t M, int64_t N);   // the tiled route takes its 128-token kernel, and fills the chip with it
+bool q6k_fills_wide(int64_t K, int64_t M, int64_t N);
 size_t stream_scratch_bytes(int type, int64_t K, int64_t M, int n, const int64_t *N);   // for the n matrices of a call
 size_t q8k_scratch_room(int64_t M, int64_t K);   // bytes of the allocation-free entry point's buffer beside M x K Q8_K planes
 hipError_t launch_gemm_stream(int n, const WeightView *w, const ActView &a, int64_t M, float *const *y, const Scratch &scratch,

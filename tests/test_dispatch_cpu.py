@@ -149,7 +149,7 @@ def test_q8_0_matrices_share_a_launch_only_while_their_partial_results_have_room
     assert qproj.plan_mul_mat(Q8_0, k // 2, ns, 256).count("(same launch)") == 3
 
 
-@pytest.mark.parametrize("qtype,m", [(Q4_K, 64), (Q6_K, 48), (Q6_K, 128), (Q6_K, 256)])
+@pytest.mark.parametrize("qtype,m", [(Q4_K, 64), (Q6_K, 48), (Q6_K, 96), (Q6_K, 192)])
 def test_outputs_beyond_32_bit_indices_stay_on_the_kernels_with_64_bit_ones(qtype, m):
     """The streaming kernel indexes a tile's outputs with 32 bits (127 rows * N + 31 at most): matrices beyond 2^24 rows
     take the tiled kernels, whose output index has 64."""
@@ -195,7 +195,7 @@ def test_a_matrix_is_cut_the_same_way_alone_and_beside_others(qtype):
             together, alone = cuts(ns, k, m), [cuts((n,), k, m) for n in ns]
             if qtype != Q8_0 and any("gemm_stream_kernel" not in a[0] for a in alone):
                 continue
-            assert together == sum(alone, []), (k, m, ns)
+            assert sorted(together) == sorted(sum(alone, [])), (k, m, ns)
             checked += 1
     assert checked > 30
 

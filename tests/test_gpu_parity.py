@@ -404,7 +404,7 @@ def test_streamed_batches_of_33_to_256_rows(ctx, orc, qtype, m, k, ns, tile):
     (Q6_K, 40, 2304, (33001,), "2 token tiles, 1 K parts", 256),
     (Q6_K, 96, 2304, (16511,), "3 token tiles, 1 K parts", 128),
     (Q6_K, 70, 2304, (33001,), "3 token tiles, 1 K parts", 256),
-    (Q6_K, 128, 2304, (16511,), "4 token tiles, 1 K parts", 128),
+    (Q6_K, 128, 4352, (16511,), "4 token tiles, 1 K parts", 128),
     (Q6_K, 100, 2304, (33001,), "4 token tiles, 1 K parts", 256),
 ])
 def test_streamed_workgroups_of_four_and_eight_waves(ctx, orc, qtype, m, k, ns, tile, rows):

@@ -121,7 +121,7 @@ def test_noalloc_scratch_belongs_to_one_context_at_a_time(ctx):
     w.free()
 
 
-@pytest.mark.parametrize("qtype,k,ns,m", [(Q6_K, 8192, (2048, 1024, 1024), 256), (Q6_K, 8192, (1024, 1024, 2048, 77), 250)])
+@pytest.mark.parametrize("qtype,k,ns,m", [(Q6_K, 8192, (4096, 4096), 256), (Q6_K, 8192, (77, 4096, 4096), 250)])
 def test_noalloc_streams_matrices_one_after_the_other_where_their_partial_tiles_do_not_fit_together(ctx, qtype, k, ns, m):
     """The partial tiles of all matrices are 67 MB, the room beside the activation planes is 61.8 MiB: they go in two
     launches through the same bytes.  Bar: the call is served and every matrix has the bits of a call of its own."""
