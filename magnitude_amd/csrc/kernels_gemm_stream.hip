@@ -197,17 +197,23 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_stream_kernel(const StreamArg
         }
     };
     const uint8_t *msbase = nullptr;
-    uint32_t msoff = 0;
     if constexpr (kQ4) {
         static_assert(KW * JT <= NW, "a wave requests one tile of the min-term plane at most");
         msbase = scalar_pointer(reinterpret_cast<const uint8_t *>(g.a.msum) + (int64_t)m0 * nb * 32);
-        msoff = (uint32_t)(min((wave % JT) * 32 + (lane >> 1), mcap) * nb * 32 + 16 * (lane & 1));
     }
+    // (three token tiles: worked out at every request from the lane counter.  Kept in a register it was spilled, and the wait
+    // for its reload was one for everything outstanding; 4096 -> 40960 at 96 rows 66.6 -> 64.6 us)
+    auto ms_offset = [&]() {
+        int zero = 0;
+        if constexpr (JT >= 3) asm volatile("" : "+v"(zero));
+        const int l = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
+        return (uint32_t)(min((wave % JT) * 32 + (l >> 1), mcap) * nb * 32 + 16 * (l & 1));
+    };
     auto request_ms = [&](int s) {
         if constexpr (kQ4) {
             if (wave < KW * JT) {
                 const uint32_t sb = (uint32_t)min(sb_begin + s * KW + wave / JT, sb_end - 1);
-                global_to_lds16(msbase + (msoff + sb * 32u), smem + L::kOffMs + ((s & 1) * KW + wave / JT) * L::kMs + (wave % JT) * 1024);
+                global_to_lds16(msbase + (ms_offset() + sb * 32u), smem + L::kOffMs + ((s & 1) * KW + wave / JT) * L::kMs + (wave % JT) * 1024);
             }
         }
     };
@@ -326,14 +332,9 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_stream_kernel(const StreamArg
             }
         };
         if constexpr (JT >= 4) {   // tile by tile: both chains of four tiles do not fit the registers
-            min_convert();
+            static_assert(!kQ4, "Q4_K takes three token tiles at most");
 #pragma unroll
             for (int p = 0; p < 8; ++p) convert(p);
-#pragma unroll
-            for (int j = 0; j < JT; ++j) {
-                min_multiply(j, 0);
-                min_add(j, 0);
-            }
         } else {
             // Pinned step by step: the activation fragments of two products are in flight, the next product's weights
             // are converted between the matrix instructions of this one.
