@@ -1097,6 +1097,18 @@ hipError_t launch_gemv_mfma(const GemvArgs &args, const Scratch &scratch, hipStr
     return launch_typed<kDense>(g, args.t[0].w.type, args.M <= 8 ? 1 : args.M <= 16 ? 2 : 4, W, s);
 }
 
+// few pairs an expert: 8 staged rows a pass are enough
+// more than 16 pairs an expert (prompt-sized batches): 32 staged rows a pass halve the passes over an expert's
+// weights (Q4_K experts whose K fits LDS beside 32 rows; eight waves, one workgroup a compute unit)
+// (only with K in one part a wave: the partial tiles of K parts, 32 rows x 32 x two tensors, would not fit a wave's region)
+int mfma_grouped_pass_rows(int type, int64_t K, int64_t N, int64_t E, int64_t n_pairs) {
+    static const bool no_wide_pass = tuning_int("QPROJ_MOE_NO_32_ROW_PASS", 0) != 0;
+    if (n_pairs <= 4 * E) return 8;
+    const bool wide = !no_wide_pass && type == kTypeQ4_K && K / 256 <= kMaxSb16 / 2 && n_pairs > 16 * E &&
+                      plan(K, 32, std::min<int64_t>(E, n_pairs) * ((N + 31) / 32), 8).kw == 1;
+    return wide ? 32 : 16;
+}
+
 // Expert-grouped form: args.order / args.offsets list each expert's pairs; `swiglu` takes tensors 0 and 1
 // as gate and up.  n_pairs only steers the launch shape (how many experts can be busy at once).
 hipError_t launch_gemv_mfma_grouped(const GemvArgs &args, int64_t n_pairs, bool swiglu, hipStream_t s, const Scratch &scratch) {
@@ -1116,13 +1128,8 @@ hipError_t launch_gemv_mfma_grouped(const GemvArgs &args, int64_t n_pairs, bool 
     // 128-expert FFN against eight waves: 23.2 -> 21.1 us at one token, 121.9 -> 115.5 us at 64.
     static const int moe_waves = tuning_int("QPROJ_MOE_WAVES", 4);
     const int64_t rg_e = (w.N + 31) / 32;
-    const bool small = n_pairs <= 4 * w.E;   // few pairs an expert: 8 staged rows a pass are enough
-    // more than 16 pairs an expert (prompt-sized batches): 32 staged rows a pass halve the passes over an expert's
-    // weights (Q4_K experts whose K fits LDS beside 32 rows; eight waves, one workgroup a compute unit)
-    static const bool no_wide_pass = tuning_int("QPROJ_MOE_NO_32_ROW_PASS", 0) != 0;
-    bool wide_pass = !no_wide_pass && !args.ids && type == kTypeQ4_K && w.K / 256 <= kMaxSb16 / 2 && n_pairs > 16 * w.E;
-    // (only with K in one part a wave: the partial tiles of K parts, 32 rows x 32 x two tensors, would not fit a wave's region)
-    if (wide_pass && plan(w.K, 32, std::min<int64_t>(w.E, n_pairs) * rg_e, 8).kw != 1) wide_pass = false;
+    const int pass_rows = mfma_grouped_pass_rows(type, w.K, w.N, w.E, n_pairs);
+    const bool small = pass_rows == 8, wide_pass = !args.ids && pass_rows == 32;
     const int W = wide_pass ? 8 : type == kTypeQ4_K && (moe_waves == 4 || moe_waves == 8) ? moe_waves : waves_per_wg(type);
     Split p = plan(w.K, small ? 8 : wide_pass ? 32 : 16, std::min<int64_t>(w.E, n_pairs) * rg_e, W);
     const int nb = (int)(w.K / 256);

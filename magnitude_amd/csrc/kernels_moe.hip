@@ -9,7 +9,7 @@ namespace qproj {
 
 // Counting sort of (token, slot) pairs by expert id, one workgroup.  offsets[e]..offsets[e+1]
 // indexes the pairs of expert e inside order[]; active[0..active[n_expert]) lists the experts that
-// have pairs (those with more than pass_rows pairs first: launch_moe_group, ascending within both parts).  Ids outside [0, n_expert) raise *error_flag and
+// have pairs (those with more than heavy_above pairs first: launch_moe_group, ascending within both parts).  Ids outside [0, n_expert) raise *error_flag and
 // their pairs are left out (their outputs are not written).  Pairs of one expert keep ascending
 // pair order so repeated runs produce the same launch geometry.  Each of the 16 waves takes every
 // 16th expert and sweeps the pair list 64 ids at a time (consecutive lanes on consecutive ids):
@@ -22,7 +22,7 @@ constexpr int kGroupLdsIds = 8192;   // pair ids staged in LDS up to this many, 
 // cnt[e] = pairs of expert e on entry; on exit cnt[e] = offsets[e] = its first slot, active[] lists the
 // experts that have pairs.  All threads of the workgroup call it; the caller synchronizes afterwards.
 __device__ __forceinline__ void group_scan(int n_expert, int32_t *cnt, int32_t *wsum, int32_t *__restrict__ offsets,
-                                           int32_t *__restrict__ active, int pass_rows) {
+                                           int32_t *__restrict__ active, int heavy_above) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // exclusive scans over the workgroup (shuffles inside a wave, wave totals through LDS) of the pair
     // counts (-> offsets) and of the non-empty flags (-> compact list of the experts that have work);
@@ -44,7 +44,7 @@ __device__ __forceinline__ void group_scan(int n_expert, int32_t *cnt, int32_t *
     // neighbouring experts.)
     int local_h = 0;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) local_h += pass_rows > 0 && tot[i] > pass_rows;
+    for (int i = 0; i < 8; ++i) local_h += heavy_above > 0 && tot[i] > heavy_above;
     int incl = local, incl_f = local_f, incl_h = local_h;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -78,7 +78,7 @@ __device__ __forceinline__ void group_scan(int n_expert, int32_t *cnt, int32_t *
             offsets[e] = before;
             before += tot[i];
             if (tot[i] > 0) {
-                const bool heavy = pass_rows > 0 && tot[i] > pass_rows;
+                const bool heavy = heavy_above > 0 && tot[i] > heavy_above;
                 const int pos = heavy ? before_h : n_heavy + (before_f - before_h);
                 active[pos] = e;
                 reinterpret_cast<int4 *>(active + active_slots_offset(n_expert))[pos] = make_int4(e, before - tot[i], tot[i], 0);
@@ -96,7 +96,7 @@ __device__ __forceinline__ void group_scan(int n_expert, int32_t *cnt, int32_t *
 template <bool STAGED>
 __device__ __forceinline__ void group_sweeps(const int32_t *__restrict__ ids, const int32_t *sid, int n_pairs, int n_expert,
                                              int32_t *cnt, int32_t *wsum, int32_t *__restrict__ order,
-                                             int32_t *__restrict__ offsets, int32_t *__restrict__ active, int pass_rows) {
+                                             int32_t *__restrict__ offsets, int32_t *__restrict__ active, int heavy_above) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     constexpr int kWaves = kGroupThreads / 64;
     auto id_at = [&](int p) { return p < n_pairs ? (STAGED ? sid[p] : ids[p]) : -1; };
@@ -116,7 +116,7 @@ __device__ __forceinline__ void group_sweeps(const int32_t *__restrict__ ids, co
         }
     }
     __syncthreads();
-    group_scan(n_expert, cnt, wsum, offsets, active, pass_rows);
+    group_scan(n_expert, cnt, wsum, offsets, active, heavy_above);
     __syncthreads();
     // sweep 2: placement, ascending pair order inside every expert (cnt[e] = the expert's next free slot)
     for (int base = 0; base < n_pairs; base += 64 * kHeld) {
@@ -152,7 +152,7 @@ __global__ __launch_bounds__(kGroupThreads) void moe_group_kernel(const int32_t 
                                                                   int32_t *__restrict__ offsets,
                                                                   int32_t *__restrict__ active,
                                                                   int32_t *__restrict__ error_flag, int by_block,
-                                                                  int pass_rows, const RowQuantJob job) {
+                                                                  int heavy_above, const RowQuantJob job) {
     // Workgroups past the first have nothing to do with the grouping: they quantize the activation rows the
     // grouped projection is going to read (one 256-wide chunk a wave, ggml's quantize_row_q8_K as in the
     // standalone quantizer), so that the two passes, which depend only on the call's inputs, share a launch.
@@ -181,8 +181,8 @@ __global__ __launch_bounds__(kGroupThreads) void moe_group_kernel(const int32_t 
         for (int e = tid; e < n_expert; e += kGroupThreads) cnt[e] = 0;
         if (bad) atomicOr(error_flag, 1);
         __syncthreads();
-        if (staged) group_sweeps<true>(ids, tab, n_pairs, n_expert, cnt, wsum, order, offsets, active, pass_rows);
-        else group_sweeps<false>(ids, tab, n_pairs, n_expert, cnt, wsum, order, offsets, active, pass_rows);
+        if (staged) group_sweeps<true>(ids, tab, n_pairs, n_expert, cnt, wsum, order, offsets, active, heavy_above);
+        else group_sweeps<false>(ids, tab, n_pairs, n_expert, cnt, wsum, order, offsets, active, heavy_above);
         return;
     }
     const int n_blocks = (n_pairs + 63) / 64;
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(kGroupThreads) void moe_group_kernel(const int32_t 
         cnt[e] = run;
     }
     __syncthreads();
-    group_scan(n_expert, cnt, wsum, offsets, active, pass_rows);
+    group_scan(n_expert, cnt, wsum, offsets, active, heavy_above);
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < kBlocksPerWave; ++i) {
@@ -244,15 +244,22 @@ __global__ __launch_bounds__(kGroupThreads) void moe_group_kernel(const int32_t 
 }
 
 hipError_t launch_moe_group(const int32_t *ids, int64_t n_pairs, int64_t n_expert, int32_t *order,
-                            int32_t *offsets, int32_t *active, int32_t *error_flag, const RowQuantJob *quantize,
-                            hipStream_t s) {
+                            int32_t *offsets, int32_t *active, int32_t *error_flag, int64_t pass_rows,
+                            const RowQuantJob *quantize, hipStream_t s) {
     if (n_expert > 8192 || n_pairs > 0x7fffffff) return hipErrorInvalidValue;
     const size_t table = (size_t)((n_pairs + 63) / 64) * (size_t)n_expert;
     const bool by_block = n_pairs <= 64 * 16 * kBlocksPerWave && table <= 24 * 1024;   // at most 96 KB of LDS
     const size_t lds = ((size_t)n_expert + 48 + (by_block ? table : n_pairs <= kGroupLdsIds ? (size_t)n_pairs : 0)) * sizeof(int32_t);
+    // Which experts start first: those that need a pass over their weights more than the average one.  `pass_rows`: rows a
+    // pass of the grouped kernel behind this stages (mfma_grouped_pass_rows); the line is the multiple of that below the
+    // average, or above it from three eighths of a pass on, where nearly every expert would be beyond the one below (at 31 pairs
+    // an expert and 32 rows those with more than 32 take two passes; with the line at 16 nothing was ordered there and the
+    // launches waited for two-pass experts begun last: 500 tokens, 128 experts, top-8 of 2048 x 768 234 -> 207 us; 16 rows, line
+    // below / above the average: 22 pairs 257 / 229, 50 pairs 375 / 406, 19 pairs 299 / 324, 87 pairs 474 / 452).
+    const int64_t heavy = pass_rows * std::max<int64_t>(1, (n_pairs / n_expert + pass_rows * 5 / 8) / pass_rows);
     if (dry_run()) {
-        plan_note("moe_group_kernel: %lld pairs over %lld experts (%s)%s", (long long)n_pairs, (long long)n_expert,
-                  by_block ? "ballot per bit of the id, prefix over 64-pair blocks" : "ballot sweeps per expert",
+        plan_note("moe_group_kernel: %lld pairs over %lld experts (%s), those with more than %lld first%s", (long long)n_pairs, (long long)n_expert,
+                  by_block ? "ballot per bit of the id, prefix over 64-pair blocks" : "ballot sweeps per expert", (long long)heavy,
                   quantize ? ", spare workgroups quantize the token rows" : "");
         return hipSuccess;
     }
@@ -267,12 +274,6 @@ hipError_t launch_moe_group(const int32_t *ids, int64_t n_pairs, int64_t n_exper
     if (quantize) job = *quantize;
     const int64_t extra = (job.n_super + kGroupThreads / 64 - 1) / (kGroupThreads / 64);
     if (extra >= 0x7fffffff) return hipErrorInvalidValue;
-    // Which experts start first: those that need a pass over their weights more than the average one.  A pass of the
-    // grouped matrix-core kernel stages 8, 16 or 32 rows, so the line is the multiple of that nearest the average (at 31
-    // pairs an expert those with more than 32 take two passes; with the line at 16 nothing was ordered there and the
-    // launches waited for two-pass experts begun last: 500 tokens, 128 experts, top-8 234 -> 207 us).
-    const int64_t pass = n_pairs <= 4 * n_expert ? 8 : n_pairs <= 16 * n_expert ? 16 : 32;
-    const int64_t heavy = pass * std::max<int64_t>(1, (n_pairs / n_expert + pass / 2) / pass);
     hipLaunchKernelGGL(moe_group_kernel, dim3((unsigned)(1 + extra)), dim3(kGroupThreads), lds, s, ids, (int)n_pairs,
                        (int)n_expert, order, offsets, active, error_flag, by_block ? 1 : 0,
                        (int)heavy, job);

@@ -1407,7 +1407,7 @@ int qproj_mul_mat_id(qproj_ctx *ctx, const qproj_weight *w, const float *x_dev, 
     if (!fuse && !joined) QP_HIP(ctx, run_quantize(ctx, p, wsp.base, x_dev, rows, K, false));
     if (!pair_mode)
         QP_HIP(ctx, launch_moe_group(ids_dev, n_pairs, w->E, order, offsets, active, ctx->flag_dev,
-                                     joined ? &job : nullptr, ctx->stream));
+                                     mfma_grouped_pass_rows(w->type, K, w->N, w->E, n_pairs), joined ? &job : nullptr, ctx->stream));
     GemvArgs g{};
     g.n_targets = 1;
     g.t[0].w = w->view;
@@ -1519,8 +1519,9 @@ int qproj_moe_ffn(qproj_ctx *ctx, const qproj_weight *gate, const qproj_weight *
     const RowQuantJob job = quantize_job(px, ws, x_dev, B, d_model);
     if (!fuse_x && !joined) QP_HIP(ctx, run_quantize(ctx, px, ws, x_dev, B, d_model, false));
     if (!pair_mode)
+        // (the order suits the passes of gate and up, two thirds of the work)
         QP_HIP(ctx, launch_moe_group(ids_dev, n_pairs, E, order, offsets, active, ctx->flag_dev,
-                                     joined ? &job : nullptr, ctx->stream));
+                                     mfma_grouped_pass_rows(gate->type, d_model, d_ff, E, n_pairs), joined ? &job : nullptr, ctx->stream));
     GemvArgs g{};
     if (pair_mode) {
         g.ids = ids_dev;

@@ -201,9 +201,12 @@ struct RowQuantJob {
     float *d;
     int16_t *bsums;
 };
+// pass_rows: mfma_grouped_pass_rows of the launch behind it
 hipError_t launch_moe_group(const int32_t *ids, int64_t n_pairs, int64_t n_expert, int32_t *order,
-                            int32_t *offsets, int32_t *active, int32_t *error_flag, const RowQuantJob *quantize,
-                            hipStream_t s);
+                            int32_t *offsets, int32_t *active, int32_t *error_flag, int64_t pass_rows,
+                            const RowQuantJob *quantize, hipStream_t s);
+// rows of an expert's pairs that a pass of the grouped matrix-core kernel stages (8, 16 or 32)
+int mfma_grouped_pass_rows(int type, int64_t K, int64_t N, int64_t E, int64_t n_pairs);
 hipError_t launch_moe_swiglu_gemv(const GemvArgs &gate_up, int mt, int n_experts_grid, hipStream_t s);
 // One or two decode tokens (at most 16 pairs) through expert stacks of Q4_K / Q6_K rows of K <= 4096 on the vector
 // ALU: args as for the pair mode of the grouped kernel (t[0], and t[1] = up when `swiglu`; x fp32 rows, x_div, ids,

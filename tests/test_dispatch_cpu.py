@@ -205,3 +205,13 @@ def test_streamed_launches_that_would_fill_half_the_chip_take_half_the_rows_a_wo
                                   (Q6_K, 4096, (14336, 14336), 160, 256), (Q4_K, 4096, (32000,), 96, 128)]:
         plan = qproj.plan_mul_mat(qtype, k, ns, m)
         assert plan.count(f"x {rows} rows") == len(ns), plan
+
+
+@pytest.mark.parametrize("qtype,d,tokens,first", [(Q4_K, 2048, 500, 32), (Q4_K, 2048, 640, 32), (Q4_K, 2048, 1000, 64), (Q4_K, 4096, 640, 48),
+                                                  (Q6_K, 2048, 640, 48), (Q6_K, 2048, 360, 32), (Q6_K, 2048, 300, 16), (Q4_K, 2048, 64, 8),
+                                                  (Q4_K, 2048, 160, 16)])
+def test_experts_that_start_first_are_those_with_a_pass_more_than_the_average(qtype, d, tokens, first):
+    """The line is a multiple of the rows a pass of the grouped launch stages: 32 only for Q4_K experts of up to 2048 weights
+    a row with more than 16 pairs on average, 16 for the others, 8 up to four pairs."""
+    plan = qproj.plan_moe_ffn(qtype, qtype, d, 768, 128, 8, tokens)
+    assert f"those with more than {first} first" in plan, plan
