@@ -112,7 +112,20 @@ def routing_table() -> str:
         dense("config 4 (ggml activations) config 1's matrix", Q8_0, 4096, (4096,), m)
     for name, qt, k, ns in layer:
         dense(f"prompt batch of the engine (512 tokens) {name}", qt, k, ns, 512)
-    for b in (1, 8, 64):
+    # batches of 33..256 rows: streamed K-quants (one matrix alone, both workgroup sizes), shared Q8_0 launches
+    for m in (48, 96, 128, 187, 256):
+        for name, qt, k, ns in layer:
+            dense(f"serving batch {name}", qt, k, ns, m)
+    for m in (48, 187, 256):
+        dense("serving batch gate alone", Q4_K, 4096, (14336,), m)
+        dense("serving batch, Q6_K q/k/v", Q6_K, 4096, (4096, 1024, 1024), m)
+        dense("serving batch, Q6_K gate/up", Q6_K, 4096, (14336, 14336), m)
+        dense("serving batch, output head", Q6_K, 4096, (32000,), m)
+        dense("serving batch, long rows", Q6_K, 8192, (8192, 1024, 1024), m)
+        dense("serving batch, long rows", Q4_K, 28672, (8192,), m)
+        for name, k, ns in (("q/k/v", 3072, (3072, 1024, 1024)), ("o", 3072, (3072,)), ("gate/up", 3072, (8192, 8192)), ("down", 8192, (3072,))):
+            dense(f"serving batch, Q8_0 {name}", Q8_0, k, ns, m)
+    for b in (1, 8, 64, 500):
         out.append(f"## config 5: 128 experts, top-8, d_model 2048, d_ff 768, Q4_K, B={b}")
         out.append(qproj.plan_moe_ffn(Q4_K, Q4_K, 2048, 768, 128, 8, b).rstrip())
     return "\n".join(out) + "\n"
