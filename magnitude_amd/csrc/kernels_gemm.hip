@@ -1029,6 +1029,9 @@ int per32_splits(int type, int64_t K, int64_t M, int64_t N) {
     // four -> two, us: 4096 -> 1024 at 64 tokens 21.2 -> 16.8, 2560 x 2560 at 250 27.2 -> 22.5, 4096 x 4096 at 100 24.5 -> 22.4.
     const int least = type == kTypeQ8_0 ? 2 : 4;
     while (n > 1 && K / 256 < least * n) --n;
+    // no stretch without work: 12 times 256 weights in five stretches of three leave the fifth empty (the same sums with four)
+    const int64_t units = (K + 255) / 256;
+    while (n > 1 && (units + n - 2) / (n - 1) == (units + n - 1) / n) --n;
     return n;
 }
 size_t per32_scratch_bytes(int type, int64_t K, int64_t M, int64_t N) {

@@ -228,3 +228,10 @@ def test_experts_that_start_first_are_those_with_a_pass_more_than_the_average(qt
     a row with more than 16 pairs on average, 16 for the others, 8 up to four pairs."""
     plan = qproj.plan_moe_ffn(qtype, qtype, d, 768, 128, 8, tokens)
     assert f"those with more than {first} first" in plan, plan
+
+
+def test_no_q8_0_stretch_of_k_is_empty():
+    for k, n, m in itertools.product(range(512, 6144, 128), (1024, 3072, 8192), (64, 187, 500)):
+        line = [l for l in qproj.plan_mul_mat(Q8_0, k, (n,), m).splitlines() if "gemm_per32_kernel" in l][0]
+        stretches, units = int(re.search(r"x (\d+) K stretches", line)[1]), (k + 255) // 256
+        assert (stretches - 1) * -(-units // stretches) < units, (k, n, m, line)
