@@ -653,11 +653,11 @@ def main():
                           # What bounds this format (not the matrix cores): both operands change scale every 32 weights, so
                           # an int32 result is good for ONE matrix instruction and each of its 16 outputs a lane costs
                           # two fmas on the vector ALU (the sum arrives as float bits): 32 vector instructions behind every
-                          # 32 x 32 x 32 product, 42.5 with addresses, staging and scales (85 a pair of products).  With a matrix
-                          # instruction holding the issue port 16 of its 32 cycles and a vector instruction 4, the floor is
-                          # 5000 TOPS x 32 / (16 + 4 x 42.5) = 860 TOPS.
-                          "bound": "valu", "floor_tops": 860.0,
-                          "floor": "5000 x 32 / (16 + 4 x 42.5): 32 of 42.5 vector instr. per matrix instr. are the per-32 flush",
+                          # 32 x 32 x 32 product.  With a matrix instruction holding the issue port 16 of its 32 cycles and a vector
+                          # instruction 4, the format's bound is 5000 TOPS x 32 / (16 + 4 x 32) = 1111 TOPS.  (The kernel issues 41
+                          # a product, and the clock sinks under this load: profiles/prefill_gemm_kernels.txt, section 6.)
+                          "bound": "valu", "floor_tops": 1111.0,
+                          "floor": "5000 x 32 / (16 + 4 x 32): the per-32 flush is 32 vector instr. behind every matrix instr.",
                           "peak_tops": INT8_PEAK_TOPS, "shapes": res}
         # the same shapes in the ggml activation format (Q8_K, one scale per 256): the reference's own arithmetic
         # (plus the layer's Q6_K down projection, which a Q4_K_M model runs through the same operator, and

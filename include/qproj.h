@@ -119,7 +119,7 @@ int qproj_dequantize(qproj_ctx *ctx, const qproj_weight *w, float *out_dev);
  * 256 for Q8_K and Q8X32 (both carry one msum record per 256 weights of a row); qproj_act_bytes returns 0 and
  * qproj_quantize_activations QPROJ_ERR_INVALID_ARG otherwise.  Activations may have any finite size; the weight
  * side of the same term is carried as fp16 pairs of dmin * min, which wants dmin * 63 < 65504 (GGUF files are
- * orders of magnitude inside that). */
+ * orders of magnitude inside that); block scales have to be finite (with an infinite one the per-32 format answers NaN). */
 size_t qproj_act_bytes(int kind, int wtype, int64_t M, int64_t K);
 int qproj_quantize_activations(qproj_ctx *ctx, int kind, int wtype, const float *x_dev, int64_t M,
                                int64_t K, void *out_dev);
@@ -174,7 +174,7 @@ int qproj_ffn(qproj_ctx *ctx, const qproj_weight *gate, const qproj_weight *up, 
               const float *x_dev, const float *gamma_dev, float eps, int use_norm, int64_t M, float *y_dev, int act);
 
 /* GGML_OP_MUL_MAT: y_dev[M][N] = x_dev[M][K] . W^T.  Picks the decode (M=1), small-batch
- * (M<=16) or prefill kernel from M.  W must have n_expert == 1. */
+ * (M<=32) or a matrix-core kernel from M (qproj_plan_mul_mat names it).  W must have n_expert == 1. */
 int qproj_mul_mat(qproj_ctx *ctx, const qproj_weight *w, const float *x_dev, int64_t M, float *y_dev,
                   int act);
 

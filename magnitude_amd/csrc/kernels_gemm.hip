@@ -7,8 +7,8 @@
 // sub-tile = two v_mfma_i32_32x32x32_i8 products per 32-wide sub-block.  Both operands change
 // scale every 32 K-elements, so an int32 accumulator is meaningful for ONE product only: each
 // product is folded into the fp32 accumulators right away.  That fp32 work, not the matrix cores,
-// bounds this kernel (the vector ALU issues in 91 % of its cycles; at this load the clock sinks to
-// 1.8 - 2.05 GHz), so everything else is kept off the vector ALU:
+// bounds this kernel (the vector ALU issues in 94 % of its cycles; at this load the clock sinks to
+// 1.8 GHz), so everything else is kept off the vector ALU:
 //   - two instructions an output and block instead of three (see `product`);
 //   - activations go from global memory straight into LDS, addresses are one register an operand
 //     and immediate offsets, the four sub-blocks of a K-step are unrolled;
@@ -18,7 +18,7 @@
 //   - LDS holds only the two int8 operand tiles and the transposed scales, double buffered over
 //     K-steps of 128 so that the global loads of step s+1 overlap step s.
 // Measured, three instructions and operands through registers -> this, same card in turn:
-// 4096 x 4096 against 14336 rows 783 -> 684 us (614 -> 703 TOPS), vector instructions 105 -> 85 a pair of products.
+// 4096 x 4096 against 14336 rows 783 -> 684 us (614 -> 703 TOPS), 61.5 -> 41.2 vector instructions beside a product.
 #include <cstdlib>
 #include <type_traits>
 #include "gemm_convert.h"
@@ -67,7 +67,7 @@ constexpr float kMagic = 12582912.f;   // 1.5 * 2^23: one integer step is one st
 // out[stretch][M][N] and an adding pass puts the stretches together in order.  The matrices of a call (q/k/v, gate/up)
 // share a launch: at 33 .. 256 tokens one of them alone leaves most of the chip's 512 places (two workgroups a compute
 // unit) empty, and every launch pays the latency of its K loop again.  Four layers of 3072 / 1024 / 8192 Q8_0 weights
-// at 187 tokens, a launch and an adding pass a matrix -> this: 828 -> 565 us.
+// at 187 tokens, a launch and an adding pass a matrix -> this: 828 -> 564 .. 579 us.
 struct Per32Target {
     WeightView w;
     float *out;   // the output, or [n_split][M][N] partial tiles
@@ -979,6 +979,7 @@ hipError_t launch_sum_parts(const float *part, int n_split, size_t n, float *y, 
     return launch_sum_parts(g, s);
 }
 
+// (The figures at 33 .. 256 tokens below were taken when those batches came here; most of them stream now, stream_takes.)
 // K stretches for the kernels that take ggml-format activations (64-token x 128-row tiles, two workgroups per
 // compute unit = 512 places): below 384 tiles K is cut in 2, below 192 in 3, below 96 in 4, below 64 in 8, never under twelve super-blocks a
 // stretch (K = 4096 cut in two measured slower than whole: the pass that adds the partial tiles costs more

@@ -448,6 +448,8 @@ struct Q6Plan {
     bool wide;
     int n_split;
 };
+// (The figures at up to 256 tokens below and in launch_gemm_q6k_q8k were taken when those batches came here; most of them
+// stream now, stream_takes.)
 // Stretches of K for the 64-token tiles (128 rows, two workgroups a compute unit = 512 places).  This kernel's
 // workgroups are slow next to the pass that adds the partial tiles, so under 192 tiles it takes as many stretches as
 // fill the places once, eight at most, four super-blocks a stretch at least.  14336 -> 4096, per call, us, stretches of

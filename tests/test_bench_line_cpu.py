@@ -3,6 +3,8 @@ stdout): every contract field, the roofline and CPU-baseline objects, one headli
 whatever the legs hold; tables and raw samples go to the details file, as the reference keeps raw
 samples in evidence files (inference/parity/README.md:110)."""
 import json
+import os
+import re
 
 import bench
 from magnitude_amd import evidence
@@ -39,8 +41,8 @@ def full_result(nshapes=9, nsamples=400):
         "q8_0": {"shape": "4096x4096, M=1", "us_per_launch": 6.07123, "GBps": 2940.12, "frac_hbm_peak": 0.3675},
         "norm": {"M=1": {"separate_us": 17.9, "fused_us": 16.2, "fused_swiglu_us": 16.3}},
         "prefill": {"act_format": "per-32", "mfma": "m", "headline_tops": 520.123, "headline_frac_int8_peak": 0.104,
-                    "headline_rel_mad": 0.0041234, "samples_per_shape": 30, "bound": "valu", "floor_tops": 704.0,
-                    "floor": "5000 x 32 / (16 + 4 x 52.8): 48 of 52.8 vector instr. per matrix instr. are the per-32 flush",
+                    "headline_rel_mad": 0.0041234, "samples_per_shape": 30, "bound": "valu", "floor_tops": 1111.0,
+                    "floor": "5000 x 32 / (16 + 4 x 32): the per-32 flush is 32 vector instr. behind every matrix instr.",
                     "peak_tops": 5000.0, "shapes": shapes},
         "prefill_ggml_acts": {"act_format": "q8k", "mfma": "m" * 200, "headline_tops": 911.6, "headline_frac_int8_peak": 0.1823,
                               "headline_rel_mad": 0.0061234, "samples_per_shape": 30, "shapes": ggml_shapes},
@@ -91,7 +93,7 @@ def test_final_line_is_compact_and_complete():
     assert line["prefill_q8x32"]["rel_mad"] == 0.0041 and line["prefill_q8k"]["rel_mad"] == 0.0061
     assert line["prefill_q8x32"]["samples"] == 30 and line["prefill_q8k"]["samples"] == 30
     # config 4's own format is bounded by the vector ALU: the line says so, with the floor, and keeps frac against 5 POPS
-    assert line["prefill_q8x32"]["bound"] == "valu" and line["prefill_q8x32"]["floor_tops"] == 704.0
+    assert line["prefill_q8x32"]["bound"] == "valu" and line["prefill_q8x32"]["floor_tops"] == 1111.0
     assert "floor" in line["prefill_q8x32"] and line["prefill_q8x32"]["peak_tops"] == 5000.0
     assert line["moe_ffn"]["B64"]["rel_mad"] == 0.0071
     assert cb["host_physical_cores"] == 64 and cb["cores"] == 16 and "physical-cores" in cb["thread_policy"] and cb["rel_mad"] == 0.0123
@@ -136,3 +138,10 @@ def test_traffic_figure_is_withheld_when_the_kernel_sources_changed(tmp_path, mo
     monkeypatch.setattr(bench, "source_digest", lambda *a: "0" * 16)
     traffic, source = bench.measured_traffic()
     assert traffic is None and ("stale" in source or "not recorded" in source)
+
+
+def test_the_per32_bound_on_the_line_is_the_arithmetic_beside_it():
+    text = open(os.path.join(os.path.dirname(__file__), "..", "bench.py")).read()
+    value = float(re.search(r'"floor_tops": ([0-9.]+)', text)[1])
+    peak, k, mfma, vec, n = map(float, re.search(r'"floor": "(\d+) x (\d+) / \((\d+) \+ (\d+) x (\d+)\)', text).groups())
+    assert abs(peak * k / (mfma + vec * n) - value) < 1.0
