@@ -1,7 +1,9 @@
 // Batches between the small-batch kernel and the wide prefill tiles: weights streamed from HBM once for up to 128
 // tokens, Q4_K / Q6_K weights x ggml Q8_K activations on the int8 matrix cores.
 //
-// Bound: HBM (33 .. ~100 tokens).  What kept the 64-token tiles below half of that was latency, not arithmetic: one
+// Bound on paper: HBM (33 .. ~100 tokens).  Measured, no unit alone: gate + up of 14336 rows at 48 tokens move 68.3 MB (the
+// weights once) in 28.4 us = 2.4 TB/s, the vector pipe busy a third and the matrix pipe a quarter of the cycles, a wave waiting
+// for 39 % of its own.  What kept the 64-token tiles further below (49 us there) was latency, not arithmetic: one
 // super-block of weights in flight a wave, a launch a matrix, too few workgroups.  So here
 //   - raw weight blocks go from global memory straight into wave-private LDS strips, two super-blocks ahead of the
 //     arithmetic (Q4_K; one ahead for the larger Q6_K strips): a wave reads its strip into registers at the top of a
@@ -9,9 +11,9 @@
 //   - activations of a step (one super-block a K part) are double-buffered in LDS, shared by the row groups of the
 //     workgroup, one barrier a step;
 //   - a workgroup is 8 waves (4 where the launch leaves room for twice the workgroups) = RW row groups of 32 weight
-//     rows x KW K parts (summed through LDS at the end), K is cut
-//     further over workgroups where the tiles would not fill the chip, and all matrices of a call (q/k/v, gate/up)
-//     share the launch and the launch that adds the partial tiles.
+//     rows x KW K parts (summed through LDS at the end), K is cut further over workgroups where the tiles would not
+//     fill the chip, and all matrices of a call (q/k/v, gate/up) share the launch and the launch that adds the partial
+//     tiles.
 // The arithmetic is that of the tiled kernels: Q4_K scales in base 8 as two int8 operands, Q6_K products as high and
 // low bytes, both chains inside the matrix cores for a whole super-block, one flush per 256 weights, the Q4_K min
 // term on the fp16 cores from the plane the quantizer wrote.
@@ -558,6 +560,8 @@ StreamPlan stream_plan(int type, int64_t K, int64_t M, int64_t N) {
     // (gate / up) and takes half the chip, a square one (q, o) leaves room for k and v, a down projection or a matrix of
     // long rows takes all of it.  Measured, us, 160 / 256 workgroups: q/k/v of 4096 at 96 tokens 21.5 / 25.6, o 17.4 / 15.9;
     // gate + up 4096 -> 14336 at 64 tokens 27.3 / 38.3; 14336 -> 4096 39.0 / 26.3 at 96 tokens; 8192 x 8192 40.1 / 28.3.
+    // (Rows of 8192 and more stay cut beside a sibling of their size too: 8192 -> 2 x 28672 at 80 tokens takes 154 us in two
+    // stretches each and 139 whole, 182 in the tiled kernels, but whole its sums run over 32 super-blocks instead of 16.)
     const bool whole_chip = K > N || K >= 8192 || (K == N && type == kTypeQ6_K);
     const int64_t wgs = tuning_int("QPROJ_STREAM_WGS", whole_chip ? (int)cus : (int)(K == N ? cus * 5 / 8 : cus / 2));
     int64_t n = std::max<int64_t>(1, wgs / stream_tiles(M, N, p.jt, p.kw));
