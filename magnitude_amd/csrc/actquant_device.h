@@ -99,13 +99,18 @@ __device__ __forceinline__ uint32_t wave_quantize_q8_32(const float4 v, int &isu
 // One wave quantizes 256 consecutive floats (lane l holds elements 4l..4l+3 in `v`) as ggml's block_q8_K and
 // writes super-block `sb` of the planes qs, d, bsums (the min-term plane is made afterwards, row by row:
 // minterm_rows_kernel)
+// `hsum` non-null: the sums of 16 codes go there as fp16 integers instead
 __device__ __forceinline__ void wave_store_q8k(const float4 &v, int lane, int64_t sb, int8_t *__restrict__ qs,
-                                               float *__restrict__ d, int16_t *__restrict__ bsums) {
+                                               float *__restrict__ d, int16_t *__restrict__ bsums,
+                                               uint16_t *__restrict__ hsum = nullptr) {
     int bsum;
     float dd;
     const uint32_t packed = wave_quantize_q8k(v, lane, bsum, dd);
     reinterpret_cast<uint32_t *>(qs + sb * 256)[lane] = packed;
-    if ((lane & 3) == 0) bsums[sb * 16 + (lane >> 2)] = (int16_t)bsum;
+    if ((lane & 3) == 0) {
+        if (hsum) hsum[sb * 16 + (lane >> 2)] = f2h((float)(int16_t)bsum);
+        else bsums[sb * 16 + (lane >> 2)] = (int16_t)bsum;
+    }
     if (lane == 0) d[sb] = dd;
 }
 

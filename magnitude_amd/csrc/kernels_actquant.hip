@@ -30,13 +30,13 @@ __device__ __forceinline__ void zero_rows(const ZeroJob &z) {
 
 __global__ __launch_bounds__(256) void quant_q8k_kernel(const float *__restrict__ x, const float *__restrict__ u, int64_t n_super,
                                                         int8_t *__restrict__ qs, float *__restrict__ d,
-                                                        int16_t *__restrict__ bsums, const ZeroJob zero) {
+                                                        int16_t *__restrict__ bsums, uint16_t *__restrict__ hsum, const ZeroJob zero) {
     zero_rows(zero);
     const int64_t sb = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (sb >= n_super) return;  // whole wave leaves together
     const float4 v = load_rows4(x, u, sb * 256 + 4 * lane);
-    wave_store_q8k(v, lane, sb, qs, d, bsums);
+    wave_store_q8k(v, lane, sb, qs, d, bsums, hsum);
 }
 
 // FP16_SCALE: ggml Q8_0 blocks (scale rounded through fp16).  Otherwise the prefill format:
@@ -155,7 +155,7 @@ hipError_t launch_minterm_rows(int kind, const float *d, const int16_t *bsums, c
 // sums themselves)
 hipError_t launch_quantize_act(int kind, const float *x, int64_t M, int64_t K, int8_t *qs, float *d,
                                int16_t *bsums, uint16_t *msum, int32_t *isum, float *rs, hipStream_t s, const float *u,
-                               const ZeroJob *zero) {
+                               const ZeroJob *zero, uint16_t *hsum) {
     const int64_t n = M * K;
     if (n == 0) return hipSuccess;
     if (kind != kActKindQ8_K && kind != kActKindQ8_0 && kind != kActKindQ8X32) return hipErrorInvalidValue;
@@ -166,9 +166,9 @@ hipError_t launch_quantize_act(int kind, const float *x, int64_t M, int64_t K, i
             if (zj.n[i] % 4 != 0 || (reinterpret_cast<uintptr_t>(zj.p[i]) & 15) != 0) return hipErrorInvalidValue;
     }
     if (dry_run()) {
-        plan_note("quantizer: %lld x %lld -> %s%s%s%s", (long long)M, (long long)K,
+        plan_note("quantizer: %lld x %lld -> %s%s%s%s%s", (long long)M, (long long)K,
                   kind == kActKindQ8_K ? "Q8_K" : kind == kActKindQ8_0 ? "Q8_0 blocks" : "per-32 int8",
-                  msum && rs ? " + min-term plane" : "", u ? ", rows = silu(x) * u" : "",
+                  msum && rs ? " + min-term plane" : "", hsum ? " + fp16 sums" : "", u ? ", rows = silu(x) * u" : "",
                   zj.count ? ", clears the output rows of a projection that adds its two K parts" : "");
         return hipSuccess;
     }
@@ -189,7 +189,7 @@ hipError_t launch_quantize_act(int kind, const float *x, int64_t M, int64_t K, i
     const int64_t chunks = (n + 255) / 256;
     const dim3 grid((unsigned)((chunks + 3) / 4)), block(256);
     if (kind == kActKindQ8_K) {
-        hipLaunchKernelGGL(quant_q8k_kernel, grid, block, 0, s, x, u, n / 256, qs, d, bsums, zj);
+        hipLaunchKernelGGL(quant_q8k_kernel, grid, block, 0, s, x, u, n / 256, qs, d, bsums, hsum, zj);
     } else if (kind == kActKindQ8_0) {
         hipLaunchKernelGGL(quant_q8_32_kernel<true>, grid, block, 0, s, x, u, chunks, n, qs, d, isum, zj);
     } else {

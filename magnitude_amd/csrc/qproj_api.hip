@@ -219,30 +219,34 @@ ActView act_view(const ActPlanes &p, uint8_t *base, int64_t K) {
     a.msum = p.kind == kActKindQ8_K || p.kind == kActKindQ8X32 ? reinterpret_cast<const uint16_t *>(base + p.off_msum) : nullptr;
     a.isum = p.kind == kActKindQ8X32 ? reinterpret_cast<const int32_t *>(base + p.off_aux) : nullptr;
     a.rs = a.msum ? reinterpret_cast<const float *>(base + p.off_rs) : nullptr;
+    a.hsum = p.kind == kActKindQ8_K ? a.msum : nullptr;   // one plane, filled for whichever kernel comes next
     return a;
 }
 
 // the same work as run_quantize (Q8_K planes only), described for the grouping launch to carry
-RowQuantJob quantize_job(const ActPlanes &p, uint8_t *base, const float *x, int64_t M, int64_t K) {
+// (hsum: with the fp16 sums of the expert tiles, in the place of the min-term plane that those do not read)
+RowQuantJob quantize_job(const ActPlanes &p, uint8_t *base, const float *x, int64_t M, int64_t K, bool hsum) {
     RowQuantJob j{};
     j.x = x;
     j.n_super = M * K / 256;
     j.qs = reinterpret_cast<int8_t *>(base + p.off_qs);
     j.d = reinterpret_cast<float *>(base + p.off_d);
     j.bsums = reinterpret_cast<int16_t *>(base + p.off_aux);
+    if (hsum) j.hsum = reinterpret_cast<uint16_t *>(base + p.off_msum);
     return j;
 }
 
 // minterm: also the min-term plane and the row normalisers that only the tiled Q4_K kernels read (a second, small launch)
 hipError_t run_quantize(qproj_ctx *ctx, const ActPlanes &p, uint8_t *base, const float *x, int64_t M, int64_t K,
-                        bool minterm = true, const float *swiglu_u = nullptr, const ZeroJob *zero = nullptr) {
+                        bool minterm = true, const float *swiglu_u = nullptr, const ZeroJob *zero = nullptr, bool hsum = false) {
     const bool mt = minterm && (p.kind == kActKindQ8_K || p.kind == kActKindQ8X32);
     return launch_quantize_act(p.kind, x, M, K, reinterpret_cast<int8_t *>(base + p.off_qs),
                                reinterpret_cast<float *>(base + p.off_d),
                                reinterpret_cast<int16_t *>(base + p.off_aux),
                                mt ? reinterpret_cast<uint16_t *>(base + p.off_msum) : nullptr,
                                reinterpret_cast<int32_t *>(base + p.off_aux),
-                               mt ? reinterpret_cast<float *>(base + p.off_rs) : nullptr, ctx->stream, swiglu_u, zero);
+                               mt ? reinterpret_cast<float *>(base + p.off_rs) : nullptr, ctx->stream, swiglu_u, zero,
+                               hsum ? reinterpret_cast<uint16_t *>(base + p.off_msum) : nullptr);
 }
 
 ActView act_rows(const ActView &a, int64_t m0) {
@@ -669,6 +673,19 @@ int grouped_mt(int64_t n_pairs, int64_t E) {
     if (n_pairs <= 4 * E) return 4;
     if (n_pairs <= 8 * E) return 8;
     return 16;
+}
+
+// Expert batches in tiles of up to 64 pairs on the matrix cores (moe_stream_kernel): beyond four pairs an expert, where the
+// grouped kernel stages 16 rows a pass instead of 8, and from three and a half on where the row tiles of the experts fill the chip
+// (two workgroups of 64 rows a compute unit).  us a call, grouped / tiles: 128 experts of 2048 x 768, 40 / 64 / 100 / 500
+// tokens (2.5 / 4 / 6.2 / 31 pairs an expert) 89 / 91.5, 103 / 94, 105 / 97, 208 / 127; 64 of 1024 x 512 at 3.8 pairs
+// 41.8 / 33.2; 32 of 4096 x 512 at 4 / 6.2 pairs 42.7 / 45.8, 50.5 / 46.4; 256 of 1024 x 2048 at 2.8 / 7.8 pairs 202 / 214, 277 / 239.
+// Popular experts take tiles of their own: the 128 experts with popularity e^N(0,1), 500 tokens, 462 / 162.
+bool moe_stream_route(int type, int64_t K, int64_t N, int64_t n_pairs, int64_t E) {
+    static const int per_4_experts = tuning_int("QPROJ_MOE_STREAM_PAIRS_PER_4_EXPERTS", 0);
+    const bool many = per_4_experts ? 4 * n_pairs >= per_4_experts * E
+                                    : n_pairs > 4 * E || (2 * n_pairs >= 7 * E && E * N >= (int64_t)2 * 64 * cu_count());
+    return many && moe_stream_fits(type, K, N);
 }
 
 }  // namespace
@@ -1388,26 +1405,29 @@ int qproj_mul_mat_id(qproj_ctx *ctx, const qproj_weight *w, const float *x_dev, 
     const size_t off_order = p.total;
     const size_t off_offsets = off_order + align_up((size_t)n_pairs * 4);
     const size_t off_active = off_offsets + align_up((size_t)(w->E + 1) * 4);
-    const size_t off_parts = off_active + align_up(active_list_bytes(w->E));
-    const bool long_rows = grouped_long_rows(w, n_pairs);
+    const bool tiles = moe_stream_route(w->type, K, w->N, n_pairs, w->E);
+    const int64_t tile_rows = tiles ? kMoeTileRows : 0;
+    const size_t off_parts = off_active + align_up(active_list_bytes(moe_list_capacity(w->E, n_pairs, tile_rows)));
+    const bool long_rows = !tiles && grouped_long_rows(w, n_pairs);
     const size_t parts_bytes = long_rows ? mfma_grouped_scratch_bytes(K, w->N, n_pairs, w->E) : 0;
     const size_t total = off_parts + align_up(parts_bytes);
     Workspace wsp = ctx_workspace(ctx);
     int rc = reserve(ctx, wsp, total);
     if (rc) return rc;
     // few pairs an expert: the grouped kernel quantizes the rows it needs in its prologue
-    const bool fuse = grouped_fuses_quantizer(w->type, K, n_pairs, w->E);
+    const bool fuse = !tiles && grouped_fuses_quantizer(w->type, K, n_pairs, w->E);
     int32_t *order = reinterpret_cast<int32_t *>(wsp.base + off_order);
     int32_t *offsets = reinterpret_cast<int32_t *>(wsp.base + off_offsets);
     int32_t *active = reinterpret_cast<int32_t *>(wsp.base + off_active);
-    const bool pair_mode = grouped_pair_mode(w->type, K, n_pairs, w->E);
+    const bool pair_mode = !tiles && grouped_pair_mode(w->type, K, n_pairs, w->E);
     // the quantizer and the grouping pass read only the call's inputs: one launch carries both
     const bool joined = !fuse && !pair_mode && p.kind == kActKindQ8_K;
-    const RowQuantJob job = quantize_job(p, wsp.base, x_dev, rows, K);
+    const RowQuantJob job = quantize_job(p, wsp.base, x_dev, rows, K, tiles);
     if (!fuse && !joined) QP_HIP(ctx, run_quantize(ctx, p, wsp.base, x_dev, rows, K, false));
     if (!pair_mode)
         QP_HIP(ctx, launch_moe_group(ids_dev, n_pairs, w->E, order, offsets, active, ctx->flag_dev,
-                                     mfma_grouped_pass_rows(w->type, K, w->N, w->E, n_pairs), joined ? &job : nullptr, ctx->stream));
+                                     mfma_grouped_pass_rows(w->type, K, w->N, w->E, n_pairs), joined ? &job : nullptr, ctx->stream,
+                                     tile_rows));
     GemvArgs g{};
     g.n_targets = 1;
     g.t[0].w = w->view;
@@ -1423,7 +1443,9 @@ int qproj_mul_mat_id(qproj_ctx *ctx, const qproj_weight *w, const float *x_dev, 
     g.offsets = offsets;
     g.active = active;
     g.x_div = nb1 == 1 ? (int)n_used : 1;
-    if (use_mfma_grouped(w->type, K))
+    if (tiles)
+        QP_HIP(ctx, launch_moe_stream(g, n_pairs, false, ctx->stream));
+    else if (use_mfma_grouped(w->type, K))
         QP_HIP(ctx, launch_gemv_mfma_grouped(g, n_pairs, false, ctx->stream));
     else if (long_rows)
         QP_HIP(ctx, launch_gemv_mfma_grouped(g, n_pairs, false, ctx->stream,
@@ -1457,7 +1479,10 @@ int qproj_moe_ffn(qproj_ctx *ctx, const qproj_weight *gate, const qproj_weight *
     const size_t off_offsets = off;
     off += align_up((size_t)(E + 1) * 4);
     const size_t off_active = off;
-    off += align_up(active_list_bytes(E));
+    // (both products or neither: they share the work list)
+    const bool tiles = moe_stream_route(gate->type, d_model, d_ff, n_pairs, E) && moe_stream_route(down->type, d_ff, d_model, n_pairs, E);
+    const int64_t tile_rows = tiles ? kMoeTileRows : 0;
+    off += align_up(active_list_bytes(moe_list_capacity(E, n_pairs, tile_rows)));
     const size_t off_h = off;
     off += align_up((size_t)(n_pairs * d_ff) * 4);
     const size_t off_hq = off;
@@ -1466,7 +1491,7 @@ int qproj_moe_ffn(qproj_ctx *ctx, const qproj_weight *gate, const qproj_weight *
     off += align_up((size_t)(n_pairs * d_model) * 4);
     // rows too long for one pass of the grouped matrix-core kernel go in K chunks (grouped_long_rows); gate and up then
     // take a launch each (the SwiGLU epilogue needs whole sums) and the swiglu is formed by the quantizer behind them
-    const bool long_down = grouped_long_rows(down, n_pairs), long_gate = grouped_long_rows(gate, n_pairs);
+    const bool long_down = !tiles && grouped_long_rows(down, n_pairs), long_gate = !tiles && grouped_long_rows(gate, n_pairs);
     const size_t parts_bytes = std::max(long_down ? mfma_grouped_scratch_bytes(d_ff, d_model, n_pairs, E) : 0,
                                         long_gate ? mfma_grouped_scratch_bytes(d_model, d_ff, n_pairs, E) : 0);
     const size_t off_parts = off;
@@ -1510,18 +1535,18 @@ int qproj_moe_ffn(qproj_ctx *ctx, const qproj_weight *gate, const qproj_weight *
         return QPROJ_OK;
     }
 
-    const bool fuse_x = grouped_fuses_quantizer(gate->type, d_model, n_pairs, E);
-    const bool fuse_h = grouped_fuses_quantizer(down->type, d_ff, n_pairs, E);
-    const bool pair_mode = grouped_pair_mode(gate->type, d_model, n_pairs, E) &&
+    const bool fuse_x = !tiles && grouped_fuses_quantizer(gate->type, d_model, n_pairs, E);
+    const bool fuse_h = !tiles && grouped_fuses_quantizer(down->type, d_ff, n_pairs, E);
+    const bool pair_mode = !tiles && grouped_pair_mode(gate->type, d_model, n_pairs, E) &&
                            grouped_pair_mode(down->type, d_ff, n_pairs, E);
     // the quantizer of x and the grouping pass read only the call's inputs: one launch carries both
     const bool joined = !fuse_x && !pair_mode && px.kind == kActKindQ8_K;
-    const RowQuantJob job = quantize_job(px, ws, x_dev, B, d_model);
+    const RowQuantJob job = quantize_job(px, ws, x_dev, B, d_model, tiles);
     if (!fuse_x && !joined) QP_HIP(ctx, run_quantize(ctx, px, ws, x_dev, B, d_model, false));
     if (!pair_mode)
         // (the order suits the passes of gate and up, two thirds of the work)
         QP_HIP(ctx, launch_moe_group(ids_dev, n_pairs, E, order, offsets, active, ctx->flag_dev,
-                                     mfma_grouped_pass_rows(gate->type, d_model, d_ff, E, n_pairs), joined ? &job : nullptr, ctx->stream));
+                                     mfma_grouped_pass_rows(gate->type, d_model, d_ff, E, n_pairs), joined ? &job : nullptr, ctx->stream, tile_rows));
     GemvArgs g{};
     if (pair_mode) {
         g.ids = ids_dev;
@@ -1540,7 +1565,9 @@ int qproj_moe_ffn(qproj_ctx *ctx, const qproj_weight *gate, const qproj_weight *
     g.active = active;
     g.x_div = (int)n_used;
     const float *swiglu_u = nullptr;   // non-null: h holds the gate products, this the up products
-    if (use_mfma_grouped(gate->type, d_model)) {
+    if (tiles) {
+        QP_HIP(ctx, launch_moe_stream(g, n_pairs, true, ctx->stream));
+    } else if (use_mfma_grouped(gate->type, d_model)) {
         QP_HIP(ctx, launch_gemv_mfma_grouped(g, n_pairs, true, ctx->stream));
     } else if (long_gate) {
         float *h2 = reinterpret_cast<float *>(ws + off_h2);
@@ -1560,7 +1587,7 @@ int qproj_moe_ffn(qproj_ctx *ctx, const qproj_weight *gate, const qproj_weight *
     } else {
         QP_HIP(ctx, launch_moe_swiglu_gemv(g, mt, (int)E, ctx->stream));
     }
-    if (!fuse_h) QP_HIP(ctx, run_quantize(ctx, ph, ws + off_hq, h, n_pairs, d_ff, false, swiglu_u));
+    if (!fuse_h) QP_HIP(ctx, run_quantize(ctx, ph, ws + off_hq, h, n_pairs, d_ff, false, swiglu_u, nullptr, tiles));
     GemvArgs gd{};
     if (pair_mode) {
         gd.ids = ids_dev;
@@ -1576,7 +1603,9 @@ int qproj_moe_ffn(qproj_ctx *ctx, const qproj_weight *gate, const qproj_weight *
     gd.offsets = offsets;
     gd.active = active;
     gd.x_div = 1;
-    if (use_mfma_grouped(down->type, d_ff))
+    if (tiles)
+        QP_HIP(ctx, launch_moe_stream(gd, n_pairs, false, ctx->stream));
+    else if (use_mfma_grouped(down->type, d_ff))
         QP_HIP(ctx, launch_gemv_mfma_grouped(gd, n_pairs, false, ctx->stream));
     else if (long_down)
         QP_HIP(ctx, launch_gemv_mfma_grouped(gd, n_pairs, false, ctx->stream,

@@ -45,6 +45,7 @@ struct ActView {
                            //       sub-blocks, high parts, then the 8 low parts (v - high); prefill min term
     const int32_t *isum;   // Q8X32: [rows][K/32]
     const float *rs;       // Q8_K, Q8X32: [rows] the power of two the row's msum entries are normalised by
+    const uint16_t *hsum;  // Q8_K: [rows][K/16] fp16: the sums of 16 codes (|.| <= 2032: exact), min term of the expert tiles
 };
 constexpr float kMinPrescale = 0.0625f;  // (d / rs) * sum / 16 <= 2 * 4064 / 16: well inside fp16 whatever the activations
 constexpr int kActKindQ8_0 = 0;
@@ -132,11 +133,17 @@ inline int wide_tile_splits(int64_t tiles, int64_t nsb, int64_t M, int64_t N, in
     return best;
 }
 
-// The busy-expert list of the grouping pass: n_expert + 1 ints (the list, then its length), then from a 16-byte boundary
-// one int4 {expert, its first slot in order[], its pairs, 0} per list position, so that a workgroup of the grouped
-// kernels learns all three from ONE load instead of a chain of two.
-__host__ __device__ inline int64_t active_slots_offset(int64_t n_expert) { return (n_expert + 1 + 3) & ~(int64_t)3; }   // in ints
-inline size_t active_list_bytes(int64_t n_expert) { return (size_t)(active_slots_offset(n_expert) + 4 * n_expert) * 4; }
+// The work list of the grouping pass: `capacity` + 1 ints (the busy experts, then at [capacity] the length of the list),
+// then from a 16-byte boundary one int4 {expert, first slot in order[], pairs, 0} per list position, so that a workgroup
+// of the grouped kernels learns all three from ONE load instead of a chain of two.  Either a position per expert that has
+// pairs (tile_rows = 0, capacity = experts), or one per tile of at most tile_rows pairs of an expert (records only).
+__host__ __device__ inline int64_t active_slots_offset(int64_t capacity) { return (capacity + 1 + 3) & ~(int64_t)3; }   // in ints
+inline size_t active_list_bytes(int64_t capacity) { return (size_t)(active_slots_offset(capacity) + 4 * capacity) * 4; }
+inline int64_t moe_list_capacity(int64_t n_expert, int64_t n_pairs, int64_t tile_rows) {
+    return tile_rows == 0 ? n_expert : (n_expert < n_pairs ? n_expert : n_pairs) + n_pairs / tile_rows;
+}
+constexpr int kMoeTileRows = 64;      // pairs of an expert that a pass of moe_stream_kernel takes
+constexpr int kMoeStreamMaxSb = 32;   // super-blocks of a row whose activation scales it keeps in LDS
 
 // Compute units of the current device (256 when no device can be asked, e.g. in a dry run on a host without one).
 int cu_count();
@@ -165,7 +172,7 @@ struct ZeroJob {
 // zero: see ZeroJob (carried by the first launch of the quantizer)
 hipError_t launch_quantize_act(int kind, const float *x, int64_t M, int64_t K, int8_t *qs, float *d,
                                int16_t *bsums, uint16_t *msum, int32_t *isum, float *rs, hipStream_t s,
-                               const float *u = nullptr, const ZeroJob *zero = nullptr);
+                               const float *u = nullptr, const ZeroJob *zero = nullptr, uint16_t *hsum = nullptr);
 // the min-term plane and the row normalisers from planes already quantized (one wave per row)
 hipError_t launch_minterm_rows(int kind, const float *d, const int16_t *bsums, const int32_t *isum, int64_t M, int64_t K,
                                uint16_t *msum, float *rs, hipStream_t s);
@@ -200,13 +207,18 @@ struct RowQuantJob {
     int8_t *qs;
     float *d;
     int16_t *bsums;
+    uint16_t *hsum;   // null: not written
 };
-// pass_rows: mfma_grouped_pass_rows of the launch behind it
+// pass_rows: mfma_grouped_pass_rows of the launch behind it; tile_rows: see the work list above (0: a position per expert)
 hipError_t launch_moe_group(const int32_t *ids, int64_t n_pairs, int64_t n_expert, int32_t *order,
                             int32_t *offsets, int32_t *active, int32_t *error_flag, int64_t pass_rows,
-                            const RowQuantJob *quantize, hipStream_t s);
+                            const RowQuantJob *quantize, hipStream_t s, int64_t tile_rows = 0);
 // rows of an expert's pairs that a pass of the grouped matrix-core kernel stages (8, 16 or 32)
 int mfma_grouped_pass_rows(int type, int64_t K, int64_t N, int64_t E, int64_t n_pairs);
+// expert batches in tiles of kMoeTileRows pairs (`a` with its hsum plane, args.active a tile list): y[pair][N], or with
+// `swiglu` silu(t[0] . x) * (t[1] . x)
+bool moe_stream_fits(int type, int64_t K, int64_t N);
+hipError_t launch_moe_stream(const GemvArgs &args, int64_t n_pairs, bool swiglu, hipStream_t s);
 hipError_t launch_moe_swiglu_gemv(const GemvArgs &gate_up, int mt, int n_experts_grid, hipStream_t s);
 // One or two decode tokens (at most 16 pairs) through expert stacks of Q4_K / Q6_K rows of K <= 4096 on the vector
 // ALU: args as for the pair mode of the grouped kernel (t[0], and t[1] = up when `swiglu`; x fp32 rows, x_div, ids,

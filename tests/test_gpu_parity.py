@@ -729,6 +729,72 @@ def test_mul_mat_id_grouping_of_many_pairs(ctx, orc, E, B):
     w.free()
 
 
+@pytest.mark.parametrize("k,n,counts", [(256, 63, (1, 31, 32, 33, 0, 64, 65)), (768, 129, (0, 129, 1, 63, 5)),
+                                        (2048, 64, (96, 2, 2)), (8192, 40, (70, 33)), (512, 1, (40,))])
+def test_expert_tiles_at_their_edges(ctx, orc, k, n, counts):
+    """moe_stream_kernel: tiles of 1 .. 64 pairs of an expert (one and two token tiles, full and ragged, an expert without
+    pairs), rows beyond the last whole row tile, one super-block and the longest rows; a pair of a bad expert is left out
+    and reported, the others are computed.  Tolerance as for every single projection: the integer sums are exact, K / 256
+    fp32 additions in another order."""
+    from magnitude_amd import ACT_GGML, QprojError
+    E = len(counts)
+    rng = np.random.default_rng(k + n)
+    ids = rng.permutation(np.repeat(np.arange(E, dtype=np.int32), counts))[:, None]
+    blocks = encode(Q4_K, (rng.standard_normal((E * n, k)) * 0.02).astype(np.float32)).reshape(E, n, -1)
+    x = rng.standard_normal((len(ids), 1, k)).astype(np.float32)
+    w = ctx.upload(Q4_K, k, n, blocks, n_expert=E)
+    want = orc.mul_mat_id(Q4_K, blocks, k, n, E, x, ids)
+    close(ctx.mul_mat_id(w, dev(x), dev(ids), ACT_GGML).cpu().numpy(), want, 2e-5)
+    bad = ids.copy()
+    bad[len(ids) // 2] = E
+    y = torch.full((len(ids), 1, n), 7.0, dtype=torch.float32, device="cuda")
+    t, i = dev(x), dev(bad)
+    torch.cuda.synchronize()
+    assert ctx.lib.qproj_mul_mat_id(ctx.handle, w.handle, t.data_ptr(), 1, i.data_ptr(), 1, len(ids), y.data_ptr(), ACT_GGML) == 0
+    with pytest.raises(QprojError):
+        ctx.sync()
+    y = y.cpu().numpy()
+    assert (y[len(ids) // 2] == 7.0).all()
+    good = np.arange(len(ids)) != len(ids) // 2
+    close(y[good], want[good], 2e-5)
+    w.free()
+
+
+@pytest.mark.parametrize("E,top,B,d_model,d_ff", [(6, 2, 97, 512, 256), (8, 3, 60, 768, 1280), (64, 5, 64, 256, 512)])
+def test_moe_ffn_in_expert_tiles(ctx, orc, E, top, B, d_model, d_ff):
+    """Gate and up sixteen rows each in a matrix instruction, their swiglu in registers; tolerance as for the other
+    feed-forwards (a code of the re-quantized rows on a rounding tie), the half of the outputs without one to 1e-6."""
+    from magnitude_amd import ACT_GGML, qproj
+    assert qproj.plan_moe_ffn(Q4_K, Q4_K, d_model, d_ff, E, top, B).count("moe_stream_kernel") == 2
+    rng = np.random.default_rng(E + B + d_ff)
+    enc = lambda rows, cols: encode(Q4_K, (rng.standard_normal((E * rows, cols)) * 0.02).astype(np.float32)).reshape(E, rows, -1)
+    gate_b, up_b, down_b = enc(d_ff, d_model), enc(d_ff, d_model), enc(d_model, d_ff)
+    ids, wts = routing(rng, B, top, E)
+    ids[: B // 2, 0] = 1                               # a popular expert (a token may name it twice)
+    x = rng.standard_normal((B, d_model)).astype(np.float32)
+    g, u, d = (ctx.upload(Q4_K, k, n, b, n_expert=E) for k, n, b in ((d_model, d_ff, gate_b), (d_model, d_ff, up_b), (d_ff, d_model, down_b)))
+    got = ctx.moe_ffn(g, u, d, dev(x), dev(ids), dev(wts), ACT_GGML).cpu().numpy()
+    want = orc.moe_ffn(Q4_K, Q4_K, gate_b, up_b, down_b, d_model, d_ff, E, x, ids, wts, orc.ACT_GGML)
+    close(got, want, 1e-3)
+    gate(got, want)
+    assert np.median(np.abs(got - want)) <= 1e-6 * np.abs(want).max()
+    for t in (g, u, d):
+        t.free()
+
+
+def test_grouping_of_very_many_experts(ctx, orc):
+    """More experts than the grouping pass has LDS counters for: it sweeps the ids once per expert."""
+    from magnitude_amd import ACT_GGML
+    E, k, n, B, top = 2048, 256, 8, 300, 8
+    rng = np.random.default_rng(5)
+    blocks = encode(Q4_K, (rng.standard_normal((E * n, k)) * 0.02).astype(np.float32)).reshape(E, n, -1)
+    ids, _ = routing(rng, B, top, E)
+    x = rng.standard_normal((B, 1, k)).astype(np.float32)
+    w = ctx.upload(Q4_K, k, n, blocks, n_expert=E)
+    close(ctx.mul_mat_id(w, dev(x), dev(ids), ACT_GGML).cpu().numpy(), orc.mul_mat_id(Q4_K, blocks, k, n, E, x, ids), 2e-5)
+    w.free()
+
+
 def test_mul_mat_id_reports_bad_expert_ids(ctx, orc, moe):
     from magnitude_amd import ACT_GGML, QprojError
     E, k, n = moe["E"], moe["d_model"], moe["d_ff"]
