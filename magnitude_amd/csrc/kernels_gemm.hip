@@ -1036,6 +1036,7 @@ int per32_splits(int type, int64_t K, int64_t M, int64_t N) {
     return n;
 }
 size_t per32_scratch_bytes(int type, int64_t K, int64_t M, int64_t N) {
+    if (type == kTypeQ8_0 && q8_0_tokens_takes(K, M, N)) return q8_0_tokens_scratch_bytes(K, M, N);
     const int n = per32_splits(type, K, M, N);
     return n > 1 ? (size_t)n * M * N * 4 : 0;
 }
@@ -1047,9 +1048,25 @@ hipError_t launch_gemm_q8x32(const WeightView &w, const ActView &a, int64_t M, f
 
 // Q8_0 weights x ggml Q8_0 activation blocks (planes in `a`), K a multiple of 128
 hipError_t launch_gemm_q8_0(int n, const WeightView *w, const ActView &a, int64_t M, float *const *y, const Scratch &scratch, hipStream_t s) {
-    for (int i = 0; i < n; ++i)
+    WeightView tokens[kMaxTargets], tiled[kMaxTargets];
+    float *yt[kMaxTargets], *yl[kMaxTargets];
+    int nt = 0, nl = 0;
+    if (n < 1 || n > kMaxTargets) return hipErrorInvalidValue;
+    for (int i = 0; i < n; ++i) {
         if (w[i].type != kTypeQ8_0 || a.kind != kActKindQ8_0 || w[i].K % BK != 0 || M <= 0) return hipErrorInvalidValue;
-    return launch_per32<kTypeQ8_0>(n, w, a, M, y, scratch, s);
+        if (q8_0_tokens_takes(w[i].K, M, w[i].N)) {
+            tokens[nt] = w[i];
+            yt[nt++] = y[i];
+        } else {
+            tiled[nl] = w[i];
+            yl[nl++] = y[i];
+        }
+    }
+    if (nt) {
+        const hipError_t e = launch_gemm_q8_0_tokens(nt, tokens, a, M, yt, scratch, s);
+        if (e != hipSuccess) return e;
+    }
+    return nl ? launch_per32<kTypeQ8_0>(nl, tiled, a, M, yl, scratch, s) : hipSuccess;
 }
 
 // Which Q4_K kernel and how many stretches of K (one rule for the launcher and for the scratch sizing).  The

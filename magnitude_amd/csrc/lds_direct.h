@@ -13,6 +13,12 @@ __device__ __forceinline__ void global_to_lds16(const void *g, void *l) {
                                      (__attribute__((address_space(3))) void *)l, 16, 0, 0);
 }
 
+// the same with 4 bytes a lane, at l + 4*l
+__device__ __forceinline__ void global_to_lds4(const void *g, void *l) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)g,
+                                     (__attribute__((address_space(3))) void *)l, 4, 0, 0);
+}
+
 // a wave-uniform pointer pinned to scalar registers: what is added to it afterwards stays a 32-bit lane
 // offset (scalar base + vector offset addressing) instead of becoming a 64-bit pointer per lane
 template <typename T>

@@ -673,6 +673,31 @@ def test_q8_0_matrices_of_a_call_share_a_launch(ctx, orc, m, k, ns):
         w.free()
 
 
+@pytest.mark.parametrize("m,k,ns", [(129, 1152, (2050,)), (187, 1280, (1025, 1031)), (192, 1536, (1284,)), (160, 2048, (1100,)),
+                                    (33, 1280, (1028,)), (64, 4352, (1026,)), (65, 1408, (1100,)), (96, 2560, (1030, 1300)),
+                                    (130, 1152, (33000,))])
+def test_q8_0_tiles_of_96_and_64_tokens(ctx, orc, m, k, ns):
+    """gemm_per32_kernel_q8_0: both token tiles with ragged tokens and rows, K in parts and stretches with an odd number of steps of
+    128, outputs whose rows are no whole float4s, workgroups of 64 and 128 rows, more tiles than compute units (K in one part).
+    Against the oracle (5e-5 of the larger of 1 and the result, exact block sums and K / 32 fp32 additions in another order);
+    nothing written behind an output."""
+    from magnitude_amd import ACT_GGML, qproj
+    plan = qproj.plan_mul_mat(Q8_0, k, list(ns), m, ACT_GGML)
+    assert plan.count("gemm_per32_kernel_q8_0") == len(ns), plan
+    rng = np.random.default_rng(m + k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    blocks = [make_weight(orc, Q8_0, n, k, seed=6400 + i) for i, n in enumerate(ns)]
+    ws = [ctx.upload(Q8_0, k, n, b) for n, b in zip(ns, blocks)]
+    bufs = [torch.full((m * n + 64,), 7.0, dtype=torch.float32, device="cuda") for n in ns]
+    ctx.mul_mat_multi(ws, dev(x), ACT_GGML, outs=[b[: m * n].view(m, n) for b, n in zip(bufs, ns)])
+    some = np.unique([0, 31, 32, min(63, m - 1), min(95, m - 1), m // 2, m - 1])
+    for w, n, b, bl in zip(ws, ns, bufs, blocks):
+        close(b[: m * n].view(m, n).cpu().numpy()[some], orc.mul_mat(Q8_0, bl, k, x[some], orc.ACT_GGML), 5e-5)
+        assert bool((b[m * n:] == 7.0).all())
+        assert torch.equal(b[: m * n].view(m, n), ctx.mul_mat(w, dev(x), ACT_GGML))
+        w.free()
+
+
 # ---------------------------------------------------------------- MUL_MAT_ID and the MoE FFN
 
 @pytest.fixture(scope="module")
