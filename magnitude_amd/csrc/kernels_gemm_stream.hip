@@ -66,10 +66,7 @@ struct Strip<kTypeQ4_K> {
             off[c] = (uint32_t)(min(p / 9, cap) * nb * 144 + 16 * (p % 9));
         }
     }
-    __device__ __forceinline__ void request(uint32_t sb, uint8_t *strip) const {
-#pragma unroll
-        for (int c = 0; c < 5; ++c) global_to_lds16(base + (off[c] + sb * 144u), strip + 1024 * c);
-    }
+    __device__ __forceinline__ void request(uint32_t sb, uint8_t *strip, int c) const { global_to_lds16(base + (off[c] + sb * 144u), strip + 1024 * c); }
     static __device__ __forceinline__ Raw read(const uint8_t *strip, int l32, int lh) {
         Raw r;
         r.hdr = *reinterpret_cast<const v4i *>(strip + l32 * 144);
@@ -112,12 +109,10 @@ struct Strip<kTypeQ6_K> {
         off_s = (uint32_t)(min(lane & 31, cap) * nb * 16);
         off_d = (uint32_t)(min(lane & 31, cap) * nb);
     }
-    __device__ __forceinline__ void request(uint32_t sb, uint8_t *strip) const {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) global_to_lds16(bl + (off_l[c] + sb * 128u), strip + 1024 * c);
-#pragma unroll
-        for (int c = 0; c < 2; ++c) global_to_lds16(bh + (off_h[c] + sb * 64u), strip + 4096 + 1024 * c);
-        global_to_lds16(bs + (off_s + sb * 16u), strip + 6144);   // the upper half lands behind: not read
+    __device__ __forceinline__ void request(uint32_t sb, uint8_t *strip, int c) const {
+        if (c < 4) global_to_lds16(bl + (off_l[c & 3] + sb * 128u), strip + 1024 * c);
+        else if (c < 6) global_to_lds16(bh + (off_h[c & 1] + sb * 64u), strip + 1024 * c);
+        else global_to_lds16(bs + (off_s + sb * 16u), strip + 6144);   // the upper half lands behind: not read
     }
     __device__ __forceinline__ uint32_t scale(uint32_t sb) const { return load_global<uint16_t>(bd, 2u * (off_d + sb)); }
     static __device__ __forceinline__ Raw read(const uint8_t *strip, int l32, int lh) {
@@ -191,12 +186,17 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_stream_kernel(const StreamArg
         const int row = 4 * (wave + NW * j) + (lane >> 4), seg = (lane & 15) ^ (row & 15);
         aoff[j] = (uint32_t)(min(row, mcap) * (int)K + 16 * seg);
     }
+    auto request_act = [&](int s, int p) {
+        const uint32_t sb = (uint32_t)min(sb_begin + s * KW + p / AP, sb_end - 1);
+        global_to_lds16(abase + (aoff[p % AP] + sb * 256u), smem + ((s & 1) * KW + p / AP) * L::kAct + (wave + NW * (p % AP)) * 1024);
+    };
     auto request_acts = [&](int s) {
 #pragma unroll
-        for (int p = 0; p < KW * AP; ++p) {
-            const uint32_t sb = (uint32_t)min(sb_begin + s * KW + p / AP, sb_end - 1);
-            global_to_lds16(abase + (aoff[p % AP] + sb * 256u), smem + ((s & 1) * KW + p / AP) * L::kAct + (wave + NW * (p % AP)) * 1024);
-        }
+        for (int p = 0; p < KW * AP; ++p) request_act(s, p);
+    };
+    auto request_strip = [&](int s, uint8_t *dst) {
+#pragma unroll
+        for (int c = 0; c < S::kLoads; ++c) strip_src.request(my_sb(s), dst, c);
     };
     const uint8_t *msbase = nullptr;
     if constexpr (kQ4) {
@@ -285,7 +285,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_stream_kernel(const StreamArg
             for (int j = 0; j < JT; ++j) flush_tile(j, j, s);
         }
     };
-    auto products = [&](const typename S::Raw &raw, bool live, int s) {
+    auto products = [&](const typename S::Raw &raw, bool live, int s, auto &&requests_of) {
         const uint8_t *ab = smem + ((s & 1) * KW + kp) * L::kAct;
         auto frag = [&](int j, int i) { return *reinterpret_cast<const v4i *>(ab + j * 8192 + (aoffl ^ (16 * i))); };
         v4i cl[8], ch[8];
@@ -355,6 +355,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_stream_kernel(const StreamArg
                     for (int j = 0; j < JT; ++j) af[(p + 2) % 3][j] = frag(j, kOrder[p + 2]);
                 }
                 if (p + 1 < 8 && (kQ4 || (p & 1))) convert(p + 1);
+                requests_of(p);
                 if (p == 2) min_convert();
 #pragma unroll
                 for (int j = 0; j < JT; ++j) {
@@ -379,6 +380,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_stream_kernel(const StreamArg
 #pragma unroll
                 for (int p = 0; p < 8; ++p) {
                     const int i = kOrder[p];
+                    if (j == 0) requests_of(p);
                     const v4i a4 = frag(j, i);
                     ilo[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a4, cl[i], p == 0 ? zi : ilo[0], 0, 0, 0);
                     ihi[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a4, ch[i], p == 0 ? zi : ihi[0], 0, 0, 0);
@@ -390,12 +392,12 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_stream_kernel(const StreamArg
     };
 
     // ---- prologue: everything of step 0 and the strips of the steps the buffers hold
-    strip_src.request(my_sb(0), strip);
+    request_strip(0, strip);
     request_acts(0);
     request_ms(0);
     load_scales(sb_begin);
     if constexpr (SW == 2) {
-        strip_src.request(my_sb(1), strip + NW * S::kBytes);
+        request_strip(1, strip + NW * S::kBytes);
         wait_vmcnt<S::kLoads>();
     } else {
         wait_vmcnt<0>();
@@ -411,12 +413,24 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_stream_kernel(const StreamArg
             uint8_t *sbuf = strip + (SW == 2 ? (s & 1) * NW * S::kBytes : 0);
             const typename S::Raw raw = S::read(sbuf, l32, lh);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the strip has been read: it may be overwritten
-            if constexpr (MORE1) {
-                request_acts(s + 1);
-                request_ms(s + 1);
-            }
-            if constexpr (MORE2) strip_src.request(my_sb(s + SW), sbuf);
-            __builtin_amdgcn_sched_barrier(0);   // the requests stay ahead of the arithmetic they overlap with
+            // The step's requests, activations first, spread over its eight products: sent in one go they hold up all waves of the
+            // workgroup at once (a compute unit takes 64 bytes of them a cycle).  14336 -> 4096 at 192 tokens 53.6 -> 48.8 us, gate +
+            // up 4096 -> 2 x 14336 at 96 54.9 -> 51.0.  Q6_K in two K parts has its conversions to hide them: level to 2 % slower.
+            constexpr bool kSpread = kQ4 || KW == 1;
+            constexpr int kRequests = KW * AP + S::kLoads, kSlots = kSpread ? 8 : 1;
+            auto requests_of = [&](int p) {
+#pragma unroll
+                for (int i = p * kRequests / kSlots; i < std::min((p + 1) * kRequests / kSlots, kRequests); ++i) {
+                    if (i < KW * AP) {
+                        if constexpr (MORE1) request_act(s + 1, i);
+                    } else {
+                        if constexpr (MORE2) strip_src.request(my_sb(s + SW), sbuf, i - KW * AP);
+                    }
+                }
+            };
+            if constexpr (MORE1) request_ms(s + 1);
+            if constexpr (!kSpread) requests_of(0);
+            __builtin_amdgcn_sched_barrier(0);
             if constexpr (LATE) {
                 if (s > 0) flush(s - 1);
                 __builtin_amdgcn_sched_barrier(0);
@@ -426,7 +440,9 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_stream_kernel(const StreamArg
                 load_scales(sb_begin + s * KW);
                 __syncthreads();
             }
-            products(raw, sb_begin + s * KW + kp < sb_end, s);
+            products(raw, sb_begin + s * KW + kp < sb_end, s, [&](int p) {
+                if constexpr (kSpread) requests_of(p);
+            });
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (!LATE) {
                 flush(s);
