@@ -1,5 +1,5 @@
-// Batches between the small-batch kernel and the wide prefill tiles: weights streamed from HBM once for up to 128
-// tokens, Q4_K / Q6_K weights x ggml Q8_K activations on the int8 matrix cores.
+// Batches between the small-batch kernel and the wide prefill tiles, and matrices too small for those: weights streamed
+// from HBM once for up to 128 tokens, Q4_K / Q6_K weights x ggml Q8_K activations on the int8 matrix cores.
 //
 // Bound on paper: HBM (33 .. ~100 tokens).  Measured, no unit alone: gate + up of 14336 rows at 48 tokens move 68.3 MB (the
 // weights once) in 28.4 us = 2.4 TB/s, the vector pipe busy a third and the matrix pipe a quarter of the cycles, a wave waiting
@@ -581,6 +581,13 @@ StreamPlan stream_plan(int type, int64_t K, int64_t M, int64_t N) {
     const bool whole_chip = K > N || K >= 8192 || (K == N && type == kTypeQ6_K);
     const int64_t wgs = tuning_int("QPROJ_STREAM_WGS", whole_chip ? (int)cus : (int)(K == N ? cus * 5 / 8 : cus / 2));
     int64_t n = std::max<int64_t>(1, wgs / stream_tiles(M, N, p.jt, p.kw));
+    // Beyond 256 tokens k and v stay whole where q and they are one round together, or nearly one and a half: cut, they cost the
+    // adding pass and more starts than they fill (q/k/v of 3072 at 384 tokens 37.4 -> 26.6 us, of 4096 at 512 56.8 -> 52.3, of 2048
+    // at 640 29.5 -> 22.4; 1.1 rounds, 4096 at 384 tokens, 46.0 cut and 50.1 whole).
+    if (M > 256 && N <= 1024 && K > N) {
+        const int64_t together = stream_tiles(M, K, p.jt, p.kw) + 2 * stream_tiles(M, N, p.jt, p.kw);
+        if (together <= cus || together * 5 >= cus * 7) n = 1;
+    }
     n = tuning_int("QPROJ_STREAM_SPLIT", (int)n);
     n = std::min<int64_t>(n, std::max<int64_t>(1, nb / (2 * p.kw)));   // two steps a stretch at least
     // never more partial tiles than the allocation-free entry point has room for beside the activation planes
@@ -607,8 +614,14 @@ hipError_t launch_stream_kernel(const StreamArgs &g, int wgs, hipStream_t s) {
 
 }  // namespace
 
-// Which products the streaming kernel takes.  From 33 tokens (below, the small-batch kernel) to 256; of the grids beyond
-// one round of workgroups Q4_K keeps the older tiles from 97 tokens on, where arithmetic and not latency is the limit
+// Which products the streaming kernel takes.  From 33 tokens (below, the small-batch kernel) to 256, and Q4_K beyond while its
+// 64-token tiles are one round of workgroups: square and narrow matrices, which the 64-token tiles of
+// gemm_q4k_q8k_direct_kernel walk a super-block at a time with one in flight.  us a call, there / here: 4096 x 4096 at 257 / 384 / 512
+// tokens 34.5 / 27.9, 36.7 / 29.7, 40.1 / 32.5; 3072 x 3072 at 320 29.1 / 19.5; 2048 x 2048 at 1024 27.0 / 23.2; 8192 -> 3072 at 448 75.3 /
+// 46.7; 4096 -> 1024 at 1536 40.6 / 32.9; q/k/v of 4096 at 320 / 384 / 512 65.8 / 31.6, 53.0 / 46.1, 56.3 / 52.9, of 2048 at 512 39.4 / 20.1, at
+// 1024 35.7 / 35.0.  k and v follow q: streamed without it, 4096 -> 4096 / 1024 / 1024 at 640 tokens 58.9 / 86.  (Q6_K would gain as much,
+// 3072 q/k/v at 320 tokens 61.8 / 32.8, but with sums 1 to 4 % further from 64 bits than the stretches of its 64-token tiles.)
+// Of the grids beyond one round of workgroups Q4_K keeps the older tiles from 97 tokens on, where arithmetic and not latency is the limit
 // (4096 -> 32000 at 128 tokens 51.0 us there, 54.0 here; at 96 tokens 50.1 against 45.3).  The 128-token kernels
 // keep the grids they fill (q4k_fills_wide, q6k_fills_wide) where they are as fast or faster, us there / here: Q4_K beyond
 // 128 tokens (28672 -> 8192 at 192 / 256 tokens 147 / 159, 151 / 166) and from 65 on for very long rows (28672 -> 16384 at 112
@@ -616,7 +629,7 @@ hipError_t launch_stream_kernel(const StreamArgs &g, int wgs, hipStream_t s) {
 // 91.5 / 96.1) and from 65 on for long rows (12288 x 12288 at 96 tokens 79 / 88, 16384 x 16384 109 / 124).  At 129..192 tokens
 // Q6_K has tiles of 96 here: 4096 -> 32000 at 160 tokens 91.7 / 83.
 bool stream_takes(int type, int64_t K, int64_t M, int64_t N) {
-    const int lo = tuning_int("QPROJ_STREAM_MIN_M", 33), hi = tuning_int("QPROJ_STREAM_MAX_M", 256);
+    const int lo = tuning_int("QPROJ_STREAM_MIN_M", 33), hi = tuning_int("QPROJ_STREAM_MAX_M", type == kTypeQ4_K ? 2048 : 256);
     if ((type != kTypeQ4_K && type != kTypeQ6_K) || K % 256 != 0 || K > (1 << 22) || M < lo || M > hi) return false;
     if (N > (1 << 24)) return false;   // row and tile numbers are ints, a tile's outputs are indexed with 32 bits: 127 * N + 31 at most
     if (type == kTypeQ6_K) {
@@ -626,7 +639,10 @@ bool stream_takes(int type, int64_t K, int64_t M, int64_t N) {
         return !alone && !((jt == 4 || (jt == 3 && M <= 96 && K >= 12288)) && q6k_fills_wide(K, M, N));
     }
     if ((M > 128 || (M > 64 && K >= 16384)) && q4k_fills_wide(K, M, N)) return false;
-    return M <= 96 || stream_tiles(M, N, 2, 2) <= cu_count();
+    if (M <= 96) return true;
+    if (M > 256 && N <= 1024 && stream_tiles(M, K, 2, 2) > cu_count()) return false;   // k and v go with q
+    // (beyond 256 tokens up rides along with gate: 1024 -> 2 x 4096 at 320 tokens 21.2 / 22.7)
+    return stream_tiles(M, N, 2, 2) * (M > 256 && N > K ? 2 : 1) <= cu_count();
 }
 
 namespace {

@@ -275,7 +275,7 @@ inline void add_sum(SumTargets &g, const float *part, float *y, int n_split, int
     g.threads += (t.n4 + 255) / 256 * 256;
 }
 hipError_t launch_sum_parts(const SumTargets &g, hipStream_t s);
-// 33..256 rows of Q4_K / Q6_K weights: all matrices of a call in one launch, K cut per matrix
+// 33..256 rows of Q4_K / Q6_K weights, Q4_K up to 2048 (stream_takes): all matrices of a call in one launch, K cut per matrix
 bool stream_takes(int type, int64_t K, int64_t M, int64_t N);
 bool q4k_fills_wide(int64_t K, int64_t M, int64_t N);   // the tiled route takes its 128-token kernel, and fills the chip with it
 bool q6k_fills_wide(int64_t K, int64_t M, int64_t N);

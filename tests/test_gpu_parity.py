@@ -698,6 +698,29 @@ def test_q8_0_tiles_of_96_and_64_tokens(ctx, orc, m, k, ns):
         w.free()
 
 
+@pytest.mark.parametrize("m,k,ns", [(257, 512, (512, 130)), (1030, 1024, (1024, 260)), (2048, 256, (256,)), (300, 4352, (1100,)),
+                                    (512, 2048, (2048, 512, 512))])
+def test_streamed_q4k_batches_beyond_256_tokens(ctx, orc, m, k, ns):
+    """The streaming kernel's token tiles past the 256 tokens it took before, up to its last one: ragged tokens and rows, one
+    super-block, several matrices.  Against the oracle as every tiled product (2e-5: exact integer sums, K / 256 additions of
+    two terms in another order); the bits of separate calls; nothing written behind an output."""
+    from magnitude_amd import ACT_GGML, qproj
+    plan = qproj.plan_mul_mat(Q4_K, k, list(ns), m, ACT_GGML)
+    assert plan.count("gemm_stream_kernel") == len(ns), plan
+    rng = np.random.default_rng(m + k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    blocks = [make_weight(orc, Q4_K, n, k, seed=6500 + i) for i, n in enumerate(ns)]
+    ws = [ctx.upload(Q4_K, k, n, b) for n, b in zip(ns, blocks)]
+    bufs = [torch.full((m * n + 64,), 7.0, dtype=torch.float32, device="cuda") for n in ns]
+    ctx.mul_mat_multi(ws, dev(x), ACT_GGML, outs=[b[: m * n].view(m, n) for b, n in zip(bufs, ns)])
+    some = np.unique([0, 31, 63, 64, 255, 256, m // 2, m - 1])
+    for w, n, b, bl in zip(ws, ns, bufs, blocks):
+        close(b[: m * n].view(m, n).cpu().numpy()[some], orc.mul_mat(Q4_K, bl, k, x[some], orc.ACT_GGML), 2e-5)
+        assert bool((b[m * n:] == 7.0).all())
+        assert torch.equal(b[: m * n].view(m, n), ctx.mul_mat(w, dev(x), ACT_GGML))
+        w.free()
+
+
 # ---------------------------------------------------------------- MUL_MAT_ID and the MoE FFN
 
 @pytest.fixture(scope="module")
