@@ -1,5 +1,6 @@
-// Q8_0 weights x ggml Q8_0 activation blocks on the int8 matrix cores in tiles of 96 or 64 tokens x 128 weight rows: the
-// batches that the 128 x 128 tiles of gemm_per32_kernel would fill with padding to a quarter and more.
+// Q8_0 weights x ggml Q8_0 activation blocks on the int8 matrix cores in tiles of 96, 64 or 32 tokens x 128 weight rows: the
+// batches that the 128 x 128 tiles of gemm_per32_kernel would fill with padding to a quarter and more, and matrices too small
+// to fill the chip with those.
 //
 // Both operands change scale every 32 weights, so an int32 sum is valid for ONE matrix instruction and is folded into the
 // fp32 sums right away: a float from the integer, the product of the two fp16 scales (exact), one fma.  Bound: that vector
@@ -8,10 +9,11 @@
 //   - the weights are the rows of the matrix instruction, the tokens its columns: the scale of a token is one register a
 //     token column, and the sixteen scales a lane needs of its weight rows are read once for all columns of the wave;
 //   - a wave owns 32 weight rows of the tile and all of its tokens: its weights pass through a wave-private LDS strip straight
-//     from global memory, and only the activations are shared (one step of 128 weights ahead), one barrier a step;
+//     from global memory, two steps of 128 ahead (one: q/k/v of 3072 at 187 tokens, weights from HBM, 24.0 -> 29.5 us), and only the
+//     activations are shared, one step ahead, one barrier a step;
 //   - the requests to global memory go out one a product: in one go at the top of a step they hold up all waves of the workgroup
 //     (3072 -> 2 x 8192 at 187 tokens 41.5 -> 37.6 us);
-//   - at 96 tokens the addend of the matrix instruction is the bits of 1.5 * 2^23, so its sums are floats already and a
+//   - the addend of the matrix instruction is the bits of 1.5 * 2^23, so its sums are floats already and a
 //     subtraction (exact) takes the place of the conversion;
 //   - K goes in two parts over the waves of a workgroup (KW = 2) while there is at most a workgroup a compute unit, the parts
 //     meeting in LDS, and in stretches over workgroups (partial tiles, an adding pass) beyond that.
@@ -53,19 +55,18 @@ struct Q8Args {
 // [2][KW][tokens, 64 at a time][4], strips [2][wave], the scales of a step [wave][4][32] as floats
 template <int WT, int KW, int RG>
 struct Q8Lds {
-    static constexpr int kSw = WT <= 2 ? 1 : 2 /* strips a wave: one where four waves a SIMD fill each other's waits */, NW = RG * KW, kAct = WT * 4096, kDx = (WT + 1) / 2 * 1024;
-    static constexpr int kOffDx = 2 * KW * kAct, kOffStrip = kOffDx + 2 * KW * kDx, kOffWs = kOffStrip + kSw * NW * kStripBytes,
+    static constexpr int NW = RG * KW, kAct = WT * 4096, kDx = (WT + 1) / 2 * 1024;
+    static constexpr int kOffDx = 2 * KW * kAct, kOffStrip = kOffDx + 2 * KW * kDx, kOffWs = kOffStrip + 2 * NW * kStripBytes,
                          kTotal = kOffWs + NW * 512;
-    static_assert(kTotal <= 160 * 1024 / (KW == 1 ? 2 : 1) / (WT <= 2 ? 2 : 1), "eight waves a compute unit, sixteen of the smaller tile");
+    static_assert(kTotal <= 160 * 1024 / (KW == 1 ? 2 : 1), "eight waves a compute unit");
     static_assert(KW == 1 || (WT + 1) / 2 * NW * 4096 <= kOffWs, "the K parts meet in the same LDS at the end");
 };
 
 // WT columns of 32 tokens, KW K parts, RG row groups of 32 weight rows
 template <int WT, int KW, int RG>
-__global__ __launch_bounds__(64 * RG * KW, WT <= 2 ? 4 : 2) void gemm_per32_kernel_q8_0(const Q8Args g) {
+__global__ __launch_bounds__(64 * RG * KW, 2) void gemm_per32_kernel_q8_0(const Q8Args g) {
     using L = Q8Lds<WT, KW, RG>;
-    constexpr int NW = L::NW, TM = 32 * WT, SW = L::kSw;
-    constexpr bool kDeep = WT > 2;
+    constexpr int NW = L::NW, TM = 32 * WT;
     extern __shared__ __align__(16) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, lh = lane >> 5, rg = wave % RG, kp = wave / RG;
@@ -128,22 +129,38 @@ __global__ __launch_bounds__(64 * RG * KW, WT <= 2 ? 4 : 2) void gemm_per32_kern
         global_to_lds16(xbase + (xoff + ks * 4u), smem + L::kOffDx + buf * L::kDx + xg * 1024);
     };
 
-    float sum[WT][16];
+    // One column: the sums of two steps are added up by themselves first.  Such tiles take K whole, in chains of K / 64 blocks,
+    // where the 128-token tiles cut it in up to eight stretches; added eight at a time their error is no larger.
+    constexpr bool kTwoLevel = WT == 1;
+    float sum[WT][16], total[kTwoLevel ? 16 : 1];
 #pragma unroll
     for (int j = 0; j < WT; ++j)
 #pragma unroll
         for (int v = 0; v < 16; ++v) sum[j][v] = 0.f;
+    if constexpr (kTwoLevel) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) total[v] = 0.f;
+    }
+    auto fold_sums = [&]() {
+        if constexpr (kTwoLevel) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                total[v] += sum[0][v];
+                sum[0][v] = 0.f;
+            }
+        }
+    };
     v16i addend;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) addend[v] = kDeep ? __float_as_int(kMagic) : 0;
-    if constexpr (kDeep) asm volatile("" : "+v"(addend));   // in registers: rebuilt for every product it costs eight moves
+    for (int v = 0; v < 16; ++v) addend[v] = __float_as_int(kMagic);
+    asm volatile("" : "+v"(addend));   // in registers: rebuilt for every product it costs eight moves
     float *const ws_tab = reinterpret_cast<float *>(smem + L::kOffWs + wave * 512);
     // segment 2 * kb + lh of row l32 (of the strip, of a token tile): offset ^ 32 * kb
     const int foff = l32 * BK + 16 * (lh ^ ((l32 >> 1) & 7));
 
     auto step = [&](int s, auto more1, auto more2) {
         constexpr bool MORE1 = decltype(more1)::value, MORE2 = decltype(more2)::value;
-        uint8_t *const sbuf = strip + (SW == 2 ? (s & 1) * NW * kStripBytes : 0);
+        uint8_t *const sbuf = strip + (s & 1) * NW * kStripBytes;
         v4i wf[4];
 #pragma unroll
         for (int kb = 0; kb < 4; ++kb) wf[kb] = *reinterpret_cast<const v4i *>(sbuf + (foff ^ (32 * kb)));
@@ -158,7 +175,7 @@ __global__ __launch_bounds__(64 * RG * KW, WT <= 2 ? 4 : 2) void gemm_per32_kern
                 if (i < AR) global_to_lds16(abase + (aoff[i < AR ? i : 0] + ks * BK), smem + buf * L::kAct + (rg + RG * i) * 1024);
                 else global_to_lds16(xbase + (xoff + ks * 4u), smem + L::kOffDx + buf * L::kDx + xg * 1024);
             } else if (MORE2 && i > AR && i <= AR + kStripLoads) {
-                const uint32_t ks = (uint32_t)my_ks(s + SW);
+                const uint32_t ks = (uint32_t)my_ks(s + 2);
                 const int c = i - AR - 1;
                 if (c < 4) global_to_lds16(wbase + (woff[c < 4 ? c : 0] + ks * BK), sbuf + 1024 * c);
                 else global_to_lds4(dbase + (doff + ks * 4u), sbuf + 4096);
@@ -180,27 +197,6 @@ __global__ __launch_bounds__(64 * RG * KW, WT <= 2 ? 4 : 2) void gemm_per32_kern
             v4i dx[WT];   // the token's four scales
 #pragma unroll
             for (int j = 0; j < WT; ++j) dx[j] = *reinterpret_cast<const v4i *>(xb + (j * 32 + l32) * 16);
-            if constexpr (!kDeep) {   // four waves a SIMD: they fill each other's waits
-#pragma unroll
-                for (int kb = 0; kb < 4; ++kb) {
-                    v4i ws[4], af[WT];
-#pragma unroll
-                    for (int j = 0; j < WT; ++j) af[j] = *reinterpret_cast<const v4i *>(ab + j * 4096 + (foff ^ (32 * kb)));
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) ws[i] = *reinterpret_cast<const v4i *>(ws_tab + kb * 32 + 8 * i + 4 * lh);
-#pragma unroll
-                    for (int j = 0; j < WT; ++j) {
-                        const v16i I = __builtin_amdgcn_mfma_i32_32x32x32_i8(wf[kb], af[j], addend, 0, 0, 0);
-                        requests_of(kb * WT + j);
-                        const float da = __int_as_float(dx[j][kb]);
-#pragma unroll
-                        for (int v = 0; v < 16; ++v) sum[j][v] = fmaf((float)I[v], __int_as_float(ws[v >> 2][v & 3]) * da, sum[j][v]);
-#pragma unroll
-                        for (int v = 0; v < 16; ++v) asm volatile("" : "+v"(sum[j][v]));
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            } else {
             // Pinned product by product: the next one's matrix instruction goes out ahead of this one's fold, the operands of
             // the next 32 weights are read during the fold of this block's first.
             v4i ws[2][4], af[2][WT];
@@ -234,7 +230,6 @@ __global__ __launch_bounds__(64 * RG * KW, WT <= 2 ? 4 : 2) void gemm_per32_kern
                 for (int v = 0; v < 16; ++v) asm volatile("" : "+v"(sum[j][v]));
                 __builtin_amdgcn_sched_barrier(0);
             }
-            }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         } else {
 #pragma unroll
@@ -242,7 +237,7 @@ __global__ __launch_bounds__(64 * RG * KW, WT <= 2 ? 4 : 2) void gemm_per32_kern
         }
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (MORE1) {
-            if constexpr (MORE2 && SW == 2) wait_vmcnt<kStripLoads>();   // all but the strip just asked for
+            if constexpr (MORE2) wait_vmcnt<kStripLoads>();   // all but the strip just asked for
             else wait_vmcnt<0>();
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         }
@@ -250,19 +245,22 @@ __global__ __launch_bounds__(64 * RG * KW, WT <= 2 ? 4 : 2) void gemm_per32_kern
     if (n_steps > 0) {
         request_strip(0, strip);
         request_acts(0);
-        if constexpr (SW == 2) {
-            request_strip(1, strip + NW * kStripBytes);   // (of a single step: once more)
-            wait_vmcnt<kStripLoads>();
-        } else {
-            wait_vmcnt<0>();
-        }
+        request_strip(1, strip + NW * kStripBytes);   // (of a single step: once more)
+        wait_vmcnt<kStripLoads>();
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         int s = 0;
-        for (; s + SW < n_steps; ++s) step(s, std::true_type{}, std::true_type{});
-        if (SW == 2 && s + 1 < n_steps) step(s++, std::true_type{}, std::false_type{});
+        for (; s + 2 < n_steps; ++s) {
+            step(s, std::true_type{}, std::true_type{});
+            if (s & 1) fold_sums();
+        }
+        if (s + 1 < n_steps) step(s++, std::true_type{}, std::false_type{});
         step(s, std::false_type{}, std::false_type{});
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (a single step leaves its second strip request behind)
+    if constexpr (kTwoLevel) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sum[0][v] += total[v];
+    }
 
     // ---- the K parts meet in LDS: part q keeps token tiles j % 2 == q, the other hands its sums over
     if constexpr (KW == 2) {
@@ -315,23 +313,28 @@ struct Q8Plan {
     int64_t tiles;
 };
 
+// q, k, v and o: square matrices and small ones, whose launch holds a matrix and a half of K rows as a rule
+bool rider(int64_t K, int64_t N) { return K == N || N <= 1024; }
+int64_t rider_tiles(int64_t K, int64_t M) { return (M + 31) / 32 * ((K + K / 2 + 127) / 128); }
+
 // Tile and cut of a matrix this kernel takes, by the matrix and the row count alone (the bits of its results do not depend on
 // what rides along).
 Q8Plan q8_plan(int64_t K, int64_t M, int64_t N) {
     const int64_t cus = cu_count(), units = (K + 255) / 256;
     Q8Plan p{};
-    p.wt = tuning_int("QPROJ_Q8_WT", M <= 64 ? 2 : 3);
+    p.wt = tuning_int("QPROJ_Q8_WT", rider(K, N) ? 1 : M <= 64 ? 2 : 3);
     const int64_t tiles_m = (M + 32 * p.wt - 1) / (32 * p.wt);
     p.tiles = tiles_m * ((N + 127) / 128);
     // (a matrix taller than its rows are long has a sibling in the launch as a rule: up beside gate)
-    const int64_t tiles = N > K ? 2 * p.tiles : p.tiles;
+    const int64_t tiles = rider(K, N) ? rider_tiles(K, M) : N > K ? 2 * p.tiles : p.tiles;
     // Up to a workgroup a compute unit K goes in two parts inside the workgroup, and in stretches that fill the chip once; beyond
     // that workgroups of four waves share a compute unit out of step (3072 -> 2 x 8192 at 187 tokens 37.6 against 44.9 us, 4096 ->
     // 2 x 14336 122 either way).
     p.kw = tuning_int("QPROJ_Q8_KW", tiles > cus ? 1 : 2);
     int64_t n = std::max<int64_t>(1, std::min<int64_t>(8, cus / tiles));
-    // never longer sums than the 128 x 128 tiles have (their error against 64 bits grows with the length)
-    n = std::max<int64_t>(n, (per32_splits(kTypeQ8_0, K, M, N) + p.kw - 1) / p.kw);
+    // never longer sums than the 128 x 128 tiles have (their error against 64 bits grows with the length; the tiles of 32 tokens
+    // add theirs up in two levels instead)
+    if (p.wt > 1) n = std::max<int64_t>(n, (per32_splits(kTypeQ8_0, K, M, N) + p.kw - 1) / p.kw);
     n = tuning_int("QPROJ_Q8_SPLIT", (int)n);
     n = std::max<int64_t>(1, std::min<int64_t>(n, units / 2));   // two times 256 weights a stretch at least
     if ((M * N) % 4 != 0) n = 1;
@@ -358,10 +361,16 @@ hipError_t launch(const Q8Args &g, int wgs, hipStream_t s) {
 // the tiles of 96 or 64 tokens are not.  129 .. 192 tokens, and rows longer than the matrix is tall up to 96 tokens.
 // us a call at 160 tokens, 128-token tiles / here: 3072 -> 2 x 8192 50.3 / 39.2, 4096 -> 2 x 14336 96 / 80, 4096 -> 32000 100 / 84,
 // 8192 -> 3072 38.0 / 33.4, 14336 -> 4096 66.2 / 52.3, 28672 -> 8192 210 / 143; at 64 tokens 8192 -> 3072 26.4 / 23.8, 28672 -> 8192
-// 114 / 86.  Square and small matrices gained nothing (4096 x 4096 at 160 tokens 29.2 / 32.4), nor did 1024 -> 2 x 2816 (19.1 / 19.9).
+// 114 / 86.  Not 1024 -> 2 x 2816 (19.1 / 19.9).
+// Square and small matrices take tiles of 32 tokens while they are one round of workgroups: the grid is filled with few
+// stretches of K or none, so the partial tiles and their adding pass go.  q/k/v of 2048 at 33 / 128 / 250 tokens 16.6 / 14.1,
+// 19.4 / 16.7, 23.6 / 18.4, of 3072 at 64 / 187 21.7 / 18.0, 30.0 / 24.0 (at 128 24.2 / 23.5 but 3072 x 3072 21.6 / 22.7: not taken), of 4096 at 64
+// 26.7 / 22.4 (at 128 26.9 / 28.5: not taken).
 bool q8_0_tokens_takes(int64_t K, int64_t M, int64_t N) {
     if (K % BK != 0 || K > (1 << 24)) return false;   // 32-bit lane offsets: 128 rows of K bytes
-    if (K == N || N <= 1024 || K <= 1024) return false;   // q, k, v, o: small grids that want many short stretches
+    if (tuning_int("QPROJ_Q8_TAKE", 0)) return true;
+    if (K <= 1024) return false;
+    if (rider(K, N)) return (K <= 3072 && rider_tiles(K, M) * (M > 128 ? 1 : 2) <= cu_count()) || (K <= 4096 && M <= 64);
     return (M > 128 && M <= 192) || (M > 32 && M <= 96 && K > N && N <= 32768);
 }
 
@@ -434,10 +443,17 @@ hipError_t launch_gemm_q8_0_tokens(int n, const WeightView *w, const ActView &a,
         hipError_t e = hipErrorInvalidValue;
 #define QP_Q8(WT, KW, RG) \
     if (p0.wt == WT && p0.kw == KW && rg == RG) e = launch<WT, KW, RG>(g, (int)wg, s)
+        QP_Q8(1, 2, 4);
         QP_Q8(2, 2, 4);
         QP_Q8(3, 1, 4);
         QP_Q8(3, 2, 4);
         QP_Q8(3, 2, 2);
+#ifdef QPROJ_TUNING
+        QP_Q8(1, 1, 4);
+        QP_Q8(2, 1, 4);
+        QP_Q8(4, 1, 4);
+        QP_Q8(4, 2, 4);
+#endif
 #undef QP_Q8
         if (e == hipSuccess && sums.n) e = launch_sum_parts(sums, s);
         if (e != hipSuccess) return e;

@@ -675,9 +675,10 @@ def test_q8_0_matrices_of_a_call_share_a_launch(ctx, orc, m, k, ns):
 
 @pytest.mark.parametrize("m,k,ns", [(129, 1152, (2050,)), (187, 1280, (1025, 1031)), (192, 1536, (1284,)), (160, 2048, (1100,)),
                                     (33, 1280, (1028,)), (64, 4352, (1026,)), (65, 1408, (1100,)), (96, 2560, (1030, 1300)),
-                                    (130, 1152, (33000,))])
-def test_q8_0_tiles_of_96_and_64_tokens(ctx, orc, m, k, ns):
-    """gemm_per32_kernel_q8_0: both token tiles with ragged tokens and rows, K in parts and stretches with an odd number of steps of
+                                    (130, 1152, (33000,)), (33, 1152, (1152, 130)), (65, 1280, (1280,)), (187, 2048, (2048, 510, 6)),
+                                    (250, 2176, (2176, 4))])
+def test_q8_0_tiles_of_96_64_and_32_tokens(ctx, orc, m, k, ns):
+    """gemm_per32_kernel_q8_0: the token tiles with ragged tokens and rows, K in parts and stretches with an odd number of steps of
     128, outputs whose rows are no whole float4s, workgroups of 64 and 128 rows, more tiles than compute units (K in one part).
     Against the oracle (5e-5 of the larger of 1 and the result, exact block sums and K / 32 fp32 additions in another order);
     nothing written behind an output."""
