@@ -180,7 +180,7 @@ int qproj_mul_mat(qproj_ctx *ctx, const qproj_weight *w, const float *x_dev, int
 
 /* Several MUL_MATs that share one activation (q/k/v, gate/up) in one launch: y_dev[i] is
  * [M][N_i].  Same results as n separate qproj_mul_mat calls: bit for bit for Q8_0 and Q6_K tensors from 33 rows on and
- * for Q4_K tensors wherever the streaming kernel serves them (33..256 rows, see qproj_plan_mul_mat), where the tile and
+ * for Q4_K tensors wherever the streaming kernel serves them (33..256 rows, smaller ones up to 2048: qproj_plan_mul_mat), where the tile and
  * the cut of K follow from a tensor and the row count alone.  Elsewhere (5..32 rows, larger Q4_K batches) K may be cut
  * differently beside other tensors: the same integer dot products, their fp32 sums in another order. */
 int qproj_mul_mat_multi(qproj_ctx *ctx, int n, const qproj_weight *const *w, const float *x_dev,
