@@ -681,11 +681,14 @@ int grouped_mt(int64_t n_pairs, int64_t E) {
 // tokens (2.5 / 4 / 6.2 / 31 pairs an expert) 89 / 91.5, 103 / 94, 105 / 97, 208 / 127; 64 of 1024 x 512 at 3.8 pairs
 // 41.8 / 33.2; 32 of 4096 x 512 at 4 / 6.2 pairs 42.7 / 45.8, 50.5 / 46.4; 256 of 1024 x 2048 at 2.8 / 7.8 pairs 202 / 214, 277 / 239.
 // Popular experts take tiles of their own: the 128 experts with popularity e^N(0,1), 500 tokens, 462 / 162.
+// A tile has one running sum over the whole row.  Where the grouped kernel cuts K over waves or chunks (few experts, few
+// rows), rows beyond 1024 weights stay with it: error against 64 bits, tiles over grouped, 8 experts x 512 rows of 1024 / 1280 /
+// 1536 / 2048 / 4096 / 8192 weights 0.95 / 0.98 / 1.006 / 1.05 / 1.12 / 1.35.
 bool moe_stream_route(int type, int64_t K, int64_t N, int64_t n_pairs, int64_t E) {
     static const int per_4_experts = tuning_int("QPROJ_MOE_STREAM_PAIRS_PER_4_EXPERTS", 0);
     const bool many = per_4_experts ? 4 * n_pairs >= per_4_experts * E
                                     : n_pairs > 4 * E || (2 * n_pairs >= 7 * E && E * N >= (int64_t)2 * 64 * cu_count());
-    return many && moe_stream_fits(type, K, N);
+    return many && moe_stream_fits(type, K, N) && (K <= 1024 || mfma_grouped_whole_rows(type, K, N, E, n_pairs));
 }
 
 }  // namespace

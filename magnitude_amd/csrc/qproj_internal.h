@@ -215,6 +215,7 @@ hipError_t launch_moe_group(const int32_t *ids, int64_t n_pairs, int64_t n_exper
                             const RowQuantJob *quantize, hipStream_t s, int64_t tile_rows = 0);
 // rows of an expert's pairs that a pass of the grouped matrix-core kernel stages (8, 16 or 32)
 int mfma_grouped_pass_rows(int type, int64_t K, int64_t N, int64_t E, int64_t n_pairs);
+bool mfma_grouped_whole_rows(int type, int64_t K, int64_t N, int64_t E, int64_t n_pairs);
 // expert batches in tiles of kMoeTileRows pairs (`a` with its hsum plane, args.active a tile list): y[pair][N], or with
 // `swiglu` silu(t[0] . x) * (t[1] . x)
 bool moe_stream_fits(int type, int64_t K, int64_t N);

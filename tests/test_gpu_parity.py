@@ -779,10 +779,10 @@ def test_mul_mat_id_grouping_of_many_pairs(ctx, orc, E, B):
 
 
 @pytest.mark.parametrize("k,n,counts", [(256, 63, (1, 31, 32, 33, 0, 64, 65)), (768, 129, (0, 129, 1, 63, 5)),
-                                        (2048, 64, (96, 2, 2)), (8192, 40, (70, 33)), (512, 1, (40,))])
+                                        (1024, 64, (96, 2, 2)), (2304, 1024, (70, 33) + (1,) * 30), (512, 1, (40,))])
 def test_expert_tiles_at_their_edges(ctx, orc, k, n, counts):
     """moe_stream_kernel: tiles of 1 .. 64 pairs of an expert (one and two token tiles, full and ragged, an expert without
-    pairs), rows beyond the last whole row tile, one super-block and the longest rows; a pair of a bad expert is left out
+    pairs), rows beyond the last whole row tile, one super-block and rows beyond 1024 weights (whole in the grouped kernel too); a pair of a bad expert is left out
     and reported, the others are computed.  Tolerance as for every single projection: the integer sums are exact, K / 256
     fp32 additions in another order."""
     from magnitude_amd import ACT_GGML, QprojError
@@ -809,7 +809,7 @@ def test_expert_tiles_at_their_edges(ctx, orc, k, n, counts):
     w.free()
 
 
-@pytest.mark.parametrize("E,top,B,d_model,d_ff", [(6, 2, 97, 512, 256), (8, 3, 60, 768, 1280), (64, 5, 64, 256, 512)])
+@pytest.mark.parametrize("E,top,B,d_model,d_ff", [(6, 2, 97, 512, 256), (8, 3, 60, 768, 1024), (64, 5, 64, 256, 512)])
 def test_moe_ffn_in_expert_tiles(ctx, orc, E, top, B, d_model, d_ff):
     """Gate and up sixteen rows each in a matrix instruction, their swiglu in registers; tolerance as for the other
     feed-forwards (a code of the re-quantized rows on a rounding tie), the half of the outputs without one to 1e-6."""
