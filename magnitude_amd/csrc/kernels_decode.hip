@@ -445,6 +445,7 @@ hipError_t launch_decode_mt(const GemvArgs &args, int mt, hipStream_t s) {
 }  // namespace
 
 int cu_count() {
+    if (plan_cu_count() > 0) return plan_cu_count();
     static int n = [] {
         int dev = 0, v = 0;
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) v = 256;

@@ -329,8 +329,9 @@ Q8Plan q8_plan(int64_t K, int64_t M, int64_t N) {
     const int64_t tiles = rider(K, N) ? rider_tiles(K, M) : N > K ? 2 * p.tiles : p.tiles;
     // Up to a workgroup a compute unit K goes in two parts inside the workgroup, and in stretches that fill the chip once; beyond
     // that workgroups of four waves share a compute unit out of step (3072 -> 2 x 8192 at 187 tokens 37.6 against 44.9 us, 4096 ->
-    // 2 x 14336 122 either way).
-    p.kw = tuning_int("QPROJ_Q8_KW", tiles > cus ? 1 : 2);
+    // 2 x 14336 122 either way).  The tiles of 32 and 64 tokens are built with two parts only:
+    // q8_0_tokens_takes leaves their larger grids to the 128-token tiles.
+    p.kw = tuning_int("QPROJ_Q8_KW", p.wt >= 3 && tiles > cus ? 1 : 2);
     int64_t n = std::max<int64_t>(1, std::min<int64_t>(8, cus / tiles));
     // never longer sums than the 128 x 128 tiles have (their error against 64 bits grows with the length; the tiles of 32 tokens
     // add theirs up in two levels instead)
@@ -355,6 +356,25 @@ hipError_t launch(const Q8Args &g, int wgs, hipStream_t s) {
     return hipGetLastError();
 }
 
+using LaunchFn = hipError_t (*)(const Q8Args &, int, hipStream_t);
+LaunchFn instance(int wt, int kw, int rg) {   // null: not built
+#define QP_Q8(WT, KW, RG) \
+    if (wt == WT && kw == KW && rg == RG) return &launch<WT, KW, RG>
+    QP_Q8(1, 2, 4);
+    QP_Q8(2, 2, 4);
+    QP_Q8(3, 1, 4);
+    QP_Q8(3, 2, 4);
+    QP_Q8(3, 2, 2);
+#ifdef QPROJ_TUNING
+    QP_Q8(1, 1, 4);
+    QP_Q8(2, 1, 4);
+    QP_Q8(4, 1, 4);
+    QP_Q8(4, 2, 4);
+#endif
+#undef QP_Q8
+    return nullptr;
+}
+
 }  // namespace
 
 // Which products this kernel takes from the 128 x 128 tiles: where a 128-token tile is padding for a quarter and more and
@@ -370,8 +390,9 @@ bool q8_0_tokens_takes(int64_t K, int64_t M, int64_t N) {
     if (K % BK != 0 || K > (1 << 24)) return false;   // 32-bit lane offsets: 128 rows of K bytes
     if (tuning_int("QPROJ_Q8_TAKE", 0)) return true;
     if (K <= 1024) return false;
-    if (rider(K, N)) return (K <= 3072 && rider_tiles(K, M) * (M > 128 ? 1 : 2) <= cu_count()) || (K <= 4096 && M <= 64);
-    return (M > 128 && M <= 192) || (M > 32 && M <= 96 && K > N && N <= 32768);
+    const int64_t cus = cu_count();
+    if (rider(K, N)) return (K <= 3072 && rider_tiles(K, M) * (M > 128 ? 1 : 2) <= cus) || (K <= 4096 && M <= 64 && rider_tiles(K, M) <= cus);
+    return (M > 128 && M <= 192) || (M > 32 && M <= 96 && K > N && N <= 128 * cus);
 }
 
 size_t q8_0_tokens_scratch_bytes(int64_t K, int64_t M, int64_t N) { return partial_bytes(q8_plan(K, M, N), M, N); }
@@ -402,6 +423,8 @@ hipError_t launch_gemm_q8_0_tokens(int n, const WeightView *w, const ActView &a,
         int64_t halves = 0;
         for (int i = first; i < n && shares(i); ++i) halves += tiles_pad(i, 64) * plans[i].n_split;
         const int rg = tuning_int("QPROJ_Q8_RG", p0.wt == 3 && p0.kw == 2 && halves <= cu_count() ? 2 : 4);
+        const LaunchFn run = instance(p0.wt, p0.kw, rg);
+        if (!run) return hipErrorInvalidValue;   // (in a dry run too)
         SumTargets sums{};
         size_t used = 0;
         int64_t wg = 0;
@@ -440,21 +463,7 @@ hipError_t launch_gemm_q8_0_tokens(int n, const WeightView *w, const ActView &a,
             if (sums.n) plan_note_cut();
             continue;
         }
-        hipError_t e = hipErrorInvalidValue;
-#define QP_Q8(WT, KW, RG) \
-    if (p0.wt == WT && p0.kw == KW && rg == RG) e = launch<WT, KW, RG>(g, (int)wg, s)
-        QP_Q8(1, 2, 4);
-        QP_Q8(2, 2, 4);
-        QP_Q8(3, 1, 4);
-        QP_Q8(3, 2, 4);
-        QP_Q8(3, 2, 2);
-#ifdef QPROJ_TUNING
-        QP_Q8(1, 1, 4);
-        QP_Q8(2, 1, 4);
-        QP_Q8(4, 1, 4);
-        QP_Q8(4, 2, 4);
-#endif
-#undef QP_Q8
+        hipError_t e = run(g, (int)wg, s);
         if (e == hipSuccess && sums.n) e = launch_sum_parts(sums, s);
         if (e != hipSuccess) return e;
     }

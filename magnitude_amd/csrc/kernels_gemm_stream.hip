@@ -612,6 +612,27 @@ hipError_t launch_stream_kernel(const StreamArgs &g, int wgs, hipStream_t s) {
     return hipGetLastError();
 }
 
+using LaunchFn = hipError_t (*)(const StreamArgs &, int, hipStream_t);
+LaunchFn instance(int type, int jt, int kw, int waves) {   // null: not built
+#define QP_STREAM(QT, JT, KW, SW, NW) \
+    if (type == QT && jt == JT && kw == KW && waves == NW) return &launch_stream_kernel<QT, JT, KW, SW, NW>
+    // (64-token tiles with K in one part are only taken by grids beyond a round of the halves)
+    QP_STREAM(kTypeQ4_K, 2, 1, 2, 8);
+    QP_STREAM(kTypeQ4_K, 2, 2, 2, 8);
+    QP_STREAM(kTypeQ4_K, 2, 2, 2, 4);
+    QP_STREAM(kTypeQ4_K, 3, 1, 2, 8);
+    QP_STREAM(kTypeQ4_K, 3, 1, 2, 4);
+    QP_STREAM(kTypeQ6_K, 2, 1, 2, 8);
+    QP_STREAM(kTypeQ6_K, 2, 2, 1, 8);
+    QP_STREAM(kTypeQ6_K, 2, 2, 1, 4);
+    QP_STREAM(kTypeQ6_K, 3, 1, 1, 8);
+    QP_STREAM(kTypeQ6_K, 3, 1, 1, 4);
+    QP_STREAM(kTypeQ6_K, 4, 1, 1, 8);
+    QP_STREAM(kTypeQ6_K, 4, 1, 1, 4);
+#undef QP_STREAM
+    return nullptr;
+}
+
 }  // namespace
 
 // Which products the streaming kernel takes.  From 33 tokens (below, the small-batch kernel) to 256, and Q4_K beyond while its
@@ -735,25 +756,10 @@ hipError_t launch_group(int n, const WeightView *w, const StreamPlan *plans, con
                       t.n_split > 1 ? " + sum_parts_kernel" : "");
         }
         if (wg >= 0x7fffffff) return hipErrorInvalidValue;
+        const LaunchFn run = instance(w[0].type, p0.jt, p0.kw, waves);
+        if (!run) return hipErrorInvalidValue;   // (in a dry run too)
         if (dry_run()) continue;
-        hipError_t e = hipErrorInvalidValue;
-#define QP_STREAM(QT, JT, KW, SW, NW)                                             \
-    if (w[0].type == QT && p0.jt == JT && p0.kw == KW && waves == NW)             \
-        e = launch_stream_kernel<QT, JT, KW, SW, NW>(g, (int)wg, s)
-        // (64-token tiles with K in one part are only taken by grids beyond a round of the halves)
-        QP_STREAM(kTypeQ4_K, 2, 1, 2, 8);
-        QP_STREAM(kTypeQ4_K, 2, 2, 2, 8);
-        QP_STREAM(kTypeQ4_K, 2, 2, 2, 4);
-        QP_STREAM(kTypeQ4_K, 3, 1, 2, 8);
-        QP_STREAM(kTypeQ4_K, 3, 1, 2, 4);
-        QP_STREAM(kTypeQ6_K, 2, 1, 2, 8);
-        QP_STREAM(kTypeQ6_K, 2, 2, 1, 8);
-        QP_STREAM(kTypeQ6_K, 2, 2, 1, 4);
-        QP_STREAM(kTypeQ6_K, 3, 1, 1, 8);
-        QP_STREAM(kTypeQ6_K, 3, 1, 1, 4);
-        QP_STREAM(kTypeQ6_K, 4, 1, 1, 8);
-        QP_STREAM(kTypeQ6_K, 4, 1, 1, 4);
-#undef QP_STREAM
+        const hipError_t e = run(g, (int)wg, s);
         if (e != hipSuccess) return e;
     }
     if (dry_run() || sg.n == 0) return hipSuccess;

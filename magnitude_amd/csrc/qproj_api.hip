@@ -20,12 +20,14 @@ namespace qproj {
 namespace {
 thread_local bool g_dry_run = false;
 thread_local size_t g_scratch_shave = 0;    // dry runs only: bytes withheld from what the launchers are told they have
+thread_local int g_plan_cus = 0;            // dry runs only: compute units to plan for, 0 = the device's
 thread_local int g_plan_cuts = 0;           // dry runs only: launches noted that cut K into parts kept in scratch
 thread_local std::string *g_plan = nullptr;   // where plan_note writes; null: nobody is listening
 }
 bool dry_run() { return g_dry_run; }
 size_t scratch_shave() { return g_dry_run ? g_scratch_shave : 0; }
 void set_dry_run(bool on) { g_dry_run = on; }
+int plan_cu_count() { return g_dry_run ? g_plan_cus : 0; }
 
 void plan_note_cut() { ++g_plan_cuts; }
 
@@ -694,6 +696,10 @@ bool moe_stream_route(int type, int64_t K, int64_t N, int64_t n_pairs, int64_t E
 }  // namespace
 
 extern "C" {
+
+// For the tests of the dispatch: the plans and scratch sizes that this thread asks for are those of a GPU (or a partition of
+// one) with this many compute units; 0 = the device's again.  Calls that launch are not affected.
+void qproj_internal_plan_cus(int cus) { g_plan_cus = cus; }
 
 const char *qproj_version(void) { return "qproj-0.1-gfx950"; }
 

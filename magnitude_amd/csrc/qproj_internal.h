@@ -145,8 +145,10 @@ inline int64_t moe_list_capacity(int64_t n_expert, int64_t n_pairs, int64_t tile
 constexpr int kMoeTileRows = 64;      // pairs of an expert that a pass of moe_stream_kernel takes
 constexpr int kMoeStreamMaxSb = 32;   // super-blocks of a row whose activation scales it keeps in LDS
 
-// Compute units of the current device (256 when no device can be asked, e.g. in a dry run on a host without one).
+// Compute units of the current device (256 when no device can be asked, e.g. in a dry run on a host without one; a dry run
+// may be told another number, qproj_internal_plan_cus).
 int cu_count();
+int plan_cu_count();   // 0: not told
 
 // Tuning knobs read from the environment exist only in builds made with -DQPROJ_TUNING (kernel-selection sweeps in
 // the lab); in the shipped library this returns `dflt` and no environment variable can change a numerics path.

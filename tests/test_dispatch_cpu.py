@@ -235,3 +235,20 @@ def test_no_q8_0_stretch_of_k_is_empty():
         line = [l for l in qproj.plan_mul_mat(Q8_0, k, (n,), m).splitlines() if "gemm_per32_kernel" in l][0]
         stretches, units = int(re.search(r"x (\d+) K stretches", line)[1]), (k + 255) // 256
         assert (stretches - 1) * -(-units // stretches) < units, (k, n, m, line)
+
+
+@pytest.mark.parametrize("cus", [16, 32, 38, 64, 76, 128, 152, 256, 304])
+def test_every_call_is_served_whatever_the_number_of_compute_units(cus):
+    """A partition of the GPU has fewer compute units (32 and 64 in its smaller modes), and the plans follow their number:
+    what they name has to be there, and what a GPU of 256 units serves is served on the others."""
+    lib = qproj.load_library()
+    lib.qproj_internal_plan_cus(cus)
+    try:
+        for qt, m, k, ns in itertools.product([Q8_0, Q4_K, Q6_K], [3, 16, 33, 48, 64, 65, 96, 128, 129, 187, 192, 250, 300, 512, 2048],
+                                              [512, 1536, 2048, 3072, 4096, 8192, 28672],
+                                              [(512,), (1024,), (4096,), (6144,), (20480,), (32000,), (32768,), (4096, 1024, 1024), (8192, 8192), (3072, 3072, 3072)]):
+            qproj.workspace_bytes(qt, k, ns, m)     # (raises where a launcher refuses)
+        for tokens, experts, d, ff in itertools.product([1, 16, 64, 300], [8, 64, 256], [1024, 4096], [768, 2048]):
+            qproj.plan_moe_ffn(Q4_K, Q4_K, d, ff, experts, 4, tokens)
+    finally:
+        lib.qproj_internal_plan_cus(0)
