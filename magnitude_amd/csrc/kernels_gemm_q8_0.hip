@@ -1,5 +1,5 @@
-// Q8_0 weights x ggml Q8_0 activation blocks on the int8 matrix cores in tiles of 96, 64 or 32 tokens x 128 weight rows: the
-// batches that the 128 x 128 tiles of gemm_per32_kernel would fill with padding to a quarter and more, and matrices too small
+// Q8_0 weights x ggml Q8_0 activation blocks on the int8 matrix cores in tiles of 96 or 64 tokens x 128 weight rows or 32
+// tokens x 64: the batches that the 128 x 128 tiles of gemm_per32_kernel would fill with padding to a quarter and more, and matrices too small
 // to fill the chip with those.
 //
 // Both operands change scale every 32 weights, so an int32 sum is valid for ONE matrix instruction and is folded into the
@@ -58,7 +58,7 @@ struct Q8Lds {
     static constexpr int NW = RG * KW, kAct = WT * 4096, kDx = (WT + 1) / 2 * 1024;
     static constexpr int kOffDx = 2 * KW * kAct, kOffStrip = kOffDx + 2 * KW * kDx, kOffWs = kOffStrip + 2 * NW * kStripBytes,
                          kTotal = kOffWs + NW * 512;
-    static_assert(kTotal <= 160 * 1024 / (KW == 1 ? 2 : 1), "eight waves a compute unit");
+    static_assert(kTotal <= 160 * 1024 / (KW == 1 || (WT == 1 && NW == 4) ? 2 : 1), "eight waves a compute unit");
     static_assert(KW == 1 || (WT + 1) / 2 * NW * 4096 <= kOffWs, "the K parts meet in the same LDS at the end");
 };
 
@@ -360,12 +360,13 @@ using LaunchFn = hipError_t (*)(const Q8Args &, int, hipStream_t);
 LaunchFn instance(int wt, int kw, int rg) {   // null: not built
 #define QP_Q8(WT, KW, RG) \
     if (wt == WT && kw == KW && rg == RG) return &launch<WT, KW, RG>
-    QP_Q8(1, 2, 4);
+    QP_Q8(1, 2, 2);
     QP_Q8(2, 2, 4);
     QP_Q8(3, 1, 4);
     QP_Q8(3, 2, 4);
     QP_Q8(3, 2, 2);
 #ifdef QPROJ_TUNING
+    QP_Q8(1, 2, 4);
     QP_Q8(1, 1, 4);
     QP_Q8(2, 1, 4);
     QP_Q8(4, 1, 4);
@@ -422,7 +423,11 @@ hipError_t launch_gemm_q8_0_tokens(int n, const WeightView *w, const ActView &a,
         // compute units (a matrix is cut as if its sibling rode along; 3072 -> 8192 alone at 187 tokens 35.0 -> 27.8 us).
         int64_t halves = 0;
         for (int i = first; i < n && shares(i); ++i) halves += tiles_pad(i, 64) * plans[i].n_split;
-        const int rg = tuning_int("QPROJ_Q8_RG", p0.wt == 3 && p0.kw == 2 && halves <= cu_count() ? 2 : 4);
+        // Tiles of 32 tokens always: two workgroups of four waves share a compute unit (56 KB of LDS each) and hide each other's
+        // barriers, and q/k/v a little beyond a round of eight-wave workgroups do not take two.  us a call, tiles of 128 tokens / 128
+        // rows a workgroup / 64: q/k/v of 2560 with 1024 for k and v at 97 tokens 21.8 / 28.0 / 23.5, of 3072 at 187 30.7 / 25.1 / 24.3
+        // and at 193 30.9 / 38.6 / 33.6, three of 2048 at 80 21.0 / 24.5 / 21.9; 3072 -> 1024 alone at 187 18.8 / 22.4 / 17.8.
+        const int rg = tuning_int("QPROJ_Q8_RG", p0.wt == 1 || (p0.wt == 3 && p0.kw == 2 && halves <= cu_count()) ? 2 : 4);
         const LaunchFn run = instance(p0.wt, p0.kw, rg);
         if (!run) return hipErrorInvalidValue;   // (in a dry run too)
         SumTargets sums{};

@@ -252,3 +252,12 @@ def test_every_call_is_served_whatever_the_number_of_compute_units(cus):
             qproj.plan_moe_ffn(Q4_K, Q4_K, d, ff, experts, 4, tokens)
     finally:
         lib.qproj_internal_plan_cus(0)
+
+
+@pytest.mark.parametrize("m,k,ns", [(97, 2560, (2560, 1024, 1024)), (193, 3072, (3072, 1024, 1024)), (80, 2048, (2048, 2048, 2048)),
+                                    (187, 3072, (1024,)), (48, 4096, (1024,))])
+def test_q8_0_tiles_of_32_tokens_are_half_a_compute_unit(m, k, ns):
+    """Workgroups of four waves: q/k/v beyond one round of larger ones would take two, and k or v alone would leave most of
+    the chip idle."""
+    plan = qproj.plan_mul_mat(Q8_0, k, ns, m)
+    assert plan.count("gemm_per32_kernel_q8_0<1 token tiles") == plan.count("tile 32 tokens x 64 rows") == len(ns), plan
