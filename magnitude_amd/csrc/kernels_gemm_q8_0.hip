@@ -310,7 +310,6 @@ __global__ __launch_bounds__(64 * RG * KW, 2) void gemm_per32_kernel_q8_0(const 
 
 struct Q8Plan {
     int wt, kw, n_split;
-    int64_t tiles;
 };
 
 // q, k, v and o: square matrices and small ones, whose launch holds a matrix and a half of K rows as a rule
@@ -324,9 +323,12 @@ Q8Plan q8_plan(int64_t K, int64_t M, int64_t N) {
     Q8Plan p{};
     p.wt = tuning_int("QPROJ_Q8_WT", rider(K, N) ? 1 : M <= 64 ? 2 : 3);
     const int64_t tiles_m = (M + 32 * p.wt - 1) / (32 * p.wt);
-    p.tiles = tiles_m * ((N + 127) / 128);
+    // workgroups of a stretch, the same number on each of the 8 XCDs: 8192 -> 2304 at 160 tokens is 36 tiles, five on four of
+    // the XCDs; seven stretches of them are 252 workgroups, but 35 for the 32 units of those (32.8 us in 128-token tiles, 39.5 in
+    // seven stretches, 30.5 in six)
+    const int64_t stretch = (tiles_m * ((N + 127) / 128) + 7) / 8 * 8;
     // (a matrix taller than its rows are long has a sibling in the launch as a rule: up beside gate)
-    const int64_t tiles = rider(K, N) ? rider_tiles(K, M) : N > K ? 2 * p.tiles : p.tiles;
+    const int64_t tiles = rider(K, N) ? rider_tiles(K, M) : N > K ? 2 * stretch : stretch;
     // Up to a workgroup a compute unit K goes in two parts inside the workgroup, and in stretches that fill the chip once; beyond
     // that workgroups of four waves share a compute unit out of step (3072 -> 2 x 8192 at 187 tokens 37.6 against 44.9 us, 4096 ->
     // 2 x 14336 122 either way).  The tiles of 32 and 64 tokens are built with two parts only:

@@ -261,3 +261,21 @@ def test_q8_0_tiles_of_32_tokens_are_half_a_compute_unit(m, k, ns):
     the chip idle."""
     plan = qproj.plan_mul_mat(Q8_0, k, ns, m)
     assert plan.count("gemm_per32_kernel_q8_0<1 token tiles") == plan.count("tile 32 tokens x 64 rows") == len(ns), plan
+
+
+def q8_0_launch_workgroups(k, ns, m):
+    """workgroups a launch of 96- or 64-token tiles with two K parts puts on the 8 XCDs (one a compute unit), 0 for other kernels"""
+    lines = re.findall(r"gemm_per32_kernel_q8_0<[23] token tiles, 2 K parts>.* (\d+) tiles x (\d+) K stretches", qproj.plan_mul_mat(Q8_0, k, ns, m))
+    return sum((int(tiles) + 7) // 8 * 8 * int(stretches) for tiles, stretches in lines)
+
+
+def test_q8_0_stretches_are_one_round_on_every_xcd():
+    """The stretches of a matrix are counted in workgroups as the XCDs get them: 36 tiles are five on four of them, so seven
+    stretches are 35 workgroups for 32 compute units there."""
+    seen = 0
+    for k, n, m in itertools.product(range(1536, 16384, 512), range(1280, 8192, 256), (33, 64, 96, 129, 192)):
+        if k > n:
+            wgs = q8_0_launch_workgroups(k, (n,), m)
+            assert wgs <= 256, (k, n, m, wgs)
+            seen += wgs > 0
+    assert seen > 500
