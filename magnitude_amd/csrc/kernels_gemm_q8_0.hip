@@ -310,6 +310,7 @@ __global__ __launch_bounds__(64 * RG * KW, 2) void gemm_per32_kernel_q8_0(const 
 
 struct Q8Plan {
     int wt, kw, n_split;
+    bool one_round;   // of workgroups, one a compute unit (two K parts)
 };
 
 // q, k, v and o: square matrices and small ones, whose launch holds a matrix and a half of K rows as a rule
@@ -343,6 +344,7 @@ Q8Plan q8_plan(int64_t K, int64_t M, int64_t N) {
     if ((M * N) % 4 != 0) n = 1;
     while (n > 1 && (units + n - 2) / (n - 1) == (units + n - 1) / n) --n;   // no stretch without work
     p.n_split = (int)n;
+    p.one_round = tiles * n <= cus;
     return p;
 }
 
@@ -389,13 +391,19 @@ LaunchFn instance(int wt, int kw, int rg) {   // null: not built
 // stretches of K or none, so the partial tiles and their adding pass go.  q/k/v of 2048 at 33 / 128 / 250 tokens 16.6 / 14.1,
 // 19.4 / 16.7, 23.6 / 18.4, of 3072 at 64 / 187 21.7 / 18.0, 30.0 / 24.0 (at 128 24.2 / 23.5 but 3072 x 3072 21.6 / 22.7: not taken), of 4096 at 64
 // 26.7 / 22.4 (at 128 26.9 / 28.5: not taken).
+// Gate and up whose sums have to be cut to be as short as those of the 128-token tiles, so that they are two rounds of workgroups,
+// stay there: 2048 -> 2 x 5120 at 160 tokens 33.4 / 41.9, 1536 -> 2 x 4608 at 192 29.6 / 39.5.
 bool q8_0_tokens_takes(int64_t K, int64_t M, int64_t N) {
     if (K % BK != 0 || K > (1 << 24)) return false;   // 32-bit lane offsets: 128 rows of K bytes
     if (tuning_int("QPROJ_Q8_TAKE", 0)) return true;
     if (K <= 1024) return false;
     const int64_t cus = cu_count();
     if (rider(K, N)) return (K <= 3072 && rider_tiles(K, M) * (M > 128 ? 1 : 2) <= cus) || (K <= 4096 && M <= 64 && rider_tiles(K, M) <= cus);
-    return (M > 128 && M <= 192) || (M > 32 && M <= 96 && K > N && N <= 128 * cus);
+    if (M > 128 && M <= 192) {
+        const Q8Plan p = q8_plan(K, M, N);
+        return p.kw == 1 || p.one_round;
+    }
+    return M > 32 && M <= 96 && K > N && N <= 128 * cus;
 }
 
 size_t q8_0_tokens_scratch_bytes(int64_t K, int64_t M, int64_t N) { return partial_bytes(q8_plan(K, M, N), M, N); }

@@ -279,3 +279,14 @@ def test_q8_0_stretches_are_one_round_on_every_xcd():
             assert wgs <= 256, (k, n, m, wgs)
             seen += wgs > 0
     assert seen > 500
+
+
+def test_q8_0_gate_and_up_in_token_tiles_are_one_round_or_whole():
+    """Cut in two so that its sums are no longer than those of the 128-token tiles, a gate / up pair of one round would be two."""
+    seen = 0
+    for k, f, m in itertools.product(range(1280, 4096, 256), (2.5, 3, 3.5, 4), (129, 160, 192)):
+        n = 256 * round(k * f / 256)
+        wgs = q8_0_launch_workgroups(k, (n, n), m)
+        assert wgs <= 256, (k, n, m, wgs)
+        seen += wgs > 0
+    assert seen > 20
