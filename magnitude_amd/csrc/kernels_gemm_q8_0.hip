@@ -16,7 +16,7 @@
 //   - the addend of the matrix instruction is the bits of 1.5 * 2^23, so its sums are floats already and a
 //     subtraction (exact) takes the place of the conversion;
 //   - K goes in two parts over the waves of a workgroup (KW = 2) while there is at most a workgroup a compute unit, the parts
-//     meeting in LDS, and in stretches over workgroups (partial tiles, an adding pass) beyond that.
+//     meeting in LDS, and in stretches over workgroups (partial tiles, an adding pass) where the tiles leave units idle.
 #include <algorithm>
 #include <type_traits>
 
@@ -62,8 +62,11 @@ struct Q8Lds {
     static_assert(KW == 1 || (WT + 1) / 2 * NW * 4096 <= kOffWs, "the K parts meet in the same LDS at the end");
 };
 
-// WT columns of 32 tokens, KW K parts, RG row groups of 32 weight rows
-template <int WT, int KW, int RG>
+// WT columns of 32 tokens, KW K parts, RG row groups of 32 weight rows.  TWO_LEVEL: shorter chains of sums.  The tiles of 32
+// tokens take K whole, in chains of K / 64 blocks, where the 128-token tiles cut it in up to eight stretches: the sums of two steps
+// are added up by themselves first, and their error is no larger.  The 96-token tiles set theirs aside in LDS halfway (a second set
+// of 48 registers made the compiler pass its products through accumulator registers: 8 % slower).
+template <int WT, int KW, int RG, bool TWO_LEVEL>
 __global__ __launch_bounds__(64 * RG * KW, 2) void gemm_per32_kernel_q8_0(const Q8Args g) {
     using L = Q8Lds<WT, KW, RG>;
     constexpr int NW = L::NW, TM = 32 * WT;
@@ -129,24 +132,48 @@ __global__ __launch_bounds__(64 * RG * KW, 2) void gemm_per32_kernel_q8_0(const 
         global_to_lds16(xbase + (xoff + ks * 4u), smem + L::kOffDx + buf * L::kDx + xg * 1024);
     };
 
-    // One column: the sums of two steps are added up by themselves first.  Such tiles take K whole, in chains of K / 64 blocks,
-    // where the 128-token tiles cut it in up to eight stretches; added eight at a time their error is no larger.
-    constexpr bool kTwoLevel = WT == 1;
-    float sum[WT][16], total[kTwoLevel ? 16 : 1];
+    float sum[WT][16], total[WT == 1 ? 16 : 1];
 #pragma unroll
     for (int j = 0; j < WT; ++j)
 #pragma unroll
         for (int v = 0; v < 16; ++v) sum[j][v] = 0.f;
-    if constexpr (kTwoLevel) {
+    if constexpr (WT == 1) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) total[v] = 0.f;
     }
+    v4i *const aside = reinterpret_cast<v4i *>(smem + L::kTotal + wave * (WT * 4096)) + lane;
     auto fold_sums = [&]() {
-        if constexpr (kTwoLevel) {
+        if constexpr (TWO_LEVEL) {
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                total[v] += sum[0][v];
-                sum[0][v] = 0.f;
+            for (int j = 0; j < WT; ++j) {
+                if constexpr (WT > 1) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        aside[(4 * j + i) * 64] = v4i{__float_as_int(sum[j][4 * i]), __float_as_int(sum[j][4 * i + 1]), __float_as_int(sum[j][4 * i + 2]),
+                                                      __float_as_int(sum[j][4 * i + 3])};
+                }
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    if constexpr (WT == 1) total[v] += sum[0][v];
+                    sum[j][v] = 0.f;
+                }
+            }
+        }
+    };
+    auto add_folded = [&](int n_steps) {
+        if constexpr (TWO_LEVEL && WT == 1) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) sum[0][v] += total[v];
+        } else if constexpr (TWO_LEVEL) {
+            if (n_steps >= 3) {
+#pragma unroll
+                for (int j = 0; j < WT; ++j)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const v4i o = aside[(4 * j + i) * 64];
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) sum[j][4 * i + r] += __int_as_float(o[r]);
+                    }
             }
         }
     };
@@ -251,16 +278,13 @@ __global__ __launch_bounds__(64 * RG * KW, 2) void gemm_per32_kernel_q8_0(const 
         int s = 0;
         for (; s + 2 < n_steps; ++s) {
             step(s, std::true_type{}, std::true_type{});
-            if (s & 1) fold_sums();
+            if (WT == 1 ? (s & 1) != 0 : s + 1 == n_steps / 2) fold_sums();   // (of three steps and more)
         }
         if (s + 1 < n_steps) step(s++, std::true_type{}, std::false_type{});
         step(s, std::false_type{}, std::false_type{});
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (a single step leaves its second strip request behind)
-    if constexpr (kTwoLevel) {
-#pragma unroll
-        for (int v = 0; v < 16; ++v) sum[0][v] += total[v];
-    }
+    add_folded(n_steps);
 
     // ---- the K parts meet in LDS: part q keeps token tiles j % 2 == q, the other hands its sums over
     if constexpr (KW == 2) {
@@ -311,6 +335,7 @@ __global__ __launch_bounds__(64 * RG * KW, 2) void gemm_per32_kernel_q8_0(const 
 struct Q8Plan {
     int wt, kw, n_split;
     bool one_round;   // of workgroups, one a compute unit (two K parts)
+    bool two_level;   // in workgroups of 64 rows, the sums added up in two levels
 };
 
 // q, k, v and o: square matrices and small ones, whose launch holds a matrix and a half of K rows as a rule
@@ -336,9 +361,23 @@ Q8Plan q8_plan(int64_t K, int64_t M, int64_t N) {
     // q8_0_tokens_takes leaves their larger grids to the 128-token tiles.
     p.kw = tuning_int("QPROJ_Q8_KW", p.wt >= 3 && tiles > cus ? 1 : 2);
     int64_t n = std::max<int64_t>(1, std::min<int64_t>(8, cus / tiles));
-    // never longer sums than the 128 x 128 tiles have (their error against 64 bits grows with the length; the tiles of 32 tokens
-    // add theirs up in two levels instead)
-    if (p.wt > 1) n = std::max<int64_t>(n, (per32_splits(kTypeQ8_0, K, M, N) + p.kw - 1) / p.kw);
+    // never longer sums than the 128 x 128 tiles have (their error against 64 bits grows with the length; two levels of them instead
+    // in the tiles of 32 tokens)
+    const int64_t least = p.wt > 1 ? (per32_splits(kTypeQ8_0, K, M, N) + p.kw - 1) / p.kw : 1;
+    p.two_level = p.wt == 1;
+    // Where that leaves a workgroup two to four steps, most of it the start of a pipeline, half as many stretches in workgroups of
+    // half the rows, still one round, walk twice as far, their sums in two levels (error against 64 bits 0.68 to 0.94 of the
+    // 128-token tiles'; up to 1.02 of the short stretches').  us a call, 128-token tiles / eight waves, short stretches / four waves:
+    // 3072 -> 1536 at 160 tokens 19.2 / 21.1 / 17.5, 4096 -> 1280 20.6 / 21.7 / 18.9, 3584 -> 2304 26.9 / 32.3 / 23.7, 5120 -> 1280 23.6 /
+    // 23.5 / 20.2; 4096 -> 3072 at 80 21.4 / 21.8 / 19.1, 8192 -> 4096 28.1 / 27.4 / 26.6.
+    if (p.wt == 3 && p.kw == 2 && K > N && !rider(K, N) && (units + n - 1) / n <= 4) {
+        const int64_t halves = cus / ((tiles_m * ((N + 63) / 64) + 7) / 8 * 8);
+        if (halves >= least) {
+            n = std::min<int64_t>(8, halves);
+            p.two_level = true;
+        }
+    }
+    n = std::max<int64_t>(n, least);
     n = tuning_int("QPROJ_Q8_SPLIT", (int)n);
     n = std::max<int64_t>(1, std::min<int64_t>(n, units / 2));   // two times 256 weights a stretch at least
     if ((M * N) % 4 != 0) n = 1;
@@ -350,10 +389,11 @@ Q8Plan q8_plan(int64_t K, int64_t M, int64_t N) {
 
 size_t partial_bytes(const Q8Plan &p, int64_t M, int64_t N) { return p.n_split > 1 ? (size_t)p.n_split * M * N * 4 : 0; }
 
-template <int WT, int KW, int RG>
+template <int WT, int KW, int RG, bool TWO_LEVEL>
 hipError_t launch(const Q8Args &g, int wgs, hipStream_t s) {
-    constexpr int lds = Q8Lds<WT, KW, RG>::kTotal;
-    const auto kern = &gemm_per32_kernel_q8_0<WT, KW, RG>;
+    constexpr int lds = Q8Lds<WT, KW, RG>::kTotal + (TWO_LEVEL && WT > 1 ? RG * KW * WT * 4096 : 0);
+    static_assert(lds <= 160 * 1024, "one workgroup's LDS");
+    const auto kern = &gemm_per32_kernel_q8_0<WT, KW, RG, TWO_LEVEL>;
     static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (attr != hipSuccess) return attr;
     hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(64 * RG * KW), lds, s, g);
@@ -361,20 +401,21 @@ hipError_t launch(const Q8Args &g, int wgs, hipStream_t s) {
 }
 
 using LaunchFn = hipError_t (*)(const Q8Args &, int, hipStream_t);
-LaunchFn instance(int wt, int kw, int rg) {   // null: not built
-#define QP_Q8(WT, KW, RG) \
-    if (wt == WT && kw == KW && rg == RG) return &launch<WT, KW, RG>
-    QP_Q8(1, 2, 2);
-    QP_Q8(2, 2, 4);
-    QP_Q8(3, 1, 4);
-    QP_Q8(3, 2, 4);
-    QP_Q8(3, 2, 2);
+LaunchFn instance(int wt, int kw, int rg, bool two_level) {   // null: not built
+#define QP_Q8(WT, KW, RG, TWO_LEVEL) \
+    if (wt == WT && kw == KW && rg == RG && two_level == TWO_LEVEL) return &launch<WT, KW, RG, TWO_LEVEL>
+    QP_Q8(1, 2, 2, true);
+    QP_Q8(2, 2, 4, false);
+    QP_Q8(3, 1, 4, false);
+    QP_Q8(3, 2, 4, false);
+    QP_Q8(3, 2, 2, false);
+    QP_Q8(3, 2, 2, true);
 #ifdef QPROJ_TUNING
-    QP_Q8(1, 2, 4);
-    QP_Q8(1, 1, 4);
-    QP_Q8(2, 1, 4);
-    QP_Q8(4, 1, 4);
-    QP_Q8(4, 2, 4);
+    QP_Q8(1, 2, 4, true);
+    QP_Q8(1, 1, 4, true);
+    QP_Q8(2, 1, 4, false);
+    QP_Q8(4, 1, 4, false);
+    QP_Q8(4, 2, 4, false);
 #endif
 #undef QP_Q8
     return nullptr;
@@ -427,7 +468,7 @@ hipError_t launch_gemm_q8_0_tokens(int n, const WeightView *w, const ActView &a,
         g.K = (int)w[0].K;
         const Q8Plan &p0 = plans[first];
         const int64_t tiles_m = (M + 32 * p0.wt - 1) / (32 * p0.wt);
-        const auto shares = [&](int i) { return plans[i].kw == p0.kw && plans[i].wt == p0.wt; };
+        const auto shares = [&](int i) { return plans[i].kw == p0.kw && plans[i].wt == p0.wt && plans[i].two_level == p0.two_level; };
         const auto tiles_pad = [&](int i, int rows) { return ((w[i].N + rows - 1) / rows * tiles_m + 7) / 8 * 8; };
         // Half the weight rows a workgroup where that many workgroups are still one a compute unit: the same sums on twice the
         // compute units (a matrix is cut as if its sibling rode along; 3072 -> 8192 alone at 187 tokens 35.0 -> 27.8 us).
@@ -437,8 +478,8 @@ hipError_t launch_gemm_q8_0_tokens(int n, const WeightView *w, const ActView &a,
         // barriers, and q/k/v a little beyond a round of eight-wave workgroups do not take two.  us a call, tiles of 128 tokens / 128
         // rows a workgroup / 64: q/k/v of 2560 with 1024 for k and v at 97 tokens 21.8 / 28.0 / 23.5, of 3072 at 187 30.7 / 25.1 / 24.3
         // and at 193 30.9 / 38.6 / 33.6, three of 2048 at 80 21.0 / 24.5 / 21.9; 3072 -> 1024 alone at 187 18.8 / 22.4 / 17.8.
-        const int rg = tuning_int("QPROJ_Q8_RG", p0.wt == 1 || (p0.wt == 3 && p0.kw == 2 && halves <= cu_count()) ? 2 : 4);
-        const LaunchFn run = instance(p0.wt, p0.kw, rg);
+        const int rg = tuning_int("QPROJ_Q8_RG", p0.two_level || (p0.wt == 3 && p0.kw == 2 && halves <= cu_count()) ? 2 : 4);
+        const LaunchFn run = instance(p0.wt, p0.kw, rg, p0.two_level);
         if (!run) return hipErrorInvalidValue;   // (in a dry run too)
         SumTargets sums{};
         size_t used = 0;

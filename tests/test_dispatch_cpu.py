@@ -290,3 +290,16 @@ def test_q8_0_gate_and_up_in_token_tiles_are_one_round_or_whole():
         assert wgs <= 256, (k, n, m, wgs)
         seen += wgs > 0
     assert seen > 20
+
+
+@pytest.mark.parametrize("m,k,n,stretches", [(160, 3072, 1536, 4), (129, 4096, 1280, 6), (80, 4096, 3072, 4), (96, 8192, 4096, 4), (192, 2560, 2304, 3)])
+def test_q8_0_short_stretches_are_walked_in_halves_of_the_rows(m, k, n, stretches):
+    """Eight waves and two to four steps of K a workgroup are mostly the start of a pipeline: half the rows and about half the
+    stretches instead, never fewer than the 128-token tiles would make."""
+    plan = qproj.plan_mul_mat(Q8_0, k, (n,), m)
+    assert f"x 64 rows, {-(-m // 96) * (n // 64)} tiles x {stretches} K stretches" in plan, plan
+
+
+@pytest.mark.parametrize("m,k,n", [(160, 6144, 3072), (160, 14336, 4096), (64, 4096, 3072)])
+def test_q8_0_longer_stretches_keep_eight_waves(m, k, n):
+    assert "x 128 rows" in qproj.plan_mul_mat(Q8_0, k, (n,), m)

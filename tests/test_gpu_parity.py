@@ -699,6 +699,29 @@ def test_q8_0_tiles_of_96_64_and_32_tokens(ctx, orc, m, k, ns):
         w.free()
 
 
+@pytest.mark.parametrize("m,k,ns", [(80, 1536, (1284,)), (65, 2560, (2320,)), (130, 2560, (1800,)), (187, 2432, (1290,)), (192, 3072, (1536, 1440)),
+                                    (96, 3584, (2308,)), (161, 4224, (1157,)), (129, 8192, (1060,))])
+def test_q8_0_tiles_of_96_tokens_in_halves(ctx, orc, m, k, ns):
+    """The 96-token tiles of 64 rows that set their sums aside halfway: stretches of two, three and more steps, an odd number of
+    steps of 128 (the second K part idle in the last), whole K where M * N is no multiple of 4, ragged tokens and rows, two matrices.
+    Oracle and tolerance as above."""
+    from magnitude_amd import ACT_GGML, qproj
+    plan = qproj.plan_mul_mat(Q8_0, k, list(ns), m, ACT_GGML)
+    assert plan.count("gemm_per32_kernel_q8_0<3 token tiles, 2 K parts>") == plan.count("tile 96 tokens x 64 rows") == len(ns), plan
+    rng = np.random.default_rng(m + k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    blocks = [make_weight(orc, Q8_0, n, k, seed=6600 + i) for i, n in enumerate(ns)]
+    ws = [ctx.upload(Q8_0, k, n, b) for n, b in zip(ns, blocks)]
+    bufs = [torch.full((m * n + 64,), 7.0, dtype=torch.float32, device="cuda") for n in ns]
+    ctx.mul_mat_multi(ws, dev(x), ACT_GGML, outs=[b[: m * n].view(m, n) for b, n in zip(bufs, ns)])
+    some = np.unique([0, 31, 32, min(95, m - 1), min(96, m - 1), m // 2, m - 1])
+    for w, n, b, bl in zip(ws, ns, bufs, blocks):
+        close(b[: m * n].view(m, n).cpu().numpy()[some], orc.mul_mat(Q8_0, bl, k, x[some], orc.ACT_GGML), 5e-5)
+        assert bool((b[m * n:] == 7.0).all())
+        assert torch.equal(b[: m * n].view(m, n), ctx.mul_mat(w, dev(x), ACT_GGML))
+        w.free()
+
+
 @pytest.mark.parametrize("m,k,ns", [(257, 512, (512, 130)), (1030, 1024, (1024, 260)), (2048, 256, (256,)), (300, 4352, (1100,)),
                                     (512, 2048, (2048, 512, 512))])
 def test_streamed_q4k_batches_beyond_256_tokens(ctx, orc, m, k, ns):
