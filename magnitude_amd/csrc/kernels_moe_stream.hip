@@ -3,7 +3,7 @@
 //
 // Bound on paper: HBM over the bytes of the experts a call touches.
 //   - The grouping pass lists tiles {expert, first pair, up to 64 pairs}; a workgroup (4 waves, two workgroups a compute
-//     unit) takes one tile and `tiles_n` row tiles of its expert as ONE stream of (row tile, super-block) steps, so the
+//     unit up to 7936 weights a row) takes one tile and `tiles_n` row tiles of its expert as ONE stream of (row tile, super-block) steps, so the
 //     pipeline never restarts: raw weight blocks go straight from global memory into wave-private LDS strips two steps
 //     ahead, the gathered activation rows (any row per lane: the loads into LDS take an address each) one step ahead into
 //     a buffer that the four waves share, one barrier a step.
@@ -27,7 +27,7 @@ namespace {
 
 constexpr int kWaves = 4, kThreads = 64 * kWaves;
 constexpr int kMaxJT = kMoeTileRows / 32;
-constexpr int kStripBytes = 5 * 1024, kStripLoads = 5;
+constexpr int kStripBytes = 32 * 144, kStripLoads = 5;
 
 struct MoeStreamArgs {
     const uint8_t *w0, *w1;   // blocks of the expert stack; w1: the up projection of the SwiGLU launch
@@ -49,6 +49,7 @@ struct MoeStreamArgs {
 constexpr int kOffSum = 2 * kMaxJT * 8192, kOffStrip = kOffSum + 2 * kMaxJT * 1024,
               kOffPair = kOffStrip + 2 * kWaves * kStripBytes, kOffDx = kOffPair + kMoeTileRows * 4;
 constexpr int moe_stream_lds(int nb) { return kOffDx + nb * kMoeTileRows * 4; }
+constexpr int workgroups_per_cu(int nb) { return 2 * moe_stream_lds(nb) <= 160 * 1024 ? 2 : 1; }   // (the launch bounds: two at most)
 
 // eight fp16 integers: the four bytes of `w` (below 128), each twice
 __device__ __forceinline__ v8h bytes_twice_to_f16(uint32_t w) {
@@ -75,14 +76,16 @@ __device__ __forceinline__ void moe_stream_tile(const MoeStreamArgs &g, uint8_t 
     const int n_rt = (int)min((int64_t)g.row_tiles, n_row_tiles - rt0);
     if (n_rt <= 0) return;   // the whole workgroup
 
-    // ---- weights: piece p = lane + 64 c of a strip is bytes 16 (p % 9).. of row p / 9 (the last request repeats piece 287)
+    // ---- weights: piece p of a strip is bytes 16 (p % 9).. of row p / 9.  The 288 pieces are four and a half requests: the fifth
+    // asks for the last 64, half of them a second time with the same bytes for the same place, so that a strip ends where its rows
+    // end (with 512 spare bytes behind each of the eight, a second workgroup did not fit beside rows of 4096 weights)
     uint8_t *const strip = smem + kOffStrip + wave * kStripBytes;   // second buffer kWaves * kStripBytes further on
     const uint8_t *src[kStripLoads];
     auto strip_row_tile = [&](int rt) {
         const int64_t row0 = ((rt0 + rt) * kWaves + wave) * kRows;
 #pragma unroll
         for (int c = 0; c < kStripLoads; ++c) {
-            const int p = min(lane + 64 * c, 287), r = p / 9;
+            const int p = lane + (c < 4 ? 64 * c : 288 - 64), r = p / 9;
             const int64_t row = min(row0 + (r & (kRows - 1)), N - 1);   // rows past the edge repeat the last (never stored)
             src[c] = (SWIGLU && r >= 16 ? g.w1 : g.w0) + ((int64_t)tile.x * N + row) * nb * 144 + 16 * (p - 9 * r);
         }
@@ -91,7 +94,7 @@ __device__ __forceinline__ void moe_stream_tile(const MoeStreamArgs &g, uint8_t 
     int req_rt = 0, req_sb = 0;   // the step that was requested last
     auto request_strip = [&](uint8_t *dst) {
 #pragma unroll
-        for (int c = 0; c < kStripLoads; ++c) global_to_lds16(src[c], dst + 1024 * c);
+        for (int c = 0; c < kStripLoads; ++c) global_to_lds16(src[c], dst + (c < 4 ? 1024 * c : kStripBytes - 1024));
     };
     auto advance = [&]() {   // (past the last step: stays there)
         if (++req_sb < nb) {
@@ -306,6 +309,7 @@ hipError_t launch(const MoeStreamArgs &g, unsigned wgs, hipStream_t s) {
 }  // namespace
 
 static_assert(moe_stream_lds(kMoeStreamMaxSb) <= 160 * 1024, "one workgroup's LDS");
+static_assert(workgroups_per_cu(kMoeStreamMaxSb - 1) == 2, "two workgroups a compute unit up to 7936 weights a row");
 
 bool moe_stream_fits(int type, int64_t K, int64_t N) {
     return type == kTypeQ4_K && K % 256 == 0 && K / 256 <= kMoeStreamMaxSb && N >= 1;
@@ -343,11 +347,11 @@ hipError_t launch_moe_stream(const GemvArgs &args, int64_t n_pairs, bool swiglu,
     // 361 / 365 / 366 / 367 / 407.
     const int64_t busy = std::min<int64_t>(w.E, n_pairs);
     const int64_t expected = std::max<int64_t>(busy, busy / 2 + n_pairs / kMoeTileRows);   // tiles: the last one of an expert half full
-    const int64_t cus = cu_count();
+    const int64_t cus = cu_count(), resident = workgroups_per_cu(g.nb);
     int64_t walk = 1, best = INT64_MAX;
     for (int64_t c = 1; c <= std::min<int64_t>(row_tiles, 64); ++c) {
         const int64_t per_cu = (expected * ((row_tiles + c - 1) / c) + cus - 1) / cus;
-        const int64_t cost = per_cu * c * g.nb + 5 * ((per_cu + 1) / 2) + (per_cu > 1 ? 0 : n_pairs > 16 * w.E ? c * g.nb / 2 : 3);
+        const int64_t cost = per_cu * c * g.nb + 5 * ((per_cu + resident - 1) / resident) + (std::min(per_cu, resident) > 1 ? 0 : n_pairs > 16 * w.E ? c * g.nb / 2 : 3);
         if (cost < best) {
             best = cost;
             walk = c;
@@ -359,8 +363,8 @@ hipError_t launch_moe_stream(const GemvArgs &args, int64_t n_pairs, bool swiglu,
     const int64_t wgs = (cap + 7) / 8 * 8 * g.wgs_per_tile;
     if (wgs >= 0x7fffffff) return hipErrorInvalidValue;
     if (dry_run()) {
-        plan_note("moe_stream_kernel<Q4_K%s>: tiles of up to %d pairs of an expert, %lld workgroups, %d a tile, %d row tiles of %lld each", swiglu ? ", gate + up + swiglu" : "",
-                  kMoeTileRows, (long long)wgs, g.wgs_per_tile, g.row_tiles, (long long)rows);
+        plan_note("moe_stream_kernel<Q4_K%s>: tiles of up to %d pairs of an expert, %lld workgroups, %d a tile, %d row tiles of %lld each, %lld a compute unit", swiglu ? ", gate + up + swiglu" : "",
+                  kMoeTileRows, (long long)wgs, g.wgs_per_tile, g.row_tiles, (long long)rows, (long long)resident);
         return hipSuccess;
     }
     if (!g.hsum || !args.order || !args.active) return hipErrorInvalidValue;

@@ -303,3 +303,12 @@ def test_q8_0_short_stretches_are_walked_in_halves_of_the_rows(m, k, n, stretche
 @pytest.mark.parametrize("m,k,n", [(160, 6144, 3072), (160, 14336, 4096), (64, 4096, 3072)])
 def test_q8_0_longer_stretches_keep_eight_waves(m, k, n):
     assert "x 128 rows" in qproj.plan_mul_mat(Q8_0, k, (n,), m)
+
+
+@pytest.mark.parametrize("d,resident", [(2048, 2), (4096, 2), (7936, 2), (8192, 1)])
+def test_expert_tiles_leave_room_for_a_second_workgroup(d, resident):
+    """Two workgroups a compute unit, each filling the other's waits, but for the longest rows; the row tiles a workgroup walks are
+    chosen by it."""
+    plan = qproj.plan_moe_ffn(Q4_K, Q4_K, d, 1024, 128, 8, 64)
+    gate = [l for l in plan.splitlines() if "moe_stream_kernel<Q4_K, gate" in l]
+    assert len(gate) == 1 and gate[0].endswith(f"each, {resident} a compute unit"), plan
