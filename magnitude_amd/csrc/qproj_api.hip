@@ -678,10 +678,12 @@ int grouped_mt(int64_t n_pairs, int64_t E) {
 }
 
 // Expert batches in tiles of up to 64 pairs on the matrix cores (moe_stream_kernel): beyond four pairs an expert, where the
-// grouped kernel stages 16 rows a pass instead of 8, and from three and a half on where the row tiles of the experts fill the chip
-// (two workgroups of 64 rows a compute unit).  us a call, grouped / tiles: 128 experts of 2048 x 768, 40 / 64 / 100 / 500
-// tokens (2.5 / 4 / 6.2 / 31 pairs an expert) 89 / 91.5, 103 / 94, 105 / 97, 208 / 127; 64 of 1024 x 512 at 3.8 pairs
-// 41.8 / 33.2; 32 of 4096 x 512 at 4 / 6.2 pairs 42.7 / 45.8, 50.5 / 46.4; 256 of 1024 x 2048 at 2.8 / 7.8 pairs 202 / 214, 277 / 239.
+// grouped kernel stages 16 rows a pass instead of 8, and with 32 experts and more, whose row tiles fill the chip (two workgroups of
+// 64 rows a compute unit), from three and three quarters on, where some expert has more than the 8 pairs of a pass in almost every
+// draw.  Grouped = 1, mean of six draws of the pairs, 82 shapes each (8 to 256 experts of 1024 to 4096 x 512 to 2048): all in tiles 1.00
+// at 3 pairs an expert, 0.99 at 3.5 (128 of 2048 x 2048 201 us / 217, 256 of 2048 x 512 134 / 124), 0.96 at 3.75 and 4, 0.94 at 4.5 and 5,
+// 0.91 at 8.  At 3.75 to 4 pairs the slowest left is 256 of 1024 x 2048, 219 / 224; 16 experts, which seldom need a second pass,
+// lost: of 4096 x 2048 63.7 / 68.3.  128 experts of 2048 x 768, 64 / 100 / 500 tokens 102.4 / 96.8, 106.1 / 98.8, 213.6 / 127.4.
 // Popular experts take tiles of their own: the 128 experts with popularity e^N(0,1), 500 tokens, 462 / 162.
 // A tile has one running sum over the whole row.  Where the grouped kernel cuts K over waves or chunks (few experts, few
 // rows), rows beyond 1024 weights stay with it: error against 64 bits, tiles over grouped, 8 experts x 512 rows of 1024 / 1280 /
@@ -689,7 +691,7 @@ int grouped_mt(int64_t n_pairs, int64_t E) {
 bool moe_stream_route(int type, int64_t K, int64_t N, int64_t n_pairs, int64_t E) {
     static const int per_4_experts = tuning_int("QPROJ_MOE_STREAM_PAIRS_PER_4_EXPERTS", 0);
     const bool many = per_4_experts ? 4 * n_pairs >= per_4_experts * E
-                                    : n_pairs > 4 * E || (2 * n_pairs >= 7 * E && E * N >= (int64_t)2 * 64 * cu_count());
+                                    : n_pairs > 4 * E || (4 * n_pairs >= 15 * E && E >= 32 && E * N >= (int64_t)2 * 64 * cu_count());
     return many && moe_stream_fits(type, K, N) && (K <= 1024 || mfma_grouped_whole_rows(type, K, N, E, n_pairs));
 }
 

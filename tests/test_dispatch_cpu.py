@@ -312,3 +312,11 @@ def test_expert_tiles_leave_room_for_a_second_workgroup(d, resident):
     plan = qproj.plan_moe_ffn(Q4_K, Q4_K, d, 1024, 128, 8, 64)
     gate = [l for l in plan.splitlines() if "moe_stream_kernel<Q4_K, gate" in l]
     assert len(gate) == 1 and gate[0].endswith(f"each, {resident} a compute unit"), plan
+
+
+@pytest.mark.parametrize("experts,used,d,ff,tokens,tiles", [(128, 8, 2048, 2048, 56, False), (256, 8, 1024, 2048, 112, False), (64, 8, 4096, 2048, 28, False),
+                                                            (16, 4, 4096, 2048, 16, False), (16, 4, 2048, 2048, 15, False), (16, 4, 4096, 2048, 17, True),
+                                                            (128, 8, 2048, 768, 60, True), (32, 4, 4096, 1024, 32, True), (64, 8, 2048, 1024, 30, True)])
+def test_expert_tiles_start_where_the_grouped_kernel_needs_second_passes(experts, used, d, ff, tokens, tiles):
+    plan = qproj.plan_moe_ffn(Q4_K, Q4_K, d, ff, experts, used, tokens)
+    assert plan.count("moe_stream_kernel") == (2 if tiles else 0), plan
