@@ -1261,6 +1261,26 @@ int qproj_plan_moe_ffn(int gate_type, int down_type, int64_t d_model, int64_t d_
     return finish_plan(text, rc, scratch_bytes, buf, buf_bytes);
 }
 
+// The launches of a qproj_mul_mat_id of this shape, for the tests: as qproj_plan_moe_ffn.
+int qproj_internal_plan_mul_mat_id(int type, int64_t K, int64_t N, int64_t n_expert, int64_t nb1, int64_t n_used, int64_t B, char *buf, size_t buf_bytes) {
+    if (!type_ok(type) || K <= 0 || N <= 0 || n_expert <= 0 || K % block_elems(type) != 0) return QPROJ_ERR_INVALID_ARG;
+    qproj_ctx ctx;
+    qproj_weight w;
+    fake_weight(w, type, K, N, n_expert);
+    std::string text;
+    set_dry_run(true);
+    g_plan = &text;
+    ctx.flag_dev = reinterpret_cast<int32_t *>(uintptr_t(256));   // never dereferenced in a dry run
+    const int rc = qproj_mul_mat_id(&ctx, &w, reinterpret_cast<const float *>(uintptr_t(256)), nb1, reinterpret_cast<const int32_t *>(uintptr_t(256)), n_used, B,
+                                    reinterpret_cast<float *>(uintptr_t(256)), kActGGML);
+    g_plan = nullptr;
+    set_dry_run(false);
+    const size_t scratch_bytes = ctx.ws_bytes;
+    ctx.ws_bytes = 0;
+    ctx.flag_dev = nullptr;
+    return finish_plan(text, rc, scratch_bytes, buf, buf_bytes);
+}
+
 int qproj_rms_norm_mul_mat(qproj_ctx *ctx, int n, const qproj_weight *const *w, const float *x_dev, const float *gamma_dev,
                            float eps, int64_t M, float *const *y_dev, int act) {
     const NormSpec norm{gamma_dev, eps};

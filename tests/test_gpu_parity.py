@@ -783,11 +783,10 @@ def test_mul_mat_id_matches_oracle(ctx, orc, moe, B):
 
 @pytest.mark.parametrize("E,B", [(16, 600), (16, 1100), (512, 500)])
 def test_mul_mat_id_grouping_of_many_pairs(ctx, orc, E, B):
-    """The three ways the grouping pass sorts pairs by expert, on small expert matrices so that the oracle
-    stays quick: 4800 pairs (ranks inside blocks of 64 pairs, several blocks per wave), 8800 pairs (more
-    than the per-block path holds: sweeps over the ids in global memory) and 4000 pairs over 512 experts
-    (block table too large for LDS: sweeps over ids staged in LDS).  Experts get hundreds of rows each, so
-    the grouped kernel also runs its several-passes-per-expert loop."""
+    """The grouping pass with hundreds of pairs an expert, on small expert matrices so that the oracle stays quick: a counter a
+    wave and expert, with every block of a wave's pairs held in registers (4000 and 4800 pairs) and with blocks that are
+    counted a second time when they are placed (8800), over few experts and over 512.  The launch behind it takes several
+    tiles an expert."""
     from magnitude_amd import ACT_GGML
     k, n, top = 256, 32, 8
     blocks = encode(Q4_K, (np.random.default_rng(E + B).standard_normal((E * n, k)) * 0.02).astype(np.float32)).reshape(E, n, -1)
@@ -801,6 +800,14 @@ def test_mul_mat_id_grouping_of_many_pairs(ctx, orc, E, B):
     w.free()
 
 
+def plan_mul_mat_id(k, n, n_expert, nb1, n_used, batch):
+    import ctypes as C
+    from magnitude_amd import qproj
+    buf, i = C.create_string_buffer(8192), C.c_int64
+    assert qproj.load_library().qproj_internal_plan_mul_mat_id(Q4_K, i(k), i(n), i(n_expert), i(nb1), i(n_used), i(batch), buf, C.c_size_t(len(buf))) == 0
+    return buf.value.decode()
+
+
 @pytest.mark.parametrize("k,n,counts", [(256, 63, (1, 31, 32, 33, 0, 64, 65)), (768, 129, (0, 129, 1, 63, 5)),
                                         (1024, 64, (96, 2, 2)), (2304, 1024, (70, 33) + (1,) * 30), (512, 1, (40,))])
 def test_expert_tiles_at_their_edges(ctx, orc, k, n, counts):
@@ -810,6 +817,7 @@ def test_expert_tiles_at_their_edges(ctx, orc, k, n, counts):
     fp32 additions in another order."""
     from magnitude_amd import ACT_GGML, QprojError
     E = len(counts)
+    assert "moe_stream_kernel" in plan_mul_mat_id(k, n, E, 1, 1, sum(counts))
     rng = np.random.default_rng(k + n)
     ids = rng.permutation(np.repeat(np.arange(E, dtype=np.int32), counts))[:, None]
     blocks = encode(Q4_K, (rng.standard_normal((E * n, k)) * 0.02).astype(np.float32)).reshape(E, n, -1)
@@ -829,6 +837,39 @@ def test_expert_tiles_at_their_edges(ctx, orc, k, n, counts):
     assert (y[len(ids) // 2] == 7.0).all()
     good = np.arange(len(ids)) != len(ids) // 2
     close(y[good], want[good], 2e-5)
+    w.free()
+
+
+@pytest.mark.parametrize("k,n,counts,walk", [(4096, 1040, (70, 33, 64, 0) + (1,) * 28, 1), (4096, 2064, (70, 32, 0) + (2,) * 29, 3),
+                                             (4352, 1040, (33, 32, 0) + (2,) * 29, 1), (8192, 1040, (66, 4) + (2,) * 29 + (0,), 2)])
+def test_expert_tiles_of_long_rows(ctx, orc, k, n, counts, walk):
+    """moe_stream_kernel at 16, 17 and 32 super-blocks a row (the LDS image and the table of activation scales grow with them;
+    one workgroup a compute unit at 32), one and several row tiles a workgroup, the last one ragged.  Tolerance as above."""
+    from magnitude_amd import ACT_GGML
+    E = len(counts)
+    plan = plan_mul_mat_id(k, n, E, 1, 1, sum(counts))
+    assert "moe_stream_kernel" in plan and f" {walk} row tiles of 128" in plan, plan
+    rng = np.random.default_rng(k + sum(counts))
+    two = encode(Q4_K, (rng.standard_normal((2 * n, k)) * 0.02).astype(np.float32)).reshape(2, n, -1)
+    blocks = np.ascontiguousarray(two[rng.integers(0, 2, size=E)])   # (an encoder in C on 32 experts would take most of the test)
+    ids = rng.permutation(np.repeat(np.arange(E, dtype=np.int32), counts))[:, None]
+    x = rng.standard_normal((len(ids), 1, k)).astype(np.float32)
+    w = ctx.upload(Q4_K, k, n, blocks, n_expert=E)
+    close(ctx.mul_mat_id(w, dev(x), dev(ids), ACT_GGML).cpu().numpy(), orc.mul_mat_id(Q4_K, blocks, k, n, E, x, ids), 2e-5)
+    w.free()
+
+
+def test_expert_tiles_with_a_row_for_every_slot(ctx, orc):
+    """Activation rows of their own for the slots of a token (nb1 = n_used), as the down projection of a graph has them."""
+    from magnitude_amd import ACT_GGML
+    E, k, n, B, top = 5, 768, 129, 50, 4
+    assert "moe_stream_kernel" in plan_mul_mat_id(k, n, E, top, top, B)
+    rng = np.random.default_rng(50)
+    blocks = encode(Q4_K, (rng.standard_normal((E * n, k)) * 0.02).astype(np.float32)).reshape(E, n, -1)
+    ids, _ = routing(rng, B, top, E)
+    x = rng.standard_normal((B, top, k)).astype(np.float32)
+    w = ctx.upload(Q4_K, k, n, blocks, n_expert=E)
+    close(ctx.mul_mat_id(w, dev(x), dev(ids), ACT_GGML).cpu().numpy(), orc.mul_mat_id(Q4_K, blocks, k, n, E, x, ids), 2e-5)
     w.free()
 
 
@@ -854,10 +895,14 @@ def test_moe_ffn_in_expert_tiles(ctx, orc, E, top, B, d_model, d_ff):
         t.free()
 
 
-def test_grouping_of_very_many_experts(ctx, orc):
-    """More experts than the grouping pass has LDS counters for: it sweeps the ids once per expert."""
+@pytest.mark.parametrize("B", [300, 1100])
+def test_grouping_of_very_many_experts(ctx, orc, B):
+    """More experts than the grouping pass has LDS counters for: it sweeps the ids once per expert, staged in LDS (2400 pairs)
+    or from global memory (8800, which the launch behind it takes in tiles)."""
     from magnitude_amd import ACT_GGML
-    E, k, n, B, top = 2048, 256, 8, 300, 8
+    E, k, n, top = 2048, 256, 8, 8
+    plan = plan_mul_mat_id(k, n, E, 1, top, B)
+    assert "ballot sweeps per expert" in plan and ("moe_stream_kernel" in plan) == (B == 1100), plan
     rng = np.random.default_rng(5)
     blocks = encode(Q4_K, (rng.standard_normal((E * n, k)) * 0.02).astype(np.float32)).reshape(E, n, -1)
     ids, _ = routing(rng, B, top, E)
