@@ -387,8 +387,8 @@ __global__ __launch_bounds__(512, 1) void gemm_q6k_q8k_wide_kernel(const WeightV
                 }
             }
             if (LATE) {
-                // the next super-block's strip was requested at the top of this trip; of the requests made since then
-                // (PA activation chunks) none needs to have landed
+                // the next super-block's strip was requested in the steps of the first tile; the only requests since then are
+                // the PA activation chunks behind it, and none of them needs to have landed
                 static_assert(PA == 4, "the wait below counts the activation requests");
                 __builtin_amdgcn_sched_barrier(0);
                 asm volatile("s_waitcnt vmcnt(4)" ::: "memory");

@@ -3,9 +3,11 @@
 // to fill the chip with those.
 //
 // Both operands change scale every 32 weights, so an int32 sum is valid for ONE matrix instruction and is folded into the
-// fp32 sums right away: a float from the integer, the product of the two fp16 scales (exact), one fma.  Bound: that vector
-// work.  A loop of nothing but matrix instruction and fold takes 70 ns a product and SIMD on random operands (58 on constant
-// ones: the clock) at two or four waves a SIMD and 95 at one, the matrix instruction hidden behind it.  So
+// fp32 sums right away: a float from the integer, the product of the two fp16 scales (exact), one fma.  Bound of the 96-token
+// tiles: that vector work.  48 vector instructions a product, 53 with everything else; 3072 -> 2 x 8192 at 187 tokens keep the vector
+// pipe busy 82 % of the launch, 8192 -> 3072 62 % (the matrix pipe 12 and 9).  The tiles of 32 tokens have 62 a product and wait as
+// well, for the step's strip, its barrier and activations that are one step ahead only: 55 % busy for q/k/v of 3072 at 187 tokens,
+// 37 % for o, a wave waiting for 36 % of its cycles.  So
 //   - the weights are the rows of the matrix instruction, the tokens its columns: the scale of a token is one register a
 //     token column, and the sixteen scales a lane needs of its weight rows are read once for all columns of the wave;
 //   - a wave owns 32 weight rows of the tile and all of its tokens: its weights pass through a wave-private LDS strip straight
@@ -423,17 +425,21 @@ LaunchFn instance(int wt, int kw, int rg, bool two_level) {   // null: not built
 
 }  // namespace
 
-// Which products this kernel takes from the 128 x 128 tiles: where a 128-token tile is padding for a quarter and more and
-// the tiles of 96 or 64 tokens are not.  129 .. 192 tokens, and rows longer than the matrix is tall up to 96 tokens.
+// Which products this kernel takes from the 128 x 128 tiles: of those where a 128-token tile is padding for a quarter and more
+// and the tiles of 96 or 64 tokens are not, 129 .. 192 tokens, and rows longer than the matrix is tall up to 96 tokens.
 // us a call at 160 tokens, 128-token tiles / here: 3072 -> 2 x 8192 50.3 / 39.2, 4096 -> 2 x 14336 96 / 80, 4096 -> 32000 100 / 84,
 // 8192 -> 3072 38.0 / 33.4, 14336 -> 4096 66.2 / 52.3, 28672 -> 8192 210 / 143; at 64 tokens 8192 -> 3072 26.4 / 23.8, 28672 -> 8192
 // 114 / 86.  Not 1024 -> 2 x 2816 (19.1 / 19.9).
 // Square and small matrices take tiles of 32 tokens while they are one round of workgroups: the grid is filled with few
-// stretches of K or none, so the partial tiles and their adding pass go.  q/k/v of 2048 at 33 / 128 / 250 tokens 16.6 / 14.1,
-// 19.4 / 16.7, 23.6 / 18.4, of 3072 at 64 / 187 21.7 / 18.0, 30.0 / 24.0 (at 128 24.2 / 23.5 but 3072 x 3072 21.6 / 22.7: not taken), of 4096 at 64
-// 26.7 / 22.4 (at 128 26.9 / 28.5: not taken).
+// stretches of K or none, so the partial tiles and their adding pass go.  q/k/v with 512 (2048) and 1024 rows for k and v: of 2048 at
+// 33 / 128 / 250 tokens 16.6 / 13.2, 19.6 / 16.0, 23.6 / 17.8, of 3072 at 64 / 187 21.7 / 17.6, 30.7 / 24.3, of 4096 at 64 27.0 / 22.1.  Left slower, by up to 9 %: launches a little beyond a round,
+// q/k/v of 3072 with 1024 for k and v at 193 .. 224 tokens (30.9 / 33.6), of 2560 at 97 .. 128 (21.8 / 23.5), three of 3072 at 80.
 // Gate and up whose sums have to be cut to be as short as those of the 128-token tiles, so that they are two rounds of workgroups,
 // stay there: 2048 -> 2 x 5120 at 160 tokens 33.4 / 41.9, 1536 -> 2 x 4608 at 192 29.6 / 39.5.
+// Not taken, though measured faster here: gate and up at 33 .. 96 tokens (3072 -> 2 x 8192 at 33 / 64 / 96 32.2 / 25.3, 34.6 / 28.2, 36.6 /
+// 33.6, 4096 -> 2 x 14336 at 48 60.8 / 42.3), 257 .. 288 tokens (4096 -> 2 x 14336 147 / 129, 14336 -> 4096 101 / 74), squares beyond 64
+// tokens: 3072 at 128 21.5 / 18.0, 3584 at 97 / 160 22.1 / 19.6, 27.3 / 22.1, 4096 at 128 / 160 24.1 / 22.2, 29.0 / 25.1 (as q/k/v at
+// 192, beyond a round, 36.8 / 43.6).
 bool q8_0_tokens_takes(int64_t K, int64_t M, int64_t N) {
     if (K % BK != 0 || K > (1 << 24)) return false;   // 32-bit lane offsets: 128 rows of K bytes
     if (tuning_int("QPROJ_Q8_TAKE", 0)) return true;

@@ -583,7 +583,9 @@ StreamPlan stream_plan(int type, int64_t K, int64_t M, int64_t N) {
     int64_t n = std::max<int64_t>(1, wgs / stream_tiles(M, N, p.jt, p.kw));
     // Beyond 256 tokens k and v stay whole where q and they are one round together, or nearly one and a half: cut, they cost the
     // adding pass and more starts than they fill (q/k/v of 3072 at 384 tokens 37.4 -> 26.6 us, of 4096 at 512 56.8 -> 52.3, of 2048
-    // at 640 29.5 -> 22.4; 1.1 rounds, 4096 at 384 tokens, 46.0 cut and 50.1 whole).
+    // at 640 29.5 -> 22.4; 1.1 rounds, 4096 at 384 tokens, 46.0 cut and 50.1 whole).  In a call of its own a small one is the
+    // slower for it: 4096 -> 256 / 512 / 1024 at 288 tokens 19.6 us in the 64-token tiles, cut in stretches, and 22.0 whole here, 20.3 / 22.2,
+    // 22.3 / 22.5; 5120 -> 512 at 288 21.8 / 26.0; 4096 -> 1024 at 512 24.6 / 23.9.
     if (M > 256 && N <= 1024 && K > N) {
         const int64_t together = stream_tiles(M, K, p.jt, p.kw) + 2 * stream_tiles(M, N, p.jt, p.kw);
         if (together <= cus || together * 5 >= cus * 7) n = 1;
@@ -642,6 +644,9 @@ LaunchFn instance(int type, int jt, int kw, int waves) {   // null: not built
 // 46.7; 4096 -> 1024 at 1536 40.6 / 32.9; q/k/v of 4096 at 320 / 384 / 512 65.8 / 31.6, 53.0 / 46.1, 56.3 / 52.9, of 2048 at 512 39.4 / 20.1, at
 // 1024 35.7 / 35.0.  k and v follow q: streamed without it, 4096 -> 4096 / 1024 / 1024 at 640 tokens 58.9 / 86.  (Q6_K would gain as much,
 // 3072 q/k/v at 320 tokens 61.8 / 32.8, but with sums 1 to 4 % further from 64 bits than the stretches of its 64-token tiles.)
+// Left slower: q/k/v of fewer than 2048 weights a row where the three are more than one round together, which a matrix does not
+// know of: three of 1280 at 576 / 1024 tokens 25.2 / 28.7, 29.1 / 32.3, 1536 with 1024 for k and v at 768 28.5 / 29.6; the same square matrix alone (o) gains at those
+// sizes, 1280 at 1024 19.9 / 18.8.  Four waves a workgroup there are slower still.
 // Of the grids beyond one round of workgroups Q4_K keeps the older tiles from 97 tokens on, where arithmetic and not latency is the limit
 // (4096 -> 32000 at 128 tokens 51.0 us there, 54.0 here; at 96 tokens 50.1 against 45.3).  The 128-token kernels
 // keep the grids they fill (q4k_fills_wide, q6k_fills_wide) where they are as fast or faster, us there / here: Q4_K beyond

@@ -1109,8 +1109,6 @@ int mfma_grouped_pass_rows(int type, int64_t K, int64_t N, int64_t E, int64_t n_
     return wide ? 32 : 16;
 }
 
-// Expert-grouped form: args.order / args.offsets list each expert's pairs; `swiglu` takes tensors 0 and 1
-// as gate and up.  n_pairs only steers the launch shape (how many experts can be busy at once).
 // Whether the grouped launch gives every output one running sum over the whole row, as the expert tiles do.
 bool mfma_grouped_whole_rows(int type, int64_t K, int64_t N, int64_t E, int64_t n_pairs) {
     const int pass_rows = mfma_grouped_pass_rows(type, K, N, E, n_pairs), W = pass_rows == 32 ? 8 : type == kTypeQ4_K ? 4 : waves_per_wg(type);
@@ -1118,6 +1116,8 @@ bool mfma_grouped_whole_rows(int type, int64_t K, int64_t N, int64_t E, int64_t 
            plan(K, pass_rows, std::min<int64_t>(E, n_pairs) * ((N + 31) / 32), W).kw == 1;
 }
 
+// Expert-grouped form: args.order / args.offsets list each expert's pairs; `swiglu` takes tensors 0 and 1
+// as gate and up.  n_pairs only steers the launch shape (how many experts can be busy at once).
 hipError_t launch_gemv_mfma_grouped(const GemvArgs &args, int64_t n_pairs, bool swiglu, hipStream_t s, const Scratch &scratch) {
     MfmaArgs g{};
     g.n_targets = swiglu ? 2 : 1;

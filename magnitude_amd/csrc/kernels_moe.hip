@@ -9,13 +9,16 @@ namespace qproj {
 
 // Counting sort of (token, slot) pairs by expert id, one workgroup.  offsets[e]..offsets[e+1]
 // indexes the pairs of expert e inside order[]; active[] is the work list (active_slots_offset): the experts that
-// have pairs, or tiles of them (those with more than heavy_above pairs first: launch_moe_group, ascending within both parts).  Ids outside [0, n_expert) raise *error_flag and
-// their pairs are left out (their outputs are not written).  Pairs of one expert keep ascending
-// pair order so repeated runs produce the same launch geometry.  Each of the 16 waves takes every
-// 16th expert and sweeps the pair list 64 ids at a time (consecutive lanes on consecutive ids):
-// a ballot of the matches gives the count in the first sweep and, with the number of matching
-// lanes below one's own, the slot in the second.  (A version that read the ids from LDS inside the
-// sweeps was a chain of dependent loads: 19 us for 512 pairs and 128 experts.)
+// have pairs, or tiles of them (those with more than heavy_above pairs first: launch_moe_group, ascending within both parts).
+// Ids outside [0, n_expert) raise *error_flag and their pairs are left out (their outputs are not written).  Offsets and work
+// list follow from the counts alone, so repeated runs produce the same launch geometry; the order of an expert's pairs inside
+// order[] does not (moe_group_kernel below), and nothing that reads order[] may depend on it.
+//
+// Two ways to sort.  Up to 1536 experts a counter a wave and expert in LDS (moe_group_kernel).  Beyond, sweeps: each of
+// the 16 waves takes every 16th expert and sweeps the pair list 64 ids at a time (consecutive lanes on consecutive ids);
+// a ballot of the matches gives the count in the first sweep and, with the number of matching lanes below one's own, the slot
+// in the second: ascending pair order.  (A version that read the ids from LDS inside the sweeps was a chain of dependent loads:
+// 19 us for 512 pairs and 128 experts.)
 constexpr int kGroupThreads = 1024;
 constexpr int kGroupLdsIds = 8192;   // pair ids staged in LDS up to this many, read from global beyond
 

@@ -248,7 +248,7 @@ uint32_t q4k_multi_adds(int n, const WeightView *w, int64_t M, bool have_scratch
 hipError_t launch_gemm_q8k(const WeightView &w, const ActView &a, int64_t M, float *y, const Scratch &scratch, hipStream_t s);
 hipError_t launch_gemm_q8k_multi(int n, const WeightView *w, const ActView &a, int64_t M, float *const *y,
                                  const Scratch &scratch, hipStream_t s);
-// Q8_0 in tiles of 96 or 64 tokens x 128 rows (kernels_gemm_q8_0.hip); launch_gemm_q8_0 hands it the matrices it takes
+// Q8_0 in tiles of 96, 64 or 32 tokens (kernels_gemm_q8_0.hip); launch_gemm_q8_0 hands it the matrices it takes
 bool q8_0_tokens_takes(int64_t K, int64_t M, int64_t N);
 size_t q8_0_tokens_scratch_bytes(int64_t K, int64_t M, int64_t N);
 hipError_t launch_gemm_q8_0_tokens(int n, const WeightView *w, const ActView &a, int64_t M, float *const *y, const Scratch &scratch, hipStream_t s);
