@@ -367,23 +367,26 @@ Q8Plan q8_plan(int64_t K, int64_t M, int64_t N) {
     // in the tiles of 32 tokens)
     const int64_t least = p.wt > 1 ? (per32_splits(kTypeQ8_0, K, M, N) + p.kw - 1) / p.kw : 1;
     p.two_level = p.wt == 1;
-    // Where that leaves a workgroup two to four steps, most of it the start of a pipeline, half as many stretches in workgroups of
-    // half the rows, still one round, walk twice as far, their sums in two levels (error against 64 bits 0.68 to 0.94 of the
+    const auto tidy = [&](int64_t parts) {
+        parts = std::max<int64_t>(1, std::min<int64_t>(parts, units / 2));   // two times 256 weights a stretch at least
+        if ((M * N) % 4 != 0) parts = 1;
+        while (parts > 1 && (units + parts - 2) / (parts - 1) == (units + parts - 1) / parts) --parts;   // no stretch without work
+        return parts;
+    };
+    n = tidy(tuning_int("QPROJ_Q8_SPLIT", (int)std::max<int64_t>(n, least)));
+    // Where that leaves a workgroup two to four steps, most of it the start of a pipeline, about half as many stretches in workgroups
+    // of half the rows, still one round, walk twice as far, their sums in two levels (error against 64 bits 0.68 to 0.94 of the
     // 128-token tiles'; up to 1.02 of the short stretches').  us a call, 128-token tiles / eight waves, short stretches / four waves:
     // 3072 -> 1536 at 160 tokens 19.2 / 21.1 / 17.5, 4096 -> 1280 20.6 / 21.7 / 18.9, 3584 -> 2304 26.9 / 32.3 / 23.7, 5120 -> 1280 23.6 /
-    // 23.5 / 20.2; 4096 -> 3072 at 80 21.4 / 21.8 / 19.1, 8192 -> 4096 28.1 / 27.4 / 26.6.
+    // 23.5 / 20.2; 4096 -> 3072 at 80 21.4 / 21.8 / 19.1, 8192 -> 4096 28.1 / 27.4 / 26.6.  (Stretches that are one round in such workgroups
+    // as they are get them from the launcher and stay as they are: two levels would cost 4 % there.)
     if (p.wt == 3 && p.kw == 2 && K > N && !rider(K, N) && (units + n - 1) / n <= 4) {
-        const int64_t halves = cus / ((tiles_m * ((N + 63) / 64) + 7) / 8 * 8);
-        if (halves >= least) {
-            n = std::min<int64_t>(8, halves);
+        const int64_t half_stretch = (tiles_m * ((N + 63) / 64) + 7) / 8 * 8, halves = cus / half_stretch;
+        if (n * half_stretch > cus && halves >= least) {
+            n = tidy(std::min<int64_t>(8, halves));
             p.two_level = true;
         }
     }
-    n = std::max<int64_t>(n, least);
-    n = tuning_int("QPROJ_Q8_SPLIT", (int)n);
-    n = std::max<int64_t>(1, std::min<int64_t>(n, units / 2));   // two times 256 weights a stretch at least
-    if ((M * N) % 4 != 0) n = 1;
-    while (n > 1 && (units + n - 2) / (n - 1) == (units + n - 1) / n) --n;   // no stretch without work
     p.n_split = (int)n;
     p.one_round = tiles * n <= cus;
     return p;
@@ -516,8 +519,9 @@ hipError_t launch_gemm_q8_0_tokens(int n, const WeightView *w, const ActView &a,
             t.first_wg = (int)wg;
             wg += pad * p.n_split;
             if (dry_run())
-                plan_note("gemm_per32_kernel_q8_0<%d token tiles, %d K parts>%s: tile %d tokens x %d rows, %lld tiles x %d K stretches%s", p.wt, p.kw,
-                          g.n > 1 ? " (same launch)" : "", 32 * p.wt, 32 * rg, (long long)(t.tiles_n * tiles_m), p.n_split, p.n_split > 1 ? " + sum_parts_kernel" : "");
+                plan_note("gemm_per32_kernel_q8_0<%d token tiles, %d K parts>%s: tile %d tokens x %d rows, %lld tiles x %d K stretches%s%s", p.wt, p.kw,
+                          g.n > 1 ? " (same launch)" : "", 32 * p.wt, 32 * rg, (long long)(t.tiles_n * tiles_m), p.n_split,
+                          p.wt > 1 && p.two_level ? " of two levels of sums" : "", p.n_split > 1 ? " + sum_parts_kernel" : "");
         }
         first = i;
         g.tiles_m = (int)tiles_m;

@@ -297,12 +297,13 @@ def test_q8_0_short_stretches_are_walked_in_halves_of_the_rows(m, k, n, stretche
     """Eight waves and two to four steps of K a workgroup are mostly the start of a pipeline: half the rows and about half the
     stretches instead, never fewer than the 128-token tiles would make."""
     plan = qproj.plan_mul_mat(Q8_0, k, (n,), m)
-    assert f"x 64 rows, {-(-m // 96) * (n // 64)} tiles x {stretches} K stretches" in plan, plan
+    assert f"x 64 rows, {-(-m // 96) * (n // 64)} tiles x {stretches} K stretches of two levels of sums" in plan, plan
 
 
-@pytest.mark.parametrize("m,k,n", [(160, 6144, 3072), (160, 14336, 4096), (64, 4096, 3072)])
-def test_q8_0_longer_stretches_keep_eight_waves(m, k, n):
-    assert "x 128 rows" in qproj.plan_mul_mat(Q8_0, k, (n,), m)
+@pytest.mark.parametrize("m,k,n,rows", [(160, 6144, 3072, 128), (160, 14336, 4096, 128), (64, 4096, 3072, 128), (96, 5120, 1792, 64), (80, 5120, 1536, 64)])
+def test_q8_0_longer_stretches_and_those_of_one_round_keep_one_level(m, k, n, rows):
+    plan = qproj.plan_mul_mat(Q8_0, k, (n,), m)
+    assert f"x {rows} rows" in plan and "two levels" not in plan, plan
 
 
 @pytest.mark.parametrize("d,resident", [(2048, 2), (4096, 2), (7936, 2), (8192, 1)])

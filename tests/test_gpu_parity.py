@@ -699,15 +699,15 @@ def test_q8_0_tiles_of_96_64_and_32_tokens(ctx, orc, m, k, ns):
         w.free()
 
 
-@pytest.mark.parametrize("m,k,ns", [(80, 1536, (1284,)), (65, 2560, (2320,)), (130, 2560, (1800,)), (187, 2432, (1290,)), (192, 3072, (1536, 1440)),
-                                    (96, 3584, (2308,)), (161, 4224, (1157,)), (129, 8192, (1060,))])
-def test_q8_0_tiles_of_96_tokens_in_halves(ctx, orc, m, k, ns):
-    """The 96-token tiles of 64 rows that set their sums aside halfway: stretches of two, three and more steps, an odd number of
-    steps of 128 (the second K part idle in the last), whole K where M * N is no multiple of 4, ragged tokens and rows, two matrices.
+@pytest.mark.parametrize("m,k,ns", [(130, 2560, (1540,)), (187, 2432, (1668,)), (192, 3072, (1536, 1440)), (96, 3584, (2308,)), (160, 4224, (1540,)),
+                                    (129, 8192, (1060,)), (65, 8192, (2052,)), (161, 2944, (2564,))])
+def test_q8_0_tiles_of_96_tokens_in_two_levels_of_sums(ctx, orc, m, k, ns):
+    """The 96-token tiles of 64 rows that set their sums aside halfway: stretches of three to eight steps and last ones of one or two
+    (nothing set aside), an odd number of steps of 128 (the second K part idle in the last), ragged tokens and rows, two matrices.
     Oracle and tolerance as above."""
     from magnitude_amd import ACT_GGML, qproj
     plan = qproj.plan_mul_mat(Q8_0, k, list(ns), m, ACT_GGML)
-    assert plan.count("gemm_per32_kernel_q8_0<3 token tiles, 2 K parts>") == plan.count("tile 96 tokens x 64 rows") == len(ns), plan
+    assert plan.count("tile 96 tokens x 64 rows") == plan.count("two levels of sums") == len(ns), plan
     rng = np.random.default_rng(m + k)
     x = rng.standard_normal((m, k)).astype(np.float32)
     blocks = [make_weight(orc, Q8_0, n, k, seed=6600 + i) for i, n in enumerate(ns)]
