@@ -1,4 +1,4 @@
-// Small-batch projection (2..16 activation rows, the speculative-verify regime) on the int8 matrix
+// Small-batch projection (3..32 activation rows, the speculative-verify regime) on the int8 matrix
 // cores: the weights are streamed from HBM once and every row of activations is applied to them.
 //
 // One v_mfma_i32_32x32x32_i8 (Q4_K, Q8_0) or v_mfma_i32_32x32x16_i8 (Q6_K) multiplies the int8
@@ -15,9 +15,9 @@
 // super-block with fully coalesced 16-byte loads (consecutive lanes = consecutive 16-byte pieces
 // of a row's block), two super-blocks ahead of the arithmetic, parks the registers in a
 // wave-private LDS region and reads the region back in operand order.  The quantized
-// activations of the workgroup's K range are staged in LDS once.
+// activations of the workgroup's K range are staged in LDS once, ahead of the weights.
 //
-// Work split.  A workgroup is 4 waves = rw row groups (32 rows each) x kw K-parts; the K-parts
+// Work split.  A workgroup is 8 waves = rw row groups (32 rows each) x kw K-parts; the K-parts
 // of a row group are summed through LDS in a fixed order.  When one workgroup cannot hold the
 // whole K range (LDS) or there would be too few workgroups, K is also cut into chunks whose
 // results go to a scratch buffer that a second small kernel sums in chunk order, so results do
@@ -26,13 +26,16 @@
 // nothing returned): two addends on zero give the same sum in either order, so this does not
 // depend on scheduling either, and the summing launch goes.  (The memory-side adder may flush a
 // sum below the smallest normal float to zero.)
+#include <limits.h>
 #include <stdlib.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "qproj_device.h"
 #include "qproj_internal.h"
 #include "actquant_device.h"
+#include "lds_direct.h"
 
 namespace qproj {
 
@@ -42,24 +45,42 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
 
+// Dense launch: y[m][n] of up to four matrices for M rows of quantized activations.  What every workgroup reads first
+// stands together: the arguments come from memory a 64-byte line at a time, and each line is a trip of its own.
+struct DenseTarget {
+    const uint8_t *p[4];   // Q4_K: blocks; Q6_K: ql, qh, scales, d; Q8_0: quants, d
+    float *y;
+    float *part;           // [n_chunks][M][N] when n_chunks > 1
+    int64_t N;
+};
+
+struct DenseArgs {
+    const int8_t *qs;      // activation planes
+    const float *d;
+    const int16_t *bsums;
+    int M, nb, n_chunks, chunk_sb, kw_log2, rw;   // nb: super-blocks of a row; 2^kw_log2 x rw waves a workgroup
+    int rpg;               // weight rows a row group: 32 fill the matrix instruction, fewer even out a small grid
+    int add_out;           // two chunks, output rows cleared before the launch: both chunks add to y
+    int first_wg[kMaxTargets];     // of the launch's matrices; INT_MAX where there is none
+    int n_rowsets[kMaxTargets];
+    DenseTarget t[kMaxTargets];
+    int n_targets;
+};
+
 struct MfmaTarget {
     WeightView w;
     float *y;
-    float *part;       // [n_chunks][M][N] when n_chunks > 1
-    int first_wg;
-    int n_rowsets;
+    float *part;       // [n_chunks][n_pairs][N] when n_chunks > 1
 };
 
+// expert-grouped launch (MUL_MAT_ID)
 struct MfmaArgs {
-    int n_targets;
-    MfmaTarget t[kMaxTargets];
+    MfmaTarget t[2];
     ActView a;
     const float *x;        // non-null: fp32 activation rows [rows][K], quantized by every workgroup in its prologue
-    int M, n_chunks, chunk_sb, kw, rw, n_wgs;
-    int rpg;               // weight rows a row group (32 fill the matrix instruction; dense launches may take fewer, below)
-    int add_out;           // dense mode, two chunks, output rows cleared before the launch: both chunks add to y
-    int64_t part_plane;    // expert-grouped mode with K in chunks: floats of one chunk's results, [n_pairs][N], in t[0].part
-    // expert-grouped mode (MUL_MAT_ID): activation rows of expert e are the pairs order[offsets[e]..offsets[e+1])
+    int n_chunks, chunk_sb, kw, rw, n_wgs;
+    int64_t part_plane;    // K in chunks: floats of one chunk's results, [n_pairs][N], in t[0].part
+    // activation rows of expert e are the pairs order[offsets[e]..offsets[e+1])
     const int32_t *order;
     const int32_t *offsets;
     const int32_t *active;  // experts that have pairs; active[n_expert] = how many
@@ -382,16 +403,40 @@ __device__ __forceinline__ void split_sum(int s, uint32_t &hi, uint32_t &lo, int
     lo |= (uint32_t)(s & 63) << (8 * pos);
 }
 
+// the sixteen block sums of a super-block (two a word) as the kernels' auxiliary operand: Q4_K sums of 32 (8 high bytes, 8 low
+// ones), Q6_K sums of 16 (16 and 16)
+template <int QT>
+__device__ __forceinline__ void split_sums(const uint32_t (&w)[8], uint8_t *dst) {
+    if constexpr (QT == kTypeQ4_K) {
+        uint32_t hi[2] = {0, 0}, lo[2] = {0, 0};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int s = (int)(int16_t)(w[j] & 0xffff) + (int)(int16_t)(w[j] >> 16);
+            split_sum(s, hi[j >> 2], lo[j >> 2], j & 3);
+        }
+        *reinterpret_cast<uint4 *>(dst) = make_uint4(hi[0], hi[1], lo[0], lo[1]);
+    } else {
+        uint32_t hi[4] = {0, 0, 0, 0}, lo[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int s = (int)(int16_t)((w[j >> 1] >> (16 * (j & 1))) & 0xffff);
+            split_sum(s, hi[j >> 2], lo[j >> 2], j & 3);
+        }
+        *reinterpret_cast<uint4 *>(dst) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        *reinterpret_cast<uint4 *>(dst + 16) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+    }
+}
+
 // Copies the quantized activations of super-blocks [c0, c0 + nsb) into LDS: staged row m (< n_rows) comes from
 // activation row src_row(m).
-template <int QT, int MT, int kThreads, bool MAPPED>
+template <int QT, int MT, int kThreads>
 __device__ __forceinline__ void stage_activations(const MfmaArgs &g, uint8_t *smem, const Layout &L, int c0, int nsb,
-                                                  int n_rows, int m0) {
+                                                  int n_rows) {
     const int tid = threadIdx.x;
     const int nb = (int)(g.a.K >> 8);
     const int row16 = nsb * 16;
     const int *map = reinterpret_cast<const int *>(smem + L.off_map);
-    auto src_row = [&](int m) -> size_t { return MAPPED ? (size_t)(map[m] / g.x_div) : (size_t)(m0 + m); };
+    auto src_row = [&](int m) -> size_t { return (size_t)(map[m] / g.x_div); };
     const int total = n_rows * row16;
     for (int base = 0; base < total; base += 4 * kThreads) {
         uint4 v[4];
@@ -419,25 +464,7 @@ __device__ __forceinline__ void stage_activations(const MfmaArgs &g, uint8_t *sm
             const uint4 *src = reinterpret_cast<const uint4 *>(g.a.bsums + (src_row(m) * nb + c0 + sb) * 16);
             const uint4 b0 = src[0], b1 = src[1];
             const uint32_t w[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
-            uint8_t *dst = smem + L.off_aux + (sb * MT + m) * Cfg<QT>::kAux;
-            if constexpr (QT == kTypeQ4_K) {
-                uint32_t hi[2] = {0, 0}, lo[2] = {0, 0};
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int s = (int)(int16_t)(w[j] & 0xffff) + (int)(int16_t)(w[j] >> 16);
-                    split_sum(s, hi[j >> 2], lo[j >> 2], j & 3);
-                }
-                *reinterpret_cast<uint4 *>(dst) = make_uint4(hi[0], hi[1], lo[0], lo[1]);
-            } else {
-                uint32_t hi[4] = {0, 0, 0, 0}, lo[4] = {0, 0, 0, 0};
-#pragma unroll
-                for (int j = 0; j < 16; ++j) {
-                    const int s = (int)(int16_t)((w[j >> 1] >> (16 * (j & 1))) & 0xffff);
-                    split_sum(s, hi[j >> 2], lo[j >> 2], j & 3);
-                }
-                *reinterpret_cast<uint4 *>(dst) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-                *reinterpret_cast<uint4 *>(dst + 16) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-            }
+            split_sums<QT>(w, smem + L.off_aux + (sb * MT + m) * Cfg<QT>::kAux);
         }
     }
 }
@@ -497,25 +524,7 @@ struct StagedRows {
             if (tid < n_rows * nsb) {
                 const int m = tid / nsb, sb = tid - m * nsb;
                 const uint32_t w[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
-                uint8_t *dstb = smem + L.off_aux + (sb * MT + m) * Cfg<QT>::kAux;
-                if constexpr (QT == kTypeQ4_K) {
-                    uint32_t hi[2] = {0, 0}, lo[2] = {0, 0};
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        const int s = (int)(int16_t)(w[j] & 0xffff) + (int)(int16_t)(w[j] >> 16);
-                        split_sum(s, hi[j >> 2], lo[j >> 2], j & 3);
-                    }
-                    *reinterpret_cast<uint4 *>(dstb) = make_uint4(hi[0], hi[1], lo[0], lo[1]);
-                } else {
-                    uint32_t hi[4] = {0, 0, 0, 0}, lo[4] = {0, 0, 0, 0};
-#pragma unroll
-                    for (int j = 0; j < 16; ++j) {
-                        const int s = (int)(int16_t)((w[j >> 1] >> (16 * (j & 1))) & 0xffff);
-                        split_sum(s, hi[j >> 2], lo[j >> 2], j & 3);
-                    }
-                    *reinterpret_cast<uint4 *>(dstb) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-                    *reinterpret_cast<uint4 *>(dstb + 16) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-                }
+                split_sums<QT>(w, smem + L.off_aux + (sb * MT + m) * Cfg<QT>::kAux);
             }
         }
     }
@@ -524,13 +533,13 @@ struct StagedRows {
 // The same LDS image made from fp32 rows: each wave quantizes whole 256-element chunks (ggml's
 // quantize_row_q8_K, or eight quantize_row_q8_0 blocks for Q8_0 weights) exactly as the standalone
 // quantizer kernels do, so both routes stage identical bytes.  Two chunks are in flight per wave.
-template <int QT, int MT, int kThreads, bool MAPPED>
+template <int QT, int MT, int kThreads>
 __device__ __forceinline__ void stage_quantize(const MfmaArgs &g, uint8_t *smem, const Layout &L, int c0, int nsb,
-                                               int n_rows, int m0) {
+                                               int n_rows) {
     constexpr int NWAVES = kThreads / 64;
     const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
     const int *map = reinterpret_cast<const int *>(smem + L.off_map);
-    auto src_row = [&](int m) -> size_t { return MAPPED ? (size_t)(map[m] / g.x_div) : (size_t)(m0 + m); };
+    auto src_row = [&](int m) -> size_t { return (size_t)(map[m] / g.x_div); };
     float *dxs = reinterpret_cast<float *>(smem + L.off_dx);
     const int total = n_rows * nsb;
     for (int base = 0; base < total; base += 2 * NWAVES) {
@@ -578,71 +587,49 @@ __device__ __forceinline__ void stage_quantize(const MfmaArgs &g, uint8_t *smem,
 
 constexpr int kDense = 0, kGrouped = 1, kGroupedSwiglu = 2;
 
-// MODE kDense: y[m][n] for the M rows of `a`.  kGrouped: the workgroup's expert e multiplies its
-// own pairs, y[pair][n].  kGroupedSwiglu: tensors 0 and 1 are gate and up of the same expert and
-// y[pair][n] = silu(gate . x) * (up . x).
-// FLAT (expert-grouped launches with K in one part, kw = 1): the wave's row groups as one stream of items.
+// kGrouped: the workgroup's expert e multiplies its own pairs, y[pair][n].  kGroupedSwiglu: tensors 0 and 1 are gate
+// and up of the same expert and y[pair][n] = silu(gate . x) * (up . x).  (kDense: gemv_mfma_dense_kernel.)
+// FLAT (K in one part, kw = 1): the wave's row groups as one stream of items.
 template <int QT, int NI, int W, int MODE, bool FLAT = false>
 __global__ __launch_bounds__(W * 64) void gemv_mfma_kernel(const MfmaArgs g) {
-    static_assert(!FLAT || MODE != kDense, "the flat item stream is for the expert-grouped modes");
+    static_assert(MODE != kDense, "dense launches have their own kernel");
     extern __shared__ __align__(16) uint8_t smem[];
     constexpr int MT = 8 * NI, NV = 4 * NI;
-    constexpr bool GROUPED = MODE != kDense, SWIGLU = MODE == kGroupedSwiglu;
+    constexpr bool SWIGLU = MODE == kGroupedSwiglu;
     constexpr int NT = SWIGLU ? 2 : 1;   // tensors streamed by one wave
     const Layout L = layout<QT, MT, W>(g.chunk_sb);
     const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
     const int h = lane >> 5, nl = lane & 31;
 
-    // workgroup -> (tensor or expert, K chunk, set of rw row groups)
-    WeightView w = g.t[0].w;
-    float *y = g.t[0].y, *part = g.t[0].part;
-    int c = 0, rs, expert = 0, pair0 = 0, n_rows = g.M;
-    if constexpr (GROUPED) {
-        const int slotc = (int)blockIdx.x / g.wgs_per_expert;   // the grid covers min(E, pairs) experts x K chunks
-        rs = (int)blockIdx.x - slotc * g.wgs_per_expert;
-        const int slot = slotc / g.n_chunks;
-        c = slotc - slot * g.n_chunks;
-        if (g.ids) {   // a workgroup set per pair
-            if (slot >= g.n_pairs) return;
-            expert = g.ids[slot];
-            if (expert < 0 || expert >= g.n_expert) {   // the pair is left out, as the grouping pass would
-                if (rs == 0 && threadIdx.x == 0) atomicOr(g.error_flag, 1);
-                return;
-            }
-            pair0 = slot;
-            n_rows = 1;
-        } else {
-            if (slot >= g.active[g.n_expert]) return;
-            const int4 rec = reinterpret_cast<const int4 *>(g.active + active_slots_offset(g.n_expert))[slot];
-            expert = rec.x;   // (one load: the list position's expert, first pair slot and pair count)
-            pair0 = rec.y;
-            n_rows = rec.z;
-            if (n_rows <= 0) return;
+    // workgroup -> (expert, K chunk, set of rw row groups)
+    const WeightView w = g.t[0].w;
+    float *y = g.t[0].y;
+    int expert, pair0, n_rows;
+    const int slotc = (int)blockIdx.x / g.wgs_per_expert;   // the grid covers min(E, pairs) experts x K chunks
+    const int rs = (int)blockIdx.x - slotc * g.wgs_per_expert;
+    const int slot = slotc / g.n_chunks, c = slotc - slot * g.n_chunks;
+    if (g.ids) {   // a workgroup set per pair
+        if (slot >= g.n_pairs) return;
+        expert = g.ids[slot];
+        if (expert < 0 || expert >= g.n_expert) {   // the pair is left out, as the grouping pass would
+            if (rs == 0 && threadIdx.x == 0) atomicOr(g.error_flag, 1);
+            return;
         }
+        pair0 = slot;
+        n_rows = 1;
     } else {
-        int ti = 0;
-#pragma unroll
-        for (int i = 1; i < kMaxTargets; ++i)
-            if (i < g.n_targets && (int)blockIdx.x >= g.t[i].first_wg) ti = i;
-        int first = g.t[0].first_wg, nrs = g.t[0].n_rowsets;
-#pragma unroll
-        for (int i = 1; i < kMaxTargets; ++i)
-            if (ti == i) {
-                w = g.t[i].w;
-                y = g.t[i].y;
-                part = g.t[i].part;
-                first = g.t[i].first_wg;
-                nrs = g.t[i].n_rowsets;
-            }
-        const int local = (int)blockIdx.x - first;
-        c = local / nrs;
-        rs = local - c * nrs;
+        if (slot >= g.active[g.n_expert]) return;
+        const int4 rec = reinterpret_cast<const int4 *>(g.active + active_slots_offset(g.n_expert))[slot];
+        expert = rec.x;   // (one load: the list position's expert, first pair slot and pair count)
+        pair0 = rec.y;
+        n_rows = rec.z;
+        if (n_rows <= 0) return;
     }
     const int N = (int)w.N;
     const int nb = (int)(g.a.K >> 8);
     const int c0 = c * g.chunk_sb, nsb = min(g.chunk_sb, nb - c0);
-    if constexpr (GROUPED)   // K in chunks: the chunk's results go to its plane of the scratch, a pass adds the planes
-        if (g.n_chunks > 1) y = part + (size_t)c * g.part_plane;
+    // K in chunks: the chunk's results go to its plane of the scratch, a pass adds the planes
+    if (g.n_chunks > 1) y = g.t[0].part + (size_t)c * g.part_plane;
 
     // wave -> (row group, K part)
     const int rgl = wave / g.kw, kp = wave - rgl * g.kw;
@@ -653,7 +640,7 @@ __global__ __launch_bounds__(W * 64) void gemv_mfma_kernel(const MfmaArgs g) {
     Stager<QT> sa, sb_;
     // the wave's rg-th row group: rows, how much of K, where its blocks start
     auto set_rowgroup = [&](int rg) {
-        row0 = ((rs * (GROUPED ? g.rg_loop : 1) + rg) * g.rw + rgl) * (GROUPED ? 32 : g.rpg);
+        row0 = ((rs * g.rg_loop + rg) * g.rw + rgl) * 32;
         rows_ok = row0 < N;
         steps = rows_ok ? s1 - s0 : 0;
         items = NT * steps;                       // (tensor, super-block) pairs this wave streams
@@ -661,7 +648,7 @@ __global__ __launch_bounds__(W * 64) void gemv_mfma_kernel(const MfmaArgs g) {
         const int64_t row = (int64_t)expert * N + (rows_ok ? row0 : 0);
         sa.rebase(0, w, row);
         sa.rebase(1, SWIGLU ? g.t[1].w : w, row);
-        const int last_row = rows_ok ? min((GROUPED ? 32 : g.rpg) - 1, N - 1 - row0) : 0;   // rows past it repeat it
+        const int last_row = rows_ok ? min(31, N - 1 - row0) : 0;   // rows past it repeat it
         sa.init(w, last_row, lane);
         sb_.rebase(0, w, row);
         sb_.rebase(1, SWIGLU ? g.t[1].w : w, row);
@@ -733,9 +720,9 @@ __global__ __launch_bounds__(W * 64) void gemv_mfma_kernel(const MfmaArgs g) {
                     }
                     rows.store(smem, L, nsb, m_cnt);
                 } else if (g.x) {
-                    stage_quantize<QT, MT, W * 64, GROUPED>(g, smem, L, c0, nsb, m_cnt, m0);
+                    stage_quantize<QT, MT, W * 64>(g, smem, L, c0, nsb, m_cnt);
                 } else {
-                    stage_activations<QT, MT, W * 64, GROUPED>(g, smem, L, c0, nsb, m_cnt, m0);
+                    stage_activations<QT, MT, W * 64>(g, smem, L, c0, nsb, m_cnt);
                 }
                 __syncthreads();
 
@@ -792,27 +779,25 @@ __global__ __launch_bounds__(W * 64) void gemv_mfma_kernel(const MfmaArgs g) {
         }
     }
 
-    // dense launches stage all (<= MT) rows at once; an expert with more than MT pairs takes several passes
+    // an expert with more than MT pairs takes several passes
     if constexpr (!FLAT)
-    for (int m0 = 0; m0 < (GROUPED ? n_rows : 1); m0 += MT)
-    for (int rg = 0; rg < (GROUPED ? g.rg_loop : 1); ++rg) {   // the rows staged for this pass serve all of the wave's row groups
+    for (int m0 = 0; m0 < n_rows; m0 += MT)
+    for (int rg = 0; rg < g.rg_loop; ++rg) {   // the rows staged for this pass serve all of the wave's row groups
         const int m_cnt = min(MT, n_rows - m0);
         set_rowgroup(rg);
         issue(sa, 0);
         issue(sb_, 1);
         if (rg == 0) {
-            if constexpr (GROUPED) {
-                if (m0 > 0) __syncthreads();   // the previous pass is done with the staged rows and the regions
-                if ((int)threadIdx.x < MT)
-                    map[threadIdx.x] = (int)threadIdx.x >= m_cnt ? 0
-                                       : g.ids      ? pair0 + m0 + (int)threadIdx.x
-                                                    : g.order[pair0 + m0 + (int)threadIdx.x];
-                __syncthreads();
-            }
+            if (m0 > 0) __syncthreads();   // the previous pass is done with the staged rows and the regions
+            if ((int)threadIdx.x < MT)
+                map[threadIdx.x] = (int)threadIdx.x >= m_cnt ? 0
+                                   : g.ids      ? pair0 + m0 + (int)threadIdx.x
+                                                : g.order[pair0 + m0 + (int)threadIdx.x];
+            __syncthreads();
             if (g.x)
-                stage_quantize<QT, MT, W * 64, GROUPED>(g, smem, L, c0, nsb, m_cnt, m0);
+                stage_quantize<QT, MT, W * 64>(g, smem, L, c0, nsb, m_cnt);
             else
-                stage_activations<QT, MT, W * 64, GROUPED>(g, smem, L, c0, nsb, m_cnt, m0);
+                stage_activations<QT, MT, W * 64>(g, smem, L, c0, nsb, m_cnt);
             __syncthreads();
         } else if (g.kw > 1) {
             __syncthreads();   // the partial tiles the previous row group left in the regions have been summed
@@ -867,29 +852,238 @@ __global__ __launch_bounds__(W * 64) void gemv_mfma_kernel(const MfmaArgs g) {
             }
         }
         if (kp == 0 && rows_ok) {
-            const bool add = !GROUPED && g.add_out;
-            float *dst = GROUPED || g.n_chunks == 1 || add ? y : part + (size_t)c * g.M * N;
             const int n = row0 + nl;
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
                 const int m = 8 * (v >> 2) + 4 * h + (v & 3);
                 float r = out[0][v];
                 if constexpr (SWIGLU) r = (r / (1.0f + expf(-r))) * out[NT - 1][v];
-                if (m < m_cnt && n < N && (GROUPED || nl < g.rpg)) {
-                    float *o = dst + (size_t)(GROUPED ? map[m] : m0 + m) * N + n;
-                    // two addends on zero: the sum does not depend on which chunk arrives first
-                    if (add) unsafeAtomicAdd(o, r);
-                    else *o = r;
-                }
+                if (m < m_cnt && n < N) y[(size_t)map[m] * N + n] = r;
             }
         }
     }
 }
 
+// What a dense workgroup needs of the quantized activation rows, asked for in ONE go and ahead of the first weights: a
+// wave's share of the codes (a super-block of a row is 16 lanes, at most eight requests a wave) and one record of scales and
+// block sums a thread.  Loads come back in the order they were asked for, over all waves of a compute unit: behind 74 KB of
+// weights, and in three rounds one after the other, these 40 KB that sit in L2 took 4 to 9 us of a workgroup's 10 to 26
+// (phase clocks; o at 8 rows, and the Q6_K down projection).  (Straight into LDS is no better: the compiler then waits for
+// every request, the weights' too, before it touches LDS.)
+template <int QT, int MT, int W>
+struct DenseRows {
+    static constexpr int ND = Cfg<QT>::kDx, kPieces = 256 / (4 * W);
+    v4i v[kPieces], b0, b1;      // b: Q8_0 the eight scales, otherwise sixteen block sums
+    float d, inv_nsb;
+    int total, nsb;              // super-blocks of all rows (at most 256)
+    // super-block u of the M x nsb: row and place in the row (the half keeps the quotient away from whole numbers)
+    __device__ __forceinline__ void place(int u, int &m, int &sb) const {
+        m = (int)(((float)u + 0.5f) * inv_nsb);
+        sb = u - m * nsb;
+    }
+    __device__ __forceinline__ int unit(int j, int wave, int lane) const { return min(4 * (wave + W * j) + (lane >> 4), total - 1); }
+    __device__ __forceinline__ void request(const DenseArgs &g, int c0, int nsb_, int wave, int lane) {
+        static_assert(W * 64 >= 256, "a record a thread");
+        nsb = nsb_;
+        total = g.M * nsb;
+        inv_nsb = __builtin_amdgcn_rcpf((float)nsb);
+        const int nb = g.nb;
+        global_ptr<int8_t> qs = (global_ptr<int8_t>)g.qs;
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile("" : "+s"(qs));   // (or every request below loads the pointer anew and waits for it)
+#endif
+        int m, sb;
+        place(min((int)threadIdx.x, total - 1), m, sb);
+        const int at = m * nb + c0 + sb;
+        if constexpr (QT == kTypeQ8_0) {
+            const v4i *src = reinterpret_cast<const v4i *>(g.d + (size_t)at * 8);
+            b0 = src[0];
+            b1 = src[1];
+            d = 0.f;
+        } else {
+            d = g.d[at];
+            const v4i *src = reinterpret_cast<const v4i *>(g.bsums + (size_t)at * 16);
+            b0 = src[0];
+            b1 = src[1];
+        }
+#pragma unroll
+        for (int j = 0; j < kPieces; ++j)
+            if (4 * (wave + W * j) < total) {   // wave-uniform
+                place(unit(j, wave, lane), m, sb);
+                v[j] = load_global<v4i>(qs, (uint32_t)(m * nb + c0 + sb) * 256u + 16u * (uint32_t)(lane & 15));
+            }
+    }
+    __device__ __forceinline__ void store(uint8_t *smem, const Layout &L, int wave, int lane) const {
+        int m, sb;
+        if ((int)threadIdx.x < total) {
+            place((int)threadIdx.x, m, sb);
+            float *dxs = reinterpret_cast<float *>(smem + L.off_dx) + sb * ND * MT + m;
+            const uint32_t w[8] = {(uint32_t)b0[0], (uint32_t)b0[1], (uint32_t)b0[2], (uint32_t)b0[3], (uint32_t)b1[0], (uint32_t)b1[1], (uint32_t)b1[2], (uint32_t)b1[3]};
+            if constexpr (QT == kTypeQ8_0) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) dxs[j * MT] = __uint_as_float(w[j]);
+            } else {
+                *dxs = d;
+                split_sums<QT>(w, smem + L.off_aux + (sb * MT + m) * Cfg<QT>::kAux);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < kPieces; ++j)
+            if (4 * (wave + W * j) < total) {
+                place(unit(j, wave, lane), m, sb);
+                *reinterpret_cast<v4i *>(smem + m * L.lda + sb * 256 + 16 * (lane & 15)) = v[j];
+            }
+    }
+};
+
+// Dense launches: a workgroup is rw row groups x kw K parts of a K chunk.  The rows beyond M are staged by nobody: what
+// lies there only reaches results that are not stored.
+// Bound: latency.  Of the 9 us of a 4096 x 4096 Q4_K launch at 8 rows the arithmetic took 1.5; the rest was one trip to
+// memory after another.  Arguments in one go, staged rows in one go ahead of the weights, K parts added by all waves, us a
+// launch before / after (4096, 14336, 8 rows): q/k/v 9.4 / 6.9, o 9.0 / 6.6, gate + up 18.4 / 16.8, Q6_K down 18.2 / 15.9.
+// (A barrier between the rows' requests and the weights': level.  K parts of 3 and 4 super-blocks instead of 4 and 0: level.)
+template <int QT, int NI, int W>
+__global__ __launch_bounds__(W * 64) void gemv_mfma_dense_kernel(const DenseArgs g) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    constexpr int MT = 8 * NI, NV = 4 * NI;
+    const Layout L = layout<QT, MT, W>(g.chunk_sb);
+    const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
+    const int h = lane >> 5, nl = lane & 31;
+
+    // every line of the arguments is asked for here, in one go: left to itself the compiler loads them where they are used,
+    // a trip to memory each time
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" ::"s"(g.qs), "s"(g.d), "s"(g.bsums), "s"(g.M), "s"(g.nb), "s"(g.n_chunks), "s"(g.chunk_sb), "s"(g.kw_log2), "s"(g.rw), "s"(g.rpg),
+                 "s"(g.add_out), "s"(g.n_rowsets[0]), "s"(g.n_rowsets[1]), "s"(g.n_rowsets[2]), "s"(g.n_rowsets[3]), "s"(g.t[0].p[0]), "s"(g.t[1].p[0]),
+                 "s"(g.t[2].p[0]), "s"(g.t[3].p[0]));
+#endif
+    // workgroup -> (tensor, K chunk, set of rw row groups)
+    int ti = 0, first = 0, nrs = g.n_rowsets[0];
+#pragma unroll
+    for (int i = 1; i < kMaxTargets; ++i)
+        if ((int)blockIdx.x >= g.first_wg[i]) {
+            ti = i;
+            first = g.first_wg[i];
+            nrs = g.n_rowsets[i];
+        }
+    const DenseTarget &t = g.t[ti];
+    const int local = (int)blockIdx.x - first;
+    const int c = g.n_chunks == 1 ? 0 : local / nrs, rs = local - c * nrs;
+    const int N = (int)t.N, c0 = c * g.chunk_sb, nsb = min(g.chunk_sb, g.nb - c0);
+
+    // wave -> (row group, K part)
+    const int rgl = wave >> g.kw_log2, kp = wave - (rgl << g.kw_log2);
+    const int part_sb = (nsb + (1 << g.kw_log2) - 1) >> g.kw_log2;
+    const int s0 = min(kp * part_sb, nsb), s1 = min(s0 + part_sb, nsb);  // range inside the chunk
+    const int row0 = (rs * g.rw + rgl) * g.rpg;
+    const bool rows_ok = row0 < N;
+    const int steps = rows_ok ? s1 - s0 : 0;
+    const int last_sb = c0 + (steps > 0 ? s1 - 1 : 0);   // loads past the range repeat its last super-block
+    WeightView w{};
+    w.K = (int64_t)g.nb * 256;
+    w.nb = QT == kTypeQ8_0 ? g.nb * 8 : g.nb;
+    w.q4k = w.q6_ql = t.p[0];
+    w.q8_qs = reinterpret_cast<const int8_t *>(t.p[0]);
+    w.q8_d = reinterpret_cast<const uint16_t *>(t.p[1]);
+    w.q6_qh = t.p[1];
+    w.q6_sc = reinterpret_cast<const int8_t *>(t.p[2]);
+    w.q6_d = reinterpret_cast<const uint16_t *>(t.p[3]);
+    Stager<QT> sa, sb_;
+    sa.rebase(0, w, rows_ok ? row0 : 0);
+    sa.init(w, rows_ok ? min(g.rpg - 1, N - 1 - row0) : 0, lane);   // rows past the group's last one repeat it
+    sb_ = sa;
+    auto issue = [&](Stager<QT> &st, int i) { st.issue(0, min(c0 + s0 + i, last_sb)); };
+    uint8_t *region = smem + L.off_w + wave * Cfg<QT>::kRegion;
+    // (the addresses stand before the first request: worked out behind it they were mixed with registers still waiting for
+    // their loads)
+    __builtin_amdgcn_sched_barrier(0);
+
+    DenseRows<QT, MT, W> rows;
+    rows.request(g, c0, nsb, wave, lane);
+    asm volatile("" ::: "memory");   // the weights' requests stay behind these, and in their order
+    __builtin_amdgcn_sched_barrier(0);
+    issue(sa, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    issue(sb_, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    rows.store(smem, L, wave, lane);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+
+    float out[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) out[v] = 0.f;
+    auto consume = [&](int i) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        compute<QT, NI>(region, smem, L, s0 + i, lane, out);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    };
+    int i = 0;
+    for (; i + 1 < steps; i += 2) {
+        sa.park(region, lane);
+        issue(sa, i + 2);
+        consume(i);
+        sb_.park(region, lane);
+        issue(sb_, i + 3);
+        consume(i + 1);
+    }
+    if (i < steps) {
+        sa.park(region, lane);
+        consume(i);
+    }
+
+    const bool add = g.add_out;
+    float *dst = g.n_chunks == 1 || add ? t.y : t.part + (size_t)c * g.M * N;
+    auto store = [&](int m, int n, float r) {
+        float *o = dst + (size_t)m * N + n;
+        // two addends on zero: the sum does not depend on which chunk arrives first
+        if (add) unsafeAtomicAdd(o, r);
+        else *o = r;
+    };
+    if (g.kw_log2 == 0) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int m = 8 * (v >> 2) + 4 * h + (v & 3);
+            if (m < g.M && nl < g.rpg && row0 + nl < N) store(m, row0 + nl, out[v]);
+        }
+        return;
+    }
+    // The K parts of a row group meet in the waves' regions and are added in a fixed order, an output a thread of ALL
+    // waves (a group's first wave alone, four outputs a lane and one part after the other, took 1.6 us of the 8-row o).
+    float *mine = reinterpret_cast<float *>(region);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) mine[(8 * (v >> 2) + 4 * h + (v & 3)) * 32 + nl] = out[v];
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    auto add_parts = [&](auto parts) {
+        constexpr int KW = decltype(parts)::value, kOut = W / KW * MT * 32;
+#pragma unroll
+        for (int e0 = 0; e0 < kOut; e0 += W * 64) {
+            const int e = e0 + (int)threadIdx.x, group = e / (MT * 32), m = e / 32 % MT, n = e % 32;
+            const int r0 = (rs * g.rw + group) * g.rpg;
+            if (e < kOut && m < g.M && n < g.rpg && r0 + n < N) {
+                const uint8_t *src = smem + L.off_w + group * KW * Cfg<QT>::kRegion + (m * 32 + n) * 4;
+                float p[KW];
+#pragma unroll
+                for (int q = 0; q < KW; ++q) p[q] = *reinterpret_cast<const float *>(src + q * Cfg<QT>::kRegion);
+                float acc = p[0];
+#pragma unroll
+                for (int q = 1; q < KW; ++q) acc += p[q];
+                store(m, r0 + n, acc);
+            }
+        }
+    };
+    if (g.kw_log2 == 1) add_parts(std::integral_constant<int, 2>{});
+    else if (g.kw_log2 == 2) add_parts(std::integral_constant<int, 4>{});
+    else if (g.kw_log2 == 3) {
+        if constexpr (W >= 8) add_parts(std::integral_constant<int, 8>{});
+    } else {
+        if constexpr (W >= 16) add_parts(std::integral_constant<int, 16>{});
+    }
+}
+
 // y[i] = sum over chunks of part[c][i], chunk order fixed
-__global__ __launch_bounds__(256) void sum_chunks_kernel(const MfmaArgs g) {
+__global__ __launch_bounds__(256) void sum_chunks_kernel(const DenseArgs g) {
     for (int ti = 0; ti < g.n_targets; ++ti) {
-        const size_t n = (size_t)g.M * g.t[ti].w.N;
+        const size_t n = (size_t)g.M * g.t[ti].N;
         for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
             float s = g.t[ti].part[i];
             for (int c = 1; c < g.n_chunks; ++c) s += g.t[ti].part[(size_t)c * n + i];
@@ -898,40 +1092,62 @@ __global__ __launch_bounds__(256) void sum_chunks_kernel(const MfmaArgs g) {
     }
 }
 
+// a workgroup's LDS: raised once per instance to the most any launch asked for
+template <typename Kernel>
+hipError_t allow_lds(Kernel kern, int bytes, int &allowed) {
+    if (bytes <= allowed) return hipSuccess;
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e == hipSuccess) allowed = bytes;
+    return e;
+}
+
+template <int QT, int NI, int W>
+hipError_t launch_dense(const DenseArgs &g, int n_wgs, hipStream_t s) {
+    // K parts of a row group are summed through the waves' regions: a wave's partial tile must fit its region
+    if (g.kw_log2 > 0 && (8 * NI) * 32 * 4 > Cfg<QT>::kRegion) return hipErrorInvalidValue;
+    if (g.M > 8 * NI || g.M * g.chunk_sb > W * 64) return hipErrorInvalidValue;   // staged rows; records, one a thread
+    if (dry_run()) {
+        if (g.n_chunks > 1 && !g.add_out) plan_note_cut();
+        plan_note("gemv_mfma_kernel<%s, %d staged rows, %d waves, dense>: %d workgroups, K in %d chunk(s) of %d super-blocks x %d parts a row group of %d rows%s",
+                  plan_type_name(QT), 8 * NI, W, n_wgs, g.n_chunks, g.chunk_sb, 1 << g.kw_log2, g.rpg,
+                  g.n_chunks == 1 ? "" : g.add_out ? ", the two chunks add themselves to cleared rows" : " + sum_chunks_kernel");
+        return hipSuccess;
+    }
+    const Layout L = layout<QT, 8 * NI, W>(g.chunk_sb);
+    static int allowed = 0;
+    hipError_t e = allow_lds(gemv_mfma_dense_kernel<QT, NI, W>, L.total, allowed);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((gemv_mfma_dense_kernel<QT, NI, W>), dim3((unsigned)n_wgs), dim3(W * 64), (size_t)L.total, s, g);
+    e = hipGetLastError();
+    if (e != hipSuccess || g.n_chunks == 1 || g.add_out) return e;
+    size_t n_out = 0;
+    for (int i = 0; i < g.n_targets; ++i) n_out = std::max(n_out, (size_t)g.M * (size_t)g.t[i].N);
+    const unsigned blocks = (unsigned)std::min<size_t>(256, (n_out + 255) / 256);
+    hipLaunchKernelGGL(sum_chunks_kernel, dim3(blocks), dim3(256), 0, s, g);
+    return hipGetLastError();
+}
+
 template <int QT, int NI, int W, int MODE, bool FLAT = false>
 hipError_t launch_one(const MfmaArgs &g, hipStream_t s) {
     // (the 16-row instances of the larger formats would spill registers in the flat form: they keep the loop per row group)
-    if constexpr (MODE != kDense && !FLAT && (QT == kTypeQ4_K || NI == 1)) {
+    if constexpr (!FLAT && (QT == kTypeQ4_K || NI == 1)) {
         static const bool no_flat = tuning_int("QPROJ_MOE_NO_FLAT", 0) != 0;
         if (g.kw == 1 && !no_flat) return launch_one<QT, NI, W, MODE, true>(g, s);
     }
     // K parts of a row group are summed through the waves' regions: a wave's partial tile must fit its region
     if (g.kw > 1 && (MODE == kGroupedSwiglu ? 2 : 1) * (8 * NI) * 32 * 4 > Cfg<QT>::kRegion) return hipErrorInvalidValue;
     if (dry_run()) {
-        if (g.n_chunks > 1 && !g.add_out) plan_note_cut();
+        if (g.n_chunks > 1) plan_note_cut();
         plan_note("gemv_mfma_kernel<%s, %d staged rows, %d waves, %s%s>: %d workgroups, K in %d chunk(s) of %d super-blocks x %d parts a row group of %d rows%s",
-                  plan_type_name(QT), 8 * NI, W, MODE == kDense ? "dense" : MODE == kGroupedSwiglu ? "expert-grouped + swiglu" : "expert-grouped",
-                  FLAT ? ", one item stream a wave" : "", g.n_wgs, g.n_chunks, g.chunk_sb, g.kw, MODE == kDense ? g.rpg : 32,
-                  g.n_chunks == 1 ? "" : g.add_out ? ", the two chunks add themselves to cleared rows"
-                                   : MODE == kDense ? " + sum_chunks_kernel" : " + sum_parts_kernel");
+                  plan_type_name(QT), 8 * NI, W, MODE == kGroupedSwiglu ? "expert-grouped + swiglu" : "expert-grouped",
+                  FLAT ? ", one item stream a wave" : "", g.n_wgs, g.n_chunks, g.chunk_sb, g.kw, 32, g.n_chunks == 1 ? "" : " + sum_parts_kernel");
         return hipSuccess;
     }
     const Layout L = layout<QT, 8 * NI, W>(g.chunk_sb);
-    auto kern = gemv_mfma_kernel<QT, NI, W, MODE, FLAT>;
     static int allowed = 0;
-    if (L.total > allowed) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, L.total);
-        if (e != hipSuccess) return e;
-        allowed = L.total;
-    }
-    hipLaunchKernelGGL(kern, dim3((unsigned)g.n_wgs), dim3(W * 64), (size_t)L.total, s, g);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || g.n_chunks == 1 || g.add_out || MODE != kDense) return e;
-    size_t n_out = 0;
-    for (int i = 0; i < g.n_targets; ++i) n_out = std::max(n_out, (size_t)g.M * (size_t)g.t[i].w.N);
-    const unsigned blocks = (unsigned)std::min<size_t>(256, (n_out + 255) / 256);
-    hipLaunchKernelGGL(sum_chunks_kernel, dim3(blocks), dim3(256), 0, s, g);
+    const hipError_t e = allow_lds(gemv_mfma_kernel<QT, NI, W, MODE, FLAT>, L.total, allowed);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((gemv_mfma_kernel<QT, NI, W, MODE, FLAT>), dim3((unsigned)g.n_wgs), dim3(W * 64), (size_t)L.total, s, g);
     return hipGetLastError();
 }
 
@@ -984,22 +1200,21 @@ hipError_t launch_w(const MfmaArgs &g, int W, hipStream_t s) {
     return launch_one<QT, NI, 8, MODE>(g, s);
 }
 
-// ni: activation rows a pass in eights -- 1, 2, or (dense launches of eight waves only) 4: all 32 token rows of the
-// matrix instruction carry a row of their own, at the same number of matrix instructions
+template <int QT>
+hipError_t launch_dense_typed(const DenseArgs &g, int n_wgs, int W, hipStream_t s) {
+    // activation rows a pass in eights; 4 (eight waves only): all 32 token rows of the matrix instruction carry a row of
+    // their own, at the same number of matrix instructions
+    if (g.M > 16) return W == 8 ? launch_dense<QT, 4, 8>(g, n_wgs, s) : hipErrorInvalidValue;
+    if constexpr (QT == kTypeQ4_K)
+        if (W == 16) return g.M <= 8 ? launch_dense<QT, 1, 16>(g, n_wgs, s) : launch_dense<QT, 2, 16>(g, n_wgs, s);
+    if (W == 4) return g.M <= 8 ? launch_dense<QT, 1, 4>(g, n_wgs, s) : launch_dense<QT, 2, 4>(g, n_wgs, s);
+    return g.M <= 8 ? launch_dense<QT, 1, 8>(g, n_wgs, s) : launch_dense<QT, 2, 8>(g, n_wgs, s);
+}
+
+// ni: activation rows a pass in eights -- 1, 2, or (Q4_K experts with K of at most eight super-blocks, eight waves) 4
 template <int MODE>
 hipError_t launch_typed(const MfmaArgs &g, int type, int ni, int W, hipStream_t s) {
-    if (ni == 4) {
-        if constexpr (MODE == kDense) {
-            if (W != 8) return hipErrorInvalidValue;
-            if (type == kTypeQ4_K) return launch_one<kTypeQ4_K, 4, 8, kDense>(g, s);
-            if (type == kTypeQ6_K) return launch_one<kTypeQ6_K, 4, 8, kDense>(g, s);
-            return launch_one<kTypeQ8_0, 4, 8, kDense>(g, s);
-        } else {
-            // expert-grouped: Q4_K experts with K of at most eight super-blocks (the staged rows of 32 pairs)
-            if (W != 8 || type != kTypeQ4_K) return hipErrorInvalidValue;
-            return launch_one<kTypeQ4_K, 4, 8, MODE>(g, s);
-        }
-    }
+    if (ni == 4) return W == 8 && type == kTypeQ4_K ? launch_one<kTypeQ4_K, 4, 8, MODE>(g, s) : hipErrorInvalidValue;
     const bool small = ni == 1;
     if (type == kTypeQ4_K) return small ? launch_w<kTypeQ4_K, 1, MODE>(g, W, s) : launch_w<kTypeQ4_K, 2, MODE>(g, W, s);
     if (type == kTypeQ6_K) return small ? launch_w<kTypeQ6_K, 1, MODE>(g, W, s) : launch_w<kTypeQ6_K, 2, MODE>(g, W, s);
@@ -1049,12 +1264,13 @@ bool mfma_gemv_two_chunks(int type, int64_t K, int64_t M, int64_t total_rg) {
 }
 
 hipError_t launch_gemv_mfma(const GemvArgs &args, const Scratch &scratch, hipStream_t s) {
-    MfmaArgs g{};
+    DenseArgs g{};
     g.n_targets = args.n_targets;
-    g.a = args.a;
-    g.x = args.x;
+    g.qs = args.a.qs;
+    g.d = args.a.d;
+    g.bsums = args.a.bsums;
     g.M = args.M;
-    g.x_div = 1;
+    g.nb = (int)(args.a.K / 256);
     int64_t total_rg = 0;
     for (int i = 0; i < args.n_targets; ++i) total_rg += (args.t[i].w.N + 31) / 32;
     if (args.M < 1 || args.M > 32) return hipErrorInvalidValue;
@@ -1062,9 +1278,8 @@ hipError_t launch_gemv_mfma(const GemvArgs &args, const Scratch &scratch, hipStr
     const Split p = plan(args.a.K, args.M, total_rg, W, 200, true, cu_count());
     g.n_chunks = p.n_chunks;
     g.chunk_sb = p.chunk_sb;
-    g.kw = p.kw;
+    while ((1 << g.kw_log2) < p.kw) ++g.kw_log2;
     g.rw = W / p.kw;
-    g.rg_loop = 1;
     g.add_out = args.y_zeroed && mfma_gemv_two_chunks(args.t[0].w.type, args.a.K, args.M, total_rg);
     // Rows a row group.  The kernel streams weights and the matrix cores idle, so a grid that leaves compute units
     // without a workgroup is evened out with row groups of fewer than the instruction's 32 rows (the spare columns
@@ -1081,20 +1296,35 @@ hipError_t launch_gemv_mfma(const GemvArgs &args, const Scratch &scratch, hipStr
         for (int r = 31; r >= 24 && wgs_with(r) <= cu_count(); --r) g.rpg = r;
     int wg = 0;
     size_t part_off = 0;
+    for (int i = 0; i < kMaxTargets; ++i) g.first_wg[i] = INT_MAX;
     for (int i = 0; i < args.n_targets; ++i) {
-        g.t[i].w = args.t[i].w;
-        g.t[i].y = args.t[i].y;
-        g.t[i].part = scratch.p ? scratch.p + part_off : nullptr;
-        part_off += (size_t)g.n_chunks * args.M * args.t[i].w.N;
-        const int n_rg = (int)((args.t[i].w.N + g.rpg - 1) / g.rpg);
-        g.t[i].n_rowsets = (n_rg + g.rw - 1) / g.rw;
-        g.t[i].first_wg = wg;
-        wg += g.t[i].n_rowsets * g.n_chunks;
+        const WeightView &w = args.t[i].w;
+        DenseTarget &t = g.t[i];
+        if (w.type == kTypeQ4_K) {
+            t.p[0] = w.q4k;
+        } else if (w.type == kTypeQ6_K) {
+            t.p[0] = w.q6_ql;
+            t.p[1] = w.q6_qh;
+            t.p[2] = reinterpret_cast<const uint8_t *>(w.q6_sc);
+            t.p[3] = reinterpret_cast<const uint8_t *>(w.q6_d);
+        } else {
+            t.p[0] = reinterpret_cast<const uint8_t *>(w.q8_qs);
+            t.p[1] = reinterpret_cast<const uint8_t *>(w.q8_d);
+        }
+        t.N = w.N;
+        t.y = args.t[i].y;
+        t.part = scratch.p ? scratch.p + part_off : nullptr;
+        part_off += (size_t)g.n_chunks * args.M * w.N;
+        const int n_rg = (int)((w.N + g.rpg - 1) / g.rpg);
+        g.n_rowsets[i] = (n_rg + g.rw - 1) / g.rw;
+        g.first_wg[i] = wg;
+        wg += g.n_rowsets[i] * g.n_chunks;
     }
-    g.n_wgs = wg;
     // the per-chunk results of all targets lie one behind the other in the scratch: refuse what would not fit
     if (g.n_chunks > 1 && !g.add_out && (!scratch.p || part_off * sizeof(float) > scratch.bytes)) return hipErrorInvalidValue;
-    return launch_typed<kDense>(g, args.t[0].w.type, args.M <= 8 ? 1 : args.M <= 16 ? 2 : 4, W, s);
+    const int type = args.t[0].w.type;
+    if (type == kTypeQ4_K) return launch_dense_typed<kTypeQ4_K>(g, wg, W, s);
+    return type == kTypeQ6_K ? launch_dense_typed<kTypeQ6_K>(g, wg, W, s) : launch_dense_typed<kTypeQ8_0>(g, wg, W, s);
 }
 
 // few pairs an expert: 8 staged rows a pass are enough
@@ -1120,10 +1350,8 @@ bool mfma_grouped_whole_rows(int type, int64_t K, int64_t N, int64_t E, int64_t 
 // as gate and up.  n_pairs only steers the launch shape (how many experts can be busy at once).
 hipError_t launch_gemv_mfma_grouped(const GemvArgs &args, int64_t n_pairs, bool swiglu, hipStream_t s, const Scratch &scratch) {
     MfmaArgs g{};
-    g.n_targets = swiglu ? 2 : 1;
     g.a = args.a;
     g.x = args.x;
-    g.M = 0;
     g.order = args.order;
     g.offsets = args.offsets;
     g.active = args.active;
@@ -1158,7 +1386,7 @@ hipError_t launch_gemv_mfma_grouped(const GemvArgs &args, int64_t n_pairs, bool 
     g.part_plane = n_pairs * w.N;
     g.kw = p.kw;
     g.rw = W / p.kw;
-    for (int i = 0; i < g.n_targets; ++i) {
+    for (int i = 0; i < (swiglu ? 2 : 1); ++i) {
         g.t[i].w = args.t[i].w;
         g.t[i].y = args.t[i].y;
         g.t[i].part = g.n_chunks > 1 ? scratch.p : nullptr;

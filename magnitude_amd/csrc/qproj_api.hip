@@ -471,15 +471,6 @@ size_t dense_scratch_bytes(int n, const qproj_weight *const *w, int64_t M) {
     return need;
 }
 
-// true when mul_mat of M fp32 rows goes to the small-batch kernel with the quantizer fused into its
-// prologue.  Off unless asked for: every one of the ~200 workgroups repeats the quantization of all M
-// rows, which costs more than the separate quantizer launch saves (gate+up, M = 4 / 8 / 16: 22.1 /
-// 26.9 / 38.5 us fused against 20.5 / 20.8 / 22.7 us).
-bool dense_fuses_quantizer(const qproj_weight *w, int64_t M) {
-    static const bool on = tuning_int("QPROJ_FUSED_QUANT_DENSE", 0) != 0;
-    return on && M <= 16 && use_mfma_kernel(w->type, M, w->K);
-}
-
 // The quantizer launch in front of the small-batch kernel clears the output rows where a pass of that kernel cuts K
 // in two chunks: the chunks then add themselves to the output and the launch that summed them goes (8B down
 // projection, 14336 -> 4096 Q6_K, at 4 and 8 rows).  Fills `z` and answers true when that is the case.
@@ -536,10 +527,9 @@ uint32_t tiled_clears_rows(int n, const qproj_weight *const *w, int64_t M, float
     return mask;
 }
 
-// x_f32: non-null when `a` carries no planes and the kernel quantizes these rows itself (small batches only);
 // y_zeroed: the output rows were cleared by the quantizer launch (dense_clears_rows)
 int run_dense_q8act(qproj_ctx *ctx, int n, const qproj_weight *const *w, const ActView &a, int64_t M,
-                    float *const *y, const Scratch &sc, const float *x_f32 = nullptr, bool y_zeroed = false) {
+                    float *const *y, const Scratch &sc, bool y_zeroed = false) {
     // Beyond the rows one pass of the small-batch kernel takes: the tiled product, weights reused across a tile of
     // tokens, K cut into stretches where the grid would leave the chip idle.  (Measured, 8B shapes, 33 rows: Q6_K
     // 14336 -> 4096 50.9 us in two passes of the small-batch kernel against 41 us tiled, Q4_K 4096 -> 14336 42 against 29.)
@@ -584,8 +574,7 @@ int run_dense_q8act(qproj_ctx *ctx, int n, const qproj_weight *const *w, const A
                 g.t[i].w = w[i]->view;
                 g.t[i].y = y[i] + m0 * w[i]->N;
             }
-            g.a = x_f32 ? a : act_rows(a, m0);
-            g.x = x_f32;   // (only with M <= 16: a single pass)
+            g.a = act_rows(a, m0);
             g.M = (int)mc;
             g.x_div = 1;
             g.y_zeroed = y_zeroed;
@@ -987,13 +976,12 @@ struct NormSpec {   // RMS norm (+ weights) applied to the rows before they are 
 }  // namespace
 
 // Can the down projection of a feed-forward block take its rows as silu(gate) * up through the quantizer?  Only the
-// routes that quantize in a launch of their own (not the decode kernel, whose prologue reads fp32 rows, nor the
-// small-batch variant that quantizes inside the projection, nor fp32 activations).
+// routes that quantize in a launch of their own (not the decode kernel, whose prologue reads fp32 rows, nor fp32
+// activations).
 static bool swiglu_quantizer_serves(const qproj_weight *w, int64_t M, int act) {
     if (act != kActGGML && act != kActQ8X32) return false;
     if (act == kActQ8X32) return w->type == kTypeQ4_K && w->K % 256 == 0;
-    if (!use_mfma_kernel(w->type, M, w->K) && use_decode_kernel(w->type, M, w->K)) return false;
-    return !dense_fuses_quantizer(w, M);
+    return use_mfma_kernel(w->type, M, w->K) || !use_decode_kernel(w->type, M, w->K);
 }
 
 // swiglu_u non-null (callers: the quantized routes beyond the decode regime only): the rows multiplied are
@@ -1037,15 +1025,6 @@ static int mul_mat_multi_impl(qproj_ctx *ctx, int n, const qproj_weight *const *
     if (act == kActGGML || act == kActQ8X32) {
         if (act == kActQ8X32 && w[0]->type != kTypeQ4_K)
             return fail(ctx, QPROJ_ERR_UNSUPPORTED, "qproj_mul_mat: the per-32 int8 path is built for Q4_K weights");
-        if (act == kActGGML && !norm && !swiglu_u && dense_fuses_quantizer(w[0], M)) {
-            const size_t extra = dense_scratch_bytes(n, w, M);
-            int rc = reserve(ctx, wsp, extra);
-            if (rc) return rc;
-            ActView a{};
-            a.kind = act_kind_for(act, w[0]->type);
-            a.K = K;
-            return run_dense_q8act(ctx, n, w, a, M, y_dev, Scratch{reinterpret_cast<float *>(wsp.base), extra - std::min(extra, scratch_shave())}, x_dev);
-        }
         const ActPlanes p = act_planes(act_kind_for(act, w[0]->type), M, K);
         const size_t extra = act == kActGGML ? dense_scratch_bytes(n, w, M) : per32_scratch_max(n, w, M);
         int rc = reserve(ctx, wsp, p.total + extra);
@@ -1074,7 +1053,7 @@ static int mul_mat_multi_impl(qproj_ctx *ctx, int n, const qproj_weight *const *
         const ActView a = act_view(p, ws, K);
         // the partial results lie behind the activation planes; `extra` is all a launcher may use of it
         const Scratch sc{extra ? reinterpret_cast<float *>(ws + p.total) : nullptr, extra - std::min(extra, scratch_shave()), tile_adds};
-        if (act == kActGGML) return run_dense_q8act(ctx, n, w, a, M, y_dev, sc, nullptr, y_zeroed);
+        if (act == kActGGML) return run_dense_q8act(ctx, n, w, a, M, y_dev, sc, y_zeroed);
         for (int i = 0; i < n; ++i) QP_HIP(ctx, launch_gemm_q8x32(w[i]->view, a, M, y_dev[i], sc, ctx->stream));
         return QPROJ_OK;
     }

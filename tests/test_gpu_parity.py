@@ -312,6 +312,31 @@ def test_small_batch_row_groups_of_fewer_than_32_rows(ctx, orc, qtype, k, ns):
             w.free()
 
 
+@pytest.mark.parametrize("qtype,k,ns,ms", [
+    (Q4_K, 8192, (70,), (8,)), (Q6_K, 4096, (33, 1), (16,)), (Q8_0, 2048, (40,), (32,)),            # 256 super-blocks staged, the most
+    (Q4_K, 8448, (65,), (6, 16)), (Q6_K, 2304, (50,), (17, 31)), (Q8_0, 8448, (31,), (5,)),          # a last chunk one shorter
+    (Q4_K, 256, (52001,), (5,)), (Q6_K, 512, (26000,), (3, 9)), (Q8_0, 768, (13001,), (7, 12)),      # K in one, two and four parts
+    (Q4_K, 4352, (33, 1, 700, 130), (3, 8)), (Q8_0, 5120, (96, 5, 33, 1), (6, 16))])                 # four matrices, 17 and 20 super-blocks
+def test_small_batch_staging_and_k_parts_at_their_edges(ctx, orc, qtype, k, ns, ms):
+    """The activation rows of a small-batch workgroup at the most it stages, in chunks of K of unequal length and with
+    super-blocks that do not divide over the waves, and the sums of one to eight K parts; rows behind the outputs stay."""
+    from magnitude_amd import ACT_GGML
+    ws, blocks = [], []
+    for i, n in enumerate(ns):
+        blocks.append(make_weight(orc, qtype, n, k, seed=5200 + k + n + i))
+        ws.append(ctx.upload(qtype, k, n, blocks[-1]))
+    for m in ms:
+        x = np.random.default_rng(m + k).standard_normal((m, k)).astype(np.float32)
+        bufs = [torch.full((m * n + 64,), 7.0, dtype=torch.float32, device="cuda") for n in ns]
+        outs = [b[: m * n].view(m, n) for b, n in zip(bufs, ns)]
+        ctx.mul_mat_multi(ws, dev(x), ACT_GGML, outs=outs)
+        for b, o, n, blk in zip(bufs, outs, ns, blocks):
+            close(o.cpu().numpy(), orc.mul_mat(qtype, blk, k, x, orc.ACT_GGML), 2e-5)
+            assert bool((b[m * n:] == 7.0).all())
+    for w in ws:
+        w.free()
+
+
 @pytest.mark.parametrize("qtype,k,n", [(Q4_K, 4096, 512), (Q4_K, 14336, 203), (Q4_K, 256, 9), (Q8_0, 4096, 384),
                                        (Q8_0, 14336, 77), (Q6_K, 4096, 130), (Q6_K, 14336, 256)])
 def test_rows_17_to_32_on_the_small_batch_kernel(ctx, orc, qtype, k, n):
