@@ -9,6 +9,8 @@
 // does a handful of operations per step and the vector unit only the dot products.
 #include "actquant_device.h"
 #include "gemv_frags.h"
+#include <limits.h>
+#include <stddef.h>
 #include <stdio.h>
 
 namespace qproj {
@@ -18,6 +20,44 @@ namespace {
 constexpr int kDecodeThreads = 1024;
 constexpr int kDecodeWaves = kDecodeThreads / 64;
 
+// Arguments of a launch.  A workgroup begins with a chain of trips to memory (arguments, activation row, weights), and
+// arguments come a 64-byte line at a time: what every workgroup needs first are the kernel's leading parameters, what it
+// needs of its matrix stands by field, so that Q4_K touches three lines and asks for them at once.  Before, 616 bytes loaded
+// where they were used, us a launch: 4096 -> 4096 / 1024 / 1024 and 4096 x 4096 Q4_K 6.3 -> 5.7, Q6_K 14336 -> 4096 12.0 -> 11.5, Q8_0
+// 2048 x 2048 4.1 -> 3.9.  (All ten lines asked for at once: 4 % slower than before.  The leading parameters preloaded into
+// scalar registers by the dispatcher: level.)
+struct DecodeArgs {
+    int first_wave[kMaxTargets];       // of each matrix, counted over the launch; INT_MAX where there is none
+    int rows_per_pair[kMaxTargets];    // consecutive rows each pair of neighbouring waves walks
+    int64_t N[kMaxTargets];
+    float *y[kMaxTargets];
+    const uint8_t *p0[kMaxTargets];    // Q4_K: blocks; Q6_K: ql, qh, scales, d; Q8_0: quants, d
+    const uint8_t *p1[kMaxTargets], *p2[kMaxTargets], *p3[kMaxTargets];
+    const int8_t *qs;                  // rows quantized earlier
+    const float *d;
+    const int16_t *bsums;
+};
+
+template <int QT>
+__device__ __forceinline__ WeightView weight_view(const DecodeArgs &args, int i, int64_t K, int nb) {
+    WeightView w{};
+    w.K = K;
+    w.nb = nb;
+    w.N = args.N[i];
+    if constexpr (QT == kTypeQ4_K) {
+        w.q4k = args.p0[i];
+    } else if constexpr (QT == kTypeQ6_K) {
+        w.q6_ql = args.p0[i];
+        w.q6_qh = args.p1[i];
+        w.q6_sc = reinterpret_cast<const int8_t *>(args.p2[i]);
+        w.q6_d = reinterpret_cast<const uint16_t *>(args.p3[i]);
+    } else {
+        w.q8_qs = reinterpret_cast<const int8_t *>(args.p0[i]);
+        w.q8_d = reinterpret_cast<const uint16_t *>(args.p1[i]);
+    }
+    return w;
+}
+
 // activations into LDS: FUSE quantizes fp32 rows here; otherwise planes quantized earlier are copied
 // 256-wide pieces of an activation row that a wave fetches ahead of its first weights: four a row for one or two
 // rows (K up to 16384 is covered; pieces fetched inside the quantizing loop instead come one after the other, a trip to
@@ -26,7 +66,7 @@ constexpr int kDecodeWaves = kDecodeThreads / 64;
 __host__ __device__ constexpr int prefetched_pieces(int mt) { return mt <= 2 ? 4 : 1; }
 
 template <int QT, int MT, bool FUSE>
-__device__ __forceinline__ void stage_activations(uint8_t *smem, const GemvArgs &args, int64_t K, int kpad,
+__device__ __forceinline__ void stage_activations(uint8_t *smem, const DecodeArgs &args, const float *rows, int M, int64_t K, int kpad,
                                                   const float4 *first = nullptr) {
     constexpr int BLK = Geo<QT>::kBlk;
     int8_t *sq = reinterpret_cast<int8_t *>(smem);
@@ -34,9 +74,9 @@ __device__ __forceinline__ void stage_activations(uint8_t *smem, const GemvArgs 
     int16_t *sb = reinterpret_cast<int16_t *>(smem + MT * kpad + MT * (kpad / BLK) * 4);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     for (int m = 0; m < MT; ++m) {
-        const bool have = m < args.M;
+        const bool have = m < M;
         if (FUSE) {
-            const float *x = args.x + (int64_t)m * K;
+            const float *x = rows + (int64_t)m * K;
             const int n_chunks = (int)((K + 255) / 256);
             for (int ch = wave; ch < n_chunks; ch += kDecodeWaves) {
                 const int e0 = ch * 256 + 4 * lane;
@@ -63,7 +103,7 @@ __device__ __forceinline__ void stage_activations(uint8_t *smem, const GemvArgs 
                 }
             }
         } else {
-            const ActView &a = args.a;
+            const DecodeArgs &a = args;
             for (int i = tid; i < K / 16; i += kDecodeThreads) {
                 uint4 v = make_uint4(0, 0, 0, 0);
                 if (have) v = *reinterpret_cast<const uint4 *>(a.qs + (int64_t)m * K + i * 16);
@@ -158,31 +198,56 @@ __device__ __forceinline__ void consume(const Raw<QT> (&raw)[R], float (&acc)[MT
 }
 
 template <int QT, int MT, int R, bool XREG, bool FUSE, bool PAIR = false>
-__global__ __launch_bounds__(kDecodeThreads) void gemv_decode_kernel(const GemvArgs args, int kpad) {
+__global__ __launch_bounds__(kDecodeThreads) void gemv_decode_kernel(const float *x, const float *norm_gamma, int K32, int nb, int kpad, int M,
+                                                                     float norm_eps, int norm, const DecodeArgs args) {
     static_assert(!PAIR || R == 2, "the gate/up pairing walks two rows a step");
     extern __shared__ __align__(16) uint8_t smem[];
+    constexpr int kPointers = QT == kTypeQ4_K ? 1 : is_q8_0<QT> ? 2 : 4;
+    fetch_arguments<40 + offsetof(DecodeArgs, p0) + kPointers * sizeof(DecodeArgs::p0)>();
     constexpr int CH = Geo<QT>::kChunk;
     constexpr int BLK = Geo<QT>::kBlk;
     const int lane = threadIdx.x & 63;
     const int wave = uniform(threadIdx.x >> 6);
     const int gw = blockIdx.x * kDecodeWaves + wave;  // global wave index
-    const int64_t K = args.t[0].w.K;
-    const int nb = (int)args.t[0].w.nb;
+    const int64_t K = K32;
     const int nch = XREG ? 1 : kpad / CH;
 
-    // this wave's target and run of rows (selected once; everything below is wave-uniform)
-    WeightView w = args.t[0].w;
-    float *y = args.t[0].y;
-    int wave_first = 0, rpp = args.t[0].rows_per_pair;
+    // The wave's piece of the activation row is requested BEFORE the first weights: loads return in order, and
+    // behind a step of weights coming from HBM the quantizing prologue would wait two microseconds for sixteen
+    // bytes that sit in L2 (phase clocks: staging 3000-4400 cycles of a workgroup's 25000).
+    float4 x_first[MT * prefetched_pieces(MT)];
+    if (FUSE) {
+        constexpr int kPer = prefetched_pieces(MT);
 #pragma unroll
-    for (int i = 1; i < kMaxTargets; ++i) {
-        if (!PAIR && i < args.n_targets && gw >= args.t[i].first_block) {
-            w = args.t[i].w;
-            y = args.t[i].y;
-            wave_first = args.t[i].first_block;
-            rpp = args.t[i].rows_per_pair;
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) {
+                const int e0 = (wave + kDecodeWaves * i) * 256 + 4 * lane;
+                x_first[m * kPer + i] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (m < M && e0 < K) x_first[m * kPer + i] = *reinterpret_cast<const float4 *>(x + (int64_t)m * K + e0);
+            }
+    }
+    // RMS norm fused in front of the quantizer (the launcher only asks for it when the prefetched pieces are the
+    // whole row): weights of the norm fetched with the row, sum of squares over the workgroup in the order of
+    // the standalone kernel, then the pieces are replaced by (x * scale) * gamma.
+    float4 g_first[prefetched_pieces(MT)];
+    if (FUSE && norm) {
+#pragma unroll
+        for (int i = 0; i < prefetched_pieces(MT); ++i) {
+            const int e0 = (wave + kDecodeWaves * i) * 256 + 4 * lane;
+            g_first[i] = make_float4(1.f, 1.f, 1.f, 1.f);
+            if (norm_gamma && e0 < K) g_first[i] = *reinterpret_cast<const float4 *>(norm_gamma + e0);
         }
     }
+
+    // this wave's target and run of rows (selected once; everything below is wave-uniform)
+    int ti = 0;
+#pragma unroll
+    for (int i = 1; i < kMaxTargets; ++i)
+        if (!PAIR && gw >= args.first_wave[i]) ti = i;
+    const WeightView w = weight_view<QT>(args, ti, K, nb);
+    float *const y = args.y[ti];
+    const int wave_first = args.first_wave[ti], rpp = args.rows_per_pair[ti];
     const int64_t N = w.N;
     // Rows are dealt to pairs of neighbouring waves: rpp consecutive rows a pair, the even wave taking the larger
     // part.  A target with 1.5 rows per wave then keeps every wave busy (2 + 1) where whole rows per wave would
@@ -202,42 +267,15 @@ __global__ __launch_bounds__(kDecodeThreads) void gemv_decode_kernel(const GemvA
     const int last_row = n_rows > 0 ? n_rows - 1 : 0;
     RowPtr<QT> rp, rp_up;
     rp.set(w, row_begin < N ? row_begin : 0);
-    rp_up.set(PAIR ? args.t[1].w : w, row_begin < N ? row_begin : 0);
+    rp_up.set(PAIR ? weight_view<QT>(args, 1, K, nb) : w, row_begin < N ? row_begin : 0);
     auto issue_rows = [&](Raw<QT> (&raw)[R], int g, int c) {
         if constexpr (PAIR) issue_pair<QT>(raw, rp, rp_up, g, c, last_row, nb, lane);
         else issue<QT, R>(raw, rp, g, c, last_row, nb, lane);
     };
 
-    // The wave's piece of the activation row is requested BEFORE the first weights: loads return in order, and
-    // behind a step of weights coming from HBM the quantizing prologue would wait two microseconds for sixteen
-    // bytes that sit in L2 (phase clocks: staging 3000-4400 cycles of a workgroup's 25000).
-    float4 x_first[MT * prefetched_pieces(MT)];
-    if (FUSE) {
-        constexpr int kPer = prefetched_pieces(MT);
-#pragma unroll
-        for (int m = 0; m < MT; ++m)
-#pragma unroll
-            for (int i = 0; i < kPer; ++i) {
-                const int e0 = (wave + kDecodeWaves * i) * 256 + 4 * lane;
-                x_first[m * kPer + i] = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (m < args.M && e0 < K) x_first[m * kPer + i] = *reinterpret_cast<const float4 *>(args.x + (int64_t)m * K + e0);
-            }
-    }
-    // RMS norm fused in front of the quantizer (the launcher only asks for it when the prefetched pieces are the
-    // whole row): weights of the norm fetched with the row, sum of squares over the workgroup in the order of
-    // the standalone kernel, then the pieces are replaced by (x * scale) * gamma.
-    float4 g_first[prefetched_pieces(MT)];
-    if (FUSE && args.norm) {
-#pragma unroll
-        for (int i = 0; i < prefetched_pieces(MT); ++i) {
-            const int e0 = (wave + kDecodeWaves * i) * 256 + 4 * lane;
-            g_first[i] = make_float4(1.f, 1.f, 1.f, 1.f);
-            if (args.norm_gamma && e0 < K) g_first[i] = *reinterpret_cast<const float4 *>(args.norm_gamma + e0);
-        }
-    }
     Raw<QT> buf_a[R], buf_b[R];
     issue_rows(buf_a, 0, 0);  // in flight while the activations are staged
-    if (FUSE && args.norm) {
+    if (FUSE && norm) {
         __shared__ double norm_partial[kDecodeWaves];
         constexpr int kPer = prefetched_pieces(MT);
 #pragma unroll
@@ -248,19 +286,19 @@ __global__ __launch_bounds__(kDecodeThreads) void gemv_decode_kernel(const GemvA
             if (m > 0) __syncthreads();   // the partial sums of the previous row have been read
             const double total = workgroup_sum16(sq, norm_partial);
             const float mean = (float)(total / (double)K);
-            const float scale = 1.0f / sqrtf(mean + args.norm_eps);
+            const float scale = 1.0f / sqrtf(mean + norm_eps);
 #pragma unroll
             for (int i = 0; i < kPer; ++i) {
                 float4 &v = x_first[m * kPer + i];
                 v.x *= scale; v.y *= scale; v.z *= scale; v.w *= scale;
-                if (args.norm_gamma) {
+                if (norm_gamma) {
                     v.x *= g_first[i].x; v.y *= g_first[i].y; v.z *= g_first[i].z; v.w *= g_first[i].w;
                 }
             }
         }
     }
 
-    stage_activations<QT, MT, FUSE>(smem, args, K, kpad, FUSE ? x_first : nullptr);
+    stage_activations<QT, MT, FUSE>(smem, args, x, M, K, kpad, FUSE ? x_first : nullptr);
     __syncthreads();
 
     XTile xt;
@@ -293,18 +331,18 @@ __global__ __launch_bounds__(kDecodeThreads) void gemv_decode_kernel(const GemvA
         for (; g + 2 < n_groups; g += 2) {
             issue_rows(buf_b, g + 1, 0);
             __builtin_amdgcn_sched_barrier(0);
-            consume<QT, MT, R, XREG, PAIR>(buf_a, acc, xr, xt, g, 0, 1, nb, n_rows, row_begin, N, y, args.M, lane);
+            consume<QT, MT, R, XREG, PAIR>(buf_a, acc, xr, xt, g, 0, 1, nb, n_rows, row_begin, N, y, M, lane);
             issue_rows(buf_a, g + 2, 0);
             __builtin_amdgcn_sched_barrier(0);
-            consume<QT, MT, R, XREG, PAIR>(buf_b, acc, xr, xt, g + 1, 0, 1, nb, n_rows, row_begin, N, y, args.M, lane);
+            consume<QT, MT, R, XREG, PAIR>(buf_b, acc, xr, xt, g + 1, 0, 1, nb, n_rows, row_begin, N, y, M, lane);
         }
         if (g + 1 < n_groups) {
             issue_rows(buf_b, g + 1, 0);
             __builtin_amdgcn_sched_barrier(0);
-            consume<QT, MT, R, XREG, PAIR>(buf_a, acc, xr, xt, g, 0, 1, nb, n_rows, row_begin, N, y, args.M, lane);
-            consume<QT, MT, R, XREG, PAIR>(buf_b, acc, xr, xt, g + 1, 0, 1, nb, n_rows, row_begin, N, y, args.M, lane);
+            consume<QT, MT, R, XREG, PAIR>(buf_a, acc, xr, xt, g, 0, 1, nb, n_rows, row_begin, N, y, M, lane);
+            consume<QT, MT, R, XREG, PAIR>(buf_b, acc, xr, xt, g + 1, 0, 1, nb, n_rows, row_begin, N, y, M, lane);
         } else if (g < n_groups) {
-            consume<QT, MT, R, XREG, PAIR>(buf_a, acc, xr, xt, g, 0, 1, nb, n_rows, row_begin, N, y, args.M, lane);
+            consume<QT, MT, R, XREG, PAIR>(buf_a, acc, xr, xt, g, 0, 1, nb, n_rows, row_begin, N, y, M, lane);
         }
         return;
     }
@@ -312,10 +350,10 @@ __global__ __launch_bounds__(kDecodeThreads) void gemv_decode_kernel(const GemvA
         for (int g = 0; g < n_groups; g += 2) {
             issue_rows(buf_b, g + 1 < n_groups ? g + 1 : n_groups - 1, 0);
             __builtin_amdgcn_sched_barrier(0);
-            consume<QT, MT, R, XREG, PAIR>(buf_a, acc, xr, xt, g, 0, 1, nb, n_rows, row_begin, N, y, args.M, lane);
+            consume<QT, MT, R, XREG, PAIR>(buf_a, acc, xr, xt, g, 0, 1, nb, n_rows, row_begin, N, y, M, lane);
             issue_rows(buf_a, g + 2 < n_groups ? g + 2 : n_groups - 1, 0);
             __builtin_amdgcn_sched_barrier(0);
-            if (g + 1 < n_groups) consume<QT, MT, R, XREG, PAIR>(buf_b, acc, xr, xt, g + 1, 0, 1, nb, n_rows, row_begin, N, y, args.M, lane);
+            if (g + 1 < n_groups) consume<QT, MT, R, XREG, PAIR>(buf_b, acc, xr, xt, g + 1, 0, 1, nb, n_rows, row_begin, N, y, M, lane);
         }
         return;
     }
@@ -331,13 +369,13 @@ __global__ __launch_bounds__(kDecodeThreads) void gemv_decode_kernel(const GemvA
         if (issued + 1 < n_iter) { advance(ig, ic); ++issued; }
         issue_rows(buf_b, uniform(ig), uniform(ic));
         __builtin_amdgcn_sched_barrier(0);  // keep the loads ahead of the arithmetic that follows
-        consume<QT, MT, R, XREG, PAIR>(buf_a, acc, xr, xt, uniform(cg), uniform(cc), nch, nb, n_rows, row_begin, N, y, args.M, lane);
+        consume<QT, MT, R, XREG, PAIR>(buf_a, acc, xr, xt, uniform(cg), uniform(cc), nch, nb, n_rows, row_begin, N, y, M, lane);
         advance(cg, cc);
         if (issued + 1 < n_iter) { advance(ig, ic); ++issued; }
         issue_rows(buf_a, uniform(ig), uniform(ic));
         __builtin_amdgcn_sched_barrier(0);
         if (it + 1 < n_iter) {
-            consume<QT, MT, R, XREG, PAIR>(buf_b, acc, xr, xt, uniform(cg), uniform(cc), nch, nb, n_rows, row_begin, N, y, args.M, lane);
+            consume<QT, MT, R, XREG, PAIR>(buf_b, acc, xr, xt, uniform(cg), uniform(cc), nch, nb, n_rows, row_begin, N, y, M, lane);
             advance(cg, cc);
         }
     }
@@ -348,13 +386,10 @@ template <int QT, int MT, int R, bool XREG, bool FUSE, bool PAIR = false>
 hipError_t launch_decode(const GemvArgs &args, hipStream_t s) {
     constexpr int CH = Geo<QT>::kChunk;
     constexpr int BLK = Geo<QT>::kBlk;
-    GemvArgs a = args;
-    if (PAIR) {   // gate and up are walked together: the waves are dealt over the rows of one of them
-        if (a.n_targets != 2 || a.t[0].w.N != a.t[1].w.N || a.t[0].w.K != a.t[1].w.K) return hipErrorInvalidValue;
-        a.n_targets = 1;
-    }
+    const int n_targets = PAIR ? 1 : args.n_targets;   // gate and up are walked together: the waves are dealt over the rows of one of them
+    if (PAIR && (args.n_targets != 2 || args.t[0].w.N != args.t[1].w.N || args.t[0].w.K != args.t[1].w.K)) return hipErrorInvalidValue;
     int64_t rows_total = 0;
-    for (int i = 0; i < a.n_targets; ++i) rows_total += a.t[i].w.N;
+    for (int i = 0; i < n_targets; ++i) rows_total += args.t[i].w.N;
     if (rows_total == 0) return hipSuccess;
     // one workgroup per CU, fewer when there are not enough rows to give every wave one
     static const int wgs_per_cu = tuning_int("QPROJ_DECODE_WGS_PER_CU", 1);
@@ -362,28 +397,48 @@ hipError_t launch_decode(const GemvArgs &args, hipStream_t s) {
     const int64_t need = (rows_total + kDecodeWaves - 1) / kDecodeWaves;  // at least one row per wave
     if (grid > need) grid = need;
     const int n_waves = (int)grid * kDecodeWaves;
+    DecodeArgs a{};
+    for (int i = 0; i < kMaxTargets; ++i) a.first_wave[i] = INT_MAX;
+    for (int i = 0; i < args.n_targets; ++i) {
+        const WeightView &w = args.t[i].w;
+        a.N[i] = w.N;
+        a.y[i] = args.t[i].y;
+        if (QT == kTypeQ4_K) {
+            a.p0[i] = w.q4k;
+        } else if (QT == kTypeQ6_K) {
+            a.p0[i] = w.q6_ql;
+            a.p1[i] = w.q6_qh;
+            a.p2[i] = reinterpret_cast<const uint8_t *>(w.q6_sc);
+            a.p3[i] = reinterpret_cast<const uint8_t *>(w.q6_d);
+        } else {
+            a.p0[i] = reinterpret_cast<const uint8_t *>(w.q8_qs);
+            a.p1[i] = reinterpret_cast<const uint8_t *>(w.q8_d);
+        }
+    }
+    a.qs = args.a.qs;
+    a.d = args.a.d;
+    a.bsums = args.a.bsums;
     // waves are dealt to the targets in proportion to their rows; a wave never straddles targets
     int given = 0;
-    for (int i = 0; i < a.n_targets; ++i) {
-        const int left_after = a.n_targets - 1 - i;  // every later target gets at least one wave
-        int share = (int)((a.t[i].w.N * n_waves + rows_total - 1) / rows_total);
+    for (int i = 0; i < n_targets; ++i) {
+        const int left_after = n_targets - 1 - i;  // every later target gets at least one wave
+        int share = (int)((a.N[i] * n_waves + rows_total - 1) / rows_total);
         if (share < 1) share = 1;
-        if (i == a.n_targets - 1 || given + share > n_waves - left_after) share = n_waves - left_after - given;
+        if (i == n_targets - 1 || given + share > n_waves - left_after) share = n_waves - left_after - given;
         if (share < 1) return hipErrorInvalidValue;
-        a.t[i].first_block = given;
-        const int rpp = (int)((2 * a.t[i].w.N + share - 1) / share);  // rows per pair of waves
-        a.t[i].rows_per_pair = rpp;
-        if ((int64_t)rpp * (int64_t)a.t[i].w.nb * 256 >= ((int64_t)1 << 31)) return hipErrorInvalidValue;  // 32-bit row offsets
+        a.first_wave[i] = given;
+        const int rpp = (int)((2 * a.N[i] + share - 1) / share);  // rows per pair of waves
+        a.rows_per_pair[i] = rpp;
+        if ((int64_t)rpp * (int64_t)args.t[i].w.nb * 256 >= ((int64_t)1 << 31)) return hipErrorInvalidValue;  // 32-bit row offsets
         given += share;
     }
-    const int64_t K = a.t[0].w.K;
+    const int64_t K = args.t[0].w.K;
     const int kpad = (int)((K + CH - 1) / CH * CH);
     const size_t smem = (size_t)MT * kpad + (size_t)MT * (kpad / BLK) * 4 + (!is_q8_0<QT> ? (size_t)MT * (kpad / 16) * 2 : 0);
-    if (PAIR) a.n_targets = 2;
     if (dry_run()) {
         char rows[96] = "";
-        for (int i = 0, o = 0; i < (PAIR ? 1 : a.n_targets) && o < 80; ++i)
-            o += snprintf(rows + o, sizeof rows - o, "%s%lld rows/%d a wave pair", i ? ", " : "", (long long)a.t[i].w.N, a.t[i].rows_per_pair);
+        for (int i = 0, o = 0; i < n_targets && o < 80; ++i)
+            o += snprintf(rows + o, sizeof rows - o, "%s%lld rows/%d a wave pair", i ? ", " : "", (long long)a.N[i], a.rows_per_pair[i]);
         plan_note("gemv_decode_kernel<%s, %d activation rows, %d weight rows a step, activations in %s, %s%s>: grid %lld x %d, %s, LDS %zu B",
                   plan_type_name(QT), MT, R, XREG ? "registers" : "LDS", FUSE ? "quantizer in the prologue" : "rows quantized earlier",
                   PAIR ? ", gate/up paired + swiglu" : "", (long long)grid, kDecodeThreads, rows, smem);
@@ -399,7 +454,8 @@ hipError_t launch_decode(const GemvArgs &args, hipStream_t s) {
             allowed = smem;
         }
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kDecodeThreads), smem, s, a, kpad);
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kDecodeThreads), smem, s, args.x, args.norm_gamma, (int)K, (int)args.t[0].w.nb, kpad, args.M,
+                       args.norm_eps, (int)args.norm, a);
     return hipGetLastError();
 }
 

@@ -56,8 +56,7 @@ constexpr int kActKindQ8X32 = 2;
 struct GemvTarget {
     WeightView w;
     float *y;              // [rows][N]
-    int first_block;       // first blockIdx.x (tiled kernels) or first wave (decode kernel) of the target
-    int rows_per_pair;     // decode kernel: consecutive rows each pair of neighbouring waves of the target walks
+    int first_block;       // first blockIdx.x of the target (fp32 and dot-product kernels)
 };
 constexpr int kMaxTargets = 4;
 
