@@ -220,9 +220,32 @@ __device__ __forceinline__ void row_minterm_finish(const float *ld, const int *l
 __device__ __forceinline__ double sum4_sq(const float4 &v) {
     return (double)(v.x * v.x) + (double)(v.y * v.y) + (double)(v.z * v.z) + (double)(v.w * v.w);
 }
+// The sum of the 64 lanes as a butterfly over lane xor 32, 16, 8, 4, 2, 1 (that tree's bits), in the vector unit: after the
+// first three levels the lanes repeat every eight, so that the last three are rotations of a row.  Six trips through the LDS
+// crossbar for the two halves of a double were 0.4 us of every launch that normalises rows.
+template <int CTRL>
+__device__ __forceinline__ double add_dpp(double s) {
+    const long long v = __double_as_longlong(s);
+    const uint32_t lo = (uint32_t)dpp_move_i<CTRL>((int)v), hi = (uint32_t)dpp_move_i<CTRL>((int)(v >> 32));
+    return s + __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+__device__ __forceinline__ double wave_sum(double s) {
+    uint32_t l0, l1, h0, h1;
+    uint64_t v = (uint64_t)__double_as_longlong(s);
+    swap32((uint32_t)v, l0, l1);
+    swap32((uint32_t)(v >> 32), h0, h1);
+    s = __longlong_as_double((long long)(((uint64_t)h0 << 32) | l0)) + __longlong_as_double((long long)(((uint64_t)h1 << 32) | l1));
+    v = (uint64_t)__double_as_longlong(s);
+    swap16((uint32_t)v, l0, l1);
+    swap16((uint32_t)(v >> 32), h0, h1);
+    s = __longlong_as_double((long long)(((uint64_t)h0 << 32) | l0)) + __longlong_as_double((long long)(((uint64_t)h1 << 32) | l1));
+    s = add_dpp<0x128>(s);    // row_ror:8 is lane xor 8
+    s = add_dpp<0x124>(s);    // row_ror:4
+    s = add_dpp<0x4E>(s);     // quad_perm [2,3,0,1]
+    return add_dpp<0xB1>(s);  // quad_perm [1,0,3,2]
+}
 __device__ __forceinline__ double workgroup_sum16(double s, double *partial) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) s += __shfl_xor(s, d);
+    s = wave_sum(s);
     if ((threadIdx.x & 63) == 0) partial[threadIdx.x >> 6] = s;
     __syncthreads();
     double total = 0.0;

@@ -39,6 +39,29 @@ __device__ __forceinline__ float dpp_move(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
 }
 
+// v + its value in lane xor 16 / xor 32: rows of 16 lanes (or halves of the wave) exchanged between two copies in the vector
+// unit, not through the LDS crossbar, whose trip a chain of these would pay each time.
+__device__ __forceinline__ void swap16(uint32_t v, uint32_t &a, uint32_t &b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    a = r[0];
+    b = r[1];
+}
+__device__ __forceinline__ void swap32(uint32_t v, uint32_t &a, uint32_t &b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    a = r[0];
+    b = r[1];
+}
+__device__ __forceinline__ float add_xor16(float v) {
+    uint32_t a, b;
+    swap16(__float_as_uint(v), a, b);
+    return __uint_as_float(a) + __uint_as_float(b);
+}
+__device__ __forceinline__ float add_xor32(float v) {
+    uint32_t a, b;
+    swap32(__float_as_uint(v), a, b);
+    return __uint_as_float(a) + __uint_as_float(b);
+}
+
 // Sum over the 64 lanes of a wave; every lane must be active.  Four DPP steps give each row of
 // 16 lanes its row sum, the four row sums are then read through SGPRs.  All lanes get the total.
 __device__ __forceinline__ float wave_sum(float v) {
@@ -66,9 +89,7 @@ __device__ __forceinline__ float wave_sum4(const float (&v)[4], int lane) {
     float t = (hi2 ? s23 : s01) + dpp_move<0x4E>(hi2 ? s01 : s23);
     t += dpp_move<0x114>(t);  // row_shr:4
     t += dpp_move<0x118>(t);  // row_shr:8  -> lanes 12..15 of each row hold the row's sums
-    t += __shfl_xor(t, 16);
-    t += __shfl_xor(t, 32);
-    return t;
+    return add_xor32(add_xor16(t));
 }
 
 // The 6-bit (scale, min) pairs of a Q4_K super-block, unpacked four at a time from the 12-byte
