@@ -17,6 +17,8 @@
 // The arithmetic is that of the tiled kernels: Q4_K scales in base 8 as two int8 operands, Q6_K products as high and
 // low bytes, both chains inside the matrix cores for a whole super-block, one flush per 256 weights, the Q4_K min
 // term on the fp16 cores from the plane the quantizer wrote.
+#include <limits.h>
+#include <stddef.h>
 #include <stdlib.h>
 
 #include <algorithm>
@@ -35,14 +37,21 @@ struct StreamTarget {
     const uint8_t *p0, *p1, *p2, *p3;   // Q4_K: blocks; Q6_K: ql, qh, scales, d
     float *out;                         // [n_split][M][N] partial tiles, or the output itself when K is whole
     int N, tiles_n, tiles_pad, n_split; // tiles_pad: workgroups of one stretch of K (a multiple of 8)
-    int first_wg;
 };
 
+// By field: arguments come a 64-byte line at a time, a trip to memory each, and Q4_K needs three of these lines; all of them are
+// asked for at once (4096 -> 2 x 14336 at 48 tokens 27.8 -> 26.5 us, 4096 x 4096 12.1 -> 11.4).
 struct StreamArgs {
-    int n;
-    StreamTarget t[kMaxTargets];
-    ActView a;
+    const int8_t *qs;                   // activations
+    const float *d;
+    const uint16_t *msum;
+    const float *rs;
     int M, nb, tiles_m;
+    int first_wg[kMaxTargets];          // of the launch's matrices; INT_MAX where there is none
+    int N[kMaxTargets], tiles_n[kMaxTargets], tiles_pad[kMaxTargets], n_split[kMaxTargets];
+    float *out[kMaxTargets];
+    const uint8_t *p0[kMaxTargets];
+    const uint8_t *p1[kMaxTargets], *p2[kMaxTargets], *p3[kMaxTargets];
 };
 
 template <int QT>
@@ -151,14 +160,17 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_stream_kernel(const StreamArg
     constexpr bool kQ4 = QT == kTypeQ4_K;
     constexpr int RW = NW / KW, TM = 32 * JT, NT = 64 * NW;
     extern __shared__ __align__(16) uint8_t smem[];
+    fetch_arguments<kQ4 ? (int)offsetof(StreamArgs, p1) : (int)sizeof(StreamArgs)>();
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, lh = lane >> 5, rg = wave % RW, kp = wave / RW;
 
-    StreamTarget t = g.t[0];
+    int ti = 0;
 #pragma unroll
     for (int i = 1; i < kMaxTargets; ++i)
-        if (i < g.n && (int)blockIdx.x >= g.t[i].first_wg) t = g.t[i];
-    const int local = (int)blockIdx.x - t.first_wg, split = local / t.tiles_pad, pid = local - split * t.tiles_pad;
+        if ((int)blockIdx.x >= g.first_wg[i]) ti = i;
+    const StreamTarget t = {g.p0[ti], kQ4 ? nullptr : g.p1[ti], kQ4 ? nullptr : g.p2[ti], kQ4 ? nullptr : g.p3[ti],
+                            g.out[ti], g.N[ti], g.tiles_n[ti], g.tiles_pad[ti], g.n_split[ti]};
+    const int local = (int)blockIdx.x - g.first_wg[ti], split = local / t.tiles_pad, pid = local - split * t.tiles_pad;
     if (pid >= t.tiles_n * g.tiles_m) return;   // padding: the whole workgroup leaves
     int tile_n, tile_m;
     tile_of_workgroup(t.tiles_n, g.tiles_m, pid, tile_n, tile_m);
@@ -179,7 +191,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_stream_kernel(const StreamArg
     // activations: request p of a wave = K part p / AP, tokens 4*(wave + NW*(p % AP)) .. +3 of the tile
     constexpr int AP = 8 * JT / NW;
     const int mcap = min(M - 1 - m0, TM - 1);
-    const int8_t *abase = scalar_pointer(g.a.qs + (int64_t)m0 * K);
+    const int8_t *abase = scalar_pointer(g.qs + (int64_t)m0 * K);
     uint32_t aoff[AP];
 #pragma unroll
     for (int j = 0; j < AP; ++j) {
@@ -201,7 +213,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_stream_kernel(const StreamArg
     const uint8_t *msbase = nullptr;
     if constexpr (kQ4) {
         static_assert(KW * JT <= NW, "a wave requests one tile of the min-term plane at most");
-        msbase = scalar_pointer(reinterpret_cast<const uint8_t *>(g.a.msum) + (int64_t)m0 * nb * 32);
+        msbase = scalar_pointer(reinterpret_cast<const uint8_t *>(g.msum) + (int64_t)m0 * nb * 32);
     }
     // (three token tiles: worked out at every request from the lane counter.  Kept in a register it was spilled, and the wait
     // for its reload was one for everything outstanding; 4096 -> 40960 at 96 rows 66.6 -> 64.6 us)
@@ -221,13 +233,13 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_stream_kernel(const StreamArg
     };
     // Scales go through LDS kScaleSb super-blocks at a time: a plain load in the loop below would make the compiler
     // wait for every outstanding request before its value is used.
-    const global_ptr<float> dxbase = scalar_global(g.a.d + (int64_t)m0 * nb);
+    const global_ptr<float> dxbase = scalar_global(g.d + (int64_t)m0 * nb);
     float *const dx_lds = reinterpret_cast<float *>(smem + L::kOffDx);
     uint16_t *const dw_lds = reinterpret_cast<uint16_t *>(smem + L::kOffDw + wave * L::kDwWave);
     float rs_mine = 1.f;   // of token tid % TM
     float inv_rs = 1.f;
     if constexpr (kQ4) {   // the min-term operand is normalised by the row: see gemm_q4k_q8k_direct_kernel
-        rs_mine = g.a.rs[m0 + min(tid % TM, mcap)];
+        rs_mine = g.rs[m0 + min(tid % TM, mcap)];
         inv_rs = 1.0f / rs_mine;
     }
     auto load_scales = [&](int sb0) {
@@ -724,7 +736,12 @@ hipError_t launch_group(int n, const WeightView *w, const StreamPlan *plans, con
         if (done[first]) continue;
         const StreamPlan &p0 = plans[first];
         StreamArgs g{};
-        g.a = a;
+        int count = 0;
+        for (int i = 0; i < kMaxTargets; ++i) g.first_wg[i] = INT_MAX;
+        g.qs = a.qs;
+        g.d = a.d;
+        g.msum = a.msum;
+        g.rs = a.rs;
         g.M = (int)M;
         g.nb = (int)(w[0].K / 256);
         g.tiles_m = (int)((M + 32 * p0.jt - 1) / (32 * p0.jt));
@@ -741,24 +758,24 @@ hipError_t launch_group(int n, const WeightView *w, const StreamPlan *plans, con
         for (int i = first; i < n; ++i) {
             if (plans[i].jt != p0.jt || plans[i].kw != p0.kw) continue;
             done[i] = true;
-            StreamTarget &t = g.t[g.n++];
-            if (q4) t.p0 = w[i].q4k;
+            const int c = count++;
+            if (q4) g.p0[c] = w[i].q4k;
             else {
-                t.p0 = w[i].q6_ql;
-                t.p1 = w[i].q6_qh;
-                t.p2 = reinterpret_cast<const uint8_t *>(w[i].q6_sc);
-                t.p3 = reinterpret_cast<const uint8_t *>(w[i].q6_d);
+                g.p0[c] = w[i].q6_ql;
+                g.p1[c] = w[i].q6_qh;
+                g.p2[c] = reinterpret_cast<const uint8_t *>(w[i].q6_sc);
+                g.p3[c] = reinterpret_cast<const uint8_t *>(w[i].q6_d);
             }
-            t.N = (int)w[i].N;
-            t.tiles_n = (int)((w[i].N + rows - 1) / rows);
-            t.tiles_pad = (int)tiles_pad(i, rows);
-            t.n_split = plans[i].n_split;
-            t.first_wg = (int)wg;
-            t.out = out[i];
-            wg += (int64_t)t.tiles_pad * t.n_split;
+            g.N[c] = (int)w[i].N;
+            g.tiles_n[c] = (int)((w[i].N + rows - 1) / rows);
+            g.tiles_pad[c] = (int)tiles_pad(i, rows);
+            g.n_split[c] = plans[i].n_split;
+            g.first_wg[c] = (int)wg;
+            g.out[c] = out[i];
+            wg += (int64_t)g.tiles_pad[c] * g.n_split[c];
             plan_note("gemm_stream_kernel<%s, %d token tiles, %d K parts>%s: tile %d tokens x %d rows, %d tiles x %d K stretches%s", plan_type_name(w[0].type),
-                      p0.jt, p0.kw, g.n > 1 ? " (same launch)" : "", 32 * p0.jt, rows, t.tiles_n * g.tiles_m, t.n_split,
-                      t.n_split > 1 ? " + sum_parts_kernel" : "");
+                      p0.jt, p0.kw, count > 1 ? " (same launch)" : "", 32 * p0.jt, rows, g.tiles_n[c] * g.tiles_m, g.n_split[c],
+                      g.n_split[c] > 1 ? " + sum_parts_kernel" : "");
         }
         if (wg >= 0x7fffffff) return hipErrorInvalidValue;
         const LaunchFn run = instance(w[0].type, p0.jt, p0.kw, waves);
