@@ -36,7 +36,16 @@ constexpr int kTypeQ8_0Wide = 1008;
 template <> struct Geo<kTypeQ8_0Wide> {
     static constexpr int kChunk = 4096, kBlk = 32, kLanesPerBlk = 2;
 };
-template <int QT> constexpr bool is_q8_0 = QT == kTypeQ8_0 || QT == kTypeQ8_0Wide;
+// The same with two or three parts, for rows that are not whole steps of four: parts past the end of a row are requested and
+// multiplied for nothing.
+constexpr int kTypeQ8_0Two = 1009, kTypeQ8_0Three = 1010;
+template <> struct Geo<kTypeQ8_0Two> {
+    static constexpr int kChunk = 2048, kBlk = 32, kLanesPerBlk = 2;
+};
+template <> struct Geo<kTypeQ8_0Three> {
+    static constexpr int kChunk = 3072, kBlk = 32, kLanesPerBlk = 2;
+};
+template <int QT> constexpr bool is_q8_0 = QT == kTypeQ8_0 || (QT >= kTypeQ8_0Wide && QT <= kTypeQ8_0Three);
 
 // block (super-block) index inside the row that `lane` works on in the chunk starting at k0
 template <int QT>
@@ -91,6 +100,8 @@ template <> struct RowPtr<kTypeQ8_0> {
     __device__ __forceinline__ const void *dummy() const { return qs; }
 };
 template <> struct RowPtr<kTypeQ8_0Wide> : RowPtr<kTypeQ8_0> {};
+template <> struct RowPtr<kTypeQ8_0Two> : RowPtr<kTypeQ8_0> {};
+template <> struct RowPtr<kTypeQ8_0Three> : RowPtr<kTypeQ8_0> {};
 
 // ------------------------------------------------------------------------------------------
 template <int QT> struct Raw;
@@ -201,14 +212,14 @@ template <> struct Frag<kTypeQ8_0> {
     }
 };
 
-template <> struct Raw<kTypeQ8_0Wide> {
-    uint4 q[4];
-    uint32_t d[4];
+template <int P> struct RawQ8Parts {   // P parts of 1024 weights
+    uint4 q[P];
+    uint32_t d[P];
     uint32_t live;   // bit j: part j's block lies inside the row (a short last chunk)
-    __device__ __forceinline__ void load(const RowPtr<kTypeQ8_0Wide> &rp, uint32_t blk_, int lane, uint32_t rel = 0) {
+    __device__ __forceinline__ void load(const RowPtr<kTypeQ8_0> &rp, uint32_t blk_, int lane, uint32_t rel = 0) {
         live = 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < P; ++j) {
             uint32_t b = blk_ + 32u * j;
             if (b < rp.nb) live |= 1u << j;
             else b = rp.nb - 1;   // in bounds, never used
@@ -219,24 +230,31 @@ template <> struct Raw<kTypeQ8_0Wide> {
     }
     __device__ __forceinline__ void zero() {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) { q[j] = make_uint4(0, 0, 0, 0); d[j] = 0; }
+        for (int j = 0; j < P; ++j) { q[j] = make_uint4(0, 0, 0, 0); d[j] = 0; }
         live = 0;
     }
 };
 
-template <> struct Frag<kTypeQ8_0Wide> {
-    uint32_t q[16];
-    float d[4];
+template <> struct Raw<kTypeQ8_0Wide> : RawQ8Parts<4> {};
+template <> struct Raw<kTypeQ8_0Two> : RawQ8Parts<2> {};
+template <> struct Raw<kTypeQ8_0Three> : RawQ8Parts<3> {};
+
+template <int P> struct FragQ8Parts {
+    uint32_t q[4 * P];
+    float d[P];
     uint32_t live;
-    __device__ __forceinline__ void unpack(const Raw<kTypeQ8_0Wide> &r, int) {
+    __device__ __forceinline__ void unpack(const RawQ8Parts<P> &r, int) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < P; ++j) {
             q[4 * j] = r.q[j].x; q[4 * j + 1] = r.q[j].y; q[4 * j + 2] = r.q[j].z; q[4 * j + 3] = r.q[j].w;
             d[j] = h2f(r.d[j]);
         }
         live = r.live;
     }
 };
+template <> struct Frag<kTypeQ8_0Wide> : FragQ8Parts<4> {};
+template <> struct Frag<kTypeQ8_0Two> : FragQ8Parts<2> {};
+template <> struct Frag<kTypeQ8_0Three> : FragQ8Parts<3> {};
 
 // ------------------------------------------------------------------------------------------
 // LDS image of staged quantized activations: MT rows, `kt` bytes of K each.
@@ -330,12 +348,12 @@ template <> struct Dot<kTypeQ8_0> {
     }
 };
 
-template <> struct Dot<kTypeQ8_0Wide> {
-    uint32_t xq[16];
-    float xd[4];
+template <int P> struct DotQ8Parts {
+    uint32_t xq[4 * P];
+    float xd[P];
     __device__ __forceinline__ void load_x(const XTile &x, int m, int c0, int lane) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < P; ++j) {
             const int xo = c0 + 1024 * j + 16 * lane;
             const uint4 a = *reinterpret_cast<const uint4 *>(x.qs + m * x.kt + xo);
             xq[4 * j] = a.x; xq[4 * j + 1] = a.y; xq[4 * j + 2] = a.z; xq[4 * j + 3] = a.w;
@@ -344,10 +362,10 @@ template <> struct Dot<kTypeQ8_0Wide> {
     }
     // the parts are added in the order of K, as four steps of the narrow geometry would add them; a part past
     // the end of the row is left out by selection (its activation bytes were never staged)
-    __device__ __forceinline__ float dot(const Frag<kTypeQ8_0Wide> &f) const {
+    __device__ __forceinline__ float dot(const FragQ8Parts<P> &f) const {
         float t = 0.f;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < P; ++j) {
             int s = 0;
 #pragma unroll
             for (int i = 0; i < 4; ++i) s = dot4(f.q[4 * j + i], xq[4 * j + i], s);
@@ -357,5 +375,8 @@ template <> struct Dot<kTypeQ8_0Wide> {
         return t;
     }
 };
+template <> struct Dot<kTypeQ8_0Wide> : DotQ8Parts<4> {};
+template <> struct Dot<kTypeQ8_0Two> : DotQ8Parts<2> {};
+template <> struct Dot<kTypeQ8_0Three> : DotQ8Parts<3> {};
 
 }  // namespace qproj

@@ -321,7 +321,7 @@ __global__ __launch_bounds__(kDecodeThreads) void gemv_decode_kernel(const float
     // (g, c) = (row group, chunk) cursors; the issue cursor runs one step ahead of the consume
     // cursor and stops on the last step, whose cache lines were just fetched, so every issue is
     // unconditional and no wait ever has to cover a maybe-issued load.
-    if constexpr (XREG && (MT == 1 || (MT == 2 && QT == kTypeQ4_K && FUSE && !PAIR))) {  // one chunk per row, one or two activation rows: the step index is the row group
+    if constexpr (XREG && (MT == 1 || (MT == 2 && (QT == kTypeQ4_K || QT == kTypeQ8_0Two) && FUSE && !PAIR))) {  // one chunk per row, one or two activation rows: the step index is the row group
         // No load is issued twice (a repeated load of the last step, cheap as it looks, costs 0.4 us of the
         // gate+up launch at one activation row and 0.8 us at two): the loop runs while two more steps follow,
         // the last one or two steps are peeled, and every block still knows exactly which loads are outstanding.
@@ -459,6 +459,13 @@ hipError_t launch_decode(const GemvArgs &args, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Q8_0: parts of 1024 weights a step.  Two for rows of at most 2048 (2048 -> 2 x 8192 13.4 -> 10.1 us, 2048 -> 2048 / 512 / 512
+// 5.7 -> 4.9 against four, half of whose requests lie past the row), three where that covers the row with fewer than four do.
+int q8_0_parts(int64_t K) {
+    const int64_t n = (K + 1023) / 1024;
+    return n <= 2 ? 2 : (n + 2) / 3 * 3 < (n + 3) / 4 * 4 ? 3 : 4;
+}
+
 template <int QT, bool FUSE>
 hipError_t launch_decode_mt(const GemvArgs &args, int mt, hipStream_t s) {
     // the wide Q8_0 geometry keeps its 20 activation registers a row only for one row and plain projections (two
@@ -486,12 +493,12 @@ hipError_t launch_decode_mt(const GemvArgs &args, int mt, hipStream_t s) {
     case 2: {
         // (two rows of the wider formats walk one weight row a step whatever the row count: their two-row steps
         // run out of registers -- Q6_K 4096 -> 14336 17.5 -> 13.9 us, Q8_0 8192 x 8192 20.1 -> 17.6)
-        const bool two = pairs && (QT == kTypeQ4_K || two_rows_env > 0);
+        const bool two = pairs && (QT == kTypeQ4_K || QT == kTypeQ8_0Two || two_rows_env > 0);
         if (one_chunk) return two ? launch_decode<QT, 2, 2, true, FUSE>(args, s) : launch_decode<QT, 2, 1, true, FUSE>(args, s);
         return two ? launch_decode<QT, 2, 2, false, FUSE>(args, s) : launch_decode<QT, 2, 1, false, FUSE>(args, s);
     }
     case 4:
-        if constexpr (QT == kTypeQ4_K)
+        if constexpr (QT == kTypeQ4_K || QT == kTypeQ8_0Two)
             if (one_chunk) return launch_decode<QT, 4, 1, true, FUSE>(args, s);
         return launch_decode<QT, 4, 1, false, FUSE>(args, s);
     default: return hipErrorInvalidValue;
@@ -527,7 +534,13 @@ hipError_t launch_gemv_decode(const GemvArgs &args, int mt, bool fuse_quantize, 
     switch (args.t[0].w.type) {
     case kTypeQ4_K: return fuse_quantize ? launch_decode_mt<kTypeQ4_K, true>(args, mt, s) : launch_decode_mt<kTypeQ4_K, false>(args, mt, s);
     case kTypeQ6_K: return fuse_quantize ? launch_decode_mt<kTypeQ6_K, true>(args, mt, s) : launch_decode_mt<kTypeQ6_K, false>(args, mt, s);
-    case kTypeQ8_0: return fuse_quantize ? launch_decode_mt<kTypeQ8_0Wide, true>(args, mt, s) : launch_decode_mt<kTypeQ8_0Wide, false>(args, mt, s);
+    case kTypeQ8_0:
+        switch (q8_0_parts(args.t[0].w.K)) {
+        case 2: return fuse_quantize ? launch_decode_mt<kTypeQ8_0Two, true>(args, mt, s) : launch_decode_mt<kTypeQ8_0Two, false>(args, mt, s);
+        case 3: return fuse_quantize ? launch_decode_mt<kTypeQ8_0Three, true>(args, mt, s) : launch_decode_mt<kTypeQ8_0Three, false>(args, mt, s);
+        default: break;
+        }
+        return fuse_quantize ? launch_decode_mt<kTypeQ8_0Wide, true>(args, mt, s) : launch_decode_mt<kTypeQ8_0Wide, false>(args, mt, s);
     default: return hipErrorInvalidValue;
     }
 }

@@ -1505,6 +1505,29 @@ def test_full_size_against_device_fp64_of_proven_parts(ctx, qtype, k, n):
     assert torch.equal(ctx.mul_mat(w, 2 * x, ACT_GGML), 2 * ctx.mul_mat(w, x, ACT_GGML))
 
 
+@pytest.mark.parametrize("k", [32, 1024, 1056, 2048, 2080, 3072, 3104, 4128, 5120, 6176, 9216])
+def test_q8_0_decode_steps_of_two_three_and_four_parts(ctx, orc, k):
+    """Rows that end inside, at and just behind the last 1024-wide part of a step, one to four activation rows, and the
+    gate / up pairing, whose two rows a step take the same parts."""
+    from magnitude_amd import ACT_GGML
+    n = 67
+    blocks = [make_weight(orc, Q8_0, n, k, seed=6100 + k + i) for i in range(2)]
+    gate, up = [ctx.upload(Q8_0, k, n, b) for b in blocks]
+    x = np.random.default_rng(k).standard_normal((4, k)).astype(np.float32)
+    want = [orc.mul_mat(Q8_0, b, k, x, orc.ACT_GGML) for b in blocks]
+    for m in (1, 2, 3, 4):
+        g, u = ctx.mul_mat_multi([gate, up], dev(x[:m]), ACT_GGML)
+        close(g.cpu().numpy(), want[0][:m], 2e-5)
+        close(u.cpu().numpy(), want[1][:m], 2e-5)
+        h = ctx.ffn_gate_up(gate, up, dev(x[:m])).cpu().numpy()
+        g64, u64 = want[0][:m].astype(np.float64), want[1][:m].astype(np.float64)
+        # 2e-5 a factor: |d(silu(g) u)| <= 1.1 |dg| |u| + |silu(g)| |du|
+        tol = 2e-5 * (1.1 * np.maximum(1, np.abs(g64)) * np.abs(u64) + np.abs(g64) * np.maximum(1, np.abs(u64)) + 1)
+        assert (np.abs(h - g64 / (1 + np.exp(-g64)) * u64) <= tol).all()
+    gate.free()
+    up.free()
+
+
 @pytest.mark.parametrize("ns", [(28677,), (4096, 1024, 1024), (14336, 14336), (9001, 5003), (12289, 1)])
 @pytest.mark.parametrize("m", [1, 2])
 def test_decode_row_dealing_at_full_grids(ctx, ns, m):
