@@ -176,41 +176,26 @@ __device__ __forceinline__ void wave_store_q8x32_row(const float4 &v, int lane, 
     }
 }
 
-// called by all kRowThreads threads of the workgroup after their stores into ld / ls; `wmax`: kRowWaves floats of LDS
+// Called by all kRowThreads threads of the workgroup after their stores into ld / ls.  Every wave finds the row's largest
+// scale by itself (one barrier) and a thread makes one value (before, a thread made the sixteen of a super-block, which left
+// one wave of sixteen at work for a microsecond: 48 rows of 4096, norm 5.1 -> 5.0 us, quantizer 4.7 -> 4.3; 512 rows 9.0 -> 8.6, 8.2 -> 7.7).
 template <bool PER32>
 __device__ __forceinline__ void row_minterm_finish(const float *ld, const int *ls, int nb, int64_t m,
-                                                   uint16_t *__restrict__ msum, float *__restrict__ rs, float *wmax) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+                                                   uint16_t *__restrict__ msum, float *__restrict__ rs) {
+    const int tid = threadIdx.x, lane = tid & 63;
     const int nd = PER32 ? nb * 8 : nb;
     __syncthreads();
     float dmax = 0.f;
-    for (int i = tid; i < nd; i += kRowThreads) dmax = fmaxf(dmax, fabsf(ld[i]));   // a Q8_K scale carries a sign
+    for (int i = lane; i < nd; i += 64) dmax = fmaxf(dmax, fabsf(ld[i]));   // a Q8_K scale carries a sign
     dmax = wave_max(dmax);
-    if (lane == 0) wmax[wave] = dmax;
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < kRowWaves; ++w) dmax = fmaxf(dmax, wmax[w]);
     const float r = pow2_floor(dmax), inv = 1.0f / r;   // exact: a power of two
     if (tid == 0) rs[m] = r;
-    for (int sb = tid; sb < nb; sb += kRowThreads) {
-        uint32_t hi[4], lo[4];
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const float dd = PER32 ? ld[sb * 8 + t] : ld[sb];
-            const float v = (dd * inv) * (float)ls[sb * 8 + t] * kMinPrescale;
-            const _Float16 h = (_Float16)v, l = (_Float16)(v - (float)h);
-            const uint32_t hb = __builtin_bit_cast(uint16_t, h), lb = __builtin_bit_cast(uint16_t, l);
-            if (t & 1) {
-                hi[t >> 1] |= hb << 16;
-                lo[t >> 1] |= lb << 16;
-            } else {
-                hi[t >> 1] = hb;
-                lo[t >> 1] = lb;
-            }
-        }
-        uint4 *dst = reinterpret_cast<uint4 *>(msum + (m * nb + sb) * 16);
-        dst[0] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-        dst[1] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+    for (int i = tid; i < nb * 8; i += kRowThreads) {
+        const float v = (ld[PER32 ? i : i >> 3] * inv) * (float)ls[i] * kMinPrescale;
+        const _Float16 h = (_Float16)v, l = (_Float16)(v - (float)h);
+        uint16_t *dst = msum + (m * nb + (i >> 3)) * 16 + (i & 7);
+        dst[0] = __builtin_bit_cast(uint16_t, h);
+        dst[8] = __builtin_bit_cast(uint16_t, l);
     }
 }
 

@@ -121,7 +121,6 @@ __global__ __launch_bounds__(kRowThreads) void quant_rows_minterm_kernel(const f
                                                                          const ZeroJob zero) {
     zero_rows(zero);
     extern __shared__ __align__(16) float row_lds[];
-    __shared__ float wmax[kRowWaves];
     float *ld = row_lds;
     int *ls = reinterpret_cast<int *>(row_lds + (PER32 ? nb * 8 : nb));
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -132,7 +131,7 @@ __global__ __launch_bounds__(kRowThreads) void quant_rows_minterm_kernel(const f
         if constexpr (PER32) wave_store_q8x32_row(v, lane, g, sb, qs, d, isum, ld, ls);
         else wave_store_q8k_row(v, lane, g, sb, qs, d, bsums, ld, ls);
     }
-    row_minterm_finish<PER32>(ld, ls, nb, m, msum, rs, wmax);
+    row_minterm_finish<PER32>(ld, ls, nb, m, msum, rs);
 }
 
 hipError_t launch_minterm_rows(int kind, const float *d, const int16_t *bsums, const int32_t *isum, int64_t M, int64_t K,

@@ -33,7 +33,6 @@ __global__ __launch_bounds__(kNormThreads) void rms_norm_kernel(const float *__r
     static_assert(kNormThreads == kRowThreads, "the row helpers assume this workgroup");
     extern __shared__ __align__(16) float row_lds[];
     __shared__ double partial[kNormWaves];
-    __shared__ float wmax[kNormWaves];
     const int nb = (int)(K / 256);
     float *ld = row_lds;
     int *ls = reinterpret_cast<int *>(row_lds + (MODE == 3 ? nb * 8 : nb));
@@ -90,7 +89,7 @@ __global__ __launch_bounds__(kNormThreads) void rms_norm_kernel(const float *__r
             wave_store_q8_32<MODE == 2>(v, lane, row * K + e0, live, qs, d, isum);
         }
     }
-    if constexpr (MT) row_minterm_finish<MODE == 3>(ld, ls, nb, row, msum, rs, wmax);
+    if constexpr (MT) row_minterm_finish<MODE == 3>(ld, ls, nb, row, msum, rs);
 }
 
 }  // namespace
