@@ -973,12 +973,19 @@ __global__ __launch_bounds__(W * 64) void gemv_mfma_dense_kernel(const DenseArgs
 
     // wave -> (row group, K part)
     const int rgl = wave >> g.kw_log2, kp = wave - (rgl << g.kw_log2);
+    // A K part takes every kw-th super-block of the chunk: the parts read neighbouring ones at the same time, and share the
+    // cache lines that hold several (Q6_K: 128 bytes are the scales of eight super-blocks, or two of the high bits, and a wave's
+    // step of 52 lines of data touched 128).  us at 8 rows, parts of consecutive super-blocks / this: Q6_K 14336 -> 4096 17.8 / 16.5,
+    // Q4_K 13.5 / 12.4, 4096 -> 14336 12.3 / 11.7; at 16 and 30 rows level.  Q8_0, whose super-blocks are whole lines, lost by it
+    // (8192 x 8192 20.9 / 22.6) and keeps consecutive ones.
+    constexpr bool kTurns = QT != kTypeQ8_0;
     const int part_sb = (nsb + (1 << g.kw_log2) - 1) >> g.kw_log2;
-    const int s0 = min(kp * part_sb, nsb), s1 = min(s0 + part_sb, nsb);  // range inside the chunk
+    const int s0 = kTurns ? kp : min(kp * part_sb, nsb), stride = kTurns ? 1 << g.kw_log2 : 1;   // first one inside the chunk, step
     const int row0 = (rs * g.rw + rgl) * g.rpg;
     const bool rows_ok = row0 < N;
-    const int steps = rows_ok ? s1 - s0 : 0;
-    const int last_sb = c0 + (steps > 0 ? s1 - 1 : 0);   // loads past the range repeat its last super-block
+    int steps = kTurns ? (nsb - kp + stride - 1) >> g.kw_log2 : min(part_sb, nsb - s0);
+    if (!rows_ok || steps < 0) steps = 0;
+    const int last_sb = c0 + (steps > 0 ? s0 + (steps - 1) * stride : 0);   // loads past the range repeat its last super-block
     WeightView w{};
     w.K = (int64_t)g.nb * 256;
     w.nb = QT == kTypeQ8_0 ? g.nb * 8 : g.nb;
@@ -992,7 +999,7 @@ __global__ __launch_bounds__(W * 64) void gemv_mfma_dense_kernel(const DenseArgs
     sa.rebase(0, w, rows_ok ? row0 : 0);
     sa.init(w, rows_ok ? min(g.rpg - 1, N - 1 - row0) : 0, lane);   // rows past the group's last one repeat it
     sb_ = sa;
-    auto issue = [&](Stager<QT> &st, int i) { st.issue(0, min(c0 + s0 + i, last_sb)); };
+    auto issue = [&](Stager<QT> &st, int i) { st.issue(0, min(c0 + s0 + i * stride, last_sb)); };
     uint8_t *region = smem + L.off_w + wave * Cfg<QT>::kRegion;
     // (the addresses stand before the first request: worked out behind it they were mixed with registers still waiting for
     // their loads)
@@ -1014,7 +1021,7 @@ __global__ __launch_bounds__(W * 64) void gemv_mfma_dense_kernel(const DenseArgs
     for (int v = 0; v < NV; ++v) out[v] = 0.f;
     auto consume = [&](int i) {
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        compute<QT, NI>(region, smem, L, s0 + i, lane, out);
+        compute<QT, NI>(region, smem, L, s0 + i * stride, lane, out);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     };
     int i = 0;
@@ -1047,8 +1054,10 @@ __global__ __launch_bounds__(W * 64) void gemv_mfma_dense_kernel(const DenseArgs
         }
         return;
     }
-    // The K parts of a row group meet in the waves' regions and are added in a fixed order, an output a thread of ALL
-    // waves (a group's first wave alone, four outputs a lane and one part after the other, took 1.6 us of the 8-row o).
+    // The K parts of a row group meet in the waves' regions and are added in pairs, an output a thread of ALL waves (a
+    // group's first wave alone, four outputs a lane, took 1.6 us of the 8-row o).  One after the other the sums of parts that
+    // take super-blocks in turns were up to 12 % further from 64 bits than before (Q6_K 3072 x 3072); in pairs they are
+    // nearer, 0.88 to 1.003 of the error over 35 shapes of K 1024 to 16384 at 8, 16 and 30 rows.
     float *mine = reinterpret_cast<float *>(region);
 #pragma unroll
     for (int v = 0; v < NV; ++v) mine[(8 * (v >> 2) + 4 * h + (v & 3)) * 32 + nl] = out[v];
@@ -1064,10 +1073,11 @@ __global__ __launch_bounds__(W * 64) void gemv_mfma_dense_kernel(const DenseArgs
                 float p[KW];
 #pragma unroll
                 for (int q = 0; q < KW; ++q) p[q] = *reinterpret_cast<const float *>(src + q * Cfg<QT>::kRegion);
-                float acc = p[0];
 #pragma unroll
-                for (int q = 1; q < KW; ++q) acc += p[q];
-                store(m, r0 + n, acc);
+                for (int d = 1; d < KW; d *= 2)   // in pairs: the shortest chain of roundings
+#pragma unroll
+                    for (int q = 0; q < KW; q += 2 * d) p[q] += p[q + d];
+                store(m, r0 + n, p[0]);
             }
         }
     };
