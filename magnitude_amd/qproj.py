@@ -245,10 +245,12 @@ class Context:
         """Device address of t made contiguous.  A copy made for that is kept alive until the next sync(): the launch
         that reads it runs on the context's own stream, which torch's allocator does not track, so a temporary freed
         when the ctypes call returns could be handed out again while the kernel is still reading it."""
-        c = t.contiguous()
-        if c is not t:
-            self._held.append(c)
-        return _ptr(c)
+        if not t.is_contiguous():
+            t = t.contiguous()
+            self._held.append(t)
+        if not t.is_cuda:
+            raise ValueError("device tensor expected")
+        return t.data_ptr()
 
     # ---- weights -------------------------------------------------------------------------
     def upload(self, qtype: int, k: int, n: int, gguf: np.ndarray, n_expert: int = 1) -> Weight:
@@ -321,10 +323,12 @@ class Context:
     def mul_mat(self, w: Weight, x: torch.Tensor, act: int = ACT_GGML, out: Optional[torch.Tensor] = None,
                 sync: bool = True) -> torch.Tensor:
         """GGML_OP_MUL_MAT: x f32 [M, K] -> y f32 [M, N]."""
-        x2 = x.reshape(-1, w.K)
+        # (rows that are already [M, K] are taken as they are: the smallest product takes the GPU 4.3 us, and a reshape that
+        # changes nothing 0.8 of the host's 5.1)
+        x2 = x if x.dim() == 2 and x.size(1) == w.K else x.reshape(-1, w.K)
         if x2.dtype != torch.float32:
             raise ValueError("activations must be float32")
-        m = x2.shape[0]
+        m = x2.size(0)
         y = out if out is not None else torch.empty((m, w.N), dtype=torch.float32, device=x.device)
         if sync:
             torch.cuda.current_stream().synchronize()
