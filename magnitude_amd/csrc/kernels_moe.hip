@@ -22,74 +22,83 @@ namespace qproj {
 constexpr int kGroupThreads = 1024;
 constexpr int kGroupLdsIds = 8192;   // pair ids staged in LDS up to this many, read from global beyond
 
+// inclusive prefix sum over the wave, in the vector unit: within a row of 16 lanes, then rows onto the next ones
+__device__ __forceinline__ int wave_prefix(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+    return v;
+}
+// sum over the 16 lanes of a row, in every lane
+__device__ __forceinline__ int row_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, true);   // row_ror:8, 4, 2, 1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x124, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x122, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x121, 0xf, 0xf, true);
+    return v;
+}
+
 // cnt[e] = pairs of expert e on entry; on exit cnt[e] = offsets[e] = its first slot, active[] lists the
 // experts that have pairs.  All threads of the workgroup call it; the caller synchronizes afterwards.
-__device__ __forceinline__ void group_scan(int n_expert, int32_t *cnt, int32_t *wsum, int32_t *__restrict__ offsets,
-                                           int32_t *__restrict__ active, int heavy_above, int tile_rows, int list_cap) {
+// PER: experts a thread (1 up to 1024 experts, 8 beyond).  The launch waits for this one workgroup: with the scans through LDS
+// shuffles, eight experts a thread whatever their number and the tiles of an expert by a division it was four of the seven
+// microseconds of the grouping launch.
+template <int PER>
+__device__ __forceinline__ void group_scan_per(int n_expert, int32_t *cnt, int32_t *wsum, int32_t *__restrict__ offsets,
+                                               int32_t *__restrict__ active, int heavy_above, bool tiled, int list_cap) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // exclusive scans over the workgroup (shuffles inside a wave, wave totals through LDS) of the pair
+    // exclusive scans over the workgroup (in the vector unit inside a wave, wave totals through LDS) of the pair
     // counts (-> offsets) and of the non-empty flags (-> compact list of the experts that have work);
-    // thread t owns experts [t * per, t * per + per)
-    const int per = (n_expert + kGroupThreads - 1) / kGroupThreads;
-    int tot[8], local = 0, local_f = 0;
+    // thread t owns experts [t * PER, t * PER + PER)
+    int tot[PER], local = 0, local_f = 0, local_h = 0;
     // list positions of an expert: one, or one per tile of its pairs
-    auto positions = [&](int pairs) { return tile_rows ? (pairs + tile_rows - 1) / tile_rows : (int)(pairs > 0); };
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int e = tid * per + i;
-        tot[i] = i < per && e < n_expert ? cnt[e] : 0;
-        local += tot[i];
-        local_f += positions(tot[i]);
-    }
+    static_assert(kMoeTileRows == 64, "tiles of an expert's pairs by a shift");
+    auto positions = [&](int pairs) { return tiled ? (pairs + 63) >> 6 : (int)(pairs > 0); };
     // The experts with more pairs than one pass of the grouped kernels stages (two passes over their weights) go
     // to the front of the list, everything else stays in ascending order: the grouped kernels hand their
     // workgroups out in list order, and a two-pass expert then starts with the grid instead of stretching its
     // tail.  A third scan, over the "heavy" flags, gives the positions.  (The whole list ordered by pair count
     // evened the launches out as well but cost the ordinary case 3 us: neighbouring workgroups no longer read
     // neighbouring experts.)
-    int local_h = 0;
+    auto is_heavy = [&](int pairs) { return heavy_above > 0 && pairs > heavy_above; };
 #pragma unroll
-    for (int i = 0; i < 8; ++i) local_h += heavy_above > 0 && tot[i] > heavy_above ? positions(tot[i]) : 0;
-    int incl = local, incl_f = local_f, incl_h = local_h;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int up = __shfl_up(incl, d), up_f = __shfl_up(incl_f, d), up_h = __shfl_up(incl_h, d);
-        if (lane >= d) {
-            incl += up;
-            incl_f += up_f;
-            incl_h += up_h;
-        }
+    for (int i = 0; i < PER; ++i) {
+        const int e = tid * PER + i;
+        tot[i] = e < n_expert ? cnt[e] : 0;
+        local += tot[i];
+        local_f += positions(tot[i]);
+        local_h += is_heavy(tot[i]) ? positions(tot[i]) : 0;
     }
+    const int incl = wave_prefix(local), incl_f = wave_prefix(local_f), incl_h = wave_prefix(local_h);
     if (lane == 63) {
         wsum[wave] = incl;
         wsum[16 + wave] = incl_f;
         wsum[32 + wave] = incl_h;
     }
     __syncthreads();
-    int before = incl - local, before_f = incl_f - local_f, before_h = incl_h - local_h, n_heavy = 0;
-    for (int w = 0; w < kGroupThreads / 64; ++w) {
-        if (w < wave) {
-            before += wsum[w];
-            before_f += wsum[16 + w];
-            before_h += wsum[32 + w];
-        }
-        n_heavy += wsum[32 + w];
-    }
+    // what the waves before this one counted: a wave total a lane of each row
+    static_assert(kGroupThreads / 64 == 16, "a row of lanes holds the totals of the waves");
+    const int w = lane & 15, w0 = wsum[w], w1 = wsum[16 + w], w2 = wsum[32 + w];
+    int before = incl - local + row_sum(w < wave ? w0 : 0), before_f = incl_f - local_f + row_sum(w < wave ? w1 : 0),
+        before_h = incl_h - local_h + row_sum(w < wave ? w2 : 0);
+    const int n_heavy = row_sum(w2);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int e = tid * per + i;
-        if (i < per && e < n_expert) {
+    for (int i = 0; i < PER; ++i) {
+        const int e = tid * PER + i;
+        if (e < n_expert) {
             cnt[e] = before;   // from here on: the expert's first slot
             offsets[e] = before;
             before += tot[i];
             if (tot[i] > 0) {
-                const bool heavy = heavy_above > 0 && tot[i] > heavy_above;
+                const bool heavy = is_heavy(tot[i]);
                 const int pos = heavy ? before_h : n_heavy + (before_f - before_h);
                 int4 *rec = reinterpret_cast<int4 *>(active + active_slots_offset(list_cap)) + pos;
                 const int n_pos = positions(tot[i]);
-                if (tile_rows) {
-                    for (int t = 0; t < n_pos; ++t)
-                        rec[t] = make_int4(e, before - tot[i] + t * tile_rows, min(tile_rows, tot[i] - t * tile_rows), 0);
+                if (tiled) {
+                    for (int t = 0; t < n_pos; ++t) rec[t] = make_int4(e, before - tot[i] + t * 64, min(64, tot[i] - t * 64), 0);
                 } else {
                     active[pos] = e;
                     *rec = make_int4(e, before - tot[i], tot[i], 0);
@@ -104,12 +113,17 @@ __device__ __forceinline__ void group_scan(int n_expert, int32_t *cnt, int32_t *
         active[list_cap] = before_f;   // positions of the list
     }
 }
+__device__ __forceinline__ void group_scan(int n_expert, int32_t *cnt, int32_t *wsum, int32_t *__restrict__ offsets,
+                                           int32_t *__restrict__ active, int heavy_above, bool tiled, int list_cap) {
+    if (n_expert <= kGroupThreads) group_scan_per<1>(n_expert, cnt, wsum, offsets, active, heavy_above, tiled, list_cap);
+    else group_scan_per<8>(n_expert, cnt, wsum, offsets, active, heavy_above, tiled, list_cap);
+}
 
 template <bool STAGED>
 __device__ __forceinline__ void group_sweeps(const int32_t *__restrict__ ids, const int32_t *sid, int n_pairs, int n_expert,
                                              int32_t *cnt, int32_t *wsum, int32_t *__restrict__ order,
                                              int32_t *__restrict__ offsets, int32_t *__restrict__ active, int heavy_above,
-                                             int tile_rows, int list_cap) {
+                                             bool tiled, int list_cap) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     constexpr int kWaves = kGroupThreads / 64;
     auto id_at = [&](int p) { return p < n_pairs ? (STAGED ? sid[p] : ids[p]) : -1; };
@@ -129,7 +143,7 @@ __device__ __forceinline__ void group_sweeps(const int32_t *__restrict__ ids, co
         }
     }
     __syncthreads();
-    group_scan(n_expert, cnt, wsum, offsets, active, heavy_above, tile_rows, list_cap);
+    group_scan(n_expert, cnt, wsum, offsets, active, heavy_above, tiled, list_cap);
     __syncthreads();
     // sweep 2: placement, ascending pair order inside every expert (cnt[e] = the expert's next free slot)
     for (int base = 0; base < n_pairs; base += 64 * kHeld) {
@@ -168,7 +182,7 @@ __global__ __launch_bounds__(kGroupThreads) void moe_group_kernel(const int32_t 
                                                                   int32_t *__restrict__ offsets,
                                                                   int32_t *__restrict__ active,
                                                                   int32_t *__restrict__ error_flag, int by_block,
-                                                                  int heavy_above, int tile_rows, int list_cap,
+                                                                  int heavy_above, int tiled, int list_cap,
                                                               const RowQuantJob job) {
     // Workgroups past the first have nothing to do with the grouping: they quantize the activation rows the
     // grouped projection is going to read (one 256-wide chunk a wave, ggml's quantize_row_q8_K as in the
@@ -198,8 +212,8 @@ __global__ __launch_bounds__(kGroupThreads) void moe_group_kernel(const int32_t 
         for (int e = tid; e < n_expert; e += kGroupThreads) cnt[e] = 0;
         if (bad) atomicOr(error_flag, 1);
         __syncthreads();
-        if (staged) group_sweeps<true>(ids, tab, n_pairs, n_expert, cnt, wsum, order, offsets, active, heavy_above, tile_rows, list_cap);
-        else group_sweeps<false>(ids, tab, n_pairs, n_expert, cnt, wsum, order, offsets, active, heavy_above, tile_rows, list_cap);
+        if (staged) group_sweeps<true>(ids, tab, n_pairs, n_expert, cnt, wsum, order, offsets, active, heavy_above, tiled, list_cap);
+        else group_sweeps<false>(ids, tab, n_pairs, n_expert, cnt, wsum, order, offsets, active, heavy_above, tiled, list_cap);
         return;
     }
     const int n_blocks = (n_pairs + 63) / 64, per_wave = (n_blocks + kGroupThreads / 64 - 1) / (kGroupThreads / 64);
@@ -247,7 +261,7 @@ __global__ __launch_bounds__(kGroupThreads) void moe_group_kernel(const int32_t 
         cnt[e] = run;
     }
     __syncthreads();
-    group_scan(n_expert, cnt, wsum, offsets, active, heavy_above, tile_rows, list_cap);
+    group_scan(n_expert, cnt, wsum, offsets, active, heavy_above, tiled, list_cap);
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < kHeldBlocks; ++i)
@@ -272,7 +286,7 @@ __global__ __launch_bounds__(kGroupThreads) void moe_group_kernel(const int32_t 
 hipError_t launch_moe_group(const int32_t *ids, int64_t n_pairs, int64_t n_expert, int32_t *order,
                             int32_t *offsets, int32_t *active, int32_t *error_flag, int64_t pass_rows,
                             const RowQuantJob *quantize, hipStream_t s, int64_t tile_rows) {
-    if (n_expert > 8192 || n_pairs > 0x7fffffff) return hipErrorInvalidValue;
+    if (n_expert > 8192 || n_pairs > 0x7fffffff || (tile_rows && tile_rows != kMoeTileRows)) return hipErrorInvalidValue;
     const size_t table = (size_t)(kGroupThreads / 64) * (size_t)n_expert;
     const bool by_block = table <= 24 * 1024;   // at most 96 KB of LDS
     const size_t lds = ((size_t)n_expert + 48 + (by_block ? table : n_pairs <= kGroupLdsIds ? (size_t)n_pairs : 0)) * sizeof(int32_t);
@@ -306,7 +320,7 @@ hipError_t launch_moe_group(const int32_t *ids, int64_t n_pairs, int64_t n_exper
     if (extra >= 0x7fffffff) return hipErrorInvalidValue;
     hipLaunchKernelGGL(moe_group_kernel, dim3((unsigned)(1 + extra)), dim3(kGroupThreads), lds, s, ids, (int)n_pairs,
                        (int)n_expert, order, offsets, active, error_flag, by_block ? 1 : 0,
-                       (int)heavy, (int)tile_rows, (int)list_cap, job);
+                       (int)heavy, tile_rows ? 1 : 0, (int)list_cap, job);
     return hipGetLastError();
 }
 
