@@ -43,6 +43,12 @@ struct MoeDecodeArgs {
 __device__ __forceinline__ float slot_sum(float v, int vlane, int lpr) {
     v += dpp_move<0xB1>(v);   // quad_perm [1,0,3,2]
     v += dpp_move<0x4E>(v);   // quad_perm [2,3,0,1]
+    if (lpr >= 16 && (lpr & (lpr - 1)) == 0) {   // (wave-uniform) slots are whole rows of 16 lanes: the same tree in the vector unit
+        if (lpr >= 64) v = add_xor32(v);
+        if (lpr >= 32) v = add_xor16(v);
+        v += dpp_move<0x108>(v);   // row_shl:8, 4
+        return v + dpp_move<0x104>(v);
+    }
 #pragma unroll
     for (int o = 32; o >= 4; o >>= 1) {
         if (o < lpr) {   // wave-uniform
