@@ -154,7 +154,7 @@ __device__ __forceinline__ void wave_store_q8k_row(const float4 &v, int lane, in
     const uint32_t packed = wave_quantize_q8k(v, lane, bsum, dd);
     reinterpret_cast<uint32_t *>(qs + g * 256)[lane] = packed;
     if ((lane & 3) == 0) bsums[g * 16 + (lane >> 2)] = (int16_t)bsum;
-    const int pair = bsum + __shfl_down(bsum, 4);   // two neighbouring groups of 16
+    const int pair = bsum + dpp_move_i<0x104>(bsum);   // row_shl:4: two neighbouring groups of 16
     if ((lane & 7) == 0) ls[sb * 8 + (lane >> 3)] = pair;
     if (lane == 0) {
         d[g] = dd;

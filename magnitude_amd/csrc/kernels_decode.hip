@@ -180,7 +180,7 @@ __device__ __forceinline__ void consume(const Raw<QT> (&raw)[R], float (&acc)[MT
             const float t = wave_sum4(q, lane);
             const int i = lane - 12;  // lanes 12..15 hold the four sums
             if constexpr (PAIR) {
-                const float up = __shfl_down(t, 1);   // sums 2m (gate) and 2m+1 (up) sit in neighbouring lanes
+                const float up = dpp_move<0x101>(t);   // row_shl:1: sums 2m (gate) and 2m+1 (up) sit in neighbouring lanes
                 if (i >= 0 && i < 4 && v0 + i < V && ((v0 + i) & 1) == 0) {
                     const int m = (v0 + i) / 2;
                     if (m < M && g < n_rows) y[(int64_t)m * N + row_begin + g] = (t / (1.0f + expf(-t))) * up;
