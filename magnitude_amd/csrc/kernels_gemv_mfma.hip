@@ -1115,7 +1115,7 @@ template <int QT, int NI, int W>
 hipError_t launch_dense(const DenseArgs &g, int n_wgs, hipStream_t s) {
     // K parts of a row group are summed through the waves' regions: a wave's partial tile must fit its region
     if (g.kw_log2 > 0 && (8 * NI) * 32 * 4 > Cfg<QT>::kRegion) return hipErrorInvalidValue;
-    if (g.M > 8 * NI || g.M * g.chunk_sb > W * 64) return hipErrorInvalidValue;   // staged rows; records, one a thread
+    if (g.M > 8 * NI || g.M * g.chunk_sb > 256) return hipErrorInvalidValue;   // staged rows and super-blocks (DenseRows)
     if (dry_run()) {
         if (g.n_chunks > 1 && !g.add_out) plan_note_cut();
         plan_note("gemv_mfma_kernel<%s, %d staged rows, %d waves, dense>: %d workgroups, K in %d chunk(s) of %d super-blocks x %d parts a row group of %d rows%s",
