@@ -460,7 +460,10 @@ hipError_t launch_decode(const GemvArgs &args, hipStream_t s) {
 }
 
 // Q8_0: parts of 1024 weights a step.  Two for rows of at most 2048 (2048 -> 2 x 8192 13.4 -> 10.1 us, 2048 -> 2048 / 512 / 512
-// 5.7 -> 4.9 against four, half of whose requests lie past the row), three where that covers the row with fewer than four do.
+// 5.7 -> 4.9 against four, half of whose requests lie past the row), three where that covers the row with fewer than four do: one
+// token through a layer of 3072 / 1024 / 8192 33.8 -> 29.5 us, of 5120 / 1024 / 13824 68.3 -> 63.4, of 2560 / 512 / 7680 30.1 -> 25.7; rows of
+// one part more or less than whole threes gain little (13824 -> 5120 16.9 / 16.7, 14336 -> 4096 12.1 / 11.8, at two rows 14.5 / 14.6).
+// Error against 64 bits 0.966 to 1.003 of that of four parts (K 5120 to 17408, one to four rows).
 int q8_0_parts(int64_t K) {
     const int64_t n = (K + 1023) / 1024;
     return n <= 2 ? 2 : (n + 2) / 3 * 3 < (n + 3) / 4 * 4 ? 3 : 4;
