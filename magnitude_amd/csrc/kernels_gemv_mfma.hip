@@ -585,14 +585,13 @@ __device__ __forceinline__ void stage_quantize(const MfmaArgs &g, uint8_t *smem,
     }
 }
 
-constexpr int kDense = 0, kGrouped = 1, kGroupedSwiglu = 2;
+constexpr int kGrouped = 1, kGroupedSwiglu = 2;
 
 // kGrouped: the workgroup's expert e multiplies its own pairs, y[pair][n].  kGroupedSwiglu: tensors 0 and 1 are gate
-// and up of the same expert and y[pair][n] = silu(gate . x) * (up . x).  (kDense: gemv_mfma_dense_kernel.)
+// and up of the same expert and y[pair][n] = silu(gate . x) * (up . x).  (Dense launches: gemv_mfma_dense_kernel.)
 // FLAT (K in one part, kw = 1): the wave's row groups as one stream of items.
 template <int QT, int NI, int W, int MODE, bool FLAT = false>
 __global__ __launch_bounds__(W * 64) void gemv_mfma_kernel(const MfmaArgs g) {
-    static_assert(MODE != kDense, "dense launches have their own kernel");
     extern __shared__ __align__(16) uint8_t smem[];
     constexpr int MT = 8 * NI, NV = 4 * NI;
     constexpr bool SWIGLU = MODE == kGroupedSwiglu;
@@ -1118,7 +1117,7 @@ hipError_t launch_dense(const DenseArgs &g, int n_wgs, hipStream_t s) {
     if (g.M > 8 * NI || g.M * g.chunk_sb > 256) return hipErrorInvalidValue;   // staged rows and super-blocks (DenseRows)
     if (dry_run()) {
         if (g.n_chunks > 1 && !g.add_out) plan_note_cut();
-        plan_note("gemv_mfma_kernel<%s, %d staged rows, %d waves, dense>: %d workgroups, K in %d chunk(s) of %d super-blocks x %d parts a row group of %d rows%s",
+        plan_note("gemv_mfma_dense_kernel<%s, %d staged rows, %d waves>: %d workgroups, K in %d chunk(s) of %d super-blocks x %d parts a row group of %d rows%s",
                   plan_type_name(QT), 8 * NI, W, n_wgs, g.n_chunks, g.chunk_sb, 1 << g.kw_log2, g.rpg,
                   g.n_chunks == 1 ? "" : g.add_out ? ", the two chunks add themselves to cleared rows" : " + sum_chunks_kernel");
         return hipSuccess;

@@ -147,6 +147,22 @@ def test_routing_table_of_the_benchmark_configurations_is_pinned():
     assert first.count("gemv_decode_kernel") == 1 and "quantizer:" not in first
 
 
+def test_plan_names_kernels_that_are_launched():
+    """A line of the plan is matched to a profile by the kernel's name: every name is one that the sources define, and the small
+    batches, whose products have a dense and an expert-grouped kernel, name the one they launch."""
+    import glob
+    import os
+    sources = "".join(open(f).read() for f in glob.glob(os.path.join(os.path.dirname(qproj.__file__), "csrc", "*.hip")))
+    defined = set(re.findall(r"__global__[^;{]*?void\s+(\w+)\s*\(", sources))
+    plans = [routing_table()] + [qproj.plan_mul_mat(qt, 4096, (4096,), m) for qt in (Q8_0, Q4_K, Q6_K) for m in (5, 8, 16, 32)]
+    named = set(re.findall(r"\b(\w+_kernel\w*)\b", "".join(plans)))
+    assert named <= defined, named - defined
+    for plan in plans[1:]:
+        assert "gemv_mfma_dense_kernel<" in plan and "gemv_mfma_kernel<" not in plan, plan
+    grouped = qproj.plan_moe_ffn(Q6_K, Q6_K, 2048, 768, 128, 8, 64)
+    assert grouped.count("gemv_mfma_kernel<") == 2 and "dense" not in grouped, grouped
+
+
 def test_plan_reports_a_refused_call():
     with pytest.raises(qproj.QprojError):
         qproj.plan_mul_mat(Q6_K, 4096, (4096,), 64, Q8X32)
