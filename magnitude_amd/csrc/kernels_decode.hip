@@ -439,8 +439,10 @@ hipError_t launch_decode(const GemvArgs &args, hipStream_t s) {
         char rows[96] = "";
         for (int i = 0, o = 0; i < n_targets && o < 80; ++i)
             o += snprintf(rows + o, sizeof rows - o, "%s%lld rows/%d a wave pair", i ? ", " : "", (long long)a.N[i], a.rows_per_pair[i]);
-        plan_note("gemv_decode_kernel<%s, %d activation rows, %d weight rows a step, activations in %s, %s%s>: grid %lld x %d, %s, LDS %zu B",
-                  plan_type_name(QT), MT, R, XREG ? "registers" : "LDS", FUSE ? "quantizer in the prologue" : "rows quantized earlier",
+        char parts[40] = "";
+        if (is_q8_0<QT>) snprintf(parts, sizeof parts, ", %d parts of 1024 weights a step", CH / 1024);
+        plan_note("gemv_decode_kernel<%s%s, %d activation rows, %d weight rows a step, activations in %s, %s%s>: grid %lld x %d, %s, LDS %zu B",
+                  plan_type_name(args.t[0].w.type), parts, MT, R, XREG ? "registers" : "LDS", FUSE ? "quantizer in the prologue" : "rows quantized earlier",
                   PAIR ? ", gate/up paired + swiglu" : "", (long long)grid, kDecodeThreads, rows, smem);
         return hipSuccess;
     }

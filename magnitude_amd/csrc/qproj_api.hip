@@ -42,7 +42,7 @@ void plan_note(const char *fmt, ...) {
     g_plan->push_back('\n');
 }
 const char *plan_type_name(int type) {
-    return type == kTypeQ4_K ? "Q4_K" : type == kTypeQ6_K ? "Q6_K" : type == kTypeQ8_0 || (type >= 1008 && type <= 1010) ? "Q8_0" : "?";
+    return type == kTypeQ4_K ? "Q4_K" : type == kTypeQ6_K ? "Q6_K" : type == kTypeQ8_0 ? "Q8_0" : "?";
 }
 
 int tuning_int(const char *name, int dflt) {

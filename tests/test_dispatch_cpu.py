@@ -163,6 +163,17 @@ def test_plan_names_kernels_that_are_launched():
     assert grouped.count("gemv_mfma_kernel<") == 2 and "dense" not in grouped, grouped
 
 
+@pytest.mark.parametrize("k,parts", [(32, 2), (1024, 2), (2048, 2), (2080, 3), (3072, 3), (3104, 4), (4096, 4), (4128, 3), (5120, 3), (6144, 3),
+                                     (6176, 4), (8192, 4), (8224, 3), (9216, 3), (9248, 4), (12288, 4), (14336, 3), (15392, 4)])
+def test_q8_0_decode_steps_of_fewest_parts(k, parts):
+    """Two parts of 1024 weights a step for rows that they cover, three where those cover the row with fewer parts than steps of
+    four do, for one to four activation rows."""
+    for m in (1, 2, 4):
+        plan = qproj.plan_mul_mat(Q8_0, k, (512, 512), m)
+        assert re.findall(r"gemv_decode_kernel<Q8_0, (\d) parts of 1024 weights a step,", plan) == [str(parts)], plan
+    assert "gemv_decode_kernel<Q4_K, 1 activation rows" in qproj.plan_mul_mat(Q4_K, k // 256 * 256 + 256, (512,), 1)
+
+
 def test_plan_reports_a_refused_call():
     with pytest.raises(qproj.QprojError):
         qproj.plan_mul_mat(Q6_K, 4096, (4096,), 64, Q8X32)
