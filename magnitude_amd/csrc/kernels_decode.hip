@@ -203,7 +203,9 @@ __global__ __launch_bounds__(kDecodeThreads) void gemv_decode_kernel(const float
     static_assert(!PAIR || R == 2, "the gate/up pairing walks two rows a step");
     extern __shared__ __align__(16) uint8_t smem[];
     constexpr int kPointers = QT == kTypeQ4_K ? 1 : is_q8_0<QT> ? 2 : 4;
-    fetch_arguments<40 + offsetof(DecodeArgs, p0) + kPointers * sizeof(DecodeArgs::p0)>();
+    using Kernel = decltype(gemv_decode_kernel<QT, MT, R, XREG, FUSE, PAIR>);
+    static_assert(offsetof(DecodeArgs, p3) == offsetof(DecodeArgs, p0) + 3 * sizeof(DecodeArgs::p0), "a format's pointers stand together");
+    fetch_arguments<Kernel, argument_block(static_cast<Kernel *>(nullptr)).last + offsetof(DecodeArgs, p0) + kPointers * sizeof(DecodeArgs::p0)>();
     constexpr int CH = Geo<QT>::kChunk;
     constexpr int BLK = Geo<QT>::kBlk;
     const int lane = threadIdx.x & 63;

@@ -160,7 +160,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_stream_kernel(const StreamArg
     constexpr bool kQ4 = QT == kTypeQ4_K;
     constexpr int RW = NW / KW, TM = 32 * JT, NT = 64 * NW;
     extern __shared__ __align__(16) uint8_t smem[];
-    fetch_arguments<kQ4 ? (int)offsetof(StreamArgs, p1) : (int)sizeof(StreamArgs)>();
+    fetch_arguments<decltype(gemm_stream_kernel<QT, JT, KW, SW, NW>), kQ4 ? offsetof(StreamArgs, p1) : sizeof(StreamArgs)>();
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, lh = lane >> 5, rg = wave % RW, kp = wave / RW;
 

@@ -7,16 +7,29 @@
 
 namespace qproj {
 
-// Asks for all of a kernel's arguments (BYTES of them) at once.  The compiler loads an argument where it is first used, and
-// every 64-byte line of them that nobody touched before is a trip to memory of half a microsecond, one after the other.
-template <int BYTES>
+// A kernel's parameters in its argument block, one after the other at their own alignment, as its signature has them
+struct ArgumentBlock {
+    size_t last, total;   // where the last parameter starts; where it ends
+};
+template <typename... P>
+constexpr ArgumentBlock argument_block(void (*)(P...)) {
+    ArgumentBlock b{0, 0};
+    ((b.last = (b.total + alignof(P) - 1) / alignof(P) * alignof(P), b.total = b.last + sizeof(P)), ...);
+    return b;
+}
+
+// Asks for the first BYTES of the arguments of the kernel that calls it, of signature `Kernel`, at once.  The compiler loads an
+// argument where it is first used, and every 64-byte line of them that nobody touched before is a trip to memory of half a
+// microsecond, one after the other.
+template <typename Kernel, size_t BYTES>
 __device__ __forceinline__ void fetch_arguments() {
+    static_assert(BYTES >= 4 && BYTES <= argument_block(static_cast<Kernel *>(nullptr)).total, "inside the kernel's arguments");
 #if defined(__HIP_DEVICE_COMPILE__)
     typedef const uint32_t __attribute__((address_space(4))) *words;
     const words w = (words)__builtin_amdgcn_kernarg_segment_ptr();
     uint32_t x = w[0];
 #pragma unroll
-    for (int i = 1; i < (BYTES + 63) / 64; ++i) x ^= w[16 * i];
+    for (size_t i = 1; i < (BYTES + 63) / 64; ++i) x ^= w[16 * i];
     asm volatile("" ::"s"(x));   // (a value, so that the loads stay; nothing reads it)
 #endif
 }
