@@ -473,14 +473,24 @@ int q8_0_parts(int64_t K) {
     return n <= 2 ? 2 : (n + 2) / 3 * 3 < (n + 3) / 4 * 4 ? 3 : 4;
 }
 
+// Rows of one chunk keep their activations in registers, longer ones read the LDS image.  Built are the instances that the
+// rule below reaches: two parts are taken for rows that they cover only, steps of two rows in the wider formats likewise.
+template <int QT, int MT, int R, bool FUSE, bool PAIR = false>
+hipError_t launch_decode_rows(const GemvArgs &args, hipStream_t s) {
+    // the wide Q8_0 geometry keeps its 20 activation registers a row only for one row and plain projections (two
+    // rows, or the gate/up pairing, would spill), four rows fit in the smallest geometries
+    constexpr bool kRegisters = QT == kTypeQ8_0Wide ? MT == 1 && !PAIR : MT <= 2 || QT == kTypeQ4_K || QT == kTypeQ8_0Two;
+    if constexpr (kRegisters)
+        if (args.t[0].w.K <= Geo<QT>::kChunk) return launch_decode<QT, MT, R, true, FUSE, PAIR>(args, s);
+    if constexpr (QT != kTypeQ8_0Two && (QT == kTypeQ4_K || R == 1 || PAIR)) return launch_decode<QT, MT, R, false, FUSE, PAIR>(args, s);
+    return hipErrorInvalidValue;   // (a chunk too long for an instance that is never asked for it)
+}
+
 template <int QT, bool FUSE>
 hipError_t launch_decode_mt(const GemvArgs &args, int mt, hipStream_t s) {
-    // the wide Q8_0 geometry keeps its 20 activation registers a row only for one row and plain projections (two
-    // rows, or the gate/up pairing, would spill); otherwise it reads them from the LDS image like a longer K
-    const bool one_chunk = args.t[0].w.K <= Geo<QT>::kChunk && !(QT == kTypeQ8_0Wide && (mt > 1 || args.swiglu_pair));
     if (args.swiglu_pair) {
-        if (mt == 1) return one_chunk ? launch_decode<QT, 1, 2, true, FUSE, true>(args, s) : launch_decode<QT, 1, 2, false, FUSE, true>(args, s);
-        if (mt == 2) return one_chunk ? launch_decode<QT, 2, 2, true, FUSE, true>(args, s) : launch_decode<QT, 2, 2, false, FUSE, true>(args, s);
+        if (mt == 1) return launch_decode_rows<QT, 1, 2, FUSE, true>(args, s);
+        if (mt == 2) return launch_decode_rows<QT, 2, 2, FUSE, true>(args, s);
         return hipErrorInvalidValue;
     }
     // two rows per step only when every wave has at least two rows to walk (with 1.5 rows per wave, split
@@ -490,24 +500,20 @@ hipError_t launch_decode_mt(const GemvArgs &args, int mt, hipStream_t s) {
     for (int i = 0; i < args.n_targets; ++i) rows_total += args.t[i].w.N;
     static const int two_rows_env = tuning_int("QPROJ_DECODE_TWO_ROWS", -1);
     const bool pairs = two_rows_env >= 0 ? two_rows_env != 0 : rows_total >= (int64_t)2 * cu_count() * kDecodeWaves;
+    // Two activation rows, or rows of several chunks, in the wider formats walk one weight row a step whatever the row count:
+    // their two-row steps run out of registers (two rows, Q6_K 4096 -> 14336 17.5 -> 13.9 us, Q8_0 8192 x 8192 20.1 -> 17.6; one
+    // row, 8192 x 8192 Q8_0 19.2 -> 16.9, Q6_K 15.6 -> 14.3).  The two-part Q8_0 steps are as small as Q4_K's.
+    constexpr bool kSmall = QT == kTypeQ4_K || QT == kTypeQ8_0Two;
     switch (mt) {
-    case 1: {
-        if (one_chunk) return pairs ? launch_decode<QT, 1, 2, true, FUSE>(args, s) : launch_decode<QT, 1, 1, true, FUSE>(args, s);
-        // (rows of several chunks in the wider formats: one row a step -- 8192 x 8192 Q8_0 19.2 -> 16.9 us, Q6_K 15.6 -> 14.3)
-        const bool two = pairs && (QT == kTypeQ4_K || two_rows_env > 0);
-        return two ? launch_decode<QT, 1, 2, false, FUSE>(args, s) : launch_decode<QT, 1, 1, false, FUSE>(args, s);
-    }
-    case 2: {
-        // (two rows of the wider formats walk one weight row a step whatever the row count: their two-row steps
-        // run out of registers -- Q6_K 4096 -> 14336 17.5 -> 13.9 us, Q8_0 8192 x 8192 20.1 -> 17.6)
-        const bool two = pairs && (QT == kTypeQ4_K || QT == kTypeQ8_0Two || two_rows_env > 0);
-        if (one_chunk) return two ? launch_decode<QT, 2, 2, true, FUSE>(args, s) : launch_decode<QT, 2, 1, true, FUSE>(args, s);
-        return two ? launch_decode<QT, 2, 2, false, FUSE>(args, s) : launch_decode<QT, 2, 1, false, FUSE>(args, s);
-    }
-    case 4:
-        if constexpr (QT == kTypeQ4_K || QT == kTypeQ8_0Two)
-            if (one_chunk) return launch_decode<QT, 4, 1, true, FUSE>(args, s);
-        return launch_decode<QT, 4, 1, false, FUSE>(args, s);
+    case 1:
+        if constexpr (!kSmall)
+            if (args.t[0].w.K > Geo<QT>::kChunk) return launch_decode_rows<QT, 1, 1, FUSE>(args, s);
+        return pairs ? launch_decode_rows<QT, 1, 2, FUSE>(args, s) : launch_decode_rows<QT, 1, 1, FUSE>(args, s);
+    case 2:
+        if constexpr (kSmall)
+            if (pairs) return launch_decode_rows<QT, 2, 2, FUSE>(args, s);
+        return launch_decode_rows<QT, 2, 1, FUSE>(args, s);
+    case 4: return launch_decode_rows<QT, 4, 1, FUSE>(args, s);
     default: return hipErrorInvalidValue;
     }
 }
