@@ -13,6 +13,7 @@ import numpy as np
 import pytest
 import torch
 
+import np_ref
 from kquant_encoders import encode
 
 pytestmark = pytest.mark.gpu
@@ -312,20 +313,38 @@ def test_small_batch_row_groups_of_fewer_than_32_rows(ctx, orc, qtype, k, ns):
             w.free()
 
 
-@pytest.mark.parametrize("qtype,k,ns,ms", [
-    (Q4_K, 8192, (70,), (8,)), (Q6_K, 4096, (33, 1), (16,)), (Q8_0, 2048, (40,), (32,)),            # 256 super-blocks staged, the most
-    (Q4_K, 8448, (65,), (6, 16)), (Q6_K, 2304, (50,), (17, 31)), (Q8_0, 8448, (31,), (5,)),          # a last chunk one shorter
-    (Q4_K, 256, (52001,), (5,)), (Q6_K, 512, (26000,), (3, 9)), (Q8_0, 768, (13001,), (7, 12)),      # K in one, two and four parts
-    (Q4_K, 4352, (33, 1, 700, 130), (3, 8)), (Q8_0, 5120, (96, 5, 33, 1), (6, 16))])                 # four matrices, 17 and 20 super-blocks
-def test_small_batch_staging_and_k_parts_at_their_edges(ctx, orc, qtype, k, ns, ms):
+def small_batch_cut(plan):
+    """(chunks of K, super-blocks a chunk, K parts a chunk) of the dense small-batch launch that the plan names, None for other kernels"""
+    m = re.search(r"gemv_mfma_dense_kernel<.*K in (\d+) chunk\(s\) of (\d+) super-blocks x (\d+) parts", plan)
+    return m and tuple(int(v) for v in m.groups())
+
+
+@pytest.mark.parametrize("qtype,k,ns,ms,cut", [
+    # 256 super-blocks staged, the most, by 8, 16 and 32 rows
+    (Q4_K, 8192, (4097,), (8,), (1, 32, 8)), (Q8_0, 8192, (4097,), (8,), (1, 32, 8)), (Q6_K, 4096, (4097,), (16,), (1, 16, 8)),
+    (Q8_0, 2048, (40,), (32,), (1, 8, 8)),
+    # chunks of equal length, too few rows for one chunk
+    (Q4_K, 8192, (70,), (8,), (4, 8, 8)), (Q6_K, 4096, (33, 1), (16,), (2, 8, 8)),
+    # a last chunk three shorter (33 super-blocks), one shorter (9, 17)
+    (Q4_K, 8448, (65,), (6, 16), (4, 9, 8)), (Q8_0, 8448, (31,), (5,), (4, 9, 8)), (Q6_K, 2304, (50,), (17, 31), (2, 5, 8)),
+    (Q4_K, 4352, (33, 1, 700, 130), (3, 8), (2, 9, 8)),      # four matrices
+    (Q8_0, 5120, (96, 5, 33, 1), (6, 16), (2, 10, 8)),
+    # K in one, two and four parts; three super-blocks over two parts
+    (Q4_K, 256, (52001,), (5,), (1, 1, 1)), (Q6_K, 512, (26000,), (5, 9), (1, 2, 2)), (Q8_0, 768, (13001,), (7, 12), (1, 3, 2)),
+    (Q4_K, 1024, (9601,), (8, 20), (1, 4, 4)), (Q6_K, 1024, (9601,), (16,), (1, 4, 4)), (Q8_0, 1024, (9601,), (7,), (1, 4, 4)),
+    (Q6_K, 512, (26000,), (3,), None)])                      # (the decode kernel's)
+def test_small_batch_staging_and_k_parts_at_their_edges(ctx, orc, qtype, k, ns, ms, cut):
     """The activation rows of a small-batch workgroup at the most it stages, in chunks of K of unequal length and with
-    super-blocks that do not divide over the waves, and the sums of one to eight K parts; rows behind the outputs stay."""
-    from magnitude_amd import ACT_GGML
+    super-blocks that do not divide over the waves, and the sums of one, two, four and eight K parts, each as the plan says;
+    rows behind the outputs stay."""
+    from magnitude_amd import ACT_GGML, qproj
     ws, blocks = [], []
     for i, n in enumerate(ns):
         blocks.append(make_weight(orc, qtype, n, k, seed=5200 + k + n + i))
         ws.append(ctx.upload(qtype, k, n, blocks[-1]))
     for m in ms:
+        plan = qproj.plan_mul_mat(qtype, k, list(ns), m, ACT_GGML)
+        assert small_batch_cut(plan) == cut, plan
         x = np.random.default_rng(m + k).standard_normal((m, k)).astype(np.float32)
         bufs = [torch.full((m * n + 64,), 7.0, dtype=torch.float32, device="cuda") for n in ns]
         outs = [b[: m * n].view(m, n) for b, n in zip(bufs, ns)]
@@ -335,6 +354,71 @@ def test_small_batch_staging_and_k_parts_at_their_edges(ctx, orc, qtype, k, ns, 
             assert bool((b[m * n:] == 7.0).all())
     for w in ws:
         w.free()
+
+
+def k_quant_terms(qtype, blocks, k, qs, d):
+    """what a super-block adds to an output, [super-block][row][n]: factor and sum in fp32 as the small-batch kernel has them, and
+    their product in 64 bits without any rounding"""
+    n = blocks.shape[0]
+    for sb in range(k // 256):
+        size = 144 if qtype == Q4_K else 210
+        b = np.ascontiguousarray(blocks[:, sb * size:(sb + 1) * size])
+        xq, dx = qs[:, sb * 256:(sb + 1) * 256].astype(np.float64), d[:, sb:sb + 1]
+        if qtype == Q4_K:
+            q, sc, mn, dw, dmin = np_ref.q4_K_ints(b)
+            isum = xq @ (q.reshape(n, 8, 32) * sc[:, :, None].astype(np.float64)).reshape(n, 256).T
+            msum = xq.reshape(-1, 8, 32).sum(2) @ mn.astype(np.float64).T
+            factor, total = np.broadcast_to(dx, isum.shape), dw * isum.astype(np.float32) - dmin * msum.astype(np.float32)
+            exact = dx.astype(np.float64) * (dw.astype(np.float64) * isum - dmin.astype(np.float64) * msum)
+        else:
+            q, sc, dw = np_ref.q6_K_ints(b)
+            isum = xq @ (q.reshape(n, 16, 16) * sc[:, :, None].astype(np.float64)).reshape(n, 256).T
+            factor, total = dx * dw, isum.astype(np.float32)
+            exact = dx.astype(np.float64) * dw.astype(np.float64) * isum
+        yield factor.astype(np.float32), total.astype(np.float32), exact
+
+
+def restated_sums(terms, chunks, chunk_sb, kw):
+    """(in turns and pairs, in consecutive stretches one after the other): the fp32 sums of a launch of `kw` K parts a chunk"""
+    def chain(sbs):
+        acc = np.zeros(terms[0][1].shape, np.float32)
+        for sb in sbs:
+            acc = (terms[sb][0].astype(np.float64) * terms[sb][1] + acc).astype(np.float32)
+        return acc
+
+    turns = other = None
+    for c in range(chunks):
+        first, last = c * chunk_sb, min((c + 1) * chunk_sb, len(terms))
+        parts = [chain(range(first + p, last, kw)) for p in range(kw)]
+        while len(parts) > 1:
+            parts = [parts[i] + parts[i + 1] for i in range(0, len(parts), 2)]
+        length = -(-(last - first) // kw)
+        serial = chain(range(first, min(first + length, last)))
+        for p in range(1, kw):
+            serial = serial + chain(range(min(first + p * length, last), min(first + (p + 1) * length, last)))
+        turns, other = (parts[0], serial) if c == 0 else (turns + parts[0], other + serial)
+    return turns, other
+
+
+@pytest.mark.parametrize("qtype,k,n,m", [(Q6_K, 3072, 3072, 8), (Q4_K, 4096, 4096, 8), (Q6_K, 14336, 1024, 8), (Q4_K, 2816, 1000, 13)])
+def test_small_batch_sums_take_super_blocks_in_turns_and_parts_in_pairs(ctx, orc, qtype, k, n, m):
+    """The order of the sums, restated here, gives the kernel's values, and they are no further from 64 bits than those of parts
+    of consecutive super-blocks added one after the other.  (Values: the fma is restated through 64 bits, whose second rounding
+    differs for one sum in 2^28.  Errors: 0.93 to 0.98 of the other order's at these shapes and
+    seeds, by the restatement; the bound is their equality.)"""
+    from magnitude_amd import ACT_GGML, qproj
+    chunks, chunk_sb, kw = small_batch_cut(qproj.plan_mul_mat(qtype, k, [n], m, ACT_GGML))
+    blocks = make_weight(orc, qtype, n, k, seed=5900 + k)
+    x = np.random.default_rng(k + m).standard_normal((m, k)).astype(np.float32)
+    w = ctx.upload(qtype, k, n, blocks)
+    q = ctx.quantize_activations(dev(x), ACT_GGML, qtype)
+    got = ctx.mul_mat(w, dev(x), ACT_GGML).cpu().numpy()
+    w.free()
+    terms = list(k_quant_terms(qtype, blocks, k, q["qs"].cpu().numpy(), q["d"].cpu().numpy()))
+    turns, other = restated_sums(terms, chunks, chunk_sb, kw)
+    exact = sum(t[2] for t in terms)
+    assert (got != turns).mean() <= 1e-5
+    assert np.linalg.norm(got - exact) <= np.linalg.norm(other - exact)
 
 
 @pytest.mark.parametrize("qtype,k,n", [(Q4_K, 4096, 512), (Q4_K, 14336, 203), (Q4_K, 256, 9), (Q8_0, 4096, 384),
