@@ -464,13 +464,15 @@ hipError_t launch_decode(const GemvArgs &args, hipStream_t s) {
 }
 
 // Q8_0: parts of 1024 weights a step.  Two for rows of at most 2048 (2048 -> 2 x 8192 13.4 -> 10.1 us, 2048 -> 2048 / 512 / 512
-// 5.7 -> 4.9 against four, half of whose requests lie past the row), three where that covers the row with fewer than four do: one
-// token through a layer of 3072 / 1024 / 8192 33.8 -> 29.5 us, of 5120 / 1024 / 13824 68.3 -> 63.4, of 2560 / 512 / 7680 30.1 -> 25.7; rows of
-// one part more or less than whole threes gain little (13824 -> 5120 16.9 / 16.7, 14336 -> 4096 12.1 / 11.8, at two rows 14.5 / 14.6).
-// Error against 64 bits 0.966 to 1.003 of that of four parts (K 5120 to 17408, one to four rows).
+// 5.7 -> 4.9 against four, half of whose requests lie past the row), three where they need a quarter fewer parts than steps of
+// four (rows of up to 3, 5, 6 and 9 parts).  Four / three, us at 1, 2, 4 rows: 3072 -> 8192 6.3 / 6.0, 7.0 / 6.3, 8.7 / 8.2;
+// 5120 -> 13824 15.5 / 14.6, 16.9 / 15.7, 22.6 / 19.9; 9216 -> 4096 8.5 / 7.8, 10.2 / 9.8, 15.8 / 14.4.  Where only a sixteenth goes they
+// lose at one and two rows (14336 -> 4096 11.3 / 11.6, 13.7 / 14.2, 21.4 / 21.0; 15360 -> 5120 17.7 / 18.4, 20.7 / 21.4, 29.1 / 28.8) and the
+// longer chain of steps costs accuracy.  Error against 64 bits, three over four parts, 2000 outputs a draw, 512 to 1024 draws: 5
+// parts 0.982, 6 0.994, 9 0.976; 13 and 14 1.001, 15 1.004, 17 (K = 16896) 1.009, 25 to 29 1.01 to 1.02.
 int q8_0_parts(int64_t K) {
-    const int64_t n = (K + 1023) / 1024;
-    return n <= 2 ? 2 : (n + 2) / 3 * 3 < (n + 3) / 4 * 4 ? 3 : 4;
+    const int64_t n = (K + 1023) / 1024, three = (n + 2) / 3 * 3, four = (n + 3) / 4 * 4;
+    return n <= 2 ? 2 : 4 * three <= 3 * four ? 3 : 4;
 }
 
 // Rows of one chunk keep their activations in registers, longer ones read the LDS image.  Built are the instances that the

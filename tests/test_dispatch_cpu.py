@@ -164,10 +164,11 @@ def test_plan_names_kernels_that_are_launched():
 
 
 @pytest.mark.parametrize("k,parts", [(32, 2), (1024, 2), (2048, 2), (2080, 3), (3072, 3), (3104, 4), (4096, 4), (4128, 3), (5120, 3), (6144, 3),
-                                     (6176, 4), (8192, 4), (8224, 3), (9216, 3), (9248, 4), (12288, 4), (14336, 3), (15392, 4)])
-def test_q8_0_decode_steps_of_fewest_parts(k, parts):
-    """Two parts of 1024 weights a step for rows that they cover, three where those cover the row with fewer parts than steps of
-    four do, for one to four activation rows."""
+                                     (6176, 4), (8192, 4), (8224, 3), (9216, 3), (9248, 4), (12288, 4), (12320, 4), (13824, 4), (14336, 4),
+                                     (15360, 4), (16896, 4), (18432, 4)])
+def test_q8_0_decode_steps_take_three_parts_where_a_quarter_fewer_are_needed(k, parts):
+    """Two parts of 1024 weights a step for rows that they cover, three where steps of four would take a third more, for one to
+    four activation rows.  Longer rows than nine parts keep four: their sums are further from 64 bits in steps of three."""
     for m in (1, 2, 4):
         plan = qproj.plan_mul_mat(Q8_0, k, (512, 512), m)
         assert re.findall(r"gemv_decode_kernel<Q8_0, (\d) parts of 1024 weights a step,", plan) == [str(parts)], plan
