@@ -449,15 +449,9 @@ hipError_t launch_decode(const GemvArgs &args, hipStream_t s) {
         return hipSuccess;
     }
     auto kern = &gemv_decode_kernel<QT, MT, R, XREG, FUSE, PAIR>;
-    if (smem > 48 * 1024) {
-        static size_t allowed = 0;
-        if (smem > allowed) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-            if (e != hipSuccess) return e;
-            allowed = smem;
-        }
-    }
+    static LdsLimit limit;
+    const hipError_t e = limit.allow(kern, smem);
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kDecodeThreads), smem, s, args.x, args.norm_gamma, (int)K, (int)args.t[0].w.nb, kpad, args.M,
                        args.norm_eps, (int)args.norm, a);
     return hipGetLastError();

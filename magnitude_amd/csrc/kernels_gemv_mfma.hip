@@ -1101,15 +1101,6 @@ __global__ __launch_bounds__(256) void sum_chunks_kernel(const DenseArgs g) {
     }
 }
 
-// a workgroup's LDS: raised once per instance to the most any launch asked for
-template <typename Kernel>
-hipError_t allow_lds(Kernel kern, int bytes, int &allowed) {
-    if (bytes <= allowed) return hipSuccess;
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    if (e == hipSuccess) allowed = bytes;
-    return e;
-}
-
 template <int QT, int NI, int W>
 hipError_t launch_dense(const DenseArgs &g, int n_wgs, hipStream_t s) {
     // K parts of a row group are summed through the waves' regions: a wave's partial tile must fit its region
@@ -1123,8 +1114,8 @@ hipError_t launch_dense(const DenseArgs &g, int n_wgs, hipStream_t s) {
         return hipSuccess;
     }
     const Layout L = layout<QT, 8 * NI, W>(g.chunk_sb);
-    static int allowed = 0;
-    hipError_t e = allow_lds(gemv_mfma_dense_kernel<QT, NI, W>, L.total, allowed);
+    static LdsLimit limit;
+    hipError_t e = limit.allow(&gemv_mfma_dense_kernel<QT, NI, W>, (size_t)L.total);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((gemv_mfma_dense_kernel<QT, NI, W>), dim3((unsigned)n_wgs), dim3(W * 64), (size_t)L.total, s, g);
     e = hipGetLastError();
@@ -1153,8 +1144,8 @@ hipError_t launch_one(const MfmaArgs &g, hipStream_t s) {
         return hipSuccess;
     }
     const Layout L = layout<QT, 8 * NI, W>(g.chunk_sb);
-    static int allowed = 0;
-    const hipError_t e = allow_lds(gemv_mfma_kernel<QT, NI, W, MODE, FLAT>, L.total, allowed);
+    static LdsLimit limit;
+    const hipError_t e = limit.allow(&gemv_mfma_kernel<QT, NI, W, MODE, FLAT>, (size_t)L.total);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((gemv_mfma_kernel<QT, NI, W, MODE, FLAT>), dim3((unsigned)g.n_wgs), dim3(W * 64), (size_t)L.total, s, g);
     return hipGetLastError();

@@ -307,13 +307,9 @@ hipError_t launch_moe_group(const int32_t *ids, int64_t n_pairs, int64_t n_exper
                   quantize ? ", spare workgroups quantize the token rows" : "");
         return hipSuccess;
     }
-    static size_t allowed = 48 * 1024;
-    if (lds > allowed) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(moe_group_kernel),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        allowed = lds;
-    }
+    static LdsLimit limit;
+    const hipError_t e = limit.allow(&moe_group_kernel, lds);
+    if (e != hipSuccess) return e;
     RowQuantJob job{};
     if (quantize) job = *quantize;
     const int64_t extra = (job.n_super + kGroupThreads / 64 - 1) / (kGroupThreads / 64);

@@ -268,12 +268,9 @@ __global__ __launch_bounds__(kThreads) void moe_decode_kernel(const MoeDecodeArg
 template <int QT, bool SWIGLU, bool COMBINE, int R = 1, bool LONGK = false>
 hipError_t launch_typed(const MoeDecodeArgs &g, unsigned grid, size_t lds, hipStream_t s) {
     auto kern = &moe_decode_kernel<QT, SWIGLU, COMBINE, R, LONGK>;
-    static size_t allowed = 48 * 1024;
-    if (lds > allowed) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        allowed = lds;
-    }
+    static LdsLimit limit;
+    const hipError_t e = limit.allow(kern, lds);
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(kThreads), lds, s, g);
     return hipGetLastError();
 }

@@ -5,6 +5,9 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <atomic>
+#include <mutex>
+
 namespace qproj {
 
 constexpr int kTypeQ8_0 = 8;
@@ -111,6 +114,23 @@ size_t scratch_shave();   // dry runs: bytes withheld from the scratch the launc
 // line.  The lines ARE the routing table: they come from the very code that serves a call.
 void plan_note(const char *fmt, ...) __attribute__((format(printf, 1, 2)));
 const char *plan_type_name(int type);
+
+// A kernel instance's limit of dynamic LDS, raised to the most that a launch has asked for: one object an instance, shared by
+// the threads that launch it (a context each).  The limit never falls: two first launches of different sizes at once, each
+// setting its own, could leave the smaller one behind the larger launch.
+struct LdsLimit {
+    std::atomic<size_t> bytes{48 * 1024};   // what needs no raising
+    std::mutex raising;
+    template <typename Kernel>
+    hipError_t allow(Kernel *kernel, size_t need) {
+        if (need <= bytes.load(std::memory_order_acquire)) return hipSuccess;
+        const std::lock_guard<std::mutex> lock(raising);
+        if (need <= bytes.load(std::memory_order_relaxed)) return hipSuccess;
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)need);
+        if (e == hipSuccess) bytes.store(need, std::memory_order_release);
+        return e;
+    }
+};
 void plan_note_cut();     // a launcher in a dry run: this launch keeps partial results of a cut K in scratch
 
 // Into how many stretches K is cut for a grid of `tiles` 128-token tiles (one workgroup a compute unit) that would

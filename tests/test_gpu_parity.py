@@ -1654,6 +1654,38 @@ def test_q8_0_decode_sums_in_steps_of_two_three_and_four_parts(ctx, orc, k, part
     assert np.linalg.norm(got - exact) <= np.linalg.norm(q8_0_decode_sums(blocks, k, qs, d, 4)[0] - exact)
 
 
+def test_contexts_of_several_threads_launch_kernels_of_growing_lds_at_once(orc):
+    """A context a thread: the same calls, whose launches take different amounts of LDS, in another order on each.  What a kernel
+    may take is one limit for all threads and is raised by whoever needs more first."""
+    import threading
+    from magnitude_amd import ACT_GGML, Context
+    calls = [(Q8_0, 20480, 64, 4), (Q8_0, 8192, 64, 4), (Q8_0, 16384, 64, 2), (Q4_K, 8192, 4097, 8), (Q4_K, 2048, 96, 16), (Q6_K, 4096, 4097, 16)]
+    blocks = [make_weight(orc, t, n, k, seed=6500 + k) for t, k, n, _ in calls]
+    xs = [dev(np.random.default_rng(k + m).standard_normal((m, k)).astype(np.float32)) for _, k, _, m in calls]
+    torch.cuda.synchronize()
+    results, start = {}, threading.Barrier(4)
+
+    def work(i):
+        c = Context(0)
+        ws = [c.upload(t, k, n, b) for (t, k, n, _), b in zip(calls, blocks)]
+        start.wait()
+        for j in (range(6), range(5, -1, -1), (2, 5, 1, 4, 0, 3), (3, 0, 4, 1, 5, 2))[i]:
+            results[i, j] = c.mul_mat(ws[j], xs[j], ACT_GGML).cpu()
+        for w in ws:
+            w.free()
+        c.close()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for j, (t, k, n, m) in enumerate(calls):
+        want = orc.mul_mat(t, blocks[j], k, xs[j].cpu().numpy(), orc.ACT_GGML)
+        for i in range(4):
+            close(results[i, j].numpy(), want, 2e-5)
+
+
 @pytest.mark.parametrize("ns", [(28677,), (4096, 1024, 1024), (14336, 14336), (9001, 5003), (12289, 1)])
 @pytest.mark.parametrize("m", [1, 2])
 def test_decode_row_dealing_at_full_grids(ctx, ns, m):
