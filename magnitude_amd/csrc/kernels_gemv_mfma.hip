@@ -3,7 +3,7 @@
 //
 // One v_mfma_i32_32x32x32_i8 (Q4_K, Q8_0) or v_mfma_i32_32x32x16_i8 (Q6_K) multiplies the int8
 // activations of up to 32 tokens (A operand) with one sub-block of 32 weight rows (B operand), so
-// that lane l ends up with the integer dots of weight row l%32 against 8 (or 16) tokens.  A
+// that lane l ends up with the integer dots of weight row l%32 against 8, 16 or 32 tokens.  A
 // sub-block's integer scale is applied with one v_mad_i32_i24 per output, the super-block's fp32
 // scales once per 256 weights.  The terms that ggml takes from the activation block sums (the
 // Q4_K mins, the -32 offset of Q6_K) are two more products each: block sums split into a signed
@@ -15,9 +15,11 @@
 // super-block with fully coalesced 16-byte loads (consecutive lanes = consecutive 16-byte pieces
 // of a row's block), two super-blocks ahead of the arithmetic, parks the registers in a
 // wave-private LDS region and reads the region back in operand order.  The quantized
-// activations of the workgroup's K range are staged in LDS once, ahead of the weights.
+// activations of the workgroup's K range are staged in LDS once: dense launches ask for them ahead of
+// the first weights, expert-grouped ones only where a thread holds its share in registers (StagedRows).
 //
-// Work split.  A workgroup is 8 waves = rw row groups (32 rows each) x kw K-parts; the K-parts
+// Work split.  A workgroup is 8 waves (Q4_K experts: 4, two workgroups a compute unit, 8 in passes of 32
+// rows) = rw row groups (32 rows each, dense launches 24 to 32) x kw K-parts; the K-parts
 // of a row group are summed through LDS in a fixed order.  When one workgroup cannot hold the
 // whole K range (LDS) or there would be too few workgroups, K is also cut into chunks whose
 // results go to a scratch buffer that a second small kernel sums in chunk order, so results do
@@ -864,7 +866,7 @@ __global__ __launch_bounds__(W * 64) void gemv_mfma_kernel(const MfmaArgs g) {
 }
 
 // What a dense workgroup needs of the quantized activation rows, asked for in ONE go and ahead of the first weights: a
-// wave's share of the codes (a super-block of a row is 16 lanes, at most eight requests a wave) and one record of scales and
+// wave's share of the codes (a super-block of a row is 16 lanes, 256 / (4 W) requests a wave at most) and one record of scales and
 // block sums a thread.  Loads come back in the order they were asked for, over all waves of a compute unit: behind 74 KB of
 // weights, and in three rounds one after the other, these 40 KB that sit in L2 took 4 to 9 us of a workgroup's 10 to 26
 // (phase clocks; o at 8 rows, and the Q6_K down projection).  (Straight into LDS is no better: the compiler then waits for
@@ -938,8 +940,9 @@ struct DenseRows {
 // Dense launches: a workgroup is rw row groups x kw K parts of a K chunk.  The rows beyond M are staged by nobody: what
 // lies there only reaches results that are not stored.
 // Bound: latency.  Of the 9 us of a 4096 x 4096 Q4_K launch at 8 rows the arithmetic took 1.5; the rest was one trip to
-// memory after another.  Arguments in one go, staged rows in one go ahead of the weights, K parts added by all waves, us a
-// launch before / after (4096, 14336, 8 rows): q/k/v 9.4 / 6.9, o 9.0 / 6.6, gate + up 18.4 / 16.8, Q6_K down 18.2 / 15.9.
+// memory after another.  Arguments in one go, staged rows in one go ahead of the weights, K parts added by all waves, and taken
+// in turns (below), us a launch before / after (4096, 14336, 8 rows; one card): q/k/v 9.3 / 7.4, o 8.7 / 6.6, gate + up 18.0 / 16.4,
+// Q6_K down 18.3 / 14.6.
 // (A barrier between the rows' requests and the weights': level.  K parts of 3 and 4 super-blocks instead of 4 and 0: level.)
 template <int QT, int NI, int W>
 __global__ __launch_bounds__(W * 64) void gemv_mfma_dense_kernel(const DenseArgs g) {
@@ -974,8 +977,8 @@ __global__ __launch_bounds__(W * 64) void gemv_mfma_dense_kernel(const DenseArgs
     const int rgl = wave >> g.kw_log2, kp = wave - (rgl << g.kw_log2);
     // A K part takes every kw-th super-block of the chunk: the parts read neighbouring ones at the same time, and share the
     // cache lines that hold several (Q6_K: 128 bytes are the scales of eight super-blocks, or two of the high bits, and a wave's
-    // step of 52 lines of data touched 128).  us at 8 rows, parts of consecutive super-blocks / this: Q6_K 14336 -> 4096 17.8 / 16.5,
-    // Q4_K 13.5 / 12.4, 4096 -> 14336 12.3 / 11.7; at 16 and 30 rows level.  Q8_0, whose super-blocks are whole lines, lost by it
+    // step of 52 lines of data touched 128).  us a call at 8 rows, quantizer launch included, parts of consecutive super-blocks /
+    // this: Q6_K 14336 -> 4096 17.8 / 16.5, Q4_K 13.5 / 12.4, 4096 -> 14336 12.3 / 11.7; at 16 and 30 rows level.  Q8_0, whose super-blocks are whole lines, lost by it
     // (8192 x 8192 20.9 / 22.6) and keeps consecutive ones.
     constexpr bool kTurns = QT != kTypeQ8_0;
     const int part_sb = (nsb + (1 << g.kw_log2) - 1) >> g.kw_log2;
